@@ -19,8 +19,10 @@ hipStream_t stream();
 // device workspace: named slots that grow on demand and live until process exit
 enum Slot {
     WS_KEY = 0,     // per-particle cell key
-    WS_SLOT,        // per-particle arrival slot in its cell
-    WS_TMP,         // per-slot particle index before stabilisation
+    WS_SLOT,        // per-particle place in its tile's list
+    WS_TMP,         // the tiles' particle lists
+    WS_TILE,        // sort tile starts
+    WS_TCOUNT,      // sort tile counts: zeroed when allocated, left zero by every sort
     WS_SCAN,        // scan tile sums
     WS_RED,         // reductions (doubles)
     WS_FLAG,        // status flags (ints)
@@ -64,6 +66,10 @@ const int32_t *hilbert_lut(const Box &b);
 
 int check_particles(const rmpcd_particles_t *p, const char *who, bool need_force);
 int check_box(const rmpcd_box_t *b, const char *who);
+
+// rmpcd_sort on sets that the caller has checked; id_to_idx may be null (not written)
+int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
+                   rmpcd_cells_t *cells, int wrap);
 
 inline unsigned blocks_for(int64_t n, int threads)
 {

@@ -86,7 +86,6 @@ int ProgramSim::setup(const rmpcd_program_config_t &c)
     }
     for (int b = 0; b < 4; ++b)
         if ((rc = alloc(&sol_force[b], 3 * n * RS))) return rc;
-    if ((rc = alloc((void **)&id_to_idx, n * 4))) return rc;
     if ((rc = alloc((void **)&cell_count, box.ncells * 4))) return rc;
     if ((rc = alloc((void **)&cell_start, box.ncells * 4))) return rc;
     if ((rc = alloc((void **)&is_md, box.ncells))) return rc;

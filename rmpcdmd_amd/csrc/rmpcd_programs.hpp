@@ -36,7 +36,7 @@ struct ProgramSim {
     void *sol_pos[2] = {}, *sol_vel[2] = {}, *sol_species[2] = {}, *sol_flags[2] = {};
     int32_t *sol_image[2] = {}, *sol_id[2] = {};
     void *sol_force[4] = {};
-    int32_t *id_to_idx = nullptr, *cell_count = nullptr, *cell_start = nullptr;
+    int32_t *cell_count = nullptr, *cell_start = nullptr;
     uint8_t *is_md = nullptr, *is_reac = nullptr;
     double *col_pos = nullptr, *col_pos_old = nullptr, *col_vel = nullptr, *col_force[2] = {};
     int32_t *col_image = nullptr, *col_id = nullptr, *col_species = nullptr, *col_flags = nullptr;
@@ -114,7 +114,8 @@ struct ProgramSim {
     {
         rmpcd_particles_t s = sv(), d = alt();
         rmpcd_cells_t c = cells();
-        int rc = rmpcd_sort(&box, &s, &d, id_to_idx, &c, pbc ? 1 : 0);
+        // no id_to_idx: nothing in these programs reads it and the state does not show it
+        int rc = sort_unchecked(&box, &s, &d, nullptr, &c, pbc ? 1 : 0);
         if (rc) return rc;
         cur = 1 - cur;  // the switch() calls of particle_system.f90:346-353
         return RMPCD_OK;

@@ -2,17 +2,19 @@
 // counting sort of the solvent (src/cell_system.f90:86-129,
 // src/particle_system.f90:304-355, src/md.f90:202-217 fused).
 //
-// Sort pipeline (all launches on the library stream):
-//   k_key_count  one thread per particle: optional periodic wrap, cell key from the
-//                box's Hilbert table, arrival slot from an atomic increment of the
-//                cell's count (the arrival order is not deterministic)
-//   scan         exclusive scan of the counts -> cell_start (wave DPP scan per tile,
-//                one block for the tile sums, then the tile offsets)
-//   k_place      tmp[cell_start[key] + slot] = particle
-//   k_gather     one thread per destination slot: the particle's rank among the
-//                cell's entries (by original index) fixes its stable position; it
-//                copies the particle there.  The result equals the reference's
-//                single-thread order, where each cell keeps increasing original index.
+// Sort pipeline (all launches on the library stream).  The unit is a tile: 2^k cells with
+// consecutive Hilbert keys, about a thousand particles.
+//   k_tile_key    per particle: optional periodic wrap, cell key from the box's Hilbert
+//                 table, and its place in its tile's list (an LDS hash counts the tiles of
+//                 1024 consecutive particles, one global atomic per tile met there)
+//   k_tile_scan   exclusive scan of the tile counts
+//   k_tile_place  list[start of the tile + place] = particle
+//   k_tile_gather one workgroup per tile: counts its cells (cell_count, cell_start), ranks
+//                 each particle among its cell's by original index, and moves the planes
+//                 through LDS, read in list order and written in slot order
+// The order within a tile's list is not deterministic, the rank does not depend on it: the
+// result equals the reference's single-thread order, where each cell keeps increasing
+// original index.
 #include "rmpcd_internal.hpp"
 
 namespace rmpcd {
@@ -40,26 +42,12 @@ __device__ inline int key_of(const Box &b, const int32_t *lut, R x, R y, R z)
 }
 
 template <class F>
-__global__ void k_key_count(Box b, const int32_t *__restrict__ lut, PView<F> p, int wrap,
-                            int32_t *__restrict__ count, int32_t *__restrict__ key,
-                            int32_t *__restrict__ slot)
+__global__ void k_key_count(Box b, const int32_t *__restrict__ lut, PView<F> p,
+                            int32_t *__restrict__ count)
 {
-    using R = typename F::real;
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.n) return;
-    R x = p.pos[i], y = p.pos[p.n + i], z = p.pos[2 * p.n + i];
-    if (wrap) {
-        int j;
-        wrap_pbc<R>(b, x, j, 0);
-        wrap_pbc<R>(b, y, j, 1);
-        wrap_pbc<R>(b, z, j, 2);
-    }
-    int k = key_of<R>(b, lut, x, y, z);
-    int s = atomicAdd(&count[k], 1);
-    if (key) {
-        key[i] = k;
-        slot[i] = s;
-    }
+    atomicAdd(&count[key_of<typename F::real>(b, lut, p.pos[i], p.pos[p.n + i], p.pos[2 * p.n + i])], 1);
 }
 
 __global__ void k_fill_i32(int32_t *a, int64_t n, int32_t v)
@@ -157,56 +145,317 @@ int exclusive_scan(const int32_t *in, int32_t *out, int64_t n)
 }
 
 // ---- counting sort ---------------------------------------------------------------
-__global__ void k_place(int64_t n, const int32_t *__restrict__ key, const int32_t *__restrict__ slot,
-                        const int32_t *__restrict__ start, int32_t *__restrict__ tmp)
+constexpr int SORT_T = 256;
+constexpr int KEY_ITEMS = 4, KEY_CHUNK = SORT_T * KEY_ITEMS;  // particles per workgroup of the key pass
+constexpr int HASH_BITS = 11, HASH = 1 << HASH_BITS;          // LDS hash entries, 2 x KEY_CHUNK
+// a thread's particles of a tile that is moved through LDS (three planes at a time): 1536
+// particles in FP32; 512 in FP64, where 1536 leave three waves per SIMD (a step of 837,000
+// particles 174 against 219 us; FP32 at 21 million 1.79 ms, 1.84 with 768 or 1024)
+template <class F>
+constexpr int TILE_ITEMS = sizeof(typename F::real) == 4 ? 6 : 2;
+template <class F>
+constexpr int TILE_MAX = SORT_T * TILE_ITEMS<F>;
+// tiles in a run that one XCD takes.  An eighth of the tiles per XCD left half of them with
+// the empty cells of a 60 x 31 x 45 box (its particles in no order: 528 us a step, 459 with
+// runs of 16, 485 with 4, 64 or 256; 21 million particles in order: 1.38 ms, 1.35 ms with
+// runs of 4 to 64).
+constexpr int TILE_RUN = 16;
+constexpr int TILE_CELLS = 128;                               // cells of a tile at most
+constexpr int SCAN1_TILES = 1 << 15;                          // tile counts that one workgroup scans
+// ints between the counts of up to SCAN1_TILES tiles: a cache line each.  Particles in no
+// order (the first sort of a run) meet a few thousand counts from everywhere, and atomics on
+// one line wait for each other.
+constexpr int COUNT_STRIDE = 16;
+
+// cell key and place in the tile's list of every particle.  A thread's positions are
+// loaded before anything is done with them; each particle then takes a place among its
+// tile's of this chunk from an LDS hash, and one global atomic per (chunk, tile) turns
+// these into places in the tile's list, so a run of consecutive particles of one tile
+// stays together there.  21 million particles FP32: 0.15 ms, 0.77 ms with an atomic per
+// particle on its cell.
+template <class F>
+__global__ void __launch_bounds__(SORT_T)
+    k_tile_key(Box b, const int32_t *__restrict__ lut, PView<F> p, int wrap, int shift,
+               int stride, int32_t *__restrict__ tile_count, int32_t *__restrict__ key, int32_t *__restrict__ slot)
+{
+    using R = typename F::real;
+    __shared__ int hkey[HASH], hcnt[HASH];
+    const int64_t base = (int64_t)blockIdx.x * KEY_CHUNK + threadIdx.x;
+    R x[KEY_ITEMS][3];
+#pragma unroll
+    for (int u = 0; u < KEY_ITEMS; ++u) {
+        const int64_t i = base + u * SORT_T;
+        if (i < p.n)
+            for (int k = 0; k < 3; ++k) x[u][k] = p.pos[k * p.n + i];
+    }
+    for (int h = threadIdx.x; h < HASH; h += SORT_T) {
+        hkey[h] = -1;
+        hcnt[h] = 0;
+    }
+    __syncthreads();
+    int at[KEY_ITEMS], in[KEY_ITEMS];
+#pragma unroll
+    for (int u = 0; u < KEY_ITEMS; ++u) {
+        const int64_t i = base + u * SORT_T;
+        if (i >= p.n) continue;
+        if (wrap) {
+            int j;
+            for (int k = 0; k < 3; ++k) wrap_pbc<R>(b, x[u][k], j, k);
+        }
+        const int c = key_of<R>(b, lut, x[u][0], x[u][1], x[u][2]);
+        key[i] = c;
+        const int t = c >> shift;
+        unsigned h = ((unsigned)t * 2654435769u) >> (32 - HASH_BITS);
+        for (;;) {  // at most KEY_CHUNK entries of the HASH are taken
+            int q = hkey[h];
+            if (q == -1) q = atomicCAS(&hkey[h], -1, t);
+            if (q == t || q == -1) break;
+            h = (h + 1) & (HASH - 1);
+        }
+        at[u] = (int)h;
+        in[u] = atomicAdd(&hcnt[h], 1);
+    }
+    __syncthreads();
+    for (int h = threadIdx.x; h < HASH; h += SORT_T)
+        if (hcnt[h] > 0) hcnt[h] = atomicAdd(&tile_count[(int64_t)hkey[h] * stride], hcnt[h]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < KEY_ITEMS; ++u) {
+        const int64_t i = base + u * SORT_T;
+        if (i < p.n) slot[i] = hcnt[at[u]] + in[u];
+    }
+}
+
+// start[t] for t in [0, nt], start[nt] = the particle count, from the counts that lie
+// COUNT_STRIDE apart; the counts are left zero, as the next sort needs them
+__global__ void __launch_bounds__(1024) k_tile_scan(int32_t *__restrict__ count, int nt, int32_t *__restrict__ start)
+{
+    __shared__ int lds[16];
+    int carry = 0;
+    for (int c = 0; c < nt; c += 1024 * 8) {
+        int v[8], s = 0;
+        const int base = c + 8 * (int)threadIdx.x;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            v[k] = base + k < nt ? count[(base + k) * COUNT_STRIDE] : 0;
+            s += v[k];
+        }
+        int tot;
+        int off = carry + block_exclusive_scan(s, lds, &tot);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (base + k < nt) {
+                start[base + k] = off;
+                count[(base + k) * COUNT_STRIDE] = 0;
+            }
+            off += v[k];
+        }
+        carry += tot;
+    }
+    if (threadIdx.x == 0) start[nt] = carry;
+}
+
+__global__ void k_tile_place(int64_t n, const int32_t *__restrict__ key, int shift,
+                             const int32_t *__restrict__ slot, const int32_t *__restrict__ start,
+                             int32_t *__restrict__ list)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    tmp[start[key[i]] + slot[i]] = (int32_t)i;
+    list[start[key[i] >> shift] + slot[i]] = (int32_t)i;
 }
 
+// one plane of a tile's particles: the loads of a thread's N particles, their way to the
+// slots in LDS, and the slots' way out
+template <int N, class T>
+__device__ inline void tile_load(T r[N], const T *__restrict__ plane, const int32_t v[N])
+{
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+        if (v[u] >= 0) r[u] = plane[v[u]];
+}
+template <int N, class T>
+__device__ inline void tile_put(T *lds, const T r[N], const int32_t v[N], const int d[N])
+{
+#pragma unroll
+    for (int u = 0; u < N; ++u)
+        if (v[u] >= 0) lds[d[u]] = r[u];
+}
+template <int N, class T>
+__device__ inline void tile_store(T *__restrict__ plane, const T *lds, int m)
+{
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const int q = (int)threadIdx.x + u * SORT_T;
+        if (q < m) plane[q] = lds[q];
+    }
+}
+
+// The cell sort's move.  Bound by memory: FP32 it reads 74 B and writes 66 B per particle,
+// and fetches 1.33 times what it uses (tiles read the edges of their neighbours' stretches),
+// 164 B in 0.67 ms for 21 million particles, 5.1 TB/s.  Moved one particle per thread
+// straight from the planes, each load touched a cache line per lane and the pass took 2.08
+// ms; in list order a tile's loads run along the source, and LDS puts them in slot order so
+// that the stores are contiguous too.  id_to_idx costs 0.42 ms of the 1.09 ms with it: its
+// 4-byte stores go anywhere once the particles have mixed.
 template <class F>
-__global__ void k_gather(Box b, PView<F> src, PView<F> dst, int wrap,
-                         const int32_t *__restrict__ key, const int32_t *__restrict__ start,
-                         const int32_t *__restrict__ count, const int32_t *__restrict__ tmp,
-                         int32_t *__restrict__ id_to_idx)
+__global__ void __launch_bounds__(SORT_T)
+    k_tile_gather(Box b, PView<F> src, PView<F> dst, int wrap, int shift, int nt, const int32_t *__restrict__ key,
+                  const int32_t *__restrict__ start, const int32_t *__restrict__ list, int32_t *__restrict__ spill,
+                  int32_t *__restrict__ cell_count, int32_t *__restrict__ cell_start, int32_t *__restrict__ id_to_idx)
 {
     using R = typename F::real;
-    int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t n = src.n;
-    if (j >= n) return;
-    int32_t v = tmp[j];
-    int c = key[v];
-    int s = start[c], m = count[c];
-    int rank = 0;
-    for (int q = s; q < s + m; ++q) rank += tmp[q] < v ? 1 : 0;
-    int64_t d = s + rank;
-    // copy particle v to slot d (wrap applied to pos/image when requested)
+    using S = typename F::small;
+    constexpr int N = TILE_ITEMS<F>, M = TILE_MAX<F>;
+    __shared__ R buf[3][M];
+    __shared__ int lv[M];
+    __shared__ int lcnt[TILE_CELLS], lstart[TILE_CELLS];
+    // consecutive workgroups go to the XCDs in turn: each XCD takes runs of TILE_RUN tiles,
+    // so that the tiles in flight there read neighbouring stretches.  The runs are short
+    // enough that the empty cells of a padded box fall to all XCDs alike.
+    const int j = (int)blockIdx.x >> 3;
+    const int t = ((j / TILE_RUN) * 8 + ((int)blockIdx.x & 7)) * TILE_RUN + j % TILE_RUN;
+    if (t >= nt) return;
+    const int tid = threadIdx.x;
+    const int64_t n = src.n;
+    const int64_t s = start[t];
+    const int m = (int)(start[t + 1] - s);
+    const int ncell = 1 << shift, cmask = ncell - 1;
+    for (int c = tid; c < ncell; c += SORT_T) lcnt[c] = 0;
+    __syncthreads();
+    int v[N], c[N], d[N];
+    R x[3][N];
+    R *const from[4] = {src.pos, src.vel, src.force, src.force_old};
+    R *const to[4] = {dst.pos, dst.vel, dst.force, dst.force_old};
+    const bool fits = m <= M;
+    if (fits) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        R x = src.pos[k * n + v];
-        int32_t im = src.image[k * n + v];
-        if (wrap) {
-            int jump;
-            wrap_pbc<R>(b, x, jump, k);
-            im += jump;
+        for (int u = 0; u < N; ++u) {
+            const int q = tid + u * SORT_T;
+            v[u] = q < m ? list[s + q] : -1;
         }
-        dst.pos[k * n + d] = x;
-        dst.image[k * n + d] = im;
-        dst.vel[k * n + d] = src.vel[k * n + v];
-        dst.force[k * n + d] = src.force[k * n + v];
-        dst.force_old[k * n + d] = src.force_old[k * n + v];
+#pragma unroll
+        for (int u = 0; u < N; ++u) c[u] = v[u] >= 0 ? key[v[u]] & cmask : 0;
+        // the positions are on their way while the particles are ranked
+        for (int k = 0; k < 3; ++k) tile_load<N>(x[k], src.pos + k * n, v);
+#pragma unroll
+        for (int u = 0; u < N; ++u) d[u] = v[u] >= 0 ? atomicAdd(&lcnt[c[u]], 1) : 0;
+    } else {
+        for (int q = tid; q < m; q += SORT_T) atomicAdd(&lcnt[key[list[s + q]] & cmask], 1);
     }
-    int32_t id = src.id[v];
-    dst.id[d] = id;
-    dst.species[d] = src.species[v];
-    dst.flags[d] = src.flags[v];
-    if ((uint32_t)id < (uint32_t)n) id_to_idx[id] = (int32_t)d;
+    __syncthreads();
+    if (tid < 64) {  // one wave scans the tile's cells
+        int carry = 0;
+        for (int c0 = 0; c0 < ncell; c0 += 64) {
+            const int k = c0 + tid, w = k < ncell ? lcnt[k] : 0;
+            const int inc = wave_inclusive_scan(w);
+            if (k < ncell) lstart[k] = carry + inc - w;
+            carry += __shfl(inc, 63);
+        }
+    }
+    __syncthreads();
+    for (int k = tid; k < ncell; k += SORT_T) {
+        cell_count[((int64_t)t << shift) + k] = lcnt[k];
+        cell_start[((int64_t)t << shift) + k] = (int32_t)s + lstart[k];
+    }
+    if (fits) {
+#pragma unroll
+        for (int u = 0; u < N; ++u)
+            if (v[u] >= 0) lv[lstart[c[u]] + d[u]] = v[u];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            if (v[u] < 0) continue;
+            const int a = lstart[c[u]], e = a + lcnt[c[u]];
+            int rank = 0;
+            for (int q = a; q < e; ++q) rank += lv[q] < v[u] ? 1 : 0;
+            d[u] = a + rank;
+        }
+        // the planes, three at a time; the next three are loaded before these are written
+        int32_t im[3][N];
+        for (int k = 0; k < 3; ++k) tile_load<N>(im[k], src.image + k * n, v);
+        if (wrap)
+            for (int k = 0; k < 3; ++k)
+                for (int u = 0; u < N; ++u)
+                    if (v[u] >= 0) {
+                        int jump;
+                        wrap_pbc<R>(b, x[k][u], jump, k);
+                        im[k][u] += jump;
+                    }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            for (int k = 0; k < 3; ++k) tile_put<N>(buf[k], x[k], v, d);
+            if (g < 3)
+                for (int k = 0; k < 3; ++k) tile_load<N>(x[k], from[(g + 1) & 3] + k * n, v);
+            __syncthreads();
+            for (int k = 0; k < 3; ++k) tile_store<N>(to[g] + k * n + s, buf[k], m);
+            __syncthreads();
+        }
+        int32_t id[N];
+        S sp[N], fl[N];
+        tile_load<N>(id, src.id, v);
+        tile_load<N>(sp, src.species, v);
+        tile_load<N>(fl, src.flags, v);
+        int32_t *ib[3] = {(int32_t *)buf[0], (int32_t *)buf[1], (int32_t *)buf[2]};
+        for (int k = 0; k < 3; ++k) tile_put<N>(ib[k], im[k], v, d);
+        __syncthreads();
+        for (int k = 0; k < 3; ++k) tile_store<N>(dst.image + k * n + s, ib[k], m);
+        __syncthreads();
+        S *sb = (S *)buf[1], *fb = (S *)buf[2];
+        tile_put<N>(ib[0], id, v, d);
+        tile_put<N>(sb, sp, v, d);
+        tile_put<N>(fb, fl, v, d);
+        if (id_to_idx)
+            for (int u = 0; u < N; ++u)
+                if (v[u] >= 0 && (uint32_t)id[u] < (uint32_t)n) id_to_idx[id[u]] = (int32_t)(s + d[u]);
+        __syncthreads();
+        tile_store<N>(dst.id + s, ib[0], m);
+        tile_store<N>(dst.species + s, sb, m);
+        tile_store<N>(dst.flags + s, fb, m);
+        return;
+    }
+    // more particles than the LDS holds: the list grouped by cell goes to memory (each
+    // workgroup writes and reads its own stretch), and each particle is ranked and moved
+    // from there
+    for (int k = tid; k < ncell; k += SORT_T) lcnt[k] = 0;
+    __syncthreads();
+    for (int q = tid; q < m; q += SORT_T) {
+        const int32_t w = list[s + q];
+        const int k = key[w] & cmask;
+        spill[s + lstart[k] + atomicAdd(&lcnt[k], 1)] = w;
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int q = tid; q < m; q += SORT_T) {
+        const int32_t w = spill[s + q];
+        const int k = key[w] & cmask;
+        const int a = lstart[k], e = a + lcnt[k];
+        int rank = 0;
+        for (int y = a; y < e; ++y) rank += spill[s + y] < w ? 1 : 0;
+        const int64_t o = s + a + rank;
+        for (int j = 0; j < 3; ++j) {
+            R x = src.pos[j * n + w];
+            int32_t im = src.image[j * n + w];
+            if (wrap) {
+                int jmp;
+                wrap_pbc<R>(b, x, jmp, j);
+                im += jmp;
+            }
+            dst.pos[j * n + o] = x;
+            dst.image[j * n + o] = im;
+            dst.vel[j * n + o] = src.vel[j * n + w];
+            dst.force[j * n + o] = src.force[j * n + w];
+            dst.force_old[j * n + o] = src.force_old[j * n + w];
+        }
+        const int32_t id = src.id[w];
+        dst.id[o] = id;
+        dst.species[o] = src.species[w];
+        dst.flags[o] = src.flags[w];
+        if (id_to_idx && (uint32_t)id < (uint32_t)n) id_to_idx[id] = (int32_t)o;
+    }
 }
 
 template <class F>
-int count_impl(const rmpcd_box_t *box, const rmpcd_particles_t *pp, rmpcd_cells_t *cells,
-               int wrap, int32_t *key, int32_t *slot)
+int count_impl(const rmpcd_box_t *box, const rmpcd_particles_t *pp, rmpcd_cells_t *cells)
 {
     Box b = make_box(box);
     PView<F> p = view<F>(pp);
@@ -215,32 +464,70 @@ int count_impl(const rmpcd_box_t *box, const rmpcd_particles_t *pp, rmpcd_cells_
     hipStream_t s = stream();
     k_fill_i32<<<blocks_for(b.ncells, 256), 256, 0, s>>>(cells->cell_count, b.ncells, 0);
     RMPCD_LAUNCHED();
-    k_key_count<F><<<blocks_for(p.n, 256), 256, 0, s>>>(b, lut, p, wrap, cells->cell_count,
-                                                          key, slot);
+    k_key_count<F><<<blocks_for(p.n, 256), 256, 0, s>>>(b, lut, p, cells->cell_count);
     RMPCD_LAUNCHED();
     return exclusive_scan(cells->cell_count, cells->cell_start, b.ncells);
+}
+
+// cells per tile (a power of two): the most whose particles, at the mean density of the
+// cells inside the box, fill at most 0.9 of the LDS (a tile above that by chance still fits:
+// three standard deviations of 1400 particles are 112), and small enough that a box has two
+// workgroups for every compute unit (a floor of 1024 or 2048 tiles made no difference)
+static int tile_shift(const Box &b, int64_t n, int tile_max)
+{
+    const double per_cell = (double)n / ((double)b.L[0] * b.L[1] * b.L[2]);
+    int shift = 0;
+    while ((2 << shift) <= TILE_CELLS && (2 << shift) <= b.ncells && per_cell * (2 << shift) <= tile_max * 0.9 &&
+           (b.ncells >> (shift + 1)) >= 512)
+        ++shift;
+    return shift;
 }
 
 template <class F>
 int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
               int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap)
 {
-    int64_t n = src->n;
+    const int64_t n = src->n;
+    const Box b = make_box(box);
+    const int shift = tile_shift(b, n, TILE_MAX<F>);
+    const int nt = b.ncells >> shift;
     int32_t *key = (int32_t *)workspace(WS_KEY, sizeof(int32_t) * n);
     int32_t *slot = (int32_t *)workspace(WS_SLOT, sizeof(int32_t) * n);
-    int32_t *tmp = (int32_t *)workspace(WS_TMP, sizeof(int32_t) * n);
-    if (!key || !slot || !tmp) return set_error(RMPCD_ERR_HIP, "rmpcd_sort: workspace allocation failed");
-    int rc = count_impl<F>(box, src, cells, wrap, key, slot);
-    if (rc) return rc;
-    Box b = make_box(box);
+    int32_t *list = (int32_t *)workspace(WS_TMP, sizeof(int32_t) * n);
+    int32_t *tstart = (int32_t *)workspace(WS_TILE, sizeof(int32_t) * ((size_t)nt + 1));
+    // zero between sorts
+    const int stride = nt <= SCAN1_TILES ? COUNT_STRIDE : 1;
+    int32_t *tcount = (int32_t *)workspace(WS_TCOUNT, sizeof(int32_t) * ((size_t)nt + 1) * stride);
+    if (!key || !slot || !list || !tstart || !tcount)
+        return set_error(RMPCD_ERR_HIP, "rmpcd_sort: workspace allocation failed");
+    const int32_t *lut = hilbert_lut(b);
+    if (!lut) return set_error(RMPCD_ERR_HIP, "rmpcd_sort: Hilbert table allocation failed");
     hipStream_t s = stream();
-    k_place<<<blocks_for(n, 256), 256, 0, s>>>(n, key, slot, cells->cell_start, tmp);
+    k_tile_key<F><<<blocks_for(n, KEY_CHUNK), SORT_T, 0, s>>>(b, lut, view<F>(src), wrap, shift, stride, tcount, key,
+                                                              slot);
     RMPCD_LAUNCHED();
-    k_gather<F><<<blocks_for(n, 256), 256, 0, s>>>(b, view<F>(src), view<F>(dst), wrap, key,
-                                                     cells->cell_start, cells->cell_count, tmp,
-                                                     id_to_idx);
+    if (nt <= SCAN1_TILES) {
+        k_tile_scan<<<1, 1024, 0, s>>>(tcount, nt, tstart);
+        RMPCD_LAUNCHED();
+    } else {
+        int rc = exclusive_scan(tcount, tstart, (int64_t)nt + 1);
+        if (rc) return rc;
+        k_fill_i32<<<blocks_for(nt, 256), 256, 0, s>>>(tcount, nt, 0);
+        RMPCD_LAUNCHED();
+    }
+    k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, key, shift, slot, tstart, list);
+    RMPCD_LAUNCHED();
+    k_tile_gather<F><<<8 * TILE_RUN * (unsigned)((nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN)), SORT_T, 0, s>>>(b, view<F>(src), view<F>(dst), wrap, shift, nt, key,
+                                                                    tstart, list, slot, cells->cell_count,
+                                                                    cells->cell_start, id_to_idx);
     RMPCD_LAUNCHED();
     return RMPCD_OK;
+}
+
+int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
+                   rmpcd_cells_t *cells, int wrap)
+{
+    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, wrap);
 }
 
 template <class F>
@@ -279,7 +566,7 @@ int rmpcd_count_particles(const rmpcd_box_t *box, const rmpcd_particles_t *p,
     if (rc) return rc;
     RMPCD_CHECK(cells && cells->cell_count && cells->cell_start,
                 "rmpcd_count_particles: null cell arrays");
-    return RMPCD_DISPATCH_FORM(p, count_impl, box, p, cells, 0, nullptr, nullptr);
+    return RMPCD_DISPATCH_FORM(p, count_impl, box, p, cells);
 }
 
 int rmpcd_cartesian_indices(const rmpcd_box_t *box, const rmpcd_particles_t *p, int32_t *xyz)
@@ -309,7 +596,7 @@ int rmpcd_sort(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_parti
                     src->force_old != dst->force_old && src->image != dst->image &&
                     src->id != dst->id && src->species != dst->species && src->flags != dst->flags,
                 "rmpcd_sort: source and destination share an array (the sort is out of place)");
-    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, apply_pbc ? 1 : 0);
+    return sort_unchecked(box, src, dst, id_to_idx, cells, apply_pbc ? 1 : 0);
 }
 
 }  // extern "C"

@@ -126,6 +126,42 @@ def test_sort_outside_box_and_empty_cells(gpu):
     assert same_bits(dst.host("id"), srt.id)
 
 
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("L,n,spread", [
+    ((4, 4, 4), 64 * 700, "even"),          # a tile is one cell, fuller than its LDS
+    ((16, 16, 16), 3000, "one cell"),       # every particle in one cell
+    ((32, 32, 32), 60000, "octant"),        # tiles of many cells fuller than their LDS
+    ((37, 5, 21), 41, "even"),              # fewer particles than tiles
+    ((256, 256, 128), 200000, "even"),      # more tiles than one workgroup scans
+])
+def test_sort_tiles(gpu, L, n, spread, form):
+    """the tile sort where tiles overflow, are empty or are many; positions and grid shift are
+    multiples of 2^-10, so both forms place them in the oracle's cells"""
+    rng = np.random.default_rng(n)
+    ps = O.PState(n)
+    hi = {"even": L, "one cell": (1, 1, 1), "octant": [v // 4 for v in L]}[spread]
+    ps.pos[:] = rng.integers(0, np.array(hi) * 1024, size=(n, 3)) / 1024.0
+    ps.vel[:] = rng.integers(-999, 999, size=(n, 3)) / 256.0
+    ps.force[:] = rng.integers(-999, 999, size=(n, 3)) / 256.0
+    ps.force_old[:] = rng.integers(-999, 999, size=(n, 3)) / 256.0
+    ps.image[:] = rng.integers(-3, 4, size=(n, 3))
+    ps.species[:] = rng.integers(0, 4, size=n)
+    ps.flags[:] = rng.integers(0, 128, size=n)
+    ps.id[:] = rng.permutation(n).astype(np.int32)
+    c = O.cells_init(L)
+    O.set_origin(c, (0.0, 0.0, 0.0) if spread == "one cell" else (-0.5, -0.25, -0.75))
+    srt, i2i, cnt, st = O.sort(c, ps)
+    src, dst = to_device(ps, form=form), ParticleSet(n, form=form)
+    i2i_d = torch.zeros(n, dtype=torch.int32, device="cuda")
+    cs = cells_to_device(c)
+    capi.call("rmpcd_sort", cs.boxp(), src.struct(), dst.struct(), ptr(i2i_d), cs.cellsp(), 0)
+    torch.cuda.synchronize()
+    assert same_bits(cs.cell_count.cpu().numpy(), cnt) and same_bits(cs.cell_start.cpu().numpy(), st)
+    for name in ("pos", "vel", "force", "force_old", "image", "id", "species", "flags"):
+        assert (dst.host(name) == getattr(srt, name)).all(), name
+    assert same_bits(i2i_d.cpu().numpy(), i2i)
+
+
 def test_maximum_displacement(gpu):
     ps = solvent_state((10, 10, 10), 10, 12)
     old = ps.pos.copy()
