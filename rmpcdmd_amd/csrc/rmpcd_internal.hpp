@@ -30,6 +30,7 @@ enum Slot {
     WS_NLCNT,       // neighbour-list per-stencil-cell counts
     WS_PART,        // per-block partial sums
     WS_AUX,         // misc
+    WS_HEAD,        // chains of list entries by particle: zeroed when allocated, left zero by compute_force
     WS_COUNT
 };
 void *workspace(Slot s, size_t bytes);

@@ -123,60 +123,71 @@ __global__ void k_roll_md(int64_t n, typename F::small *flags)
     flags[i] = (typename F::small)(f & ~MD_MASK);
 }
 
-// compute_force part 2 (neighbor_list.f90:191-222): one thread per list entry of the
-// colloids c0 .. c0 + gridDim.y - 1.  With one colloid per launch (ordered launches) each
-// solvent particle is in the list at most once, so its force is updated without atomics,
-// in the reference's colloid order, bit for bit; a launch over several colloids adds
-// with atomics (the order of two colloids' contributions to one particle is then not
-// fixed).  The colloid force and energy go to per-block partials, summed in block order by
-// k_force_nl_sum.
+// compute_force part 2 (neighbor_list.f90:191-222): the force of colloid i on entry k of
+// its list, f = 0 beyond the cutoff; true when the pair is inside it
+template <class F>
+__device__ inline bool pair_force(const PView<F64> &c, const PView<F> &sol, int i, int idx, double L0, double L1,
+                                  double L2, const LJ &lj, double f[3], double *e)
+{
+    const int s2 = (int)sol.species[idx];
+    if (s2 <= 0) return false;
+    const double d0 = min_image(c.pos[i] - (double)sol.pos[idx], L0);
+    const double d1 = min_image(c.pos[c.n + i] - (double)sol.pos[sol.n + idx], L1);
+    const double d2 = min_image(c.pos[2 * c.n + i] - (double)sol.pos[2 * sol.n + idx], L2);
+    const double r_sq = (d0 * d0 + d1 * d1) + d2 * d2;
+    const int pidx = (s2 - 1) + lj.n1 * (c.species[i] - 1);
+    if (!(r_sq <= lj.cut_sq[pidx])) return false;
+    const double fr = lj_force_over_r(r_sq, lj.eps[pidx], lj.sigma[pidx]);
+    f[0] = fr * d0;
+    f[1] = fr * d1;
+    f[2] = fr * d2;
+    *e = lj_energy(r_sq, lj.eps[pidx], lj.sigma[pidx], lj.cut_energy[pidx]);
+    return true;
+}
+
+// The colloids c0 .. c0 + gridDim.y - 1, one thread per list entry.  The reference adds
+// the forces on a solvent particle in colloid order.  One colloid meets a particle once,
+// and its thread adds the force at once (next null).  With several, the entries inside the
+// cutoff chain up per particle, head[particle] = the last to arrive, next[entry] = the one
+// before (entries counted from 1, 0 ends a chain, OUTSIDE marks the entries beyond the
+// cutoff), and k_force_nl_apply adds each chain in order.  The colloid force and energy go
+// to per-block partials, summed in block order by k_force_nl_sum.  Bound by launches and the
+// latency of the entries' reads: a launch per colloid, which kept the order before, took
+// 390 us an MD step with 52 colloids (30.0 ms a cycle of 50 steps, 10.8 with the chains).
+constexpr uint32_t OUTSIDE = 0xffffffffu;
+
 template <class F>
 __global__ void __launch_bounds__(256)
     k_force_nl(PView<F64> c, PView<F> sol, const int32_t *__restrict__ list,
                const int32_t *__restrict__ nl, int32_t nmax, double L0, double L1, double L2, LJ lj,
-               double *__restrict__ part, int c0, int atomic_add)
+               double *__restrict__ part, int c0, uint32_t *__restrict__ head, uint32_t *__restrict__ next)
 {
     using R = typename F::real;
     __shared__ double red[16];
     const int i = c0 + (int)blockIdx.y;
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     const int n_i = min(nl[i], nmax);
-    double f0 = 0, f1 = 0, f2 = 0, e = 0;
-    const double x0 = c.pos[i], x1 = c.pos[c.n + i], x2 = c.pos[2 * c.n + i];
-    const int s1 = c.species[i];
+    double *pp = part + ((int64_t)i * gridDim.x + blockIdx.x) * 4;
+    if ((int)(blockIdx.x * blockDim.x) >= n_i) {  // past the list: nothing to add
+        if (threadIdx.x < 4) pp[threadIdx.x] = 0;
+        return;
+    }
+    double f[3] = {0, 0, 0}, e = 0;
     if (k < n_i) {
         const int idx = list[(int64_t)i * nmax + k];
-        const int s2 = (int)sol.species[idx];
-        if (s2 > 0) {
-            const double d0 = min_image(x0 - (double)sol.pos[idx], L0);
-            const double d1 = min_image(x1 - (double)sol.pos[sol.n + idx], L1);
-            const double d2 = min_image(x2 - (double)sol.pos[2 * sol.n + idx], L2);
-            const double r_sq = (d0 * d0 + d1 * d1) + d2 * d2;
-            const int pidx = (s2 - 1) + lj.n1 * (s1 - 1);
-            if (r_sq <= lj.cut_sq[pidx]) {
-                const double fr = lj_force_over_r(r_sq, lj.eps[pidx], lj.sigma[pidx]);
-                f0 = fr * d0;
-                f1 = fr * d1;
-                f2 = fr * d2;
-                e = lj_energy(r_sq, lj.eps[pidx], lj.sigma[pidx], lj.cut_energy[pidx]);
-                if (atomic_add) {
-                    atomicAdd(&sol.force[idx], (R)(-f0));
-                    atomicAdd(&sol.force[sol.n + idx], (R)(-f1));
-                    atomicAdd(&sol.force[2 * sol.n + idx], (R)(-f2));
-                } else {
-                    sol.force[idx] = sol.force[idx] - (R)f0;
-                    sol.force[sol.n + idx] = sol.force[sol.n + idx] - (R)f1;
-                    sol.force[2 * sol.n + idx] = sol.force[2 * sol.n + idx] - (R)f2;
-                }
-                const int mask = MD_MASK | (s1 == 1 ? CATALYZED_MASK : 0);
-                atomic_or_flag(&sol.flags[idx], mask);
-            }
+        const bool in = pair_force<F>(c, sol, i, idx, L0, L1, L2, lj, f, &e);
+        if (next) {
+            const uint32_t ent = (uint32_t)blockIdx.y * (uint32_t)nmax + (uint32_t)k + 1;
+            next[ent - 1] = in ? atomicExch(&head[idx], ent) : OUTSIDE;
+        } else if (in) {
+            for (int q = 0; q < 3; ++q) sol.force[q * sol.n + idx] = sol.force[q * sol.n + idx] - (R)f[q];
+            sol.flags[idx] = (typename F::small)((int)sol.flags[idx] | MD_MASK |
+                                                 (c.species[i] == 1 ? CATALYZED_MASK : 0));
         }
     }
-    const double b0 = block_sum(f0, red), b1 = block_sum(f1, red), b2 = block_sum(f2, red),
+    const double b0 = block_sum(f[0], red), b1 = block_sum(f[1], red), b2 = block_sum(f[2], red),
                  be = block_sum(e, red);
     if (threadIdx.x == 0) {
-        double *pp = part + ((int64_t)i * gridDim.x + blockIdx.x) * 4;
         pp[0] = b0;
         pp[1] = b1;
         pp[2] = b2;
@@ -184,24 +195,64 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// the colloid force and energy of compute_force: colloid blockIdx.x's block partials in
-// block order, added to the force it holds (one thread per colloid)
-__global__ void k_force_nl_sum(PView<F64> c, const double *__restrict__ part, int nb, double *__restrict__ e_out)
+// the chains of k_force_nl: the thread of a chain's last arrival adds its entries in
+// colloid order (the next larger entry each time: two or three colloids meet at most) and
+// clears the head.  The other entries of the chain read a head that is not their own before
+// as after that.
+template <class F>
+__global__ void __launch_bounds__(256)
+    k_force_nl_apply(PView<F64> c, PView<F> sol, const int32_t *__restrict__ list, const int32_t *__restrict__ nl,
+                     int32_t nmax, double L0, double L1, double L2, LJ lj, int c0, uint32_t *__restrict__ head,
+                     const uint32_t *__restrict__ next)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= c.n) return;
-    double a0 = 0, a1 = 0, a2 = 0, ae = 0;
-    for (int q = 0; q < nb; ++q) {
-        const double *pp = part + ((int64_t)i * nb + q) * 4;
-        a0 += pp[0];
-        a1 += pp[1];
-        a2 += pp[2];
-        ae += pp[3];
+    using R = typename F::real;
+    const int i = c0 + (int)blockIdx.y;
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= min(nl[i], nmax)) return;
+    const uint32_t ent = (uint32_t)blockIdx.y * (uint32_t)nmax + (uint32_t)k + 1;
+    if (next[ent - 1] == OUTSIDE) return;
+    const int idx = list[(int64_t)i * nmax + k];
+    if (head[idx] != ent) return;
+    R a[3] = {sol.force[idx], sol.force[sol.n + idx], sol.force[2 * sol.n + idx]};
+    int fl = (int)sol.flags[idx];
+    uint32_t done = 0;
+    for (;;) {
+        uint32_t least = OUTSIDE;
+        for (uint32_t q = ent; q; q = next[q - 1])
+            if (q > done && q < least) least = q;
+        if (least == OUTSIDE) break;
+        done = least;
+        const int ci = c0 + (int)((least - 1) / (uint32_t)nmax);
+        double f[3] = {0, 0, 0}, e;
+        pair_force<F>(c, sol, ci, idx, L0, L1, L2, lj, f, &e);
+        for (int q = 0; q < 3; ++q) a[q] = a[q] - (R)f[q];
+        fl |= MD_MASK | (c.species[ci] == 1 ? CATALYZED_MASK : 0);
     }
-    c.force[i] = c.force[i] + a0;
-    c.force[c.n + i] = c.force[c.n + i] + a1;
-    c.force[2 * c.n + i] = c.force[2 * c.n + i] + a2;
-    e_out[i] = ae;
+    for (int q = 0; q < 3; ++q) sol.force[q * sol.n + idx] = a[q];
+    sol.flags[idx] = (typename F::small)fl;
+    head[idx] = 0;
+}
+
+// the colloid force and energy of compute_force: colloid blockIdx.x's block partials,
+// staged in LDS and added in block order by one lane per component
+__global__ void __launch_bounds__(64)
+    k_force_nl_sum(PView<F64> c, const double *__restrict__ part, int nb, double *__restrict__ e_out)
+{
+    __shared__ double lp[256][4];
+    const int i = blockIdx.x, q = threadIdx.x;
+    double a = 0;
+    for (int b0 = 0; b0 < nb; b0 += 256) {
+        const int m = min(256, nb - b0);
+        __syncthreads();
+        for (int x = q; x < 4 * m; x += 64) lp[x >> 2][x & 3] = part[4 * ((int64_t)i * nb + b0) + x];
+        __syncthreads();
+        if (q < 4)
+            for (int b = 0; b < m; ++b) a += lp[b][q];
+    }
+    if (q < 3)
+        c.force[q * c.n + i] = c.force[q * c.n + i] + a;
+    else if (q == 3)
+        e_out[i] = a;
 }
 
 __global__ void k_copy_f64(const double *__restrict__ a, double *__restrict__ b, int64_t n)
@@ -367,35 +418,40 @@ int update_list_impl(const rmpcd_box_t *box, rmpcd_cells_t *cells, const rmpcd_p
     return RMPCD_OK;
 }
 
-constexpr int FORCE_ORDERED = 64;  // colloids of compute_force taken one launch each
-
 template <class F>
 int force_impl(rmpcd_particles_t *ps1, rmpcd_particles_t *ps2, const int32_t *list, const int32_t *nl,
                int32_t nmax, const double *L, const rmpcd_lj_t *lj, double *e)
 {
     int np = (int)ps1->n;
     unsigned nb = blocks_for(nmax, 256);
+    PView<F> sol = view<F>(ps2);
+    // colloids of one launch: their entries are counted in 32 bits
+    const int group = np == 1 ? 1 : (int)(nmax >= (1 << 30) ? 1 : np < (1 << 30) / nmax ? np : (1 << 30) / nmax);
     double *part = (double *)workspace(WS_PART, sizeof(double) * 4 * (size_t)nb * np);
     double *eb = (double *)workspace(WS_RED, sizeof(double) * (np + 1));
     double *host = (double *)pinned(64);
-    if (!part || !eb || !host) return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
+    uint32_t *head = nullptr, *next = nullptr;
+    if (np > 1) {
+        head = (uint32_t *)workspace(WS_HEAD, sizeof(uint32_t) * (size_t)sol.n);
+        next = (uint32_t *)workspace(WS_AUX, sizeof(uint32_t) * (size_t)group * nmax);
+    }
+    if (!part || !eb || !host || (np > 1 && (!head || !next)))
+        return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
     hipStream_t s = stream();
-    PView<F> sol = view<F>(ps2);
     k_roll_md<F><<<blocks_for(sol.n, 256), 256, 0, s>>>(sol.n, sol.flags);
     RMPCD_LAUNCHED();
-    // up to FORCE_ORDERED colloids, one launch per colloid: the solvent forces are then
-    // updated in the reference's colloid order, without atomics
     const LJ l = make_lj(lj);
-    if (np <= FORCE_ORDERED) {
-        for (int i = 0; i < np; ++i)
-            k_force_nl<F><<<dim3(nb, 1), 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, part,
-                                                      i, 0);
-    } else {
-        k_force_nl<F><<<dim3(nb, np), 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, part, 0,
-                                                   1);
+    for (int c0 = 0; c0 < np; c0 += group) {
+        const dim3 grid(nb, group < np - c0 ? group : np - c0);
+        k_force_nl<F><<<grid, 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, part, c0, head,
+                                           next);
+        RMPCD_LAUNCHED();
+        if (np == 1) break;
+        k_force_nl_apply<F><<<grid, 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, c0, head,
+                                                 next);
+        RMPCD_LAUNCHED();
     }
-    RMPCD_LAUNCHED();
-    k_force_nl_sum<<<blocks_for(np, 64), 64, 0, s>>>(view<F64>(ps1), part, (int)nb, eb);
+    k_force_nl_sum<<<np, 64, 0, s>>>(view<F64>(ps1), part, (int)nb, eb);
     RMPCD_LAUNCHED();
     k_sum_serial<<<1, 64, 0, s>>>(eb, np, eb + np);
     RMPCD_LAUNCHED();

@@ -52,7 +52,7 @@ void *workspace(Slot s, size_t bytes)
         e.ptr = nullptr;
         return nullptr;
     }
-    if (s == WS_TCOUNT && hipMemsetAsync(e.ptr, 0, want, g_stream) != hipSuccess) {
+    if ((s == WS_TCOUNT || s == WS_HEAD) && hipMemsetAsync(e.ptr, 0, want, g_stream) != hipSuccess) {
         (void)hipFree(e.ptr);
         e.ptr = nullptr;
         return nullptr;

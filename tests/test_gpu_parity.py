@@ -461,6 +461,39 @@ def test_update_list_overflow(gpu):
     assert nlst.n.max().item() <= 50
 
 
+@pytest.mark.parametrize("n_col,nmax", [(1, 3000), (3, 2501), (70, 2600)])
+def test_compute_force_colloid_order(gpu, n_col, nmax):
+    """overlapping colloids, so that particles lie inside the cutoff of several: their forces
+    are added in the reference's colloid order, bit for bit, onto what they hold"""
+    L = (14, 12, 13)
+    c, srt, cnt, st = sorted_state(L, 10, 41, frac2=0.3)
+    rng = np.random.default_rng(n_col)
+    cp = O.PState(n_col)
+    cp.pos[:] = (np.array([6.0, 6.0, 6.0]) + rng.uniform(-3, 3, size=(n_col, 3))) % L
+    cp.force[:] = rng.normal(size=(n_col, 3))
+    cp.species[:] = rng.integers(1, 3, size=n_col)
+    sig = np.array([[1.5, 1.2], [1.4, 1.6]])
+    cut = sig * 2 ** (1 / 6)
+    eps = np.array([[1.0, 0.7], [1.3, 0.9]])
+    radius = cut.max() + 1.0
+    lj_o = O.lj_params(eps, sig, cut)
+    lst, nl, is_md, is_reac = O.update_list(c, cnt, st, cp.pos, cp.species, srt.pos, srt.species, radius,
+                                            O.make_stencil(1.0, radius), lj_o, nmax)
+    d, cd = to_device(srt), to_device(cp)
+    want_s, want_c = srt.copy(), cp.copy()
+    e_o = O.compute_force(want_c.pos, want_c.species, want_c.force, want_s.pos, want_s.species, want_s.force,
+                          want_s.flags, lst, nl, L, lj_o)
+    lj, e = lj_params(eps, sig, cut), C.c_double()
+    ld, nd = torch.as_tensor(lst).cuda(), torch.as_tensor(nl).cuda()
+    capi.call("rmpcd_compute_force", cd.struct(), d.struct(), ptr(ld), ptr(nd), nmax, capi.d3(L), C.byref(lj),
+              C.byref(e))
+    assert same_bits(d.host("force"), want_s.force)
+    assert same_bits(d.host("flags"), want_s.flags)
+    # the colloid sums run over blocks of 256 entries: 1e-12 of the sum of the magnitudes
+    assert abs(e.value - e_o) <= 1e-12 * abs(e_o)
+    assert close(cd.host("force"), want_c.force, scale=np.abs(want_c.force - cp.force).sum() + 1.0)
+
+
 def test_compute_force_and_helpers(gpu):
     L = (20, 20, 20)
     c, srt, cnt, st, cp, eps, sig, cut = dimer_setup(L, 10, 29)
