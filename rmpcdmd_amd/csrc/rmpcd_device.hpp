@@ -512,12 +512,6 @@ __device__ inline double block_max(double v, double *scratch)
     return t;
 }
 
-// atomic max on a non-negative double through its bit pattern (monotone for x >= 0)
-__device__ inline void atomic_max_nonneg(double *addr, double v)
-{
-    atomicMax((unsigned long long *)addr, (unsigned long long)__double_as_longlong(v));
-}
-
 // OR / AND into a flag of either width (a uint8 flag is updated through its aligned
 // 32-bit word; flag arrays are allocated in multiples of 256 bytes)
 __device__ inline void atomic_or_flag(int32_t *f, int m) { atomicOr(f, m); }
