@@ -72,6 +72,16 @@ int check_box(const rmpcd_box_t *b, const char *who);
 int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
                    rmpcd_cells_t *cells, int wrap);
 
+// the parts of compute_force after the roll of the MD bits, on checked sets: the solvent's
+// forces and the colloids' block partials (4 doubles per block of 256 entries), the
+// partials' sums added to the colloid forces, the energies' sum in colloid order
+int force_list_unchecked(const rmpcd_particles_t *ps1, const rmpcd_particles_t *ps2, const int32_t *list,
+                         const int32_t *nl, int32_t nmax, const double *L, const rmpcd_lj_t *lj, double *part);
+int force_sum_unchecked(const rmpcd_particles_t *ps1, const double *part, int nb, double *e_out);
+int energy_sum_unchecked(const double *e, int64_t n, double *out);
+// compute_temperature on checked sets, left in device (or pinned) memory
+int temperature_unchecked(const rmpcd_box_t *box, const rmpcd_cells_t *cells, const rmpcd_particles_t *p, double *te);
+
 inline unsigned blocks_for(int64_t n, int threads)
 {
     int64_t b = (n + threads - 1) / threads;

@@ -3,6 +3,7 @@
 // (src/md.f90:61-319, src/particle_system.f90:357-410,
 //  programs/single_dimer_pbc.f90:312-315,356-359).
 #include "rmpcd_internal.hpp"
+#include "rmpcd_steps.hpp"
 
 namespace rmpcd {
 
@@ -54,43 +55,6 @@ __global__ void k_apply_pbc(int64_t n, typename F::real *__restrict__ pos, int32
         int jump = (int)floor((double)(x / ed));
         image[k * n + i] += jump;
         pos[k * n + i] = x - (R)jump * ed;
-    }
-}
-
-// cell_md_pos / cell_md_vel / cell_md_pos_{y,z}wall (md.f90:79-263) and
-// cell_maximum_displacement (particle_system.f90:380-410) touch the particles of the cells
-// with is_md equal to md_flag.  A wave takes CELL_WAVE consecutive cells: it reads their
-// marks, starts and counts together, then goes through those that qualify, four at a time
-// with CELL_LANES lanes each, so that neighbouring lanes move neighbouring particles (a
-// thread per cell walked its ten particles one after the other, each wave's lanes ten
-// particles apart: for the velocities, positions and displacements of the md cells of an
-// L = 48 box with 52 colloids, FP64, 33, 24 and 22 us then, 16, 10 and 12 us now).
-constexpr int CELL_WAVE = 32, CELL_LANES = 16;
-
-template <class Fn>
-__device__ inline void for_md_cells(int ncells, const int32_t *__restrict__ start, const int32_t *__restrict__ count,
-                                    const uint8_t *__restrict__ is_md, int md_flag, Fn each)
-{
-    const int lane = threadIdx.x & 63, sub = lane & (CELL_LANES - 1), grp = lane / CELL_LANES;
-    const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int64_t c = wave * CELL_WAVE + (lane & (CELL_WAVE - 1));
-    int s = 0, m = 0;
-    bool on = false;
-    if (c < ncells) {
-        s = start[c];
-        m = count[c];
-        on = m > 0 && (is_md[c] != 0) == (md_flag != 0);
-    }
-    // one bit per cell (the two halves of the wave hold the same cells)
-    uint32_t todo = (uint32_t)__ballot(on);
-    while (todo) {
-        uint32_t t = todo;
-        for (int k = 0; k < grp; ++k) t &= t - 1;
-        const int from = t ? __ffs(t) - 1 : 0;
-        const int cs = __shfl(s, from), cm = __shfl(m, from);
-        const int n = t ? cm : 0;
-        for (int j = sub; j < n; j += CELL_LANES) each((int64_t)cs + j);
-        for (int k = 0; k < 64 / CELL_LANES; ++k) todo &= todo - 1;
     }
 }
 
@@ -161,17 +125,6 @@ __global__ void __launch_bounds__(256)
     });
 }
 
-// the squared displacement of particle j from pos_old (particle_system.f90:357-378)
-template <class F>
-__device__ inline double disp_sq(const PView<F> &p, const typename F::real *__restrict__ pos_old, int64_t j)
-{
-    if ((int)p.species[j] < 0) return 0;
-    const double d0 = (double)(p.pos[j] - pos_old[j]);
-    const double d1 = (double)(p.pos[p.n + j] - pos_old[p.n + j]);
-    const double d2 = (double)(p.pos[2 * p.n + j] - pos_old[2 * p.n + j]);
-    return (d0 * d0 + d1 * d1) + d2 * d2;
-}
-
 // maximum_displacement (particle_system.f90:357-378): a maximum per workgroup (a maximum
 // does not depend on the order, so the result is exact); k_max_final takes the maximum of
 // these.  With an atomic maximum on one word instead, 1280 workgroups of 327,680 FP64
@@ -203,16 +156,6 @@ __global__ void __launch_bounds__(256)
     for_md_cells(ncells, start, count, is_md, 1, [&](int64_t j) { local = fmax(local, disp_sq<F>(p, pos_old, j)); });
     const double m = block_max(local, red);
     if (threadIdx.x == 0) part[blockIdx.x] = m;
-}
-
-// the maximum of n values, written where the host reads it
-__global__ void __launch_bounds__(1024) k_max_final(const double *__restrict__ part, int64_t n, double *__restrict__ out)
-{
-    __shared__ double red[16];
-    double a = 0;
-    for (int64_t q = threadIdx.x; q < n; q += 1024) a = fmax(a, part[q]);
-    a = block_max(a, red);
-    if (threadIdx.x == 0) out[0] = a;
 }
 
 // ---- colloids (always FP64) -----------------------------------------------------
@@ -315,8 +258,6 @@ int apply_pbc_impl(rmpcd_particles_t *pp, const double *e)
     RMPCD_LAUNCHED();
     return RMPCD_OK;
 }
-static unsigned cell_blocks(int ncells) { return blocks_for(ncells, 256 / 64 * CELL_WAVE); }
-
 template <class F>
 int cell_md_pos_impl(const rmpcd_box_t *box, const rmpcd_cells_t *cells, rmpcd_particles_t *pp,
                      double dt, int md_flag, int axis)
@@ -342,7 +283,7 @@ static int fetch_max(const double *part, unsigned nb, double *r)
 {
     double *host = (double *)pinned(64);
     if (!host) return set_error(RMPCD_ERR_HIP, "pinned staging allocation failed");
-    k_max_final<<<1, 1024, 0, stream()>>>(part, nb, host);
+    k_max_final<1024><<<1, 1024, 0, stream()>>>(part, nb, host, nullptr, 0);
     RMPCD_LAUNCHED();
     RMPCD_HIP(hipStreamSynchronize(stream()));
     *r = sqrt(host[0]);

@@ -902,26 +902,41 @@ int stream_yzwall_impl(const rmpcd_box_t *box, rmpcd_particles_t *pp, double dt,
     return RMPCD_OK;
 }
 
+// compute_temperature, its result left in te (device or pinned memory)
 template <class F>
-int temperature_impl(const rmpcd_box_t *box, const rmpcd_cells_t *cells,
-                     const rmpcd_particles_t *pp, double *te, TzProfile tz)
+int temperature_launch(const rmpcd_box_t *box, const rmpcd_cells_t *cells, const rmpcd_particles_t *pp, double *te,
+                       TzProfile tz)
 {
     int nc = box->ncells;
     unsigned nb = blocks_for(nc, CELL_THREADS);
     double *part = (double *)workspace(WS_PART, sizeof(double) * 2 * nb);
-    double *red = (double *)workspace(WS_RED, 64);
-    double *host = (double *)pinned(64);
-    if (!part || !red || !host) return set_error(RMPCD_ERR_HIP, "compute_temperature: workspace allocation failed");
+    if (!part) return set_error(RMPCD_ERR_HIP, "compute_temperature: workspace allocation failed");
     hipStream_t s = stream();
     k_temperature<F><<<nb, CELL_THREADS, 0, s>>>(nc, cells->cell_start, cells->cell_count, view<F>(pp), part,
                                                  make_box(box), tz);
     RMPCD_LAUNCHED();
-    k_temperature_final<<<1, CELL_THREADS, 0, s>>>(part, nb, red);
+    k_temperature_final<<<1, CELL_THREADS, 0, s>>>(part, nb, te);
     RMPCD_LAUNCHED();
-    RMPCD_HIP(hipMemcpyAsync(host, red, sizeof(double), hipMemcpyDeviceToHost, s));
-    RMPCD_HIP(hipStreamSynchronize(s));
+    return RMPCD_OK;
+}
+
+template <class F>
+int temperature_impl(const rmpcd_box_t *box, const rmpcd_cells_t *cells,
+                     const rmpcd_particles_t *pp, double *te, TzProfile tz)
+{
+    double *host = (double *)pinned(64);
+    if (!host) return set_error(RMPCD_ERR_HIP, "compute_temperature: workspace allocation failed");
+    int rc = temperature_launch<F>(box, cells, pp, host, tz);
+    if (rc) return rc;
+    RMPCD_HIP(hipStreamSynchronize(stream()));
     *te = host[0];
     return RMPCD_OK;
+}
+
+int temperature_unchecked(const rmpcd_box_t *box, const rmpcd_cells_t *cells, const rmpcd_particles_t *p, double *te)
+{
+    const TzProfile tz{0, 0, 0, nullptr, nullptr};
+    return RMPCD_DISPATCH_FORM(p, temperature_launch, box, cells, p, te, tz);
 }
 
 // ---- compute_temperature without allocation ----------------------------------------

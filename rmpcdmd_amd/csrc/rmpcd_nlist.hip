@@ -7,6 +7,7 @@
 // the counts, and a fill pass that writes every accepted particle at its final offset.
 #include "rmpcd_internal.hpp"
 #include "rmpcd_pairforce.hpp"
+#include "rmpcd_steps.hpp"
 
 namespace rmpcd {
 
@@ -26,7 +27,11 @@ __device__ inline int stencil_key(const Box &b, const double *x, const int32_t *
 }
 
 // pass 1 (fill == 0) counts accepted particles per (point, stencil cell) and marks
-// is_md / is_reac; pass 2 (fill == 1) writes them at offset[point*ns + j]
+// is_md / is_reac; pass 2 (fill == 1) writes them at offset[point*ns + j].  NL_LANES lanes
+// take a stencil cell, a particle each (a thread per cell walked its ten particles one
+// after the other: 15 us a pass for one point with 1500 stencil cells, FP64).
+constexpr int NL_LANES = 16;
+
 template <class F>
 __global__ void __launch_bounds__(NL_THREADS)
     k_nl_pass(Box b, PView<F64> pts, PView<F> sol, const int32_t *__restrict__ start,
@@ -35,9 +40,10 @@ __global__ void __launch_bounds__(NL_THREADS)
               int32_t *__restrict__ cnt, uint8_t *__restrict__ is_md, uint8_t *__restrict__ is_reac,
               int fill, int32_t nmax, int32_t *__restrict__ list)
 {
-    int j = blockIdx.x * blockDim.x + threadIdx.x;
-    int i = blockIdx.y;
-    if (j >= ns) return;
+    const int j = (blockIdx.x * blockDim.x + threadIdx.x) / NL_LANES;
+    const int i = blockIdx.y;
+    if (j >= ns) return;  // all lanes of a cell alike
+    const int lane = threadIdx.x & 63, sub = lane & (NL_LANES - 1), first = lane - sub;
     double x[3] = {pts.pos[i], pts.pos[pts.n + i], pts.pos[2 * pts.n + i]};
     int si = pts.species[i];
     int key = stencil_key(b, x, st, j);
@@ -45,28 +51,34 @@ __global__ void __launch_bounds__(NL_THREADS)
     int64_t slot = (int64_t)i * ns + j;
     int off = fill ? cnt[slot] : 0;
     int k = 0;
-    bool md = false, noreac = false;
-    for (int q = s; q < s + n; ++q) {
-        int sp = (int)sol.species[q];
-        if (sp <= 0) continue;
-        double y0 = (double)sol.pos[q], y1 = (double)sol.pos[sol.n + q], y2 = (double)sol.pos[2 * sol.n + q];
-        double d0 = min_image(x[0] - y0, L0), d1 = min_image(x[1] - y1, L1), d2 = min_image(x[2] - y2, L2);
-        double rsq = (d0 * d0 + d1 * d1) + d2 * d2;
-        if (rsq < radiussq) {
-            md = true;
-            if (do_lj && rsq <= lj.cut_sq[(sp - 1) + lj.n1 * (si - 1)]) noreac = true;
-            if (fill) {
-                int pos = off + k;
-                if (pos < nmax) list[(int64_t)i * nmax + pos] = q;
-            }
-            ++k;
+    bool noreac = false;
+    for (int q0 = s; q0 < s + n; q0 += NL_LANES) {
+        const int q = q0 + sub;
+        const int sp = q < s + n ? (int)sol.species[q] : 0;
+        bool in = false;
+        if (sp > 0) {
+            double y0 = (double)sol.pos[q], y1 = (double)sol.pos[sol.n + q], y2 = (double)sol.pos[2 * sol.n + q];
+            double d0 = min_image(x[0] - y0, L0), d1 = min_image(x[1] - y1, L1), d2 = min_image(x[2] - y2, L2);
+            double rsq = (d0 * d0 + d1 * d1) + d2 * d2;
+            in = rsq < radiussq;
+            if (in && do_lj && rsq <= lj.cut_sq[(sp - 1) + lj.n1 * (si - 1)]) noreac = true;
         }
+        // the accepted lanes of this cell, in the cell's order
+        const unsigned m = (unsigned)(__ballot(in) >> first) & ((1u << NL_LANES) - 1);
+        if (fill && in) {
+            const int pos = off + k + __popc(m & ((1u << sub) - 1));
+            if (pos < nmax) list[(int64_t)i * nmax + pos] = q;
+        }
+        k += __popc(m);
     }
     if (!fill) {
-        cnt[slot] = k;
-        if (md) {
-            is_md[key] = 1;
-            if (noreac) is_reac[key] = 0;
+        const unsigned nr = (unsigned)(__ballot(noreac) >> first) & ((1u << NL_LANES) - 1);
+        if (sub == 0) {
+            cnt[slot] = k;
+            if (k > 0) {
+                is_md[key] = 1;
+                if (nr) is_reac[key] = 0;
+            }
         }
     }
 }
@@ -100,7 +112,7 @@ __global__ void __launch_bounds__(1024)
         // the reference stops here on overflow (neighbor_list.f90:135-137); the count is
         // clamped so that no consumer reads past the list capacity
         nout[i] = carry > nmax ? nmax : carry;
-        if (carry > nmax) atomicOr(overflow, 1);
+        if (carry > nmax) *overflow = 1;
     }
 }
 
@@ -121,28 +133,6 @@ __global__ void k_roll_md(int64_t n, typename F::small *flags)
     int f = (int)flags[i];
     f = (f & MD_MASK) ? (f | PAST_MD_MASK) : (f & ~PAST_MD_MASK);
     flags[i] = (typename F::small)(f & ~MD_MASK);
-}
-
-// compute_force part 2 (neighbor_list.f90:191-222): the force of colloid i on entry k of
-// its list, f = 0 beyond the cutoff; true when the pair is inside it
-template <class F>
-__device__ inline bool pair_force(const PView<F64> &c, const PView<F> &sol, int i, int idx, double L0, double L1,
-                                  double L2, const LJ &lj, double f[3], double *e)
-{
-    const int s2 = (int)sol.species[idx];
-    if (s2 <= 0) return false;
-    const double d0 = min_image(c.pos[i] - (double)sol.pos[idx], L0);
-    const double d1 = min_image(c.pos[c.n + i] - (double)sol.pos[sol.n + idx], L1);
-    const double d2 = min_image(c.pos[2 * c.n + i] - (double)sol.pos[2 * sol.n + idx], L2);
-    const double r_sq = (d0 * d0 + d1 * d1) + d2 * d2;
-    const int pidx = (s2 - 1) + lj.n1 * (c.species[i] - 1);
-    if (!(r_sq <= lj.cut_sq[pidx])) return false;
-    const double fr = lj_force_over_r(r_sq, lj.eps[pidx], lj.sigma[pidx]);
-    f[0] = fr * d0;
-    f[1] = fr * d1;
-    f[2] = fr * d2;
-    *e = lj_energy(r_sq, lj.eps[pidx], lj.sigma[pidx], lj.cut_energy[pidx]);
-    return true;
 }
 
 // The colloids c0 .. c0 + gridDim.y - 1, one thread per list entry.  The reference adds
@@ -233,32 +223,17 @@ __global__ void __launch_bounds__(256)
     head[idx] = 0;
 }
 
-// the colloid force and energy of compute_force: colloid blockIdx.x's block partials,
-// staged in LDS and added in block order by one lane per component
+// the colloid force and energy of compute_force: a colloid's block partials added to the
+// force it holds
 __global__ void __launch_bounds__(64)
     k_force_nl_sum(PView<F64> c, const double *__restrict__ part, int nb, double *__restrict__ e_out)
 {
-    __shared__ double lp[256][4];
     const int i = blockIdx.x, q = threadIdx.x;
-    double a = 0;
-    for (int b0 = 0; b0 < nb; b0 += 256) {
-        const int m = min(256, nb - b0);
-        __syncthreads();
-        for (int x = q; x < 4 * m; x += 64) lp[x >> 2][x & 3] = part[4 * ((int64_t)i * nb + b0) + x];
-        __syncthreads();
-        if (q < 4)
-            for (int b = 0; b < m; ++b) a += lp[b][q];
-    }
+    const double a = list_force_sum(part, nb, i);
     if (q < 3)
         c.force[q * c.n + i] = c.force[q * c.n + i] + a;
     else if (q == 3)
         e_out[i] = a;
-}
-
-__global__ void k_copy_f64(const double *__restrict__ a, double *__restrict__ b, int64_t n)
-{
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = a[i];
 }
 
 // sum of n doubles in index order by one thread (the small colloid count)
@@ -392,54 +367,51 @@ int update_list_impl(const rmpcd_box_t *box, rmpcd_cells_t *cells, const rmpcd_p
     Box b = make_box(box);
     int np = (int)points->n;
     int32_t *cnt = (int32_t *)workspace(WS_NLCNT, sizeof(int32_t) * (size_t)np * ns);
-    int32_t *flag = (int32_t *)workspace(WS_FLAG, 64);
-    int32_t *host = (int32_t *)pinned(64);
-    if (!cnt || !flag || !host) return set_error(RMPCD_ERR_HIP, "update_list: workspace allocation failed");
+    // the overflow flag, written where the host reads it: no other call uses this word, and
+    // each call of this one waits for its kernels
+    char *pin = (char *)pinned(64);
+    if (!cnt || !pin) return set_error(RMPCD_ERR_HIP, "update_list: workspace allocation failed");
     hipStream_t s = stream();
     double L0 = b.L[0] * b.a, L1 = b.L[1] * b.a, L2 = b.L[2] * b.a;  // neighbor_list.f90:92
     LJ l{};
     if (lj) l = make_lj(lj);
     k_init_cells<<<blocks_for(b.ncells, 256), 256, 0, s>>>(b.ncells, cells->is_md, cells->is_reac);
-    RMPCD_HIP(hipMemsetAsync(flag, 0, sizeof(int32_t), s));
-    dim3 grid(blocks_for(ns, NL_THREADS), np);
+    volatile int32_t *host = (int32_t *)(pin + 32);
+    *host = 0;
+    dim3 grid(blocks_for((int64_t)ns * NL_LANES, NL_THREADS), np);
     k_nl_pass<F><<<grid, NL_THREADS, 0, s>>>(b, view<F64>(points), view<F>(solvent), cells->cell_start,
                                              cells->cell_count, stencil, ns, radius * radius, L0, L1, L2,
                                              lj ? 1 : 0, l, cnt, cells->is_md, cells->is_reac, 0, nmax, list);
     RMPCD_LAUNCHED();
-    k_nl_scan<<<np, 1024, 0, s>>>(cnt, ns, nmax, n, flag);
+    k_nl_scan<<<np, 1024, 0, s>>>(cnt, ns, nmax, n, (int32_t *)(pin + 32));
     RMPCD_LAUNCHED();
     k_nl_pass<F><<<grid, NL_THREADS, 0, s>>>(b, view<F64>(points), view<F>(solvent), cells->cell_start,
                                              cells->cell_count, stencil, ns, radius * radius, L0, L1, L2,
                                              lj ? 1 : 0, l, cnt, cells->is_md, cells->is_reac, 1, nmax, list);
     RMPCD_LAUNCHED();
-    RMPCD_HIP(hipMemcpyAsync(host, flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     RMPCD_HIP(hipStreamSynchronize(s));
-    if (host[0]) return set_error(RMPCD_ERR_OVERFLOW, "maximum of neighbor list reached");
+    if (*host) return set_error(RMPCD_ERR_OVERFLOW, "maximum of neighbor list reached");
     return RMPCD_OK;
 }
 
+// the solvent's share of compute_force after the roll of the MD bits, and the colloids'
+// block partials (4 per block of 256 entries, nb blocks each)
 template <class F>
-int force_impl(rmpcd_particles_t *ps1, rmpcd_particles_t *ps2, const int32_t *list, const int32_t *nl,
-               int32_t nmax, const double *L, const rmpcd_lj_t *lj, double *e)
+int force_list(const rmpcd_particles_t *ps1, const rmpcd_particles_t *ps2, const int32_t *list, const int32_t *nl,
+               int32_t nmax, const double *L, const rmpcd_lj_t *lj, double *part)
 {
-    int np = (int)ps1->n;
-    unsigned nb = blocks_for(nmax, 256);
-    PView<F> sol = view<F>(ps2);
+    const int np = (int)ps1->n;
+    const unsigned nb = blocks_for(nmax, 256);
+    const PView<F> sol = view<F>(ps2);
     // colloids of one launch: their entries are counted in 32 bits
     const int group = np == 1 ? 1 : (int)(nmax >= (1 << 30) ? 1 : np < (1 << 30) / nmax ? np : (1 << 30) / nmax);
-    double *part = (double *)workspace(WS_PART, sizeof(double) * 4 * (size_t)nb * np);
-    double *eb = (double *)workspace(WS_RED, sizeof(double) * (np + 1));
-    double *host = (double *)pinned(64);
     uint32_t *head = nullptr, *next = nullptr;
     if (np > 1) {
         head = (uint32_t *)workspace(WS_HEAD, sizeof(uint32_t) * (size_t)sol.n);
         next = (uint32_t *)workspace(WS_AUX, sizeof(uint32_t) * (size_t)group * nmax);
     }
-    if (!part || !eb || !host || (np > 1 && (!head || !next)))
-        return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
+    if (np > 1 && (!head || !next)) return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
     hipStream_t s = stream();
-    k_roll_md<F><<<blocks_for(sol.n, 256), 256, 0, s>>>(sol.n, sol.flags);
-    RMPCD_LAUNCHED();
     const LJ l = make_lj(lj);
     for (int c0 = 0; c0 < np; c0 += group) {
         const dim3 grid(nb, group < np - c0 ? group : np - c0);
@@ -451,11 +423,48 @@ int force_impl(rmpcd_particles_t *ps1, rmpcd_particles_t *ps2, const int32_t *li
                                                  next);
         RMPCD_LAUNCHED();
     }
-    k_force_nl_sum<<<np, 64, 0, s>>>(view<F64>(ps1), part, (int)nb, eb);
+    return RMPCD_OK;
+}
+
+int energy_sum_unchecked(const double *e, int64_t n, double *out)
+{
+    k_sum_serial<<<1, 64, 0, stream()>>>(e, n, out);
     RMPCD_LAUNCHED();
-    k_sum_serial<<<1, 64, 0, s>>>(eb, np, eb + np);
+    return RMPCD_OK;
+}
+
+int force_list_unchecked(const rmpcd_particles_t *ps1, const rmpcd_particles_t *ps2, const int32_t *list,
+                         const int32_t *nl, int32_t nmax, const double *L, const rmpcd_lj_t *lj, double *part)
+{
+    return RMPCD_DISPATCH_FORM(ps2, force_list, ps1, ps2, list, nl, nmax, L, lj, part);
+}
+
+int force_sum_unchecked(const rmpcd_particles_t *ps1, const double *part, int nb, double *e_out)
+{
+    k_force_nl_sum<<<(unsigned)ps1->n, 64, 0, stream()>>>(view<F64>(ps1), part, nb, e_out);
     RMPCD_LAUNCHED();
-    RMPCD_HIP(hipMemcpyAsync(host, eb + np, sizeof(double), hipMemcpyDeviceToHost, s));
+    return RMPCD_OK;
+}
+
+template <class F>
+int force_impl(rmpcd_particles_t *ps1, rmpcd_particles_t *ps2, const int32_t *list, const int32_t *nl,
+               int32_t nmax, const double *L, const rmpcd_lj_t *lj, double *e)
+{
+    const int np = (int)ps1->n;
+    const unsigned nb = blocks_for(nmax, 256);
+    double *part = (double *)workspace(WS_PART, sizeof(double) * 4 * (size_t)nb * np);
+    double *eb = (double *)workspace(WS_RED, sizeof(double) * np);
+    double *host = (double *)pinned(64);
+    if (!part || !eb || !host) return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
+    hipStream_t s = stream();
+    const PView<F> sol = view<F>(ps2);
+    k_roll_md<F><<<blocks_for(sol.n, 256), 256, 0, s>>>(sol.n, sol.flags);
+    RMPCD_LAUNCHED();
+    int rc = force_list<F>(ps1, ps2, list, nl, nmax, L, lj, part);
+    if (rc) return rc;
+    if ((rc = force_sum_unchecked(ps1, part, (int)nb, eb))) return rc;
+    k_sum_serial<<<1, 64, 0, s>>>(eb, np, host);
+    RMPCD_LAUNCHED();
     RMPCD_HIP(hipStreamSynchronize(s));
     *e = host[0];
     return RMPCD_OK;
@@ -503,20 +512,15 @@ int rmpcd_compute_force_n2(rmpcd_particles_t *ps, const double L[3], const rmpcd
     RMPCD_CHECK(ps->form == RMPCD_FP64, "compute_force_n2: colloids must use the FP64 form");
     RMPCD_CHECK(L && lj && e, "compute_force_n2: null argument");
     int64_t n = ps->n;
-    double *fnew = (double *)workspace(WS_AUX, sizeof(double) * 3 * n);
     double *ep = (double *)workspace(WS_PART, sizeof(double) * (n + 1));
     double *host = (double *)pinned(64);
-    if (!fnew || !ep || !host) return set_error(RMPCD_ERR_HIP, "compute_force_n2: workspace allocation failed");
+    if (!ep || !host) return set_error(RMPCD_ERR_HIP, "compute_force_n2: workspace allocation failed");
     hipStream_t s = stream();
     const PView<F64> c = view<F64>(ps);
-    k_force_n2_blocks<256><<<(unsigned)n, 256, 0, s>>>(c.pos, c.species, n, c.force, L[0], L[1], L[2], make_lj(lj), fnew,
-                                                       ep);
+    k_force_n2_blocks<256><<<(unsigned)n, 256, 0, s>>>(c.pos, c.species, n, c.force, L[0], L[1], L[2], make_lj(lj), ep);
     RMPCD_LAUNCHED();
-    k_copy_f64<<<blocks_for(3 * n, 256), 256, 0, s>>>(fnew, (double *)ps->force, 3 * n);
+    k_sum_block<256><<<1, 256, 0, s>>>(ep, n, host);
     RMPCD_LAUNCHED();
-    k_sum_block<256><<<1, 256, 0, s>>>(ep, n, ep + n);
-    RMPCD_LAUNCHED();
-    RMPCD_HIP(hipMemcpyAsync(host, ep + n, sizeof(double), hipMemcpyDeviceToHost, s));
     RMPCD_HIP(hipStreamSynchronize(s));
     *e = host[0];
     return RMPCD_OK;

@@ -52,17 +52,16 @@ __device__ inline void n2_pair_sums(const double *__restrict__ pos, const int32_
 template <int T>
 __global__ void __launch_bounds__(T)
     k_force_n2_blocks(const double *__restrict__ pos, const int32_t *__restrict__ species, int64_t n,
-                      const double *__restrict__ force_in, double L0, double L1, double L2, LJ lj,
-                      double *__restrict__ fnew, double *__restrict__ e_out)
+                      double *__restrict__ force, double L0, double L1, double L2, LJ lj, double *__restrict__ e_out)
 {
     __shared__ double red[16];
     const int64_t i = blockIdx.x;
     double f0, f1, f2, e;
     n2_pair_sums<T>(pos, species, n, i, L0, L1, L2, lj, red, f0, f1, f2, e);
     if (threadIdx.x == 0) {
-        fnew[i] = force_in[i] + f0;
-        fnew[n + i] = force_in[n + i] + f1;
-        fnew[2 * n + i] = force_in[2 * n + i] + f2;
+        force[i] = force[i] + f0;
+        force[n + i] = force[n + i] + f1;
+        force[2 * n + i] = force[2 * n + i] + f2;
         e_out[i] = e;
     }
 }

@@ -20,9 +20,247 @@
 #include <new>
 #include <vector>
 
+#include "rmpcd_pairforce.hpp"
 #include "rmpcd_programs.hpp"
+#include "rmpcd_steps.hpp"
 
 namespace rmpcd {
+
+// ---- the MD steps, their passes fused ------------------------------------------------------
+// Each kernel makes the reference's passes of one region of the step in the reference's
+// order per particle.  What bounds these loops at their size (10^5 to 10^6 particles) is
+// launches and waits: one wait per step, for the displacements that decide on a sort; the
+// energies and the temperature stay on the device until a run ends.  As separate passes with
+// four waits per step a cycle of ten SPHERE steps took 0.94 ms (L = 32, FP64) and one of
+// fifty COLLOIDS steps 7.9 ms (L = 48, FP64, 52 colloids), 0.63 and 4.8 ms like this.
+constexpr unsigned STEP_BLOCKS = 1024;  // workgroups of a pass over all particles that leaves a partial each
+
+// SPHERE, before the decision: md_pos, maximum_displacement, and the solvent's force reset
+// of this step: the new force array (force_old until the switch) zeroed, the MD bits
+// rolled.  The reference makes the reset after a sort of the same step; the sort carries
+// zeros and bits along, so the state after it is the same.
+template <class F>
+__global__ void __launch_bounds__(256)
+    k_sphere_move(PView<F> p, const typename F::real *__restrict__ pos_old, double dt, double *__restrict__ part)
+{
+    using R = typename F::real;
+    __shared__ double red[16];
+    const R rdt = (R)dt, dt_sq = (R)((dt * dt) / 2);
+    double r_sq = 0;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < p.n; i += (int64_t)gridDim.x * blockDim.x) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int64_t q = k * p.n + i;
+            p.pos[q] = (p.pos[q] + rdt * p.vel[q]) + dt_sq * p.force[q];
+            p.force_old[q] = 0;
+        }
+        int f = (int)p.flags[i];
+        f = (f & MD_MASK) ? (f | PAST_MD_MASK) : (f & ~PAST_MD_MASK);
+        p.flags[i] = (typename F::small)(f & ~MD_MASK);
+        r_sq = fmax(r_sq, disp_sq<F>(p, pos_old, i));
+    }
+    const double m = block_max(r_sq, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+// SPHERE: compute_force on the list of colloid 0, and flag_particles_nl of its driver
+// (setup_single_catalytic_fixed_sphere.f90:311-329), which reads neither the velocities nor
+// the bits that md_vel writes in between
+template <class F>
+__global__ void __launch_bounds__(256)
+    k_sphere_list(PView<F64> c, PView<F> sol, const int32_t *__restrict__ list, const int32_t *__restrict__ nl,
+                  int32_t nmax, double L0, double L1, double L2, LJ lj, double prob, uint64_t seed, uint64_t step,
+                  double *__restrict__ part)
+{
+    using R = typename F::real;
+    __shared__ double red[16];
+    const int k = blockIdx.x * blockDim.x + threadIdx.x;
+    const int n = min(nl[0], nmax);
+    double f[3] = {0, 0, 0}, e = 0;
+    if (k < n) {
+        const int idx = list[k];
+        int fl = (int)sol.flags[idx];
+        const int old = fl;
+        if (pair_force<F>(c, sol, 0, idx, L0, L1, L2, lj, f, &e)) {
+            for (int q = 0; q < 3; ++q) sol.force[q * sol.n + idx] = sol.force[q * sol.n + idx] - (R)f[q];
+            fl |= MD_MASK | (c.species[0] == 1 ? CATALYZED_MASK : 0);
+        }
+        if ((int)sol.species[idx] == 1) {
+            const double d0 = min_image(c.pos[0] - (double)sol.pos[idx], L0);
+            const double d1 = min_image(c.pos[c.n] - (double)sol.pos[sol.n + idx], L1);
+            const double d2 = min_image(c.pos[2 * c.n] - (double)sol.pos[2 * sol.n + idx], L2);
+            if ((d0 * d0 + d1 * d1) + d2 * d2 < lj.cut_sq[0]) {
+                uint64_t a, b;
+                threefry2x64(step, (uint64_t)sol.id[idx], seed, STREAM_CHANGE, a, b);
+                if (u01(a) <= prob) fl |= REAC_MASK;
+            }
+        }
+        if (fl != old) sol.flags[idx] = (typename F::small)fl;
+    }
+    double *pp = part + 4 * (int64_t)blockIdx.x;
+    if ((int)(blockIdx.x * blockDim.x) >= n) {
+        if (threadIdx.x < 4) pp[threadIdx.x] = 0;
+        return;
+    }
+    const double b0 = block_sum(f[0], red), b1 = block_sum(f[1], red), b2 = block_sum(f[2], red),
+                 be = block_sum(e, red);
+    if (threadIdx.x == 0) {
+        pp[0] = b0;
+        pp[1] = b1;
+        pp[2] = b2;
+        pp[3] = be;
+    }
+}
+
+// SPHERE, the end of the step: md_vel (md.f90:219-237) and change_species
+// (setup_single_catalytic_fixed_sphere.f90:331-349)
+template <class F>
+__global__ void __launch_bounds__(256)
+    k_sphere_finish(PView<F> p, PView<F64> c, double dt, double L0, double L1, double L2, double cut_sq_c)
+{
+    using R = typename F::real;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= p.n) return;
+    const int old = (int)p.flags[i];
+    int f = old;
+    if (!(f & WALL_MASK)) {
+        const R rdt = (R)dt;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int64_t q = k * p.n + i;
+            p.vel[q] = p.vel[q] + (rdt * (p.force[q] + p.force_old[q])) / (R)2;
+        }
+    } else {
+        f &= ~WALL_MASK;
+    }
+    if (f & REAC_MASK) {
+        const double a0 = min_image(c.pos[0] - (double)p.pos[i], L0);
+        const double a1 = min_image(c.pos[c.n] - (double)p.pos[p.n + i], L1);
+        const double a2 = min_image(c.pos[2 * c.n] - (double)p.pos[2 * p.n + i], L2);
+        if ((a0 * a0 + a1 * a1) + a2 * a2 > cut_sq_c) {
+            p.species[i] = (typename F::small)2;
+            f &= ~REAC_MASK;
+        }
+    }
+    if (f != old) p.flags[i] = (typename F::small)f;
+}
+
+// COLLOIDS: cell_md_pos with md_flag true and cell_maximum_displacement over the same cells
+template <class F>
+__global__ void __launch_bounds__(256)
+    k_cells_move(int ncells, const int32_t *__restrict__ start, const int32_t *__restrict__ count,
+                 const uint8_t *__restrict__ is_md, PView<F> p, const typename F::real *__restrict__ pos_old, double dt,
+                 double *__restrict__ part)
+{
+    using R = typename F::real;
+    __shared__ double red[16];
+    const R rdt = (R)dt, dt_sq = (R)((dt * dt) / 2);
+    double r_sq = 0;
+    for_md_cells(ncells, start, count, is_md, 1, [&](int64_t j) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int64_t q = k * p.n + j;
+            p.pos[q] = (p.pos[q] + rdt * p.vel[q]) + dt_sq * p.force[q];
+        }
+        r_sq = fmax(r_sq, disp_sq<F>(p, pos_old, j));
+    });
+    const double m = block_max(r_sq, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+// COLLOIDS: the colloids' Verlet position and their displacement
+__global__ void __launch_bounds__(256)
+    k_colloids_move(PView<F64> c, const double *__restrict__ mass, const double *__restrict__ pos_old, double dt,
+                    double *__restrict__ part)
+{
+    __shared__ double red[16];
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    double r_sq = 0;
+    if (i < c.n) {
+        for (int k = 0; k < 3; ++k) {
+            const int64_t q = k * c.n + i;
+            c.pos[q] = (c.pos[q] + dt * c.vel[q]) + ((dt * dt) * c.force[q]) / (2 * mass[i]);
+        }
+        r_sq = disp_sq<F64>(c, pos_old, i);
+    }
+    const double m = block_max(r_sq, red);
+    if (threadIdx.x == 0) part[blockIdx.x] = m;
+}
+
+// the solvent's force reset of a step: zeroed, the MD bits rolled (neighbor_list.f90:180-188)
+template <class F>
+__global__ void __launch_bounds__(256) k_force_reset(PView<F> p)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= p.n) return;
+    for (int k = 0; k < 3; ++k) p.force[k * p.n + i] = 0;
+    int f = (int)p.flags[i];
+    f = (f & MD_MASK) ? (f | PAST_MD_MASK) : (f & ~PAST_MD_MASK);
+    p.flags[i] = (typename F::small)(f & ~MD_MASK);
+}
+
+// COLLOIDS, one workgroup per colloid: its list partials, compute_force_n2 and its Verlet
+// velocity
+template <int T>
+__global__ void __launch_bounds__(T)
+    k_colloids_finish(PView<F64> c, const double *__restrict__ mass, const double *__restrict__ part, int nb, double L0,
+                      double L1, double L2, LJ lj, double dt, double *__restrict__ e1, double *__restrict__ e2)
+{
+    __shared__ double red[16], sum[4];
+    const int64_t i = blockIdx.x;
+    const double a = list_force_sum(part, nb, i);
+    if (threadIdx.x < 4) sum[threadIdx.x] = a;
+    double f[3], e;
+    n2_pair_sums<T>(c.pos, c.species, c.n, i, L0, L1, L2, lj, red, f[0], f[1], f[2], e);
+    if (threadIdx.x < 3) {
+        const int64_t q = threadIdx.x * c.n + i;
+        const double s = threadIdx.x == 0 ? f[0] : threadIdx.x == 1 ? f[1] : f[2];
+        const double fn = (0.0 + a) + s;
+        c.force[q] = fn;
+        c.vel[q] = c.vel[q] + (dt * (fn + c.force_old[q])) / (2 * mass[i]);
+    }
+    if (threadIdx.x == 0) {
+        e1[i] = sum[3];
+        e2[i] = e;
+    }
+}
+
+// sqrt of the maxima of a step's displacement partials: the one wait of an MD step
+static int fetch_max2(const double *part, int64_t n, const double *part2, int64_t n2, double *r, double *r2)
+{
+    double *host = (double *)pinned(64);
+    if (!host) return set_error(RMPCD_ERR_HIP, "program: pinned staging allocation failed");
+    k_max_final<1024><<<part2 ? 2 : 1, 1024, 0, stream()>>>(part, n, host, part2, n2);
+    RMPCD_LAUNCHED();
+    RMPCD_HIP(hipStreamSynchronize(stream()));
+    *r = sqrt(host[0]);
+    if (r2) *r2 = sqrt(host[1]);
+    return RMPCD_OK;
+}
+
+int ProgramSim::fetch_scalars()
+{
+    double *host = (double *)pinned(64);
+    if (!host) return set_error(RMPCD_ERR_HIP, "program: pinned staging allocation failed");
+    hipStream_t st = stream();
+    int rc;
+    if (have_e) {
+        if ((rc = energy_sum_unchecked(dev_e1, nc, host))) return rc;
+        if (cfg.kind == RMPCD_PROG_COLLOIDS) {
+            k_sum_block<256><<<1, 256, 0, st>>>(dev_e2, nc, host + 1);
+            RMPCD_LAUNCHED();
+        }
+    }
+    if (have_te) RMPCD_HIP(hipMemcpyAsync(host + 2, dev_te, sizeof(double), hipMemcpyDeviceToHost, st));
+    RMPCD_HIP(hipStreamSynchronize(st));
+    if (have_e) {
+        e1 = host[0];
+        if (cfg.kind == RMPCD_PROG_COLLOIDS) e2 = host[1];
+    }
+    if (have_te) temperature = host[2];
+    have_e = have_te = false;
+    return RMPCD_OK;
+}
 
 int ProgramSim::setup(const rmpcd_program_config_t &c)
 {
@@ -91,6 +329,7 @@ int ProgramSim::setup(const rmpcd_program_config_t &c)
     if ((rc = alloc((void **)&is_md, box.ncells))) return rc;
     if ((rc = alloc((void **)&is_reac, box.ncells))) return rc;
     if ((rc = alloc((void **)&scratch, 1 << 16))) return rc;
+    dev_te = scratch + 64;
     if (nc) {
         size_t c3 = 3 * (size_t)nc * sizeof(double);
         if ((rc = alloc((void **)&col_pos, c3))) return rc;
@@ -105,6 +344,8 @@ int ProgramSim::setup(const rmpcd_program_config_t &c)
         if ((rc = alloc((void **)&col_mass, (size_t)nc * 8))) return rc;
         if ((rc = alloc((void **)&list, (size_t)nc * nmax * 4))) return rc;
         if ((rc = alloc((void **)&nlist, (size_t)nc * 4))) return rc;
+        if ((rc = alloc((void **)&dev_e1, (size_t)nc * 8))) return rc;
+        if ((rc = alloc((void **)&dev_e2, (size_t)nc * 8))) return rc;
         n_stencil = rmpcd_make_stencil(1.0, radius, nullptr, 0);
         std::vector<int32_t> st(3 * (size_t)n_stencil);
         rmpcd_make_stencil(1.0, radius, st.data(), n_stencil);
@@ -251,29 +492,47 @@ int ProgramSim::fluid_cycle()
 }
 
 // SPHERE MD step (setup_single_catalytic_fixed_sphere.f90:190-228)
+template <class F>
+static int sphere_step_t(ProgramSim &m)
+{
+    hipStream_t st = stream();
+    rmpcd_particles_t s = m.sv();
+    const unsigned nb = blocks_for(m.n, 256) < STEP_BLOCKS ? blocks_for(m.n, 256) : STEP_BLOCKS;
+    const unsigned lb = blocks_for(m.nmax, 256);
+    double *part = (double *)workspace(WS_PART, sizeof(double) * (4 * (size_t)lb > nb ? 4 * (size_t)lb : nb));
+    if (!part) return set_error(RMPCD_ERR_HIP, "program: workspace allocation failed");
+    k_sphere_move<F><<<nb, 256, 0, st>>>(view<F>(&s), (const typename F::real *)m.alt().pos, m.dt, part);
+    RMPCD_LAUNCHED();
+    int rc;
+    double so_max;
+    if ((rc = fetch_max2(part, nb, nullptr, 0, &so_max, nullptr))) return rc;
+    if (so_max >= m.skin) {
+        if ((rc = m.sort(true))) return rc;  // apply_pbc, sort
+        if ((rc = m.build_list())) return rc;
+        if ((rc = m.copy_pos_old())) return rc;
+        ++m.n_extra;
+    }
+    // switch(force, force_old) for both; the driver zeroes the solvent forces only
+    m.fpar = 1 - m.fpar;
+    m.cfpar = 1 - m.cfpar;
+    s = m.sv();
+    rmpcd_particles_t p = m.cv();
+    const double *L = m.box.edges;
+    k_sphere_list<F><<<lb, 256, 0, st>>>(view<F64>(&p), view<F>(&s), m.list, m.nlist, m.nmax, L[0], L[1], L[2],
+                                         make_lj(&m.lj_sc), m.cfg.prob, m.seed, (uint64_t)m.md_steps, part);
+    RMPCD_LAUNCHED();
+    if ((rc = force_sum_unchecked(&p, part, (int)lb, m.dev_e1))) return rc;
+    m.have_e = true;
+    k_sphere_finish<F><<<blocks_for(m.n, 256), 256, 0, st>>>(view<F>(&s), view<F64>(&p), m.dt, L[0], L[1], L[2],
+                                                             m.lj_sc.cut_sq[0]);
+    RMPCD_LAUNCHED();
+    ++m.md_steps;
+    return RMPCD_OK;
+}
+
 int ProgramSim::sphere_step()
 {
-    rmpcd_particles_t s = sv();
-    int rc = rmpcd_md_pos(&s, dt);
-    if (rc) return rc;
-    double so_max;
-    if ((rc = rmpcd_maximum_displacement(&s, alt().pos, &so_max))) return rc;
-    if (so_max >= skin) {
-        if ((rc = sort(true))) return rc;  // apply_pbc, sort
-        if ((rc = build_list())) return rc;
-        if ((rc = copy_pos_old())) return rc;
-        ++n_extra;
-    }
-    if ((rc = forces(false))) return rc;  // the driver zeroes the solvent forces only
-    s = sv();
-    rmpcd_particles_t p = cv();
-    if ((rc = rmpcd_md_vel(&s, dt))) return rc;
-    if ((rc = rmpcd_flag_particles_nl_prob(&s, &p, list, nlist, nmax, box.edges, lj_sc.cut_sq[0], cfg.prob,
-                                           nullptr, seed, (uint64_t)md_steps)))
-        return rc;
-    if ((rc = rmpcd_change_species_sphere(&s, &p, box.edges, lj_sc.cut_sq[0]))) return rc;
-    ++md_steps;
-    return RMPCD_OK;
+    return cfg.form == RMPCD_FP64 ? sphere_step_t<F64>(*this) : sphere_step_t<F32>(*this);
 }
 
 // SPHERE collision (:230-253): temperature, grid shift, sort without apply_pbc, list,
@@ -282,8 +541,9 @@ int ProgramSim::sphere_collide()
 {
     rmpcd_particles_t s = sv();
     rmpcd_cells_t c = cells();
-    int rc = rmpcd_compute_temperature(&box, &c, &s, &temperature);
+    int rc = temperature_unchecked(&box, &c, &s, dev_te);
     if (rc) return rc;
+    have_te = true;
     if ((rc = shift((uint64_t)cycles))) return rc;
     if ((rc = sort(false))) return rc;
     if ((rc = build_list())) return rc;
@@ -297,34 +557,59 @@ int ProgramSim::sphere_collide()
 
 // COLLOIDS MD step (n_colloids_pbc.f90:288-320): lazy streaming of the cells holding
 // list particles; the others catch up (cell_md_pos/vel with md_flag false) at a sort
+template <class F>
+static int colloids_step_t(ProgramSim &m)
+{
+    hipStream_t st = stream();
+    rmpcd_particles_t s = m.sv(), p = m.cv();
+    rmpcd_cells_t c = m.cells();
+    const unsigned nb = cell_blocks(m.box.ncells), cb = blocks_for(m.nc, 256), lb = blocks_for(m.nmax, 256);
+    const size_t moves = (size_t)nb + cb, lists = 4 * (size_t)lb * m.nc;
+    double *part = (double *)workspace(WS_PART, sizeof(double) * (moves > lists ? moves : lists));
+    if (!part) return set_error(RMPCD_ERR_HIP, "program: workspace allocation failed");
+    k_cells_move<F><<<nb, 256, 0, st>>>(m.box.ncells, c.cell_start, c.cell_count, c.is_md, view<F>(&s),
+                                        (const typename F::real *)m.alt().pos, m.dt, part);
+    RMPCD_LAUNCHED();
+    k_colloids_move<<<cb, 256, 0, st>>>(view<F64>(&p), m.col_mass, m.col_pos_old, m.dt, part + nb);
+    RMPCD_LAUNCHED();
+    const double k1 = (double)(m.md_steps + 1 - m.last_sort);
+    int rc;
+    double so_max, co_max;
+    if ((rc = fetch_max2(part, nb, part + nb, cb, &so_max, &co_max))) return rc;
+    // cell_maximum_displacement is at least max_v dt (particle_system.f90:408)
+    const double bound = m.box.max_v * (m.dt * k1);
+    if (bound > so_max) so_max = bound;
+    if (co_max >= m.skin * 0.1 || so_max >= m.skin * 0.9) {
+        if ((rc = rmpcd_cell_md_pos(&m.box, &c, &s, k1 * m.dt, 0))) return rc;
+        if ((rc = rmpcd_cell_md_vel(&m.box, &c, &s, k1 * m.dt, 0))) return rc;
+        if ((rc = rmpcd_apply_pbc(&p, m.box.edges))) return rc;
+        if ((rc = m.sort(true))) return rc;
+        m.last_sort = m.md_steps + 1;
+        if ((rc = m.build_list())) return rc;
+        if ((rc = m.copy_pos_old())) return rc;
+        ++m.n_extra;
+    }
+    // switch(force, force_old) for both systems, then the new forces from zero
+    m.fpar = 1 - m.fpar;
+    m.cfpar = 1 - m.cfpar;
+    s = m.sv();
+    p = m.cv();
+    const double *L = m.box.edges;
+    k_force_reset<F><<<blocks_for(m.n, 256), 256, 0, st>>>(view<F>(&s));
+    RMPCD_LAUNCHED();
+    if ((rc = force_list_unchecked(&p, &s, m.list, m.nlist, m.nmax, L, &m.lj_sc, part))) return rc;
+    k_colloids_finish<256><<<(unsigned)m.nc, 256, 0, st>>>(view<F64>(&p), m.col_mass, part, (int)lb, L[0], L[1], L[2],
+                                                           make_lj(&m.lj_cc), m.dt, m.dev_e1, m.dev_e2);
+    RMPCD_LAUNCHED();
+    m.have_e = true;
+    if ((rc = rmpcd_cell_md_vel(&m.box, &c, &s, m.dt, 1))) return rc;
+    ++m.md_steps;
+    return RMPCD_OK;
+}
+
 int ProgramSim::colloids_step()
 {
-    rmpcd_particles_t s = sv(), p = cv();
-    rmpcd_cells_t c = cells();
-    int rc = rmpcd_cell_md_pos(&box, &c, &s, dt, 1);
-    if (rc) return rc;
-    if ((rc = rmpcd_colloid_md_pos(&p, col_mass, dt))) return rc;
-    double k1 = (double)(md_steps + 1 - last_sort);
-    double so_max, co_max;
-    if ((rc = rmpcd_cell_maximum_displacement(&box, &c, &s, alt().pos, dt * k1, &so_max))) return rc;
-    if ((rc = rmpcd_maximum_displacement(&p, col_pos_old, &co_max))) return rc;
-    if (co_max >= skin * 0.1 || so_max >= skin * 0.9) {
-        if ((rc = rmpcd_cell_md_pos(&box, &c, &s, k1 * dt, 0))) return rc;
-        if ((rc = rmpcd_cell_md_vel(&box, &c, &s, k1 * dt, 0))) return rc;
-        if ((rc = rmpcd_apply_pbc(&p, box.edges))) return rc;
-        if ((rc = sort(true))) return rc;
-        last_sort = md_steps + 1;
-        if ((rc = build_list())) return rc;
-        if ((rc = copy_pos_old())) return rc;
-        ++n_extra;
-    }
-    if ((rc = forces(true))) return rc;
-    s = sv();
-    p = cv();
-    if ((rc = rmpcd_cell_md_vel(&box, &c, &s, dt, 1))) return rc;
-    if ((rc = rmpcd_colloid_md_vel(&p, col_mass, dt))) return rc;
-    ++md_steps;
-    return RMPCD_OK;
+    return cfg.form == RMPCD_FP64 ? colloids_step_t<F64>(*this) : colloids_step_t<F32>(*this);
 }
 
 // COLLOIDS collision (:322-344)
@@ -358,7 +643,8 @@ int ProgramSim::colloids_collide()
                                           T, cfg.hydro)))
             return rc;
     }
-    if ((rc = rmpcd_compute_temperature(&box, &c, &s, &temperature))) return rc;
+    if ((rc = temperature_unchecked(&box, &c, &s, dev_te))) return rc;
+    have_te = true;
     ++cycles;
     return RMPCD_OK;
 }
@@ -366,6 +652,16 @@ int ProgramSim::colloids_collide()
 int ProgramSim::run(int n_cycles)
 {
     if (cfg.kind == RMPCD_PROG_COLLOIDS && cfg.graph) return colloids_graph_run(*this, n_cycles);
+    const int rc = run_cycles(n_cycles);
+    // a run that stopped at a failed list build leaves the scalars of the steps before it
+    const int rf = (have_e || have_te) && rc != RMPCD_ERR_HIP ? fetch_scalars() : RMPCD_OK;
+    if (rc || rf) return rc ? rc : rf;
+    RMPCD_HIP(hipStreamSynchronize(stream()));
+    return RMPCD_OK;
+}
+
+int ProgramSim::run_cycles(int n_cycles)
+{
     int rc;
     for (int cy = 0; cy < n_cycles; ++cy) {
         switch (cfg.kind) {
@@ -383,7 +679,6 @@ int ProgramSim::run(int n_cycles)
             if ((rc = colloids_collide())) return rc;
         }
     }
-    RMPCD_HIP(hipStreamSynchronize(stream()));
     return RMPCD_OK;
 }
 

@@ -134,19 +134,11 @@ struct ProgramSim {
         if (nc) RMPCD_HIP(hipMemcpyAsync(col_pos_old, col_pos, 3 * nc * sizeof(double), hipMemcpyDeviceToDevice, st));
         return RMPCD_OK;
     }
-    int forces(bool zero_colloid)
-    {
-        hipStream_t st = stream();
-        // switch(force, force_old) for both systems, then zero the new forces
-        fpar = 1 - fpar;
-        cfpar = 1 - cfpar;
-        rmpcd_particles_t s = sv(), p = cv();
-        RMPCD_HIP(hipMemsetAsync(s.force, 0, 3 * n * rsize(cfg.form), st));
-        if (zero_colloid) RMPCD_HIP(hipMemsetAsync(p.force, 0, 3 * nc * sizeof(double), st));
-        int rc = rmpcd_compute_force(&p, &s, list, nlist, nmax, box.edges, &lj_sc, &e1);
-        if (!rc && cfg.kind == RMPCD_PROG_COLLOIDS) rc = rmpcd_compute_force_n2(&p, box.edges, &lj_cc, &e2);
-        return rc;
-    }
+    // the scalars of the last step and collision, read back at the end of a run: e1 (as one
+    // value or per colloid), e2 per colloid, the temperature
+    double *dev_e1 = nullptr, *dev_e2 = nullptr, *dev_te = nullptr;
+    bool have_e = false, have_te = false;
+    int fetch_scalars();
     int shift(uint64_t s)
     {
         double u[3];
@@ -160,6 +152,7 @@ struct ProgramSim {
     int colloids_step();
     int colloids_collide();
     int run(int n_cycles);
+    int run_cycles(int n_cycles);
 };
 
 }  // namespace rmpcd
