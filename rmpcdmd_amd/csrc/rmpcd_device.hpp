@@ -172,12 +172,21 @@ __host__ __device__ inline void compact_point(int h, int M0, int M1, int M2, int
 // ---------------------------------------------------------------------------------
 // cell of a position: floor(x/a - origin), wrapping p == L to 0 (z only without walls)
 // (src/cell_system.f90:165-175).  Computed in the precision of the position.
+// With unit cells, what every program of the reference uses, x / a is x and the three
+// divisions are left out.
+__device__ inline float floor_r(float x) { return floorf(x); }
+__device__ inline double floor_r(double x) { return floor(x); }
 template <class R>
 __device__ inline void cell_of(const Box &b, R x, R y, R z, int &p0, int &p1, int &p2)
 {
-    p0 = (int)floor((double)((R)(x / (R)b.a) - (R)b.origin[0]));
-    p1 = (int)floor((double)((R)(y / (R)b.a) - (R)b.origin[1]));
-    p2 = (int)floor((double)((R)(z / (R)b.a) - (R)b.origin[2]));
+    if (b.a != 1.0) {
+        x = x / (R)b.a;
+        y = y / (R)b.a;
+        z = z / (R)b.a;
+    }
+    p0 = (int)floor_r(x - (R)b.origin[0]);
+    p1 = (int)floor_r(y - (R)b.origin[1]);
+    p2 = (int)floor_r(z - (R)b.origin[2]);
     if (p0 == b.L[0]) p0 = 0;
     if (p1 == b.L[1]) p1 = 0;
     if (!b.has_walls && p2 == b.L[2]) p2 = 0;
@@ -189,6 +198,18 @@ __host__ __device__ inline double min_image(double r, double L)
     if (r < -0.5 * L) return r + L;
     if (r > 0.5 * L) return r - L;
     return r;
+}
+
+// x folded into [0, e) by its image floor(x / e) (md.f90:209-214); returns the image.  For
+// 0 <= x < e the rounded quotient lies in [0, 1), so the image is 0 and x stays as it is:
+// the division is made for the others only (whole waves pass by it away from the faces).
+template <class R>
+__device__ inline int fold_pbc(R &x, R e)
+{
+    if (x >= (R)0 && x < e) return 0;
+    const int jump = (int)floor_r(x / e);
+    x = x - (R)jump * e;
+    return jump;
 }
 
 // ---------------------------------------------------------------------------------
@@ -346,47 +367,94 @@ struct Acc3 {
 // smallest in magnitude, so the cell's momentum is kept to the rounding of that one
 // addition.  FP64 is left as the reference computes it.
 template <class R>
-__device__ inline void srd_rotate(R *vx, R *vy, R *vz, int m, const R *o, R u0, R u1, R u2, const Acc3<R> &old,
-                                  bool conserve)
+__device__ inline void srd_rotate_one(R v[3], const R *o, R u0, R u1, R u2)
 {
+    const R w0 = v[0] - u0, w1 = v[1] - u1, w2 = v[2] - u2;
+    R r0 = o[0] * w0;
+    r0 = r0 + o[1] * w1;
+    r0 = r0 + o[2] * w2;
+    R r1 = o[3] * w0;
+    r1 = r1 + o[4] * w1;
+    r1 = r1 + o[5] * w2;
+    R r2 = o[6] * w0;
+    r2 = r2 + o[7] * w1;
+    r2 = r2 + o[8] * w2;
+    v[0] = u0 + r0;
+    v[1] = u1 + r1;
+    v[2] = u2 + r2;
+}
+
+// the sums and smallest components of new velocities, and the compensation of a cell
+template <class R>
+struct SrdNew {
     Acc3<R> nw;
     int jmin[3] = {0, 0, 0};
     R amin[3] = {INFINITY, INFINITY, INFINITY};
-    for (int i = 0; i < m; ++i) {
-        const R w0 = vx[i] - u0, w1 = vy[i] - u1, w2 = vz[i] - u2;
-        R r0 = o[0] * w0;
-        r0 = r0 + o[1] * w1;
-        r0 = r0 + o[2] * w2;
-        R r1 = o[3] * w0;
-        r1 = r1 + o[4] * w1;
-        r1 = r1 + o[5] * w2;
-        R r2 = o[6] * w0;
-        r2 = r2 + o[7] * w1;
-        r2 = r2 + o[8] * w2;
-        const R n3[3] = {u0 + r0, u1 + r1, u2 + r2};
-        vx[i] = n3[0];
-        vy[i] = n3[1];
-        vz[i] = n3[2];
-        if constexpr (sizeof(R) == 4) {
-            for (int k = 0; k < 3; ++k) {
-                nw.add(k, n3[k]);
-                const R a = fabsf(n3[k]);
-                if (a < amin[k]) {
-                    amin[k] = a;
-                    jmin[k] = i;
-                }
+    __device__ inline void add(const R v[3], int i)
+    {
+        for (int k = 0; k < 3; ++k) {
+            nw.add(k, v[k]);
+            const R a = fabsf(v[k]);
+            if (a < amin[k]) {
+                amin[k] = a;
+                jmin[k] = i;
             }
         }
+    }
+    __device__ inline void fix(R *vx, R *vy, R *vz, const Acc3<R> &old) const
+    {
+        R *vk[3] = {vx, vy, vz};
+        for (int k = 0; k < 3; ++k) {
+            const R d = (old.s[k] - nw.s[k]) + (old.c[k] - nw.c[k]);
+            vk[k][jmin[k]] = vk[k][jmin[k]] + d;
+        }
+    }
+};
+
+// the compensation of a cell whose m velocities are already rotated
+template <class R>
+__device__ inline void srd_conserve(R *vx, R *vy, R *vz, int m, const Acc3<R> &old)
+{
+    SrdNew<R> nw;
+    for (int i = 0; i < m; ++i) {
+        const R v[3] = {vx[i], vy[i], vz[i]};
+        nw.add(v, i);
+    }
+    nw.fix(vx, vy, vz, old);
+}
+
+template <class R>
+__device__ inline void srd_rotate(R *vx, R *vy, R *vz, int m, const R *o, R u0, R u1, R u2, const Acc3<R> &old,
+                                  bool conserve)
+{
+    SrdNew<R> nw;
+    for (int i = 0; i < m; ++i) {
+        R v[3] = {vx[i], vy[i], vz[i]};
+        srd_rotate_one(v, o, u0, u1, u2);
+        vx[i] = v[0];
+        vy[i] = v[1];
+        vz[i] = v[2];
+        if constexpr (sizeof(R) == 4) nw.add(v, i);
     }
     if constexpr (sizeof(R) == 4) {
-        if (conserve) {
-            R *vk[3] = {vx, vy, vz};
-            for (int k = 0; k < 3; ++k) {
-                const R d = (old.s[k] - nw.s[k]) + (old.c[k] - nw.c[k]);
-                vk[k][jmin[k]] = vk[k][jmin[k]] + d;
-            }
-        }
+        if (conserve) nw.fix(vx, vy, vz, old);
     }
+}
+
+// omega(r,k) about the axis v as filled column-major by mpcd.f90:163-171
+template <class R>
+__device__ inline void srd_matrix(double v0, double v1, double v2, double sin_a, double cos_a, R o[9])
+{
+    const double omc = 1 - cos_a;
+    o[0] = (R)(cos_a + (v0 * v0) * omc);
+    o[1] = (R)((v1 * v0) * omc + v2 * sin_a);
+    o[2] = (R)((v2 * v0) * omc - v1 * sin_a);
+    o[3] = (R)((v0 * v1) * omc - v2 * sin_a);
+    o[4] = (R)(cos_a + (v1 * v1) * omc);
+    o[5] = (R)((v2 * v1) * omc + v0 * sin_a);
+    o[6] = (R)((v0 * v2) * omc + v1 * sin_a);
+    o[7] = (R)((v1 * v2) * omc - v0 * sin_a);
+    o[8] = (R)(cos_a + (v2 * v2) * omc);
 }
 
 // SRD rotation (mpcd.f90:120-180, default or given alpha); axes injected per cell or
@@ -419,11 +487,8 @@ __device__ inline void srd_cell(R *vx, R *vy, R *vz, const S *sp, int n, int c, 
         v1 = sph.n[1];
         v2 = sph.n[2];
     }
-    const double omc = 1 - cos_a;
-    // omega(r,k) as filled column-major by mpcd.f90:163-171
-    const R o[9] = {(R)(cos_a + (v0 * v0) * omc), (R)((v1 * v0) * omc + v2 * sin_a), (R)((v2 * v0) * omc - v1 * sin_a),
-                    (R)((v0 * v1) * omc - v2 * sin_a), (R)(cos_a + (v1 * v1) * omc), (R)((v2 * v1) * omc + v0 * sin_a),
-                    (R)((v0 * v2) * omc + v1 * sin_a), (R)((v1 * v2) * omc - v0 * sin_a), (R)(cos_a + (v2 * v2) * omc)};
+    R o[9];
+    srd_matrix(v0, v1, v2, sin_a, cos_a, o);
     srd_rotate(vx, vy, vz, n, o, u0, u1, u2, acc, n_eff == n);
 }
 

@@ -72,6 +72,11 @@ int check_box(const rmpcd_box_t *b, const char *who);
 int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
                    rmpcd_cells_t *cells, int wrap);
 
+// a plain fluid's cycle on checked sets whose forces are zero: SRD on the cells of the last
+// sort, n_md streaming steps, then the sort under the next grid shift
+int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
+                          rmpcd_cells_t *cells, uint64_t seed, uint64_t step, int n_md, double dt);
+
 // the parts of compute_force after the roll of the MD bits, on checked sets: the solvent's
 // forces and the colloids' block partials (4 doubles per block of 256 entries), the
 // partials' sums added to the colloid forces, the energies' sum in colloid order

@@ -51,10 +51,13 @@ __global__ void k_apply_pbc(int64_t n, typename F::real *__restrict__ pos, int32
     double e[3] = {e0, e1, e2};
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        R x = pos[k * n + i], ed = (R)e[k];
-        int jump = (int)floor((double)(x / ed));
-        image[k * n + i] += jump;
-        pos[k * n + i] = x - (R)jump * ed;
+        // a particle inside the box is not written: most of them, and 12 to 24 B each
+        R x = pos[k * n + i];
+        const int jump = fold_pbc<R>(x, (R)e[k]);
+        if (jump != 0) {
+            image[k * n + i] += jump;
+            pos[k * n + i] = x;
+        }
     }
 }
 

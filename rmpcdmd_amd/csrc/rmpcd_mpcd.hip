@@ -755,10 +755,9 @@ __global__ void k_stream_periodic(Box b, PView<F> p, double dt)
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         R x = p.pos[k * p.n + i] + p.vel[k * p.n + i] * (R)dt;
-        R e = (R)b.edges[k];
-        int jump = (int)floor((double)(x / e));
-        p.image[k * p.n + i] += jump;
-        p.pos[k * p.n + i] = x - (R)jump * e;
+        const int jump = fold_pbc<R>(x, (R)b.edges[k]);
+        if (jump != 0) p.image[k * p.n + i] += jump;
+        p.pos[k * p.n + i] = x;
     }
 }
 

@@ -478,14 +478,12 @@ int ProgramSim::init_solvent()
 // sort, streaming, the next grid shift, sort
 int ProgramSim::fluid_cycle()
 {
-    rmpcd_particles_t s = sv();
+    rmpcd_particles_t s = sv(), d = alt();
     rmpcd_cells_t c = cells();
-    int rc = rmpcd_simple_mpcd_step(&box, &c, &s, nullptr, seed, (uint64_t)cycles, 0, 0.0, 0, cfg.T, 1);
+    int rc = shift((uint64_t)cycles + 1);
     if (rc) return rc;
-    for (int k = 0; k < cfg.n_md; ++k)
-        if ((rc = rmpcd_mpcd_stream_periodic(&box, &s, dt))) return rc;
-    if ((rc = shift((uint64_t)cycles + 1))) return rc;
-    if ((rc = sort(false))) return rc;
+    if ((rc = fluid_cycle_unchecked(&box, &s, &d, &c, seed, (uint64_t)cycles, cfg.n_md, dt))) return rc;
+    cur = 1 - cur;
     md_steps += cfg.n_md;
     ++cycles;
     return RMPCD_OK;

@@ -16,19 +16,11 @@
 // result equals the reference's single-thread order, where each cell keeps increasing
 // original index.
 #include "rmpcd_internal.hpp"
+#include "rmpcd_srdtile.hpp"
 
 namespace rmpcd {
 
-// cell key of a position given in the particle's precision; the periodic wrap of
-// apply_pbc (md.f90:209-214) is applied first when wrap != 0
-template <class R>
-__device__ inline void wrap_pbc(const Box &b, R &x, int &jump, int k)
-{
-    R e = (R)b.edges[k];
-    jump = (int)floor((double)(x / e));
-    x = x - (R)jump * e;
-}
-
+// cell key of a position given in the particle's precision
 template <class R>
 __device__ inline int key_of(const Box &b, const int32_t *lut, R x, R y, R z)
 {
@@ -174,19 +166,51 @@ static int count_stride(int nt)
     return s;
 }
 
-// cell key and place in the tile's list of every particle.  A thread's positions are
-// loaded before anything is done with them; each particle then takes a place among its
-// tile's of this chunk from an LDS hash, and one global atomic per (chunk, tile) turns
-// these into places in the tile's list, so a run of consecutive particles of one tile
-// stays together there.  21 million particles FP32: 0.15 ms, 0.77 ms with an atomic per
-// particle on its cell.
+// Places in the tiles' lists for up to three quarters as many particles as the hash has
+// entries: each particle takes a place among its tile's of this workgroup from the LDS hash, and one
+// global atomic per tile met turns these into places in the tile's list, so a run of
+// consecutive particles of one tile stays together there.  All threads call clear, a
+// barrier, put per particle, a barrier, commit, a barrier; then place(at, in).
+template <int BITS>
+struct TileHash {
+    int key[1 << BITS], cnt[1 << BITS];
+    __device__ inline void clear()
+    {
+        for (int h = threadIdx.x; h < (1 << BITS); h += SORT_T) {
+            key[h] = -1;
+            cnt[h] = 0;
+        }
+    }
+    __device__ inline void put(int t, int &at, int &in)
+    {
+        unsigned h = ((unsigned)t * 2654435769u) >> (32 - BITS);
+        for (;;) {  // a quarter of the entries at least stays free
+            int q = key[h];
+            if (q == -1) q = atomicCAS(&key[h], -1, t);
+            if (q == t || q == -1) break;
+            h = (h + 1) & ((1 << BITS) - 1);
+        }
+        at = (int)h;
+        in = atomicAdd(&cnt[h], 1);
+    }
+    __device__ inline void commit(int32_t *__restrict__ tile_count, int stride)
+    {
+        for (int h = threadIdx.x; h < (1 << BITS); h += SORT_T)
+            if (cnt[h] > 0) cnt[h] = atomicAdd(&tile_count[(int64_t)key[h] * stride], cnt[h]);
+    }
+    __device__ inline int place(int at, int in) const { return cnt[at] + in; }
+};
+
+// cell key and place in the tile's list of every particle, a thread's positions loaded
+// before anything is done with them.  21 million particles FP32: 0.15 ms, 0.77 ms with an
+// atomic per particle on its cell.
 template <class F>
 __global__ void __launch_bounds__(SORT_T)
     k_tile_key(Box b, const int32_t *__restrict__ lut, PView<F> p, int wrap, int shift,
                int stride, int32_t *__restrict__ tile_count, int32_t *__restrict__ key, int32_t *__restrict__ slot)
 {
     using R = typename F::real;
-    __shared__ int hkey[HASH], hcnt[HASH];
+    __shared__ TileHash<HASH_BITS> hash;
     const int64_t base = (int64_t)blockIdx.x * KEY_CHUNK + threadIdx.x;
     R x[KEY_ITEMS][3];
 #pragma unroll
@@ -195,10 +219,7 @@ __global__ void __launch_bounds__(SORT_T)
         if (i < p.n)
             for (int k = 0; k < 3; ++k) x[u][k] = p.pos[k * p.n + i];
     }
-    for (int h = threadIdx.x; h < HASH; h += SORT_T) {
-        hkey[h] = -1;
-        hcnt[h] = 0;
-    }
+    hash.clear();
     __syncthreads();
     int at[KEY_ITEMS], in[KEY_ITEMS];
 #pragma unroll
@@ -206,30 +227,134 @@ __global__ void __launch_bounds__(SORT_T)
         const int64_t i = base + u * SORT_T;
         if (i >= p.n) continue;
         if (wrap) {
-            int j;
-            for (int k = 0; k < 3; ++k) wrap_pbc<R>(b, x[u][k], j, k);
+            for (int k = 0; k < 3; ++k) fold_pbc<R>(x[u][k], (R)b.edges[k]);
         }
         const int c = key_of<R>(b, lut, x[u][0], x[u][1], x[u][2]);
         key[i] = c;
-        const int t = c >> shift;
-        unsigned h = ((unsigned)t * 2654435769u) >> (32 - HASH_BITS);
-        for (;;) {  // at most KEY_CHUNK entries of the HASH are taken
-            int q = hkey[h];
-            if (q == -1) q = atomicCAS(&hkey[h], -1, t);
-            if (q == t || q == -1) break;
-            h = (h + 1) & (HASH - 1);
-        }
-        at[u] = (int)h;
-        in[u] = atomicAdd(&hcnt[h], 1);
+        hash.put(c >> shift, at[u], in[u]);
     }
     __syncthreads();
-    for (int h = threadIdx.x; h < HASH; h += SORT_T)
-        if (hcnt[h] > 0) hcnt[h] = atomicAdd(&tile_count[(int64_t)hkey[h] * stride], hcnt[h]);
+    hash.commit(tile_count, stride);
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < KEY_ITEMS; ++u) {
         const int64_t i = base + u * SORT_T;
-        if (i < p.n) slot[i] = hcnt[at[u]] + in[u];
+        if (i < p.n) slot[i] = hash.place(at[u], in[u]);
+    }
+}
+
+// A plain fluid's cycle up to its sort (setup_simple_fluid.f90:108-118): SRD on the cells
+// of the last sort, n_md steps of mpcd_stream_periodic, then key and place in the tile's
+// list under the next grid shift (b).  One workgroup takes 2^cshift cells, collides their
+// velocities in LDS while the positions are on their way to registers, and goes on with the
+// particles it holds; one with more particles than its LDS collides from memory, a thread
+// per cell, and goes through them in pieces.  Bound by instructions (0.18 ms of them for 21
+// million FP32 particles) and by their phases: 0.37 ms with eight workgroups per CU, 0.42
+// with six, 0.56 with four.  The hash takes the place of the collision's LDS for that, the
+// axes are drawn by the waves that do not add up the cells (one wave per workgroup
+// colliding its cells alone: 0.61 ms), and a position inside the box is not divided by it.
+// As separate collision, streaming and key passes: 0.55 ms.
+template <class F>
+constexpr int FLUID_ITEMS = sizeof(typename F::real) == 4 ? 3 : 2;
+template <class F>
+constexpr int FLUID_MAX = SORT_T * FLUID_ITEMS<F>;
+
+template <class F>
+__global__ void __launch_bounds__(SORT_T, 8)
+    k_fluid_key(Box b, const int32_t *__restrict__ lut, PView<F> p, const int32_t *__restrict__ start,
+                const int32_t *__restrict__ count, int cshift, uint64_t seed, uint64_t step, int n_md, double dt,
+                int shift, int stride, int32_t *__restrict__ tile_count, int32_t *__restrict__ key,
+                int32_t *__restrict__ slot)
+{
+    using R = typename F::real;
+    constexpr int N = FLUID_ITEMS<F>, M = FLUID_MAX<F>;
+    constexpr int BITS = 10;
+    static_assert(M <= 3 << (BITS - 2), "the hash holds a workgroup's particles");
+    // the hash is used after the collision, in its place
+    __shared__ union U {
+        TileHash<BITS> hash;
+        SrdTile<R, typename F::small, M> srd;
+        __device__ U() {}
+    } sh;
+    __shared__ R v[3][M];
+    const int tid = threadIdx.x;
+    const int c0 = (int)blockIdx.x << cshift, ncell = 1 << cshift;
+    const int64_t s = start[c0];
+    const int m = (int)(start[c0 + ncell - 1] + count[c0 + ncell - 1] - s);
+    if (m == 0) return;
+    R x[N][3];
+    auto load = [&](int base) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int q = base + tid + u * SORT_T;
+            if (q < m)
+                for (int k = 0; k < 3; ++k) x[u][k] = p.pos[k * p.n + s + q];
+        }
+    };
+    const R rdt = (R)dt;
+    // the particles from base on that the registers hold, their velocities from vel(k, q)
+    auto piece = [&](int base, bool write_vel, auto vel) {
+        sh.hash.clear();
+        __syncthreads();
+        int at[N], in[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int q = base + tid + u * SORT_T;
+            if (q >= m) continue;
+            const int64_t i = s + q;
+            for (int k = 0; k < 3; ++k) {
+                const R w = vel(k, q);
+                int jump = 0;
+                for (int j = 0; j < n_md; ++j) {
+                    x[u][k] = x[u][k] + w * rdt;
+                    jump += fold_pbc<R>(x[u][k], (R)b.edges[k]);
+                }
+                if (write_vel) p.vel[k * p.n + i] = w;
+                p.pos[k * p.n + i] = x[u][k];
+                if (jump != 0) p.image[k * p.n + i] += jump;
+            }
+            const int c = key_of<R>(b, lut, x[u][0], x[u][1], x[u][2]);
+            key[i] = c;
+            sh.hash.put(c >> shift, at[u], in[u]);
+        }
+        __syncthreads();
+        sh.hash.commit(tile_count, stride);
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int q = base + tid + u * SORT_T;
+            if (q < m) slot[s + q] = sh.hash.place(at[u], in[u]);
+        }
+    };
+    // the LDS and memory in separate calls, so each is addressed directly
+    if (m <= M) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int q = tid + u * SORT_T;
+            if (q < m) {
+                for (int k = 0; k < 3; ++k) v[k][q] = p.vel[k * p.n + s + q];
+                sh.srd.sp[q] = p.species[s + q];
+            }
+        }
+        load(0);
+        __syncthreads();
+        srd_tile(sh.srd, v, s, m, c0, ncell, start, count, seed, step, 1.0, 0.0);
+        piece(0, true, [&](int k, int q) { return v[k][q]; });
+        return;
+    }
+    for (int c = tid; c < ncell; c += SORT_T) {
+        const int n = count[c0 + c];
+        if (n <= 1) continue;
+        const int64_t a = start[c0 + c];
+        srd_cell(p.vel + a, p.vel + p.n + a, p.vel + 2 * p.n + a, p.species + a, n, c0 + c, b.ncells,
+                 (const double *)nullptr, seed, step, 1.0, 0.0);
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (int base = 0; base < m; base += M) {
+        load(base);
+        piece(base, false, [&](int k, int q) { return p.vel[k * p.n + s + q]; });
+        __syncthreads();
     }
 }
 
@@ -306,8 +431,9 @@ __device__ inline void tile_store(T *__restrict__ plane, const T *lds, int m)
 // straight from the planes, each load touched a cache line per lane and the pass took 2.08
 // ms; in list order a tile's loads run along the source, and LDS puts them in slot order so
 // that the stores are contiguous too.  id_to_idx costs 0.42 ms of the 1.09 ms with it: its
-// 4-byte stores go anywhere once the particles have mixed.
-template <class F>
+// 4-byte stores go anywhere once the particles have mixed.  FORCES false leaves the force
+// planes out, for a program whose forces are zero in both buffers.
+template <class F, bool FORCES>
 __global__ void __launch_bounds__(SORT_T)
     k_tile_gather(Box b, PView<F> src, PView<F> dst, int wrap, int shift, int nt, const int32_t *__restrict__ key,
                   const int32_t *__restrict__ start, const int32_t *__restrict__ list, int32_t *__restrict__ spill,
@@ -315,7 +441,7 @@ __global__ void __launch_bounds__(SORT_T)
 {
     using R = typename F::real;
     using S = typename F::small;
-    constexpr int N = TILE_ITEMS<F>, M = TILE_MAX<F>;
+    constexpr int N = TILE_ITEMS<F>, M = TILE_MAX<F>, PLANES = FORCES ? 4 : 2;
     __shared__ R buf[3][M];
     __shared__ int lv[M];
     __shared__ int lcnt[TILE_CELLS], lstart[TILE_CELLS];
@@ -386,15 +512,11 @@ __global__ void __launch_bounds__(SORT_T)
         if (wrap)
             for (int k = 0; k < 3; ++k)
                 for (int u = 0; u < N; ++u)
-                    if (v[u] >= 0) {
-                        int jump;
-                        wrap_pbc<R>(b, x[k][u], jump, k);
-                        im[k][u] += jump;
-                    }
+                    if (v[u] >= 0) im[k][u] += fold_pbc<R>(x[k][u], (R)b.edges[k]);
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
+        for (int g = 0; g < PLANES; ++g) {
             for (int k = 0; k < 3; ++k) tile_put<N>(buf[k], x[k], v, d);
-            if (g < 3)
+            if (g + 1 < PLANES)
                 for (int k = 0; k < 3; ++k) tile_load<N>(x[k], from[(g + 1) & 3] + k * n, v);
             __syncthreads();
             for (int k = 0; k < 3; ++k) tile_store<N>(to[g] + k * n + s, buf[k], m);
@@ -445,16 +567,14 @@ __global__ void __launch_bounds__(SORT_T)
         for (int j = 0; j < 3; ++j) {
             R x = src.pos[j * n + w];
             int32_t im = src.image[j * n + w];
-            if (wrap) {
-                int jmp;
-                wrap_pbc<R>(b, x, jmp, j);
-                im += jmp;
-            }
+            if (wrap) im += fold_pbc<R>(x, (R)b.edges[j]);
             dst.pos[j * n + o] = x;
             dst.image[j * n + o] = im;
             dst.vel[j * n + o] = src.vel[j * n + w];
-            dst.force[j * n + o] = src.force[j * n + w];
-            dst.force_old[j * n + o] = src.force_old[j * n + w];
+            if (FORCES) {
+                dst.force[j * n + o] = src.force[j * n + w];
+                dst.force_old[j * n + o] = src.force_old[j * n + w];
+            }
         }
         const int32_t id = src.id[w];
         dst.id[o] = id;
@@ -493,45 +613,93 @@ static int tile_shift(const Box &b, int64_t n, int tile_max)
     return shift;
 }
 
+// a sort's workspace and tiles
+struct TileSort {
+    Box b;
+    const int32_t *lut;
+    int shift, nt, stride;
+    int32_t *key, *slot, *list, *start, *count;
+};
+
+template <class F>
+static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
+{
+    t.b = make_box(box);
+    t.shift = tile_shift(t.b, n, TILE_MAX<F>);
+    t.nt = t.b.ncells >> t.shift;
+    t.stride = count_stride(t.nt);
+    t.key = (int32_t *)workspace(WS_KEY, sizeof(int32_t) * n);
+    t.slot = (int32_t *)workspace(WS_SLOT, sizeof(int32_t) * n);
+    t.list = (int32_t *)workspace(WS_TMP, sizeof(int32_t) * n);
+    t.start = (int32_t *)workspace(WS_TILE, sizeof(int32_t) * ((size_t)t.nt + 1));
+    t.count = (int32_t *)workspace(WS_TCOUNT, sizeof(int32_t) * ((size_t)t.nt + 1) * t.stride);  // zero between sorts
+    if (!t.key || !t.slot || !t.list || !t.start || !t.count)
+        return set_error(RMPCD_ERR_HIP, "rmpcd_sort: workspace allocation failed");
+    t.lut = hilbert_lut(t.b);
+    if (!t.lut) return set_error(RMPCD_ERR_HIP, "rmpcd_sort: Hilbert table allocation failed");
+    return RMPCD_OK;
+}
+
+// the sort after its keys
+template <class F, bool FORCES>
+static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
+                            int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap)
+{
+    const int64_t n = src->n;
+    hipStream_t s = stream();
+    if (t.nt <= SCAN1_TILES) {
+        k_tile_scan<<<1, 1024, 0, s>>>(t.count, t.stride, t.nt, t.start);
+        RMPCD_LAUNCHED();
+    } else {
+        int rc = exclusive_scan(t.count, t.start, (int64_t)t.nt + 1);
+        if (rc) return rc;
+        k_fill_i32<<<blocks_for(t.nt, 256), 256, 0, s>>>(t.count, t.nt, 0);
+        RMPCD_LAUNCHED();
+    }
+    k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, t.key, t.shift, t.slot, t.start, t.list);
+    RMPCD_LAUNCHED();
+    const unsigned runs = (unsigned)((t.nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
+    k_tile_gather<F, FORCES><<<8 * TILE_RUN * runs, SORT_T, 0, s>>>(t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt,
+                                                                    t.key, t.start, t.list, t.slot, cells->cell_count,
+                                                                    cells->cell_start, id_to_idx);
+    RMPCD_LAUNCHED();
+    return RMPCD_OK;
+}
+
 template <class F>
 int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
               int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap)
 {
-    const int64_t n = src->n;
-    const Box b = make_box(box);
-    const int shift = tile_shift(b, n, TILE_MAX<F>);
-    const int nt = b.ncells >> shift;
-    int32_t *key = (int32_t *)workspace(WS_KEY, sizeof(int32_t) * n);
-    int32_t *slot = (int32_t *)workspace(WS_SLOT, sizeof(int32_t) * n);
-    int32_t *list = (int32_t *)workspace(WS_TMP, sizeof(int32_t) * n);
-    int32_t *tstart = (int32_t *)workspace(WS_TILE, sizeof(int32_t) * ((size_t)nt + 1));
-    // zero between sorts
-    const int stride = count_stride(nt);
-    int32_t *tcount = (int32_t *)workspace(WS_TCOUNT, sizeof(int32_t) * ((size_t)nt + 1) * stride);
-    if (!key || !slot || !list || !tstart || !tcount)
-        return set_error(RMPCD_ERR_HIP, "rmpcd_sort: workspace allocation failed");
-    const int32_t *lut = hilbert_lut(b);
-    if (!lut) return set_error(RMPCD_ERR_HIP, "rmpcd_sort: Hilbert table allocation failed");
-    hipStream_t s = stream();
-    k_tile_key<F><<<blocks_for(n, KEY_CHUNK), SORT_T, 0, s>>>(b, lut, view<F>(src), wrap, shift, stride, tcount, key,
-                                                              slot);
+    TileSort t;
+    int rc = tile_sort_begin<F>(box, src->n, t);
+    if (rc) return rc;
+    k_tile_key<F><<<blocks_for(src->n, KEY_CHUNK), SORT_T, 0, stream()>>>(t.b, t.lut, view<F>(src), wrap, t.shift,
+                                                                          t.stride, t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    if (nt <= SCAN1_TILES) {
-        k_tile_scan<<<1, 1024, 0, s>>>(tcount, stride, nt, tstart);
-        RMPCD_LAUNCHED();
-    } else {
-        int rc = exclusive_scan(tcount, tstart, (int64_t)nt + 1);
-        if (rc) return rc;
-        k_fill_i32<<<blocks_for(nt, 256), 256, 0, s>>>(tcount, nt, 0);
-        RMPCD_LAUNCHED();
-    }
-    k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, key, shift, slot, tstart, list);
+    return tile_sort_finish<F, true>(t, src, dst, id_to_idx, cells, wrap);
+}
+
+template <class F>
+int fluid_cycle_impl(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
+                     rmpcd_cells_t *cells, uint64_t seed, uint64_t step, int n_md, double dt)
+{
+    TileSort t;
+    int rc = tile_sort_begin<F>(next, src->n, t);
+    if (rc) return rc;
+    // the collision's cells per workgroup, by the same rule as a tile's
+    int cshift = tile_shift(t.b, src->n, FLUID_MAX<F>);
+    while ((1 << cshift) > SRD_CELLS) --cshift;
+    k_fluid_key<F><<<(unsigned)(t.b.ncells >> cshift), SORT_T, 0, stream()>>>(
+        t.b, t.lut, view<F>(src), cells->cell_start, cells->cell_count, cshift, seed, step, n_md, dt, t.shift, t.stride,
+        t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    k_tile_gather<F><<<8 * TILE_RUN * (unsigned)((nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN)), SORT_T, 0, s>>>(b, view<F>(src), view<F>(dst), wrap, shift, nt, key,
-                                                                    tstart, list, slot, cells->cell_count,
-                                                                    cells->cell_start, id_to_idx);
-    RMPCD_LAUNCHED();
-    return RMPCD_OK;
+    return tile_sort_finish<F, false>(t, src, dst, nullptr, cells, 0);
+}
+
+int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
+                          rmpcd_cells_t *cells, uint64_t seed, uint64_t step, int n_md, double dt)
+{
+    return RMPCD_DISPATCH_FORM(src, fluid_cycle_impl, next, src, dst, cells, seed, step, n_md, dt);
 }
 
 int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,

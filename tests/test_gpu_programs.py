@@ -58,6 +58,44 @@ def test_fluid_matches_oracle(gpu, n_md):
     prog.close()
 
 
+@pytest.mark.parametrize("form", [capi.FP64, capi.FP32])
+@pytest.mark.parametrize("L,rho,n_md", [
+    ((13, 10, 7), 10, 2),   # workgroups of several cells, a padded box
+    ((4, 4, 4), 900, 1),    # one cell holds more particles than a workgroup's LDS
+    ((9, 8, 8), 1, 1),      # cells with one particle or none
+])
+def test_fluid_equals_entry_points(gpu, form, L, rho, n_md):
+    """the fused cycle against simple_mpcd_step, mpcd_stream_periodic and sort, bit for bit"""
+    import ctypes as C
+    import torch
+    from rmpcdmd_amd.system import CellSet, ParticleSet
+    tau, seed = 0.3, 21
+    prog = Program(PROG_FLUID, form=form, seed=seed, L=L, rho=rho, n_md=n_md, tau=tau, T=1.0)
+    st = prog.download()
+    n = st["id"].size
+    src, dst, cs = ParticleSet(n, form), ParticleSet(n, form), CellSet(L)
+    src.load(**{k: st[k] for k in ("pos", "vel", "force", "force_old", "image", "id", "species", "flags")})
+    i2i = torch.zeros(n, dtype=torch.int32, device="cuda")
+    capi.call("rmpcd_sort", cs.boxp(), src.struct(), dst.struct(), C.c_void_p(i2i.data_ptr()), cs.cellsp(), 0)
+    src, dst = dst, src
+    for cycle in range(3):
+        prog.run(1)
+        g = prog.download()
+        capi.call("rmpcd_simple_mpcd_step", cs.boxp(), cs.cellsp(), src.struct(), None, seed, cycle, 0, 0.0, 0, 1.0, 1)
+        for _ in range(n_md):
+            capi.call("rmpcd_mpcd_stream_periodic", cs.boxp(), src.struct(), tau / n_md)
+        cs.set_origin(g["origin"])
+        capi.call("rmpcd_sort", cs.boxp(), src.struct(), dst.struct(), C.c_void_p(i2i.data_ptr()), cs.cellsp(), 0)
+        torch.cuda.synchronize()
+        src, dst = dst, src
+        for k in ("pos", "vel", "force", "force_old", "image", "id", "species", "flags"):
+            assert src.host(k).tobytes() == np.ascontiguousarray(g[k]).tobytes(), "%s, cycle %d" % (k, cycle)
+        assert dst.host("pos").tobytes() == np.ascontiguousarray(g["pos_old"]).tobytes()
+        assert (cs.cell_count.cpu().numpy() == g["cell_count"]).all()
+        assert (cs.cell_start.cpu().numpy() == g["cell_start"]).all()
+    prog.close()
+
+
 def test_sphere_matches_oracle(gpu):
     from oracle.programs import SphereOracle
     L = (16, 16, 16)
