@@ -4,25 +4,25 @@
 //
 // The reference updates the links one after the other, each correction seeing the ones
 // before it, sweep after sweep until the constraints hold.  That order is kept exactly.
-// On the host the link list becomes a schedule of levels: an update's level is one more
-// than the highest level of the earlier updates that share a particle with it.  Updates
-// of one level touch disjoint particles and every earlier update of the same particle
-// sits in a lower level, so a workgroup running the levels in turn, with a barrier in
-// between, reads and writes every particle in the order of the sequential loops: the
-// results are the reference's bit for bit.
+// On the host the link list becomes a schedule: an update waits for the earlier updates
+// that share a particle with it, and updates that share none may run side by side, so that
+// every particle is read and written in the order of the sequential loops and the results
+// are the reference's bit for bit.
 //
-// Sweeps overlap.  The schedule covers a block of K consecutive sweeps as one unrolled
-// sequence, so the first links of sweep s + 1 start while the last ones of sweep s are
-// still running (on a 300-bead shell one sweep alone takes 155 levels, each further
-// sweep of the block about 16).  The stopping test of a sweep needs the state at its end:
-// the update that is a particle's last in a sweep copies the particle to that sweep's
-// snapshot, the block's tests then run on the snapshots, and the state of the first sweep
-// that passes is put back before the block's later sweeps are forgotten.  Body, links
-// and schedule live in LDS (up to 160 KiB on gfx950); bodies too large for it run the
-// one-sweep schedule from global memory.
+// The schedule covers a block of K consecutive sweeps as one unrolled sequence, so the first
+// links of sweep s + 1 start while the last ones of sweep s are still running (on a
+// 300-bead shell one sweep alone takes 155 steps, each further sweep of the block about 15),
+// and a step holds at most 64 updates, those with the longest way to go first: one wave runs
+// it, a lane per update, and needs no barrier between steps.  The stopping test of a sweep
+// needs the state at its end: the update that is a particle's last in a sweep copies the
+// particle to that sweep's snapshot in LDS, the block's tests then run on the snapshots with
+// all waves, and the state of the first sweep that passes is put back.  Bodies too large for
+// that run sweep by sweep, level by level, from global memory.
 #include <math.h>
 #include <string.h>
 
+#include <queue>
+#include <type_traits>
 #include <vector>
 
 #include "rmpcd_internal.hpp"
@@ -31,7 +31,10 @@ namespace rmpcd {
 
 constexpr int BT = 256;           // threads of the one workgroup
 constexpr int RATTLE_MAX = 1000;  // md.f90:341, :432
-constexpr int KMAX = 12;          // sweeps per block at most (4 bits of the entry)
+constexpr int KMAX = 16;          // sweeps per block at most (4 bits of the entry)
+constexpr int AHEAD = 4;          // steps that a link's constants are read ahead of their use
+constexpr int LC = 10;            // doubles per link of its constants
+constexpr int WAVE_N = 2700;      // particles of the one-wave rattle at most (16-bit offsets)
 
 struct BodyMass {
     double m[16];    // particle_system%mass by species (species s at s - 1)
@@ -44,9 +47,10 @@ __device__ inline double dot3b(const double a[3], const double b[3]) { return (a
 // Built on the host from the caller's link list and kept on the device while the list is
 // unchanged (compared by content on every call).
 struct BlockSched {
-    int K = 0, n_glev = 0;
-    uint2 *d_ent = nullptr;   // by level: {a | b << 16, l | s << 24 | last-of-a << 28 | last-of-b << 29}
-    int32_t *d_gs = nullptr;  // level starts, n_glev + 1
+    int K = 0, n_steps = 0;   // n_steps a multiple of 2 AHEAD
+    // 64 per step, all as byte offsets that a lane can use as they are: {a | b << 16 in the
+    // particles, the link's constants | sweep, where a's and b's state go in the snapshots}
+    uint4 *d_ent = nullptr;
     void *block = nullptr;
 };
 
@@ -59,11 +63,10 @@ struct Schedule {
     // one sweep by level (the global-memory rattle)
     int32_t *d_i1 = nullptr, *d_i2 = nullptr, *d_start = nullptr;
     double *d_d = nullptr;
-    // by link: a, b, a | b << 16 (when n < 65536), distance; per particle: the links
+    // by link: a, b, distance; per particle: the links
     // touching it in link order (bit 31 set where it is the second particle)
     int32_t *d_la = nullptr, *d_lb = nullptr;
-    uint32_t *d_lab = nullptr;
-    double *d_dist = nullptr;
+        double *d_dist = nullptr;
     int32_t *d_cstart = nullptr, *d_csr = nullptr;
     void *block = nullptr;
     BlockSched blocks[KMAX + 1];  // by K, built on first use
@@ -115,7 +118,6 @@ static int get_schedule(const int32_t *links, const double *dist, int n_links, i
     }
     const size_t nl = (size_t)n_links;
     std::vector<int32_t> start((size_t)n_levels + 1, 0), i1(nl), i2(nl), la(nl), lb(nl);
-    std::vector<uint32_t> lab(nl);
     std::vector<double> dd(nl);
     for (int l = 0; l < n_links; ++l) ++start[lvl[l] + 1];
     for (int v = 0; v < n_levels; ++v) start[v + 1] += start[v];
@@ -127,7 +129,6 @@ static int get_schedule(const int32_t *links, const double *dist, int n_links, i
         dd[k] = dist[l];
         la[l] = links[2 * l];
         lb[l] = links[2 * l + 1];
-        lab[l] = (uint32_t)links[2 * l] | ((uint32_t)links[2 * l + 1] << 16);
     }
     std::vector<int32_t> cstart((size_t)n + 1, 0), csr(2 * nl);
     for (int l = 0; l < n_links; ++l) {
@@ -151,7 +152,7 @@ static int get_schedule(const int32_t *links, const double *dist, int n_links, i
         RMPCD_HIP(hipSetDevice(cur));
     }
     const size_t nl1 = nl > 0 ? nl : 1;
-    const size_t bytes = nl1 * 16 + nl1 * 4 * 5 + ((size_t)n_levels + 1) * 4 + ((size_t)n + 1) * 4 + 2 * nl1 * 4 + 256;
+    const size_t bytes = nl1 * 16 + nl1 * 4 * 4 + ((size_t)n_levels + 1) * 4 + ((size_t)n + 1) * 4 + 2 * nl1 * 4 + 256;
     RMPCD_HIP(hipMalloc(&s.block, bytes));
     s.d_d = (double *)s.block;
     s.d_dist = s.d_d + nl1;
@@ -159,15 +160,14 @@ static int get_schedule(const int32_t *links, const double *dist, int n_links, i
     s.d_i2 = s.d_i1 + nl1;
     s.d_la = s.d_i2 + nl1;
     s.d_lb = s.d_la + nl1;
-    s.d_lab = (uint32_t *)(s.d_lb + nl1);
-    s.d_csr = (int32_t *)(s.d_lab + nl1);
+    s.d_csr = s.d_lb + nl1;
     s.d_cstart = s.d_csr + 2 * nl1;
     s.d_start = s.d_cstart + n + 1;
     std::vector<double> dist_v(dist, dist + n_links);
     int rc;
     if ((rc = upload(s.d_d, dd)) || (rc = upload(s.d_dist, dist_v)) || (rc = upload(s.d_i1, i1)) ||
         (rc = upload(s.d_i2, i2)) || (rc = upload(s.d_la, la)) || (rc = upload(s.d_lb, lb)) ||
-        (rc = upload(s.d_lab, lab)) || (rc = upload(s.d_csr, csr)) || (rc = upload(s.d_cstart, cstart)) ||
+        (rc = upload(s.d_csr, csr)) || (rc = upload(s.d_cstart, cstart)) ||
         (rc = upload(s.d_start, start)))
         return rc;
     s.links.assign(links, links + 2 * nl);
@@ -180,7 +180,8 @@ static int get_schedule(const int32_t *links, const double *dist, int n_links, i
     return RMPCD_OK;
 }
 
-// the unrolled schedule of K sweeps, built once per list and K
+// the unrolled schedule of K sweeps, built once per list and K: each step takes, of the
+// updates whose predecessors have run, the up to 64 with the longest chain behind them
 static int get_block(Schedule &s, int K, const BlockSched **out)
 {
     BlockSched &b = s.blocks[K];
@@ -188,50 +189,85 @@ static int get_block(Schedule &s, int K, const BlockSched **out)
         *out = &b;
         return RMPCD_OK;
     }
-    const int nl = s.n_links;
+    const int nl = s.n_links, nt = K * nl;
     const int32_t *links = s.links.data();
-    std::vector<int32_t> last((size_t)s.n, 0), lastlink((size_t)s.n, -1), lvl((size_t)K * nl);
+    // the next update of a's and of b's particle, the number of updates waited for, the
+    // length of the longest chain from here on
+    std::vector<int32_t> next(2 * (size_t)nt, -1), wait((size_t)nt, 0), height((size_t)nt, 0), last((size_t)s.n, -1),
+        lastlink((size_t)s.n, -1);
     for (int l = 0; l < nl; ++l) lastlink[links[2 * l]] = lastlink[links[2 * l + 1]] = l;
-    int n_glev = 0;
-    for (int q = 0; q < K; ++q)
-        for (int l = 0; l < nl; ++l) {
-            const int a = links[2 * l], c = links[2 * l + 1];
-            const int v = last[a] > last[c] ? last[a] : last[c];
-            lvl[(size_t)q * nl + l] = v;
-            last[a] = last[c] = v + 1;
-            if (v + 1 > n_glev) n_glev = v + 1;
+    for (int t = nt - 1; t >= 0; --t) {
+        const int x[2] = {links[2 * (t % nl)], links[2 * (t % nl) + 1]};
+        int h = 0;
+        for (int e = 0; e < 2; ++e)
+            if (last[x[e]] >= 0 && !(e == 1 && x[1] == x[0])) {
+                next[2 * (size_t)t + e] = last[x[e]];
+                ++wait[last[x[e]]];
+                if (height[last[x[e]]] > h) h = height[last[x[e]]];
+            }
+        height[t] = h + 1;
+        last[x[0]] = last[x[1]] = t;
+    }
+    // the longest chain first, the earlier update among equals
+    auto later = [&](int32_t p, int32_t q) { return height[p] != height[q] ? height[p] < height[q] : p > q; };
+    std::priority_queue<int32_t, std::vector<int32_t>, decltype(later)> ready(later);
+    for (int t = 0; t < nt; ++t)
+        if (wait[t] == 0) ready.push(t);
+    std::vector<uint4> ent;
+    const uint32_t spare = (uint32_t)(K * s.n * 24);  // in the snapshots: a place per lane
+    const uint4 idle{(uint32_t)(s.n * 24) | ((uint32_t)((s.n + 1) * 24) << 16), (uint32_t)nl * LC * 8, 0, 0};
+    std::vector<int32_t> step;
+    ent.reserve(2 * (size_t)nt);
+    while (!ready.empty()) {
+        step.clear();
+        while (!ready.empty() && step.size() < 64) {
+            step.push_back(ready.top());
+            ready.pop();
         }
-    std::vector<int32_t> gs((size_t)n_glev + 1, 0);
-    for (size_t k = 0; k < lvl.size(); ++k) ++gs[lvl[k] + 1];
-    for (int v = 0; v < n_glev; ++v) gs[v + 1] += gs[v];
-    std::vector<int32_t> fill(gs.begin(), gs.end() - 1);
-    std::vector<uint2> ent(lvl.size());
-    for (int q = 0; q < K; ++q)
-        for (int l = 0; l < nl; ++l) {
-            const int a = links[2 * l], c = links[2 * l + 1];
-            uint2 e;
-            e.x = (uint32_t)a | ((uint32_t)c << 16);
-            e.y = (uint32_t)l | ((uint32_t)q << 24) | ((lastlink[a] == l ? 1u : 0u) << 28) |
-                  ((lastlink[c] == l ? 1u : 0u) << 29);
-            ent[fill[lvl[(size_t)q * nl + l]]++] = e;
+        for (const int32_t t : step) {
+            const int l = t % nl, q = t / nl, a = links[2 * l], c = links[2 * l + 1];
+            const uint32_t lane = (uint32_t)(ent.size() % 64);
+            uint4 e;
+            e.x = (uint32_t)a * 24 | ((uint32_t)c * 24 << 16);
+            e.y = (uint32_t)l * LC * 8 | (uint32_t)q;
+            e.z = lastlink[a] == l ? (uint32_t)((q * s.n + a) * 24) : spare + lane * 24;
+            e.w = lastlink[c] == l ? (uint32_t)((q * s.n + c) * 24) : spare + lane * 24;
+            ent.push_back(e);
+            for (int k = 0; k < 2; ++k) {
+                const int32_t w = next[2 * (size_t)t + k];
+                if (w >= 0 && --wait[w] == 0) ready.push(w);
+            }
         }
-    RMPCD_HIP(hipMalloc(&b.block, ent.size() * sizeof(uint2) + gs.size() * 4 + 256));
-    b.d_ent = (uint2 *)b.block;
-    b.d_gs = (int32_t *)(b.d_ent + ent.size());
-    int rc;
-    if ((rc = upload(b.d_ent, ent)) || (rc = upload(b.d_gs, gs))) return rc;
+        auto pad = [&] {
+            uint4 e = idle;
+            e.z = e.w = spare + (uint32_t)(ent.size() % 64) * 24;
+            ent.push_back(e);
+        };
+        while (ent.size() % 64) pad();
+        if (ready.empty())  // idle steps up to a whole turn, and one more turn to read ahead
+            while (ent.size() % (64 * 2 * AHEAD)) pad();
+    }
+    const size_t n_ent = ent.size();
+    for (int k = 0; k < 64 * 2 * AHEAD; ++k) {
+        ent.push_back(idle);
+        ent.back().z = ent.back().w = spare + (uint32_t)(k % 64) * 24;
+    }
+    RMPCD_HIP(hipMalloc(&b.block, ent.size() * sizeof(uint4)));
+    b.d_ent = (uint4 *)b.block;
+    int rc = upload(b.d_ent, ent);
+    if (rc) return rc;
     b.K = K;
-    b.n_glev = n_glev;
+    b.n_steps = (int)(n_ent / 64);
     *out = &b;
     return RMPCD_OK;
 }
 
-// bytes of LDS the pipelined rattle takes: particles (P, V and for positions R, four
-// doubles each), links (distance, packed pair), the entries and level starts, flags
-static size_t pipe_lds_bytes(int64_t n, int n_links, int K, int n_glev, bool with_pr)
+// bytes of LDS the one-wave rattle takes: the particles' positions and velocities (for the
+// velocities alone: velocities) with two spare particles for idle lanes, a copy of what a
+// block starts from, K snapshots with a spare place per lane, flags
+static size_t wave_lds_bytes(int64_t n, int K, bool with_pr)
 {
-    return (size_t)n * 32 * (with_pr ? 3 : 2) + (size_t)n_links * 12 + (size_t)K * n_links * 8 +
-           ((size_t)n_glev + 1) * 4 + 16 * 4 + 64;
+    return 24 * ((size_t)(n + 2) * (with_pr ? 3 : 2) + (size_t)K * n + 64) + 2 * KMAX * 4 + 64;
 }
 
 static int lds_limit()
@@ -247,220 +283,284 @@ static int lds_limit()
     return limit;
 }
 
-// a workgroup barrier that orders LDS only: global stores stay in flight
-__device__ inline void lds_barrier()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
+constexpr int WT = 512;  // threads of the one-wave rattle: one wave updates, all set up and test
 
-struct PipeView {
-    const uint2 *ent;
-    const int32_t *gs;
-    const uint32_t *lab;
+struct WaveView {
+    const uint4 *ent;
+    const int32_t *la, *lb;
     const double *dist;
-    int n_links, n_ent, n_glev, K;
+    const int32_t *cstart;  // links per particle, to see which have any
+    int n_links, n_steps, K;
 };
 
-// ---- rattle_body_pos (kPos) / rattle_body_vel, pipelined -------------------------------
-// Staging: every particle but the first is unfolded next to particle 0 (md.f90:343-353,
-// :427-431) and folded back at the end (md.f90:400-402, :474-476); pos_rattle is left
-// unfolded, as the reference leaves it.
-template <bool kPos>
-__global__ void __launch_bounds__(BT) k_rattle_pipe(PView<F64> p, double *__restrict__ gpr, PipeView pv, BodyMass bm,
-                                                    double dt, double e0, double e1, double e2, double precision,
-                                                    int32_t *__restrict__ out, int32_t *__restrict__ gim,
-                                                    double *__restrict__ snap)
+// a / b, correctly rounded, from y = the rounded 1 / b: Markstein's correction of a quotient
+// by its exact remainder (P. W. Markstein, IBM J. Res. Dev. 34, 1990), twice; the second
+// starts from a quotient within one unit in the last place, for which it is proven.  The
+// caller keeps |a| and b away from the ends of the exponent range.
+__device__ inline double div_by(double a, double b, double y)
 {
-    extern __shared__ double smem[];
-    const int64_t n = p.n;
-    const int tid = threadIdx.x;
-    const int nl = pv.n_links, K = pv.K;
-    const double edges[3] = {e0, e1, e2};
-    double *P = smem;          // {x, y, z, 1/m}
-    double *V = P + 4 * n;     // {vx, vy, vz, linked}
-    double *R = V + 4 * n;     // {x, y, z, -} (positions only)
-    double *D = kPos ? R + 4 * n : R;
-    uint2 *E = (uint2 *)(D + nl);
-    uint32_t *LAB = (uint32_t *)(E + pv.n_ent);
-    int32_t *GS = (int32_t *)(LAB + nl);
-    int32_t *NC = GS + pv.n_glev + 1;
-    for (int64_t i = tid; i < n; i += BT) {
-        for (int k = 0; k < 3; ++k) {
-            const double x0 = p.pos[k * n], x = p.pos[k * n + i];
-            const int j = i == 0 ? 0 : (int)floor(((x - x0) / edges[k]) + 0.5);
-            gim[k * n + i] = j;
-            P[4 * i + k] = i == 0 ? x : x - j * edges[k];
-            V[4 * i + k] = p.vel[k * n + i];
-            if (kPos) {
-                const double r0 = gpr[k * n], r = gpr[k * n + i];
-                const int jr = i == 0 ? 0 : (int)floor(((r - r0) / edges[k]) + 0.5);
-                R[4 * i + k] = i == 0 ? r : r - jr * edges[k];
-            }
-        }
-        P[4 * i + 3] = bm.inv[((int)p.species[i] - 1) & 15];
-        V[4 * i + 3] = 0;
-    }
-    for (int l = tid; l < nl; l += BT) {
-        D[l] = pv.dist[l];
-        LAB[l] = pv.lab[l];
-    }
-    for (int x = tid; x < pv.n_ent; x += BT) E[x] = pv.ent[x];
-    for (int g = tid; g <= pv.n_glev; g += BT) GS[g] = pv.gs[g];
-    __syncthreads();
-    for (int l = tid; l < nl; l += BT) {
-        V[4 * (LAB[l] & 0xFFFF) + 3] = 1;
-        V[4 * (LAB[l] >> 16) + 3] = 1;
-    }
-    __syncthreads();
-    int it = RATTLE_MAX + 1;
-    // one link update of the schedule (md.f90:365-383, :435-452)
-    auto update = [&](const uint2 e, const int ns) {
-        const int q = (e.y >> 24) & 15;
-        if (q >= ns) return;
-        const int a = e.x & 0xFFFF, b = e.x >> 16, l = e.y & 0xFFFFFF;
-        const double pa[3] = {P[4 * a], P[4 * a + 1], P[4 * a + 2]};
-        const double pb[3] = {P[4 * b], P[4 * b + 1], P[4 * b + 2]};
-        const double va[3] = {V[4 * a], V[4 * a + 1], V[4 * a + 2]};
-        const double vb[3] = {V[4 * b], V[4 * b + 1], V[4 * b + 2]};
-        const double ma = P[4 * a + 3], mb = P[4 * b + 3], d = D[l];
-        double s[3], na[3], nb[3], wa[3], wb[3];
-        for (int k = 0; k < 3; ++k) s[k] = pa[k] - pb[k];
-        if (kPos) {
-            double r[3];
-            for (int k = 0; k < 3; ++k) r[k] = R[4 * a + k] - R[4 * b + k];
-            const double rsq = dot3b(r, r), ssq = dot3b(s, s), rs = dot3b(r, s);
-            double gg = rs - sqrt(rs * rs - rsq * (ssq - d * d));
-            gg = gg / ((dt * (ma + mb)) * rsq);
-            // a link from a particle to itself reads its own update, as the reference does
-            for (int k = 0; k < 3; ++k) {
-                na[k] = pa[k] - ((gg * dt) * r[k]) * ma;
-                nb[k] = (a == b ? na[k] : pb[k]) + ((gg * dt) * r[k]) * mb;
-                wa[k] = va[k] - (gg * r[k]) * ma;
-                wb[k] = (a == b ? wa[k] : vb[k]) + (gg * r[k]) * mb;
-            }
-            for (int k = 0; k < 3; ++k) {
-                P[4 * a + k] = na[k];
-                V[4 * a + k] = wa[k];
-            }
-            for (int k = 0; k < 3; ++k) {
-                P[4 * b + k] = nb[k];
-                V[4 * b + k] = wb[k];
-            }
-        } else {
-            double dv[3];
-            for (int k = 0; k < 3; ++k) dv[k] = va[k] - vb[k];
-            const double kk = dot3b(dv, s) / ((d * d) * (ma + mb));
-            for (int k = 0; k < 3; ++k) {
-                na[k] = pa[k];
-                nb[k] = pb[k];
-                wa[k] = va[k] - (kk * s[k]) * ma;
-                wb[k] = (a == b ? wa[k] : vb[k]) + (kk * s[k]) * mb;
-            }
-            for (int k = 0; k < 3; ++k) V[4 * a + k] = wa[k];
-            for (int k = 0; k < 3; ++k) V[4 * b + k] = wb[k];
-        }
-        // the last update of a particle in a sweep leaves its end-of-sweep state
-        if (e.y & (1u << 28)) {
-            double *o = snap + ((size_t)q * n + a) * 8;
-            for (int k = 0; k < 3; ++k) {
-                o[k] = na[k];
-                o[3 + k] = wa[k];
-            }
-        }
-        if (e.y & (1u << 29)) {
-            double *o = snap + ((size_t)q * n + b) * 8;
-            for (int k = 0; k < 3; ++k) {
-                o[k] = nb[k];
-                o[3 + k] = wb[k];
-            }
+    double q = a * y;
+    q = fma(fma(-b, q, a), y, q);
+    return fma(fma(-b, q, a), y, q);
+}
+
+// sqrt(x), correctly rounded, for 1e-200 < x < 1e200: a Goldschmidt step from the hardware's
+// reciprocal square root, then two corrections by the exact remainder (same source); without
+// the scaling and the special cases of sqrt()
+__device__ inline double sqrt_mid(double x)
+{
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    return fma(fma(-g, g, x), h, g);
+}
+// how far |x| lies above 1e-200 in units of its upper word, doubled; more than MID_SPAN from
+// 1e200 on, and for 0, infinities and NaN
+constexpr uint32_t MID_LOW = (1023u - 665u) << 21, MID_SPAN = (665u + 664u) << 21;
+__device__ inline uint32_t mid_off(double x) { return ((uint32_t)__double2hiint(x) << 1) - MID_LOW; }
+
+// The steps of a block for one wave.  A lane's update needs its entry, then the constants of
+// the entry's link (and with kG the update's multiplier from g): they are read from memory
+// 2 AHEAD and AHEAD steps before their use and looked at no earlier, so that a step waits
+// for LDS alone.  each(entry, constants, step) runs with every lane; the idle ones, and with
+// kLimit those of sweeps from ns on, have the two spare particles for their ends.
+template <int NC_, bool kG, bool kLimit, class Fn>
+__device__ inline void for_steps(const WaveView &w, const double *lc, const double *g, int n, int ns, Fn each)
+{
+    const int lane = threadIdx.x & 63;
+    uint4 e[2 * AHEAD];
+    double c[AHEAD][NC_ + 1];
+    auto entry = [&](int s) {
+        const uint4 *at = w.ent + (size_t)s * 64;
+        uint4 f = at[lane];
+        return f;
+    };
+    auto constants = [&](int d, uint32_t y, int s) {
+        const double *q = (const double *)((const char *)lc + (y & ~15u));
+#pragma unroll
+        for (int k = 0; k < NC_; ++k) c[d][k] = q[k];
+        if (kG) {
+            const double *at = g + (size_t)s * 64;
+            c[d][NC_] = at[lane];
         }
     };
-    const int last_ent = pv.n_ent > 0 ? pv.n_ent - 1 : 0;
-    for (int base = 0; base < RATTLE_MAX; base += K) {
-        const int ns = K < RATTLE_MAX - base ? K : RATTLE_MAX - base;
-        // each level's first entry of this thread is read one level ahead; the barrier
-        // between levels orders LDS only (the snapshots are read after the full barrier
-        // that ends the block)
-        int x0 = GS[0], x1 = pv.n_glev > 0 ? GS[1] : 0;
-        uint2 cur = E[min(x0 + tid, last_ent)];
-        for (int g = 0; g < pv.n_glev; ++g) {
-            const uint2 next = E[min(x1 + tid, last_ent)];
-            const int y1 = GS[g + 2 <= pv.n_glev ? g + 2 : pv.n_glev];
-            if (x0 + tid < x1) update(cur, ns);
-            for (int x = x0 + tid + BT; x < x1; x += BT) update(E[x], ns);
-            lds_barrier();
-            x0 = x1;
-            x1 = y1;
-            cur = next;
+#pragma unroll
+    for (int d = 0; d < 2 * AHEAD; ++d) e[d] = entry(d);
+#pragma unroll
+    for (int d = 0; d < AHEAD; ++d) constants(d, e[d].y, d);
+    for (int s0 = 0; s0 < w.n_steps; s0 += 2 * AHEAD) {
+#pragma unroll
+        for (int d = 0; d < 2 * AHEAD; ++d) {
+            const int s = s0 + d;
+            uint4 f = e[d];
+            if (kLimit && (int)(f.y & 15) >= ns) {
+                f.x = (uint32_t)(n * 24) | ((uint32_t)((n + 1) * 24) << 16);
+                f.z = f.w = (uint32_t)(w.K * n * 24 + lane * 24);
+            }
+            each(f, c[d % AHEAD], s);
+            constants(d % AHEAD, e[(d + AHEAD) % (2 * AHEAD)].y, s + AHEAD);
+            e[d] = entry(s + 2 * AHEAD);
+            // LDS serves a wave in order: what this step wrote, the next one reads
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
         }
+    }
+}
+
+// ---- rattle_body_pos (kPos) / rattle_body_vel, one wave --------------------------------
+// Every particle but the first is unfolded next to particle 0 (md.f90:343-353, :427-431) and
+// folded back at the end (md.f90:400-402, :474-476); pos_rattle is left unfolded, as the
+// reference leaves it.  What does not change during the call is made once per link: the
+// separation of pos_rattle (positions) or of the positions (velocities), its square, the
+// denominator of the multiplier and its reciprocal.  The position updates do not read the
+// velocities, so a second wave makes the velocity updates of a block, from the multipliers,
+// while the first runs the next block.
+//
+// The square root and the division of an update are made without the general forms' scaling
+// and special cases; what they leave out is watched for (the largest mid_off of their
+// operands), and a block that met it is run again from its start with the general forms.
+//
+// Bound by one wave's issue and the latency of a step's chain of LDS reads and FP64
+// operations (one update after the other along the longest chain of links): 0.21 us a step.
+// An MD step of a 300-bead shell with 1202 links, 229 and 364 sweeps: 1.9 ms for the
+// positions and 2.0 for the velocities; 256 threads with a barrier per level and 12 sweeps
+// per block took 4.8 and 5.0.
+template <bool kPos>
+__global__ void __launch_bounds__(WT)
+    k_rattle_wave(PView<F64> p, double *__restrict__ gpr, WaveView w, BodyMass bm, double dt, double e0, double e1,
+                  double e2, double precision, int32_t *__restrict__ out, int32_t *__restrict__ gim, double *lc,
+                  double *gg)
+{
+    extern __shared__ double smem[];
+    const int n = (int)p.n, n3 = 3 * (n + 2);
+    const int tid = threadIdx.x, wave = tid >> 6;
+    const int nl = w.n_links, K = w.K;
+    const double edges[3] = {e0, e1, e2};
+    double *X = smem;                  // positions (kPos) or velocities, x y z per particle
+    double *V = kPos ? X + n3 : X;     // velocities
+    double *XS = V + n3;               // X at the start of a block
+    double *SN = XS + n3;              // snapshots of X, n particles per sweep, and a place per lane
+    // failed sweeps of a block; those of the next block are cleared while a slow wave may
+    // still look at these, so they lie apart
+    int32_t *const NC2 = (int32_t *)(SN + 3 * ((size_t)K * n + 64));
+    // unfold; the velocities' positions go to the snapshots' place until the links are made
+    double *Q = kPos ? X : SN;
+    for (int i = tid; i < n; i += WT)
+        for (int k = 0; k < 3; ++k) {
+            const double x0 = p.pos[k * p.n], x = p.pos[k * p.n + i];
+            const int j = i == 0 ? 0 : (int)floor(((x - x0) / edges[k]) + 0.5);
+            gim[k * n + i] = j;
+            Q[3 * i + k] = i == 0 ? x : x - j * edges[k];
+            V[3 * i + k] = p.vel[k * p.n + i];
+            if (kPos) {
+                const double r0 = gpr[k * p.n], r = gpr[k * p.n + i];
+                const int jr = i == 0 ? 0 : (int)floor(((r - r0) / edges[k]) + 0.5);
+                gpr[k * p.n + i] = i == 0 ? r : r - jr * edges[k];
+            }
+        }
+    // the spare particles lie one apart along x; the link behind the last one, theirs, has
+    // constants that keep their update harmless and in range
+    if (tid < 6) X[3 * n + tid] = V[3 * n + tid] = tid == 0 ? 1 : 0;
+    if (tid < LC) lc[(size_t)nl * LC + tid] = tid == 0 || (tid >= 5 && tid <= 7) ? 1 : tid == 8 ? 0.75 : 0;
+    __threadfence_block();
+    __syncthreads();
+    for (int l = tid; l < nl; l += WT) {
+        const int a = w.la[l], b = w.lb[l];
+        const double ma = bm.inv[((int)p.species[a] - 1) & 15], mb = bm.inv[((int)p.species[b] - 1) & 15];
+        const double d = w.dist[l];
+        double *c = lc + (size_t)l * LC;
+        double r[3], den;
+        for (int k = 0; k < 3; ++k) {
+            r[k] = kPos ? gpr[k * p.n + a] - gpr[k * p.n + b] : Q[3 * a + k] - Q[3 * b + k];
+            c[k] = r[k];
+        }
+        const double rsq = dot3b(r, r);
+        den = kPos ? (dt * (ma + mb)) * rsq : (d * d) * (ma + mb);
+        c[3] = ma;
+        c[4] = mb;
+        c[5] = den;
+        // a NaN sends the block to the general division
+        c[6] = den > 1e-90 && den < 1e90 ? 1 / den : NAN;
+        c[7] = rsq;
+        c[8] = d * d;
+    }
+    __threadfence_block();
+    __syncthreads();
+    char *const xb = (char *)X, *const vb = (char *)V, *const sb = (char *)SN;
+    // (a link from a particle to itself has r = 0: its update is NaN, or changes nothing)
+    // velocity updates of a block up to sweep ns, from the block's multipliers
+    auto velocity = [&](const uint4 e, const double *c, int) {
+        double *va = (double *)(vb + (e.x & 0xFFFF)), *vc = (double *)(vb + (e.x >> 16));
+        const double a[3] = {va[0], va[1], va[2]}, b[3] = {vc[0], vc[1], vc[2]}, g = c[5];
+        for (int k = 0; k < 3; ++k) va[k] = a[k] - (g * c[k]) * c[3];
+        for (int k = 0; k < 3; ++k) vc[k] = b[k] + (g * c[k]) * c[4];
+    };
+    // the updates of a block; kFast: false when an operand left the range of the short forms
+    auto block = [&](double *g_now, int ns, auto fast, auto limit) {
+        constexpr bool kFast = decltype(fast)::value, kLimit = decltype(limit)::value;
+        uint32_t off = 0;
+        for_steps<kPos ? 9 : 7, false, kLimit>(w, lc, nullptr, n, ns, [&](const uint4 e, const double *c, int s) {
+            double *xa = (double *)(xb + (e.x & 0xFFFF)), *xc = (double *)(xb + (e.x >> 16));
+            double *sa = (double *)(sb + e.z), *sc = (double *)(sb + e.w);
+            const double a[3] = {xa[0], xa[1], xa[2]}, b[3] = {xc[0], xc[1], xc[2]};
+            const double d[3] = {a[0] - b[0], a[1] - b[1], a[2] - b[2]};
+            double g;  // the multiplier
+            if (kPos) {
+                const double ssq = dot3b(d, d), rs = dot3b(c, d);
+                const double disc = rs * rs - c[7] * (ssq - c[8]);
+                if (kFast) {
+                    g = rs - sqrt_mid(disc);
+                    off = max(off, max(mid_off(disc), mid_off(g)));
+                } else {
+                    g = rs - sqrt(disc);
+                }
+            } else {
+                g = dot3b(d, c);
+                if (kFast) off = max(off, mid_off(g));
+            }
+            g = kFast ? div_by(g, c[5], c[6]) : g / c[5];
+            if (kFast) off = max(off, c[6] != c[6] ? 0xffffffffu : 0u);
+            const double h = kPos ? g * dt : g;
+            double na[3], nb[3];
+            for (int k = 0; k < 3; ++k) {
+                na[k] = a[k] - (h * c[k]) * c[3];
+                nb[k] = b[k] + (h * c[k]) * c[4];
+            }
+            for (int k = 0; k < 3; ++k) xa[k] = na[k];
+            for (int k = 0; k < 3; ++k) xc[k] = nb[k];
+            for (int k = 0; k < 3; ++k) sa[k] = na[k];
+            for (int k = 0; k < 3; ++k) sc[k] = nb[k];
+            if (kPos) {
+                double *at = g_now + (size_t)s * 64;
+                at[tid & 63] = g;
+            }
+        });
+        return !__any(off > MID_SPAN);
+    };
+    const std::true_type yes{};
+    const std::false_type no{};
+    int it = RATTLE_MAX + 1, conv = -1, blk = 0, ns = 0;
+    for (int base = 0; base < RATTLE_MAX && conv < 0; base += K, ++blk) {
+        ns = K < RATTLE_MAX - base ? K : RATTLE_MAX - base;
+        int32_t *const NC = NC2 + (blk & 1) * KMAX;
+        double *g_now = gg + (size_t)(blk & 1) * w.n_steps * 64;
+        if (wave == 0) {
+            for (int i = tid; i < n3; i += 64) XS[i] = X[i];
+            if (ns < K || !block(g_now, ns, yes, no)) {
+                for (int i = tid; i < n3; i += 64) X[i] = XS[i];
+                block(g_now, ns, no, yes);
+            }
+        } else if (kPos && wave == 1 && blk > 0) {
+            for_steps<5, true, false>(w, lc, gg + (size_t)((blk - 1) & 1) * w.n_steps * 64, n, K, velocity);
+        }
+        if (tid >= WT - 64 && tid - (WT - 64) < K) NC[tid - (WT - 64)] = 0 < precision ? 0 : 1;
+        __threadfence_block();
         __syncthreads();
         // the stopping test of each sweep of the block (md.f90:385-392, :454-465): a sweep
         // passes when no link reaches the precision (a NaN never does).  Items run sweep
-        // fastest, four at a time, and skip sweeps already failed.
-        if (tid < K) NC[tid] = 0 < precision ? 0 : 1;
-        __syncthreads();
+        // fastest and skip sweeps already failed.
         const int n_items = ns * nl;
-        for (int x0c = tid; x0c < n_items; x0c += 4 * BT) {
-            double err[4];
-            int qs[4];
-            bool live[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int x = x0c + u * BT;
-                const int q = x % ns, l = x / ns;
-                qs[u] = q;
-                live[u] = x < n_items && !NC[q];
-                err[u] = 0;
-                if (!live[u]) continue;
-                const int a = LAB[l] & 0xFFFF, b = LAB[l] >> 16;
-                const double *sa = snap + ((size_t)q * n + a) * 8, *sb = snap + ((size_t)q * n + b) * 8;
-                if (kPos) {
-                    double r[3];
-                    for (int k = 0; k < 3; ++k) r[k] = sa[k] - sb[k];
-                    err[u] = fabs(sqrt(dot3b(r, r)) - D[l]);
-                } else {
-                    double sv[3], dv[3];
-                    for (int k = 0; k < 3; ++k) {
-                        sv[k] = P[4 * a + k] - P[4 * b + k];
-                        dv[k] = sa[3 + k] - sb[3 + k];
-                    }
-                    err[u] = fabs(dot3b(dv, sv) / ((D[l] * D[l]) * (P[4 * a + 3] + P[4 * b + 3])));
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (live[u] && err[u] >= precision) NC[qs[u]] = 1;
+        for (int y = tid; y < n_items; y += WT) {
+            const int q = y % ns, l = y / ns;
+            if (((volatile int32_t *)NC)[q]) continue;
+            const int a = w.la[l], b = w.lb[l];
+            double r[3], err;
+            for (int k = 0; k < 3; ++k) r[k] = SN[3 * (q * n + a) + k] - SN[3 * (q * n + b) + k];
+            if (kPos)
+                err = fabs(sqrt(dot3b(r, r)) - w.dist[l]);
+            else
+                err = fabs(dot3b(r, lc + (size_t)l * LC) / lc[(size_t)l * LC + 5]);
+            if (err >= precision) NC[q] = 1;
         }
         __syncthreads();
-        int conv = -1;
         for (int q = 0; q < ns; ++q)
             if (!NC[q]) {
                 conv = q;
                 break;
             }
-        if (conv >= 0) {
-            it = base + conv + 1;
-            for (int64_t i = tid; i < n; i += BT)
-                if (V[4 * i + 3] != 0) {
-                    const double *o = snap + ((size_t)conv * n + i) * 8;
-                    for (int k = 0; k < 3; ++k) {
-                        P[4 * i + k] = o[k];
-                        V[4 * i + k] = o[3 + k];
-                    }
-                }
-            __syncthreads();
-            break;
-        }
-        __syncthreads();
+        if (conv >= 0) it = base + conv + 1;
     }
-    for (int64_t i = tid; i < n; i += BT)
+    // the velocity updates of the last block, and the state after the sweep that passed
+    if (kPos && wave == 0 && blk > 0)
+        for_steps<5, true, true>(w, lc, gg + (size_t)((blk - 1) & 1) * w.n_steps * 64, n, conv >= 0 ? conv + 1 : ns,
+                                 velocity);
+    __syncthreads();
+    for (int i = tid; i < n; i += WT) {
+        const bool put_back = conv >= 0 && w.cstart[i + 1] > w.cstart[i];
         for (int k = 0; k < 3; ++k) {
-            p.pos[k * n + i] = i == 0 ? P[4 * i + k] : P[4 * i + k] + gim[k * n + i] * edges[k];
-            p.vel[k * n + i] = V[4 * i + k];
-            if (kPos) gpr[k * n + i] = R[4 * i + k];
+            const double x = put_back ? SN[3 * (conv * n + i) + k] : X[3 * i + k];
+            if (kPos) p.pos[k * p.n + i] = i == 0 ? x : x + gim[k * n + i] * edges[k];
+            p.vel[k * p.n + i] = kPos ? V[3 * i + k] : x;
         }
+        if (!kPos && i > 0)  // unfolded and folded back as the reference does
+            for (int k = 0; k < 3; ++k) {
+                const int j = gim[k * n + i];
+                p.pos[k * p.n + i] = (p.pos[k * p.n + i] - j * edges[k]) + j * edges[k];
+            }
+    }
     if (tid == 0) out[0] = it;
 }
 
@@ -927,26 +1027,18 @@ static int fetch_i32(const int32_t *dev, int32_t *host_out)
     return RMPCD_OK;
 }
 
-// which rattle runs: the pipelined one with the largest K whose body fits in LDS, else
-// the global one (K = 0)
+// which rattle runs: the one-wave one with the most sweeps per block whose snapshots fit in
+// LDS, else the global one
 static int pick_k(Schedule &s, bool with_pr, const BlockSched **blk, size_t *lds)
 {
     *blk = nullptr;
     *lds = 0;
-    if (s.n >= 65536 || s.n_links >= (1 << 24) || s.n_links == 0) return RMPCD_OK;
-    const size_t limit = (size_t)lds_limit();
+    if (s.n > WAVE_N || s.n_links >= (1 << 24) || s.n_links == 0) return RMPCD_OK;
     for (int K = KMAX; K >= 1; --K) {
-        // a cheap bound first: every entry could be its own level
-        if (pipe_lds_bytes(s.n, s.n_links, K, 0, with_pr) > limit) continue;
-        const BlockSched *b;
-        int rc = get_block(s, K, &b);
-        if (rc) return rc;
-        const size_t need = pipe_lds_bytes(s.n, s.n_links, K, b->n_glev, with_pr);
-        if (need <= limit) {
-            *blk = b;
-            *lds = need;
-            return RMPCD_OK;
-        }
+        const size_t need = wave_lds_bytes(s.n, K, with_pr);
+        if (need > (size_t)lds_limit()) continue;
+        *lds = need;
+        return get_block(s, K, blk);
     }
     return RMPCD_OK;
 }
@@ -972,16 +1064,18 @@ static int rattle_body(rmpcd_particles_t *p, double *pos_rattle, const int32_t *
     size_t lds = 0;
     if (s && (rc = pick_k(*s, kPos, &blk, &lds))) return rc;
     if (blk) {
-        char *w = (char *)workspace(WS_AUX, 3 * (size_t)n * 4 + (size_t)blk->K * n * 64 + 512);
+        // images, the links' constants, the updates' multipliers of two blocks
+        const size_t im_b = (3 * (size_t)n * 4 + 255) & ~(size_t)255, lc_b = ((size_t)n_links + 1) * LC * 8;
+        const size_t n_ent = (size_t)blk->n_steps * 64, ahead = 64 * AHEAD;
+        char *w = (char *)workspace(WS_AUX, im_b + lc_b + (kPos ? (2 * n_ent + ahead) * 8 : 0) + 256);
         RMPCD_CHECK(w != nullptr, "%s: workspace allocation failed", who);
-        int32_t *gim = (int32_t *)w;
-        double *snap = (double *)(w + ((3 * (size_t)n * 4 + 255) & ~(size_t)255));
         if (lds > 64 * 1024)
-            RMPCD_HIP(hipFuncSetAttribute((const void *)k_rattle_pipe<kPos>,
+            RMPCD_HIP(hipFuncSetAttribute((const void *)k_rattle_wave<kPos>,
                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        PipeView pv{blk->d_ent, blk->d_gs, s->d_lab, s->d_dist, s->n_links, blk->K * s->n_links, blk->n_glev, blk->K};
-        k_rattle_pipe<kPos><<<1, BT, lds, stream()>>>(view<F64>(p), pos_rattle, pv, bm, dt, edges[0], edges[1],
-                                                       edges[2], precision, out, gim, snap);
+        const WaveView wv{blk->d_ent, s->d_la, s->d_lb, s->d_dist, s->d_cstart, s->n_links, blk->n_steps, blk->K};
+        k_rattle_wave<kPos><<<1, WT, lds, stream()>>>(view<F64>(p), pos_rattle, wv, bm, dt, edges[0], edges[1], edges[2],
+                                                      precision, out, (int32_t *)w, (double *)(w + im_b),
+                                                      (double *)(w + im_b + lc_b));
     } else {
         char *w = (char *)workspace(WS_AUX, (size_t)n * 8 + 3 * (size_t)n * 4 + 256);
         RMPCD_CHECK(w != nullptr, "%s: workspace allocation failed", who);

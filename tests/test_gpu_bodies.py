@@ -92,6 +92,39 @@ def test_rattle_body_pos_vel(gpu, n, radius, centre, edges):
     assert same_bits(g.host("vel"), want.vel)
 
 
+@pytest.mark.parametrize("case", ["at rest", "unsatisfiable", "far too large"])
+def test_rattle_body_edges(gpu, case):
+    """where the one-wave rattle leaves its usual way: multipliers of zero (a body at rest),
+    the last, shorter block of 1000 sweeps, a body beyond its 16-bit offsets and LDS"""
+    n, radius, edges = {"far too large": (2400, 14.0, np.array([60.0] * 3))}.get(case, (24, 2.0, EDGES))
+    ps, links, d, rng = sphere_body(n, radius, edges / 2, 77)
+    mass = np.array([1.0, 2.5])
+    rattle = ps.pos.copy()
+    precision = 1e-4 if case == "far too large" else 1e-11
+    if case == "at rest":
+        ps.vel[:] = 0
+    else:
+        ps.pos[:] += 0.001 * rng.normal(size=ps.pos.shape)
+    if case == "unsatisfiable":
+        d = d * (1 + 0.002 * rng.normal(size=d.shape))
+    g = to_device(ps)
+    rt, lk, dd, m, it = dev(rattle.T), host(links), host(d), (C.c_double * 2)(*mass), C.c_int32(0)
+    want, want_r = ps.copy(), rattle.copy()
+    if case != "at rest":
+        it_p = O.rattle_body_pos(want.pos, want.vel, want_r, want.species, mass, links, d, 0.01, edges, precision)
+        print(f"rattle_body_pos {case}: {it_p} sweeps", flush=True)
+        capi.call("rmpcd_rattle_body_pos", g.struct(), ptr(rt), lk, dd, len(d), m, 2, 0.01, capi.d3(edges), precision,
+                  C.byref(it))
+        assert it.value == it_p and (case != "unsatisfiable" or it_p == 1001)
+        assert np.isfinite(want.pos).all()
+        assert same_bits(g.host("pos"), want.pos) and same_bits(g.host("vel"), want.vel)
+    it_v = O.rattle_body_vel(want.pos, want.vel, want.species, mass, links, d, 0.01, edges, precision)
+    print(f"rattle_body_vel {case}: {it_v} sweeps", flush=True)
+    capi.call("rmpcd_rattle_body_vel", g.struct(), lk, dd, len(d), m, 2, 0.01, capi.d3(edges), precision, C.byref(it))
+    assert it.value == it_v
+    assert same_bits(g.host("pos"), want.pos) and same_bits(g.host("vel"), want.vel)
+
+
 def test_rattle_body_without_links(gpu):
     """no links: the first sweep passes, and the positions still go through the
     reference's unfold next to particle 1 and fold back (md.f90:343-353, 400-402)"""
