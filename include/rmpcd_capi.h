@@ -380,9 +380,10 @@ typedef struct rmpcd_dimer_config {
                                   moved only when read (at a sort or an exact skin test), by
                                   replaying their per-step additions; the same trajectory
                                   bit for bit, without the per-step pass over all solvent */
-    int32_t extra_sort_blocks; /* fused mode launch shape, 0: sort_blocks: workgroups of the
-                                  key, place and rank passes of the sorts that may follow
-                                  each MD step (they return at once when none is due) */
+    int32_t extra_sort_blocks; /* fused mode launch shape, 0: 512 or sort_blocks if fewer: at
+                                  most so many workgroups for the key, place and rank passes
+                                  of the sorts that may follow each MD step (they return at
+                                  once when none is due) */
     int32_t sort_order;        /* fused mode launch shape: how the sort passes' workgroups
                                   take their units.  0: default (2), 1: a contiguous range
                                   per workgroup, 2: XCD-grouped (the workgroups of one XCD,
@@ -391,10 +392,11 @@ typedef struct rmpcd_dimer_config {
                                   neighbours and share its L2) */
     int32_t groups;            /* fused mode launch shape: the replicas are split into this
                                   many groups of about equal particle count, each group's
-                                  collision cycle one branch of the captured graph, so that
-                                  one group's latency-bound work (colloids, sorts after MD
-                                  steps) runs beside another's streaming.  0: default (2
-                                  with two or more replicas), at most 8 and n_replicas */
+                                  collision cycle a captured graph launched on a stream of
+                                  its own, so that one group's latency-bound work (colloids,
+                                  sorts after MD steps) runs beside another's streaming.
+                                  0: default (2 where an MD step streams 100 MB or more, 1 GB
+                                  if lazy, else 1), at most 8 and n_replicas */
     int32_t collide_cells;     /* fused mode launch shape: cells (one thread each) per
                                   workgroup of the collision kernel, 64, 128 or 256; 0:
                                   default (128) */

@@ -9,7 +9,7 @@ at a time (coordinate descent, two passes):
     extra_sort_blocks  the same for the sorts that may follow each MD step
     sort_order     the sort passes' units: a contiguous range per workgroup (1) or
                    grouped by XCD (2)
-    groups         replica groups run as concurrent branches of the captured cycle
+    groups         replica groups, each a captured cycle on a stream of its own (see rmpcd_capi.h)
     collide_cells  cells (threads) per workgroup of the collision kernel (its LDS tile)
 The result is stored in a JSON table keyed by the workload; bench.py applies the entry
 of its workload when the table exists.

@@ -42,6 +42,18 @@ constexpr int PS = 32768;          // partial-sum slots per replica
 constexpr int STREAM_BLOCKS = 16384;  // stream-role blocks per replica, default and maximum
 constexpr int LAZY_STREAM_BLOCKS = 1024;  // stream-role blocks per replica in lazy mode
 constexpr int SORT_BLOCKS = 4096;     // blocks of the particle passes of a sort (all replicas), default
+// the same for the sorts that may follow an MD step: their blocks mostly return at once, and
+// fewer return sooner (cycle of 16 x L=64 FP32: 16.88 ms at 4096, 16.45 at 512, 16.55 at 256;
+// one L=24 box: 1.52 ms, 1.40, 1.41)
+constexpr int EXTRA_BLOCKS = 512;
+// Bytes that a step's streaming moves in all replicas from which they are split into two
+// groups by default (ten times as many with lazy streaming, which moves them at sorts alone).
+// Below there is too little of it to pay for a second group's launches.  FP32 cycles in runs
+// of ten and of one cycle, one group and two: 4 x L=64 (0.38 GB) 5.17, 5.18 and 4.76, 4.85 ms;
+// 4 x L=45 (0.13 GB) 2.90, 2.92 and 2.76, 2.91; 2 x L=24 (10 MB) 1.40, 1.43 and 1.38, 1.53;
+// lazy, 16 x L=64 (1.5 GB) 7.08, 7.11 and 6.91, 6.95; 4 x L=64 2.81, 2.84 and 2.74, 2.88.  Four
+// groups are slower at each of these sizes (4 x L=64: 5.81).
+constexpr int64_t GROUP_BYTES = 100000000;
 constexpr int GATHER_GRID_MUL = 4;  // the collision sort's fused gather runs on this many times the sort grid
 constexpr int SCAN_BLOCKS = 1024;     // blocks of the cell-count tile scan (all replicas)
 constexpr int CT_DEFAULT = 128;  // cells per block in the collision kernel (64, 128 or 256; 12 particles per cell
@@ -2151,30 +2163,46 @@ static int stream_blocks(const DimerSim &s)
     return (int)std::min<int64_t>((s.nmax_rep + per - 1) / per, cap);
 }
 
+// the grid of a sort pass after an MD step: no more workgroups than R of the largest replica
+// have units (a multiple of 8 for the XCD grouping)
+static unsigned extra_grid(const DimerSim &s, int R, int kind, int cap)
+{
+    const int64_t n = s.nmax_rep, nc = s.ncmax_rep;
+    const int64_t u = kind == U_KEY     ? (n + KCHUNK - 1) / KCHUNK
+                      : kind == U_SCAN  ? (nc + SCAN_TILE - 1) / SCAN_TILE
+                      : kind == U_PLACE ? (n + PT - 1) / PT + (nc + PT - 1) / PT
+                                        : (std::max(n, nc) + GT - 1) / GT;
+    return (unsigned)std::min<int64_t>((u * R + XCDS - 1) / XCDS * XCDS, cap);
+}
+
 // (each enqueue_* works on the R replicas of b's group)
 template <class F>
 static void enqueue_sort(DimerSim &s, const FB<F> &b, const FP &p, hipStream_t st, int R, int forced)
 {
     const unsigned Rr = (unsigned)R;
-    // the sorts that may follow each MD step get their own grid: when none is due their
-    // blocks only read the plan and return, and fewer blocks return sooner
-    const int nb = forced ? s.sort_blocks : s.extra_blocks;
-    k_fz_plan<F><<<1, FT, 0, st>>>(b, forced, R);
-    if (forced)
-        k_fz_key_collision<F><<<nb, FT, 0, st>>>(b, p, R);
-    else
-        k_fz_key<F><<<nb, FT, 0, st>>>(b, p, R);
+    const int nb = s.sort_blocks, nx = s.extra_blocks;
+    if (!forced) {
+        // the sorts that may follow each MD step: when none is due their blocks only read
+        // the plan and return
+        k_fz_plan<F><<<1, FT, 0, st>>>(b, 0, R);
+        k_fz_key<F><<<extra_grid(s, R, U_KEY, nx), FT, 0, st>>>(b, p, R);
+        k_fz_scan_tiles<F><<<extra_grid(s, R, U_SCAN, SCAN_BLOCKS), SCAN_T, 0, st>>>(b, R);
+        k_fz_place<F><<<extra_grid(s, R, U_PLACE, nx), FT, 0, st>>>(b, 0, R);
+        k_fz_rank<F><<<extra_grid(s, R, U_GATHER, nx), FT, 0, st>>>(b, R);
+        k_fz_commit_list<F><<<dim3(2, Rr), 1024, 0, st>>>(b, p, 0, R);
+        return;
+    }
+    k_fz_plan<F><<<1, FT, 0, st>>>(b, 1, R);
+    k_fz_key_collision<F><<<nb, FT, 0, st>>>(b, p, R);
     k_fz_scan_tiles<F><<<SCAN_BLOCKS, SCAN_T, 0, st>>>(b, R);
-    k_fz_place<F><<<nb, FT, 0, st>>>(b, forced, R);
-    if (forced && b.fuse_srd)
+    k_fz_place<F><<<nb, FT, 0, st>>>(b, 1, R);
+    if (b.fuse_srd)
         // four times the sort grid: more tiles in flight per XCD find more of the records
         // they read in its L2 (measured fetch: 1.17x the used bytes against 1.32x)
         k_fz_gather_srd<F><<<GATHER_GRID_MUL * nb, FT, 0, st>>>(b, p, R);
-    else if (forced)
-        k_fz_gather<F><<<nb, FT, 0, st>>>(b, p, R);
     else
-        k_fz_rank<F><<<nb, FT, 0, st>>>(b, R);
-    k_fz_commit_list<F><<<dim3(2, Rr), 1024, 0, st>>>(b, p, forced, R);
+        k_fz_gather<F><<<nb, FT, 0, st>>>(b, p, R);
+    k_fz_commit_list<F><<<dim3(2, Rr), 1024, 0, st>>>(b, p, 1, R);
 }
 
 // an MD step in two parts: the step kernel (the streaming), then the colloids and the
@@ -2308,89 +2336,65 @@ static std::vector<int> group_ranges(const DimerSim &s, int G)
     return r0;
 }
 
-// One collision cycle per replica group, each group's kernels captured from its own
-// stream (forked from and joined to fstream).  Group q starts after group q - 1's first
-// step kernel and then runs free, so that the groups stay out of step: the latency-bound
+// One collision cycle per replica group, a graph of its own for each, launched on the
+// group's own stream: the groups share nothing until a run ends, so that the latency-bound
 // work after one group's step (its colloids, the sort that may follow) runs while another
-// group streams.  (A dependency between streams costs about 10 us, too much to make the
-// groups take turns at every step.)  A profiled graph keeps one group, so that every
-// timed streaming launch has the device to itself.
+// group streams, over the ends of cycles too.  (One graph with a branch per group took 0.9
+// to 1.4 ms longer to start, and joined the groups at every cycle.)  A profiled run keeps
+// one group, so that every timed streaming launch has the device to itself.
 template <class F>
-static int build_graph(DimerSim &s)
+static int build_graphs(DimerSim &s)
 {
     FP p = make_fp(s);
-    hipStream_t st = s.fstream;
     const int G = s.prof_stride > 0 ? 1 : s.groups;
     const std::vector<int> r0 = group_ranges(s, G);
     bool ok = (int)r0.size() == G + 1;
     for (int q = 0; ok && q < G; ++q) ok = r0[q] < r0[q + 1];
     RMPCD_CHECK(ok, "dimer: internal error in the replica groups");
-    if (s.graph_exec) {
-        RMPCD_HIP(hipGraphExecDestroy(s.graph_exec));
-        s.graph_exec = nullptr;
-    }
-    if (s.graph) {
-        RMPCD_HIP(hipGraphDestroy(s.graph));
-        s.graph = nullptr;
-    }
-    RMPCD_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    int rc = RMPCD_OK;
-    hipError_t e = hipSuccess;
-    if (G > 1) {
-        e = hipEventRecord(s.gevents[0], st);
-        for (int q = 1; q < G && e == hipSuccess; ++q) e = hipStreamWaitEvent(s.gstreams[q - 1], s.gevents[0], 0);
-    }
-    std::vector<FB<F>> bq;
-    std::vector<hipStream_t> sq(G);
+    s.drop_graphs();
+    s.prof_pairs = 0;
     int64_t goff = 0;
     for (int q = 0; q < G; ++q) {
-        sq[q] = q == 0 ? st : s.gstreams[q - 1];
-        bq.push_back(make_fb<F>(s, r0[q], q, goff));
+        hipStream_t st = s.gstreams[q];
+        const int Rq = r0[q + 1] - r0[q];
+        const FB<F> b = make_fb<F>(s, r0[q], q, goff);
         for (int r = r0[q]; r < r0[q + 1]; ++r) goff += gather_units(s.rep[r]);
-    }
-    // the first step streams with the last force; each later step first finishes its
-    // predecessor; the last step (mode 2) is finished right before the collision
-    for (int j = 0; j <= s.cfg.n_md && e == hipSuccess; ++j) {
-        const int mode = j == 0 ? 0 : j < s.cfg.n_md ? 1 : 2;
-        for (int q = 0; q < G && e == hipSuccess; ++q) {
-            const int Rq = r0[q + 1] - r0[q];
-            // group q starts after group q - 1's first step kernel
-            if (G > 1 && j == 0 && q > 0) e = hipStreamWaitEvent(sq[q], s.gevents[G + q - 1], 0);
-            if (e != hipSuccess) break;
-            enqueue_step_kernel<F>(s, bq[q], p, sq[q], Rq, mode);
-            if (G > 1 && j == 0) e = hipEventRecord(s.gevents[G + q], sq[q]);
-            enqueue_step_rest<F>(s, bq[q], p, sq[q], Rq, mode);
+        RMPCD_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+        // the first step streams with the last force; each later step first finishes its
+        // predecessor; the last step (mode 2) is finished right before the collision
+        for (int j = 0; j <= s.cfg.n_md; ++j) {
+            const int mode = j == 0 ? 0 : j < s.cfg.n_md ? 1 : 2;
+            enqueue_step_kernel<F>(s, b, p, st, Rq, mode);
+            enqueue_step_rest<F>(s, b, p, st, Rq, mode);
         }
-    }
-    for (int q = 0; q < G && e == hipSuccess; ++q) {
-        enqueue_collision<F>(s, bq[q], p, sq[q], r0[q + 1] - r0[q]);
-        if (q > 0) {
-            e = hipEventRecord(s.gevents[q], sq[q]);
-            if (e == hipSuccess) e = hipStreamWaitEvent(st, s.gevents[q], 0);
+        enqueue_collision<F>(s, b, p, st, Rq);
+        hipGraph_t g = nullptr;
+        const hipError_t e = hipStreamEndCapture(st, &g);
+        if (e != hipSuccess) {
+            if (g) (void)hipGraphDestroy(g);
+            return set_error(RMPCD_ERR_HIP, "dimer: graph capture failed: %s", hipGetErrorString(e));
         }
+        s.graphs.push_back(g);
+        int rc;
+        if (s.prof_stride > 0 && (rc = add_stream_timers<F>(s, g))) return rc;
+        hipGraphExec_t ge;
+        RMPCD_HIP(hipGraphInstantiate(&ge, g, nullptr, nullptr, 0));
+        s.graph_execs.push_back(ge);
     }
-    hipGraph_t g = nullptr;
-    const hipError_t e_end = hipStreamEndCapture(st, &g);
-    if (e == hipSuccess) e = e_end;
-    if (rc) {
-        if (g) (void)hipGraphDestroy(g);
-        return rc;
-    }
-    if (e != hipSuccess) {
-        if (g) (void)hipGraphDestroy(g);
-        return set_error(RMPCD_ERR_HIP, "dimer: graph capture failed: %s", hipGetErrorString(e));
-    }
-    s.graph = g;
-    s.prof_pairs = 0;
-    if (s.prof_stride > 0 && (rc = add_stream_timers<F>(s, g))) return rc;
-    RMPCD_HIP(hipGraphInstantiate(&s.graph_exec, g, nullptr, nullptr, 0));
     return RMPCD_OK;
+}
+
+static int build_cycle(DimerSim &s)
+{
+    const int rc = s.cfg.form == RMPCD_FP64 ? build_graphs<F64>(s) : build_graphs<F32>(s);
+    if (rc) s.drop_graphs();  // all groups or none
+    return rc;
 }
 
 int fused_set_profile(DimerSim &s, int stride)
 {
     if (!s.fused_ready) return set_error(RMPCD_ERR_ARG, "dimer: profiling needs the fused mode");
-    RMPCD_HIP(hipStreamSynchronize(s.fstream));
+    RMPCD_HIP(hipStreamSynchronize(s.gstreams[0]));
     for (hipEvent_t e : s.prof_ev) (void)hipEventDestroy(e);
     s.prof_ev.clear();
     s.prof_stride = stride > 0 ? stride : 0;
@@ -2399,7 +2403,7 @@ int fused_set_profile(DimerSim &s, int stride)
         s.prof_ev.resize(2 * (size_t)pairs);
         for (hipEvent_t &e : s.prof_ev) RMPCD_HIP(hipEventCreate(&e));
     }
-    return s.cfg.form == RMPCD_FP64 ? build_graph<F64>(s) : build_graph<F32>(s);
+    return build_cycle(s);
 }
 
 int fused_stream_time(DimerSim &s, double *avg_ms, int32_t *samples)
@@ -2407,7 +2411,7 @@ int fused_stream_time(DimerSim &s, double *avg_ms, int32_t *samples)
     *avg_ms = 0;
     *samples = 0;
     if (s.prof_pairs == 0) return set_error(RMPCD_ERR_ARG, "dimer: no profiled run yet");
-    RMPCD_HIP(hipStreamSynchronize(s.fstream));
+    RMPCD_HIP(hipStreamSynchronize(s.gstreams[0]));
     double tot = 0;
     for (int k = 0; k < s.prof_pairs; ++k) {
         float ms = 0;
@@ -2426,7 +2430,7 @@ int fused_prepare(DimerSim &s)
     // every per-block partial of a replica must fit its PS slots
     s.stream_blocks = s.cfg.stream_blocks > 0 ? s.cfg.stream_blocks : STREAM_BLOCKS;
     s.sort_blocks = s.cfg.sort_blocks > 0 ? s.cfg.sort_blocks : SORT_BLOCKS;
-    s.extra_blocks = s.cfg.extra_sort_blocks > 0 ? s.cfg.extra_sort_blocks : s.sort_blocks;
+    s.extra_blocks = s.cfg.extra_sort_blocks > 0 ? s.cfg.extra_sort_blocks : std::min(s.sort_blocks, EXTRA_BLOCKS);
     RMPCD_CHECK(s.cfg.sort_order >= 0 && s.cfg.sort_order <= 2, "dimer: sort_order must be 0, 1 or 2");
     RMPCD_CHECK(s.cfg.groups >= 0 && s.cfg.groups <= MAX_GROUPS, "dimer: groups must be 0 to 8");
     s.sort_order = s.cfg.sort_order > 0 ? s.cfg.sort_order : 2;
@@ -2476,17 +2480,11 @@ int fused_prepare(DimerSim &s)
     if ((rc = s.alloc((void **)&s.part, (size_t)s.R * PS * 8))) return rc;
     if ((rc = s.alloc((void **)&s.rep_dev, sizeof(RepDev) * s.R))) return rc;
     if ((rc = s.alloc((void **)&s.ctl_dev, sizeof(CtlDev) * s.R))) return rc;
-    RMPCD_HIP(hipStreamCreate(&s.fstream));
-    // replica groups: streams to capture the groups after the first from, events to fork
-    // and join them
-    // (events 0 .. groups - 1: the fork, then the joins; groups .. 2 groups - 1: each
-    // group's turn at the step kernel)
-    s.groups = std::min(s.cfg.groups > 0 ? s.cfg.groups : 2, s.R);
-    for (int q = 0; q < 2 * s.groups; ++q) {
-        hipEvent_t ev;
-        RMPCD_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
-        s.gevents.push_back(ev);
-        if (q == 0 || q >= s.groups) continue;
+    s.ctl_host.resize(s.R);
+    // replica groups, each with a stream of its own
+    const bool two = 9 * (int64_t)RS * s.ntot >= (s.cfg.lazy ? 10 : 1) * GROUP_BYTES;
+    s.groups = std::min(s.cfg.groups > 0 ? s.cfg.groups : two ? 2 : 1, s.R);
+    for (int q = 0; q < s.groups; ++q) {
         hipStream_t sq;
         RMPCD_HIP(hipStreamCreate(&sq));
         s.gstreams.push_back(sq);
@@ -2535,30 +2533,37 @@ int fused_prepare(DimerSim &s)
     RMPCD_HIP(hipMemcpy(s.rep_dev, rd.data(), sizeof(RepDev) * s.R, hipMemcpyHostToDevice));
     RMPCD_HIP(hipMemcpy(s.ctl_dev, cd.data(), sizeof(CtlDev) * s.R, hipMemcpyHostToDevice));
     if (s.cfg.form == RMPCD_FP64)
-        k_fz_memb_init<F64><<<dim3(member_blocks(s), s.R), FT, 0, s.fstream>>>(make_fb<F64>(s), make_fp(s));
+        k_fz_memb_init<F64><<<dim3(member_blocks(s), s.R), FT, 0, s.gstreams[0]>>>(make_fb<F64>(s), make_fp(s));
     else
-        k_fz_memb_init<F32><<<dim3(member_blocks(s), s.R), FT, 0, s.fstream>>>(make_fb<F32>(s), make_fp(s));
+        k_fz_memb_init<F32><<<dim3(member_blocks(s), s.R), FT, 0, s.gstreams[0]>>>(make_fb<F32>(s), make_fp(s));
     RMPCD_LAUNCHED();
     RMPCD_HIP(hipDeviceSynchronize());
-    rc = s.cfg.form == RMPCD_FP64 ? build_graph<F64>(s) : build_graph<F32>(s);
-    if (rc) return rc;
+    if ((rc = build_cycle(s))) return rc;
     s.fused_ready = true;
     return RMPCD_OK;
 }
 
 int run_fused_cycles(DimerSim &s, int n_cycles)
 {
-    if (!s.fused_ready) return set_error(RMPCD_ERR_ARG, "dimer: fused mode not prepared");
-    for (int c = 0; c < n_cycles; ++c) RMPCD_HIP(hipGraphLaunch(s.graph_exec, s.fstream));
-    RMPCD_HIP(hipStreamSynchronize(s.fstream));
+    if (!s.fused_ready || s.graph_execs.empty())
+        return set_error(RMPCD_ERR_ARG, "dimer: fused mode not prepared");
+    s.synced = false;
+    for (int c = 0; c < n_cycles; ++c)
+        for (size_t q = 0; q < s.graph_execs.size(); ++q) RMPCD_HIP(hipGraphLaunch(s.graph_execs[q], s.gstreams[q]));
     return s.sync_state();
 }
 
 int DimerSim::sync_state()
 {
     if (cfg.mode != RMPCD_SIM_FUSED || !fused_ready) return RMPCD_OK;
-    std::vector<CtlDev> cd(R);
-    RMPCD_HIP(hipMemcpy(cd.data(), ctl_dev, sizeof(CtlDev) * R, hipMemcpyDeviceToHost));
+    // the control state changes in runs alone, and every run ends here
+    if (!synced) {
+        for (size_t q = 1; q < gstreams.size(); ++q) RMPCD_HIP(hipStreamSynchronize(gstreams[q]));
+        RMPCD_HIP(hipMemcpyAsync(ctl_host.data(), ctl_dev, sizeof(CtlDev) * R, hipMemcpyDeviceToHost, gstreams[0]));
+        RMPCD_HIP(hipStreamSynchronize(gstreams[0]));
+        synced = true;
+    }
+    const CtlDev *cd = ctl_host.data();
     int err = 0;
     for (int r = 0; r < R; ++r) {
         Replica &rp = rep[r];

@@ -52,14 +52,19 @@ int DimerSim::alloc(void **p, size_t bytes)
     return RMPCD_OK;
 }
 
+void DimerSim::drop_graphs()
+{
+    for (hipGraphExec_t e : graph_execs) (void)hipGraphExecDestroy(e);
+    for (hipGraph_t g : graphs) (void)hipGraphDestroy(g);
+    graph_execs.clear();
+    graphs.clear();
+}
+
 DimerSim::~DimerSim()
 {
     (void)hipDeviceSynchronize();
-    if (graph_exec) (void)hipGraphExecDestroy(graph_exec);
-    if (graph) (void)hipGraphDestroy(graph);
-    if (fstream) (void)hipStreamDestroy(fstream);
+    drop_graphs();
     for (hipStream_t st : gstreams) (void)hipStreamDestroy(st);
-    for (hipEvent_t e : gevents) (void)hipEventDestroy(e);
     for (hipEvent_t e : prof_ev) (void)hipEventDestroy(e);
     for (void *p : allocs) (void)hipFree(p);
 }

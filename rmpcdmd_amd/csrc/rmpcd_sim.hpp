@@ -86,15 +86,16 @@ struct DimerSim {
     // fused mode
     RepDev *rep_dev = nullptr;
     CtlDev *ctl_dev = nullptr;
-    hipGraphExec_t graph_exec = nullptr;
-    hipGraph_t graph = nullptr;
-    hipStream_t fstream = nullptr;
-    // replica groups, each a branch of the captured cycle; groups after the first are
-    // captured from their own streams, forked from and joined to fstream
+    // replica groups, each with the captured collision cycle of its replicas and a stream of
+    // its own for it
     int groups = 1;
     std::vector<hipStream_t> gstreams;
-    std::vector<hipEvent_t> gevents;
+    std::vector<hipGraph_t> graphs;
+    std::vector<hipGraphExec_t> graph_execs;
+    void drop_graphs();
     bool fused_ready = false;
+    std::vector<CtlDev> ctl_host;  // copy of ctl_dev, up to date while synced
+    bool synced = false;
     int prof_stride = 0, prof_pairs = 0;  // event nodes around the streaming kernel
     std::vector<hipEvent_t> prof_ev;
     std::vector<void *> allocs;
