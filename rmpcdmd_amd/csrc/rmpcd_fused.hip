@@ -156,51 +156,6 @@ __device__ inline int64_t gindex() { return (int64_t)blockIdx.x * blockDim.x + t
 
 
 
-// ---- colloid helpers (one thread, replica r; the arithmetic of k_colloid_pos,
-// k_rattle_pos, k_max_disp, k_force_nl's last block, k_force_n2, k_colloid_vel and
-// k_rattle_vel, so that both modes agree bit for bit) --------------------------------
-__device__ inline void rattle_pos_2(double *cp, double *cv, const double *pr, const int32_t *sp,
-                                    const double *mass, double d, double dt, const double *L)
-{
-    double a1[3] = {pr[0], pr[2], pr[4]}, a2[3] = {pr[1], pr[3], pr[5]};
-    double x1[3] = {cp[0], cp[2], cp[4]}, x2[3] = {cp[1], cp[3], cp[5]};
-    double r[3], s[3];
-    for (int k = 0; k < 3; ++k) {
-        r[k] = min_image(a1[k] - a2[k], L[k]);
-        s[k] = min_image(x1[k] - x2[k], L[k]);
-    }
-    double m1 = mass[(sp[0] - 1) & 1], m2 = mass[(sp[1] - 1) & 1];
-    double inv_mass = 1 / m1 + 1 / m2;
-    double rsq = (r[0] * r[0] + r[1] * r[1]) + r[2] * r[2];
-    double ssq = (s[0] * s[0] + s[1] * s[1]) + s[2] * s[2];
-    double rs = (r[0] * s[0] + r[1] * s[1]) + r[2] * s[2];
-    double g = rs - sqrt(rs * rs - rsq * (ssq - d * d));
-    g = g / ((dt * inv_mass) * rsq);
-    for (int k = 0; k < 3; ++k) {
-        cp[2 * k] = cp[2 * k] - ((g * dt) * r[k]) / m1;
-        cp[2 * k + 1] = cp[2 * k + 1] + ((g * dt) * r[k]) / m2;
-        cv[2 * k] = cv[2 * k] - (g * r[k]) / m1;
-        cv[2 * k + 1] = cv[2 * k + 1] + (g * r[k]) / m2;
-    }
-}
-
-__device__ inline void rattle_vel_2(const double *cp, double *cv, const int32_t *sp, const double *mass,
-                                    double d, const double *L)
-{
-    double m1 = mass[(sp[0] - 1) & 1], m2 = mass[(sp[1] - 1) & 1];
-    double inv_mass = 1 / m1 + 1 / m2;
-    double s[3], dv[3];
-    for (int k = 0; k < 3; ++k) {
-        s[k] = min_image(cp[2 * k] - cp[2 * k + 1], L[k]);
-        dv[k] = cv[2 * k] - cv[2 * k + 1];
-    }
-    double kk = ((dv[0] * s[0] + dv[1] * s[1]) + dv[2] * s[2]) / ((d * d) * inv_mass);
-    for (int k = 0; k < 3; ++k) {
-        cv[2 * k] = cv[2 * k] - (kk * s[k]) / m1;
-        cv[2 * k + 1] = cv[2 * k + 1] + (kk * s[k]) / m2;
-    }
-}
-
 // ---- the MD step kernel ---------------------------------------------------------------
 // Blocks [0, nbm) take the entries of the two neighbour lists (member role: a particle in
 // both lists is taken by its colloid-0 entry, so each member is handled by one thread);
@@ -445,152 +400,6 @@ __global__ void __launch_bounds__(FT) k_fz_step(FB<F> B, FP P, int mode, int nbm
     }
 }
 
-// The colloids' share of the step, one block per replica after k_fz_step (COLLOID_T
-// threads: most of the work is one thread's, and a small block starts sooner beside
-// another replica group's streaming): the member
-// partial sums in block order (deterministic), the stream-role maxima, then the
-// colloid force, compute_force_n2, Verlet velocity and RATTLE of the previous step and
-// the Verlet position step, RATTLE and skin decision of this one.
-template <class F>
-__global__ void __launch_bounds__(COLLOID_T) k_fz_colloid(FB<F> B, FP P, int mode, int nbm, int nstream)
-{
-    __shared__ double red[16];
-    __shared__ double acc[MPV];
-    __shared__ double lp[MAX_MEMBER_BLOCKS * MPV];
-    const int r = B.r0 + blockIdx.y;
-    const RepDev &rp = B.rep[r];
-    CtlDev &C = B.ctl[r];
-    if (C.error) return;
-    const bool exact = C.need_exact != 0;
-    const double *part = B.part + (int64_t)r * PS;
-    const int moff = nbm * MPV;
-    for (int q = threadIdx.x; q < nbm * MPV; q += blockDim.x) lp[q] = part[q];
-    __syncthreads();
-    if (threadIdx.x < MPV) {
-        double a = 0;
-        for (int b = 0; b < nbm; ++b) {
-            const double t = lp[b * MPV + threadIdx.x];
-            if (threadIdx.x == 8)
-                a = t > a ? t : a;
-            else
-                a = a + t;
-        }
-        acc[threadIdx.x] = a;
-    }
-    double smax = 0;
-    if (exact && mode <= 1) {
-        for (int b = threadIdx.x; b < nstream; b += blockDim.x) {
-            const double t = part[moff + b];
-            smax = t > smax ? t : smax;
-        }
-    }
-    smax = block_max(smax, red);
-    if (threadIdx.x != 0) return;
-    // the colloid state in registers: one batch of loads, one batch of stores
-    const double *L = rp.box.edges;
-    const double dt = P.dt;
-    const int cfpar = C.cfpar, fpar = C.fpar, k_since = C.k_since;
-    const int64_t md_step = C.md_step;
-    const double vmax2 = C.vmax2;
-    double cp[6], cv[6], cf[6], cfo[6], co[6], cm[2];
-    int32_t cs[2];
-    for (int q = 0; q < 6; ++q) {
-        cp[q] = B.cpos[6 * r + q];
-        cv[q] = B.cvel[6 * r + q];
-        cf[q] = B.cforce[cfpar][6 * r + q];
-        cfo[q] = B.cforce[cfpar ^ 1][6 * r + q];
-        co[q] = B.cpos_old[6 * r + q];
-    }
-    cm[0] = B.cmass[2 * r];
-    cm[1] = B.cmass[2 * r + 1];
-    cs[0] = B.cspecies[2 * r];
-    cs[1] = B.cspecies[2 * r + 1];
-    int ncf = cfpar;
-    if (mode >= 1) {
-        // switch(force, force_old) of the colloids; the new force is the list sum
-        // (single_dimer_pbc.f90:341-352), then compute_force_n2 (neighbor_list.f90:243-262)
-        ncf = cfpar ^ 1;
-        for (int q = 0; q < 6; ++q) cfo[q] = cf[q];
-        for (int cc = 0; cc < 2; ++cc) {
-            cf[cc] = 0.0 + acc[4 * cc];
-            cf[2 + cc] = 0.0 + acc[4 * cc + 1];
-            cf[4 + cc] = 0.0 + acc[4 * cc + 2];
-        }
-        double e1 = 0;
-        e1 = e1 + acc[3];
-        e1 = e1 + acc[7];
-        C.e1 = e1;
-        {
-            const double d0 = min_image(cp[0] - cp[1], L[0]);
-            const double d1 = min_image(cp[2] - cp[3], L[1]);
-            const double d2 = min_image(cp[4] - cp[5], L[2]);
-            const double r_sq = (d0 * d0 + d1 * d1) + d2 * d2;
-            const int sa = cs[0], sb = cs[1];
-            const int pc = (sa - 1) + P.cc.n1 * (sb - 1), pe = (sb - 1) + P.cc.n1 * (sa - 1);
-            double e2 = 0, e0 = 0;
-            if (r_sq <= P.cc.cut_sq[pc]) {
-                const double fr = lj_force_over_r(r_sq, P.cc.eps[pe], P.cc.sigma[pe]);
-                cf[0] = cf[0] + fr * d0;
-                cf[2] = cf[2] + fr * d1;
-                cf[4] = cf[4] + fr * d2;
-                cf[1] = cf[1] - fr * d0;
-                cf[3] = cf[3] - fr * d1;
-                cf[5] = cf[5] - fr * d2;
-                e0 = e0 + lj_energy(r_sq, P.cc.eps[pe], P.cc.sigma[pe], P.cc.cut_energy[pe]);
-            }
-            e2 = e2 + e0;
-            e2 = e2 + 0.0;
-            C.e2 = e2;
-        }
-        // colloid velocity step and RATTLE (single_dimer_pbc.f90:356-361)
-        for (int i = 0; i < 2; ++i)
-            for (int q3 = 0; q3 < 3; ++q3) {
-                const int q = 2 * q3 + i;
-                cv[q] = cv[q] + (dt * (cf[q] + cfo[q])) / (2 * cm[i]);
-            }
-        rattle_vel_2(cp, cv, cs, P.mass, P.d, L);
-        for (int q = 0; q < 6; ++q) B.cforce[ncf][6 * r + q] = cf[q];
-        C.cfpar = ncf;
-        C.fpar = fpar ^ 1;
-        C.md_step = md_step + 1;
-    }
-    if (mode <= 1) {
-        // colloid Verlet position step and RATTLE (single_dimer_pbc.f90:311-317), with the
-        // force of the last completed step
-        double cr[6];
-        for (int q = 0; q < 6; ++q) cr[q] = cp[q];
-        for (int i = 0; i < 2; ++i)
-            for (int q3 = 0; q3 < 3; ++q3) {
-                const int q = 2 * q3 + i;
-                cp[q] = (cp[q] + dt * cv[q]) + ((dt * dt) * cf[q]) / (2 * cm[i]);
-            }
-        rattle_pos_2(cp, cv, cr, cs, P.mass, P.d, dt, L);
-        for (int q = 0; q < 6; ++q) B.cpos_rattle[6 * r + q] = cr[q];
-        // maximum displacements and the skin test (single_dimer_pbc.f90:320-323)
-        double cmax = 0;
-        for (int i = 0; i < 2; ++i) {
-            const double d0 = cp[i] - co[i], d1 = cp[2 + i] - co[2 + i], d2 = cp[4 + i] - co[4 + i];
-            const double q2 = (d0 * d0 + d1 * d1) + d2 * d2;
-            cmax = q2 > cmax ? q2 : cmax;
-        }
-        const double co_max = sqrt(cmax);
-        C.co_max = co_max;
-        const int k = k_since + 1;
-        const double per = P.dt * sqrt(vmax2) * (1.0 + 1e-6) + P.slack;
-        const double mem = acc[8];
-        C.list_max2 = mem;
-        const double so_max = exact ? sqrt(mem > smax ? mem : smax) : fmax(sqrt(mem), (double)k * per);
-        C.need_sort = (co_max >= P.skin * 0.1 || so_max >= P.skin * 0.89) ? 1 : 0;
-        C.k_since = k;
-        // is the ballistic bound conclusive for the next step?
-        C.need_exact = (double)(k + 1) * per >= P.skin * 0.89 ? 1 : 0;
-    }
-    for (int q = 0; q < 6; ++q) {
-        B.cpos[6 * r + q] = cp[q];
-        B.cvel[6 * r + q] = cv[q];
-    }
-}
-
 // ---- sort -------------------------------------------------------------------------
 // The particle passes of a sort run on a fixed grid over the replicas that sort (a
 // graph cannot branch, and a grid of blocks per replica that mostly exit at once costs
@@ -694,6 +503,184 @@ __global__ void __launch_bounds__(FT) k_fz_plan(FB<F> B, int forced, int R)
             plan[1 + kind] = csum[kind];
             plan[1 + U_KINDS + 2 * (int64_t)R + (int64_t)kind * (R + 1) + carry] = csum[kind];
         }
+    }
+}
+
+// the plan of an extra sort for a group of one replica (one thread), as k_fz_plan makes it
+template <class F>
+__device__ inline void plan_one(const FB<F> &B, const RepDev &rp, CtlDev &C, int r, int sorts)
+{
+    int64_t *plan = B.plan;
+    if (!sorts) {
+        for (int j = 0; j <= U_KINDS; ++j) plan[j] = 0;
+        return;
+    }
+    const bool dfr = C.def == 0 && rp.defer != 0;
+    C.kind = dfr ? 1 : 0;
+    C.ccount = 0;
+    plan[0] = 1;
+    plan[1 + U_KINDS] = r;
+    plan[2 + U_KINDS] = 0;
+    for (int kind = 0; kind < U_KINDS; ++kind) {
+        const int64_t u = dfr && kind != U_KEY ? 0 : units_of(rp, kind, false);
+        plan[1 + kind] = u;
+        plan[3 + U_KINDS + 2 * kind] = 0;
+        plan[3 + U_KINDS + 2 * kind + 1] = u;
+    }
+}
+
+// The colloids' share of the step, one block per replica after k_fz_step (a small block
+// starts sooner beside another replica group's streaming): the member partial sums in block
+// order (deterministic), the stream-role maxima, then the colloid force, compute_force_n2,
+// Verlet velocity and RATTLE of the previous step and the Verlet position step, RATTLE and
+// skin decision of this one.
+//
+// Bound by latency: the colloid state is read before the partials are waited for, and the
+// six components of the two colloids lie on six lanes of a wave (lane 2 k + i: axis k,
+// colloid i), so that the forty FP64 divisions of a step become eleven; what belongs to no
+// component is computed on all lanes alike.  With one replica in the group (R = 1) it also
+// makes the plan of the sort that may follow, which k_fz_plan makes for several.  One L=24
+// box FP32: 7.6 -> 6.0 us a step and one launch of 3.7 us less, 1.475 -> 1.313 ms per cycle.
+__device__ inline double lane_value(double v, int lane)
+{
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), lane);
+    return __hiloint2double(hi, lo);
+}
+// the three axes of a value that colloid 0's lanes hold
+__device__ inline double lane_dot(double a, double b, int i)
+{
+    const double p = a * b;
+    return (lane_value(p, i) + lane_value(p, 2 + i)) + lane_value(p, 4 + i);
+}
+// x of colloid 0 minus x of colloid 1, on the lanes of both
+__device__ inline double lane_diff(double x, int i)
+{
+    const double y = __shfl_xor(x, 1);
+    return i == 0 ? x - y : y - x;
+}
+
+template <class F>
+__global__ void __launch_bounds__(COLLOID_T) k_fz_colloid(FB<F> B, FP P, int mode, int nbm, int nstream, int R)
+{
+    __shared__ double red[16];
+    __shared__ double acc[MPV];
+    __shared__ double lp[MAX_MEMBER_BLOCKS * MPV];
+    const int r = B.r0 + blockIdx.y;
+    const RepDev &rp = B.rep[r];
+    CtlDev &C = B.ctl[r];
+    const bool plans = R == 1 && mode <= 1;
+    if (C.error) {
+        if (plans && threadIdx.x <= U_KINDS) B.plan[threadIdx.x] = 0;
+        return;
+    }
+    const bool exact = C.need_exact != 0;
+    const double *part = B.part + (int64_t)r * PS;
+    const int moff = nbm * MPV;
+    // the colloid state, one component per lane (the lanes from 6 on hold copies)
+    const int q = threadIdx.x < 6 ? (int)threadIdx.x : 0, i = q & 1, ax = q >> 1;
+    const int cfpar = C.cfpar, fpar = C.fpar, k_since = C.k_since;
+    const int64_t md_step = C.md_step;
+    const double vmax2 = C.vmax2, dt = P.dt, L = rp.box.edges[ax];
+    double cp = B.cpos[6 * r + q], cv = B.cvel[6 * r + q], cf = B.cforce[cfpar][6 * r + q];
+    double cfo = B.cforce[cfpar ^ 1][6 * r + q];
+    const double co = B.cpos_old[6 * r + q], cm = B.cmass[2 * r + i];
+    const int cs0 = B.cspecies[2 * r], cs1 = B.cspecies[2 * r + 1];
+    for (int x = threadIdx.x; x < nbm * MPV; x += blockDim.x) lp[x] = part[x];
+    double smax = 0;
+    if (exact && mode <= 1)
+        for (int b = threadIdx.x; b < nstream; b += blockDim.x) {
+            const double t = part[moff + b];
+            smax = t > smax ? t : smax;
+        }
+    __syncthreads();
+    if (threadIdx.x < MPV) {
+        double a = 0;
+        for (int b = 0; b < nbm; ++b) {
+            const double t = lp[b * MPV + threadIdx.x];
+            if (threadIdx.x == 8)
+                a = t > a ? t : a;
+            else
+                a = a + t;
+        }
+        acc[threadIdx.x] = a;
+    }
+    smax = block_max(smax, red);
+    if (threadIdx.x >= 64) return;
+    const bool lane0 = threadIdx.x == 0, stores = threadIdx.x < 6;
+    const double m1 = P.mass[(cs0 - 1) & 1], m2 = P.mass[(cs1 - 1) & 1], m = i == 0 ? m1 : m2;
+    const double inv_mass = 1 / m1 + 1 / m2;
+    if (mode >= 1) {
+        // switch(force, force_old) of the colloids; the new force is the list sum
+        // (single_dimer_pbc.f90:341-352), then compute_force_n2 (neighbor_list.f90:243-262)
+        cfo = cf;
+        cf = 0.0 + acc[4 * i + ax];
+        const double d = min_image(lane_diff(cp, i), L);
+        const double r_sq = lane_dot(d, d, 0);
+        const int pc = (cs0 - 1) + P.cc.n1 * (cs1 - 1), pe = (cs1 - 1) + P.cc.n1 * (cs0 - 1);
+        double e2 = 0;
+        if (r_sq <= P.cc.cut_sq[pc]) {
+            const double fr = lj_force_over_r(r_sq, P.cc.eps[pe], P.cc.sigma[pe]);
+            cf = i == 0 ? cf + fr * d : cf - fr * d;
+            e2 = lj_energy(r_sq, P.cc.eps[pe], P.cc.sigma[pe], P.cc.cut_energy[pe]);
+        }
+        // colloid velocity step and RATTLE (single_dimer_pbc.f90:356-361; md.f90:298-319)
+        cv = cv + (dt * (cf + cfo)) / (2 * cm);
+        const double s = d;  // of the same positions
+        const double kk = lane_dot(lane_diff(cv, i), s, 0) / ((P.d * P.d) * inv_mass);
+        const double c = (kk * s) / m;
+        cv = i == 0 ? cv - c : cv + c;
+        if (stores) B.cforce[cfpar ^ 1][6 * r + q] = cf;
+        if (lane0) {
+            double e1 = 0;
+            e1 = e1 + acc[3];
+            e1 = e1 + acc[7];
+            C.e1 = e1;
+            C.e2 = e2;
+            C.cfpar = cfpar ^ 1;
+            C.fpar = fpar ^ 1;
+            C.md_step = md_step + 1;
+        }
+    }
+    if (mode <= 1) {
+        // colloid Verlet position step and RATTLE (single_dimer_pbc.f90:311-317;
+        // md.f90:265-296), with the force of the last completed step
+        const double cr = cp;
+        cp = (cp + dt * cv) + ((dt * dt) * cf) / (2 * cm);
+        const double rr = min_image(lane_diff(cr, i), L), s = min_image(lane_diff(cp, i), L);
+        const double rsq = lane_dot(rr, rr, 0), ssq = lane_dot(s, s, 0), rs = lane_dot(rr, s, 0);
+        double g = rs - sqrt(rs * rs - rsq * (ssq - P.d * P.d));
+        g = g / ((dt * inv_mass) * rsq);
+        const double dx = ((g * dt) * rr) / m, dv = (g * rr) / m;
+        cp = i == 0 ? cp - dx : cp + dx;
+        cv = i == 0 ? cv - dv : cv + dv;
+        if (stores) B.cpos_rattle[6 * r + q] = cr;
+        // maximum displacements and the skin test (single_dimer_pbc.f90:320-323)
+        const double dd = cp - co;
+        double cmax = 0;
+        for (int j = 0; j < 2; ++j) {
+            const double q2 = lane_dot(dd, dd, j);
+            cmax = q2 > cmax ? q2 : cmax;
+        }
+        const double co_max = sqrt(cmax);
+        const int k = k_since + 1;
+        const double per = P.dt * sqrt(vmax2) * (1.0 + 1e-6) + P.slack;
+        const double mem = acc[8];
+        const double so_max = exact ? sqrt(mem > smax ? mem : smax) : fmax(sqrt(mem), (double)k * per);
+        const int sorts = (co_max >= P.skin * 0.1 || so_max >= P.skin * 0.89) ? 1 : 0;
+        if (lane0) {
+            C.co_max = co_max;
+            C.list_max2 = mem;
+            C.need_sort = sorts;
+            C.k_since = k;
+            // is the ballistic bound conclusive for the next step?
+            C.need_exact = (double)(k + 1) * per >= P.skin * 0.89 ? 1 : 0;
+            if (plans) plan_one(B, rp, C, r, sorts);
+        }
+    }
+    if (stores) {
+        B.cpos[6 * r + q] = cp;
+        B.cvel[6 * r + q] = cv;
     }
 }
 
@@ -2184,7 +2171,7 @@ static void enqueue_sort(DimerSim &s, const FB<F> &b, const FP &p, hipStream_t s
     if (!forced) {
         // the sorts that may follow each MD step: when none is due their blocks only read
         // the plan and return
-        k_fz_plan<F><<<1, FT, 0, st>>>(b, 0, R);
+        if (R > 1) k_fz_plan<F><<<1, FT, 0, st>>>(b, 0, R);
         k_fz_key<F><<<extra_grid(s, R, U_KEY, nx), FT, 0, st>>>(b, p, R);
         k_fz_scan_tiles<F><<<extra_grid(s, R, U_SCAN, SCAN_BLOCKS), SCAN_T, 0, st>>>(b, R);
         k_fz_place<F><<<extra_grid(s, R, U_PLACE, nx), FT, 0, st>>>(b, 0, R);
@@ -2218,7 +2205,7 @@ template <class F>
 static void enqueue_step_rest(DimerSim &s, const FB<F> &b, const FP &p, hipStream_t st, int R, int mode)
 {
     k_fz_colloid<F><<<dim3(1, (unsigned)R), COLLOID_T, 0, st>>>(b, p, mode, member_blocks(s),
-                                                            mode <= 1 ? stream_blocks(s) : 0);
+                                                            mode <= 1 ? stream_blocks(s) : 0, R);
     if (mode <= 1) enqueue_sort<F>(s, b, p, st, R, 0);
 }
 
