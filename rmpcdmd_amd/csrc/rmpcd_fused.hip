@@ -54,6 +54,14 @@ constexpr int EXTRA_BLOCKS = 512;
 // lazy, 16 x L=64 (1.5 GB) 7.08, 7.11 and 6.91, 6.95; 4 x L=64 2.81, 2.84 and 2.74, 2.88.  Four
 // groups are slower at each of these sizes (4 x L=64: 5.81).
 constexpr int64_t GROUP_BYTES = 100000000;
+// Bytes that a step's eager streaming moves in a group of several replicas from which the sort
+// after the step has a launch for each particle pass: its launches run beside the other
+// group's streaming there, and its passes are faster on their own.  One launch and four,
+// FP32, a cycle and the first one, in which all replicas sort several times: 16 x L=64 (0.75
+// GB a group) 16.18, 19.5 and 16.30, 18.9 ms; 8 x L=64 8.35, 10.3 and 8.52, 9.7; 4 x L=64
+// 4.48, 5.6 and 4.76, 5.4; FP64 8 x L=64 (0.75 GB) 15.7, 18.1 and 15.7, 17.2; lazy,
+// 16 x L=64 6.5 and 6.8 a cycle.
+constexpr int64_t CHAIN_BYTES = 500000000;
 constexpr int GATHER_GRID_MUL = 4;  // the collision sort's fused gather runs on this many times the sort grid
 constexpr int SCAN_BLOCKS = 1024;     // blocks of the cell-count tile scan (all replicas)
 constexpr int CT_DEFAULT = 128;  // cells per block in the collision kernel (64, 128 or 256; 12 particles per cell
@@ -62,9 +70,11 @@ constexpr int SCAN_T = 256, SCAN_I = 8, SCAN_TILE = SCAN_T * SCAN_I;
 constexpr int MAX_TILES = 4096;  // cells per replica up to MAX_TILES * SCAN_TILE
 constexpr int MAX_STENCIL = 2048;  // stencil cells of the fused list build
 constexpr int GPT = 1, GT = FT * GPT;  // destination slots per thread and per unit of the gather
+constexpr int RANK_UNITS = 4;          // units that a workgroup of the rank pass takes together
 constexpr int GHALO = 32;              // slots staged on either side of a gather or rank unit
 constexpr int KPT = 4, KCHUNK = FT * KPT;  // particles per thread and per chunk of the key pass
 constexpr int KHASH_BITS = 11, KHASH = 1 << KHASH_BITS;  // LDS hash entries, 2 x KCHUNK
+constexpr int RANK_LDS = RANK_UNITS * GT + 2 * GHALO;
 // a replica's error flag: a list longer than its capacity (the reference's error stop),
 // or more particles near the colloids than a deferred extra sort can collect; every
 // kernel returns at once for a replica with the flag set, so it stops at that step
@@ -128,12 +138,13 @@ struct FB {
     int64_t scan_stride;
     int32_t *mslots, *mcount;  // per replica and sort buffer: the member slots of its last lists
     int64_t *plan;             // the replicas a sort chain works on (k_fz_plan)
+    int32_t *chain;            // the counters of k_fz_extra_sort
     double *gpart;             // |v|^2 maximum per gather unit
     int32_t nmax;
     int32_t xcd_order;  // sort passes: units grouped by XCD (1) or a contiguous range per workgroup (0)
     int32_t fuse_srd;   // the collision sort's gather also makes the collision (no bulk reaction)
-    // the replica group a launch works on: replicas r0 + blockIdx.y (R of them); plan and
-    // gpart are the group's own
+    // the replica group a launch works on: replicas r0 + blockIdx.y (R of them); plan,
+    // chain and gpart are the group's own
     int32_t r0;
     const RepDev *rep;
     CtlDev *ctl;
@@ -405,6 +416,7 @@ __global__ void __launch_bounds__(FT) k_fz_step(FB<F> B, FP P, int mode, int nbm
 // graph cannot branch, and a grid of blocks per replica that mostly exit at once costs
 // microseconds per launch in a large batch).  k_fz_plan lists those replicas and the
 // prefix sums of their work units per pass; a pass's blocks take contiguous unit ranges.
+constexpr int XCDS = 8;
 enum { U_KEY = 0, U_SCAN, U_PLACE, U_GATHER, U_KINDS };
 constexpr int PT = 4 * FT;  // particles or cells per place unit
 
@@ -447,6 +459,26 @@ __device__ inline int64_t units_of(const RepDev &rp, int kind, bool fused_gather
     }
 }
 
+// k_fz_extra_sort's counters, a cache line each: per pass the units done, the XCDs that worked
+// on it (a bit each), those that have written their L2 back, each XCD's election of the
+// workgroup that does, and the next ticket of each queue
+constexpr int CHAIN_STRIDE = 32, XCCS = 16;
+enum { CH_DONE = 0, CH_XCCS, CH_WROTE, CH_ELECT, CH_NEXT = CH_ELECT + XCCS, CH_LINES = CH_NEXT + XCDS };
+constexpr int CHAIN_LEN = U_KINDS * CH_LINES * CHAIN_STRIDE;
+constexpr int CHAIN_RUNS = 8;                     // runs of units of a pass per workgroup
+constexpr int HWREG_XCC_ID = (31 << 11) | 20;     // s_getreg: all of HW_REG_XCC_ID
+__device__ inline int *chain_line(int *chain, int pass, int what)
+{
+    return chain + (pass * CH_LINES + what) * CHAIN_STRIDE;
+}
+__device__ inline int chain_load(const int *c)
+{
+    return __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline void chain_wait(const int *c, int n)
+{
+    while (chain_load(c) < n) __builtin_amdgcn_s_sleep(16);
+}
 // plan layout (int64), for a group of R replicas from r0 on: [0] active count, [1 + kind]
 // total units, then act[R] (replica of active index a), amap[R] (active index of replica
 // r0 + j at j, or -1), pre[kind][R + 1]
@@ -497,6 +529,8 @@ __global__ void __launch_bounds__(FT) k_fz_plan(FB<F> B, int forced, int R)
         }
         carry += tot;
     }
+    static_assert(CHAIN_LEN / CHAIN_STRIDE <= FT, "a thread per counter");
+    if (threadIdx.x < CHAIN_LEN / CHAIN_STRIDE) B.chain[threadIdx.x * CHAIN_STRIDE] = 0;
     if (threadIdx.x == 0) {
         plan[0] = carry;
         for (int kind = 0; kind < U_KINDS; ++kind) {
@@ -518,6 +552,7 @@ __device__ inline void plan_one(const FB<F> &B, const RepDev &rp, CtlDev &C, int
     const bool dfr = C.def == 0 && rp.defer != 0;
     C.kind = dfr ? 1 : 0;
     C.ccount = 0;
+    for (int j = 0; j < CHAIN_LEN; j += CHAIN_STRIDE) B.chain[j] = 0;
     plan[0] = 1;
     plan[1 + U_KINDS] = r;
     plan[2 + U_KINDS] = 0;
@@ -703,7 +738,6 @@ __device__ inline int find_unit(const int64_t *pre, int nact, int64_t u)
 // workgroups go to the XCDs in turn) share a contiguous eighth of the units, interleaved:
 // the units in flight on an XCD are then neighbours, whose particles come from, and go
 // to, the same stretch of memory, cached once in that XCD's L2
-constexpr int XCDS = 8;
 struct UnitRange {
     int64_t u0, u1, step;
     int nact;
@@ -737,19 +771,15 @@ __device__ inline UnitRange unit_range(const int64_t *plan, int R, int kind, int
 // then one global atomic per distinct key reserves the chunk's slots in that cell
 // (arrival order within a cell is made stable by the gather).  The block with a
 // replica's first chunk records the grid shift and wraps the colloids.
+// hbuf (3 KHASH) is the LDS hash (hkey, hcnt, occ); a collision sort stages each slab of FT
+// records in the same memory before the hash is built.
 template <class F, int kForced>
-__device__ inline void key_pass(const FB<F> &B, const FP &P, int R)
+__device__ inline void key_pass(const FB<F> &B, const FP &P, const UnitRange &w, int *hbuf, int *lds, double *red)
 {
     constexpr int forced = kForced;
     using Rl = typename F::real;
-    // the LDS hash (hkey, hcnt, occ); a collision sort stages each slab of FT records in
-    // the same memory before the hash is built
-    __shared__ __align__(16) int hbuf[3 * KHASH];
     int *hkey = hbuf, *hcnt = hbuf + KHASH, *occ = hbuf + 2 * KHASH;
     static_assert(sizeof(typename FB<F>::Rec) * FT <= sizeof(int) * 3 * KHASH, "record slab in the hash LDS");
-    __shared__ int lds[FT / 64];
-    __shared__ double red[16];
-    const UnitRange w = unit_range(B.plan, R, U_KEY, B.xcd_order);
     int a = -1;
     for (int64_t u = w.u0; u < w.u1; u += w.step) {
         if (a < 0 || u >= w.pre[a + 1]) a = find_unit(w.pre, w.nact, u);
@@ -1019,26 +1049,31 @@ __device__ inline void key_pass(const FB<F> &B, const FP &P, int R)
     }
 }
 
-// the collision sort's key pass and the extra sorts' one are separate kernels, so that
-// each is given the registers of its own path (the collision sort's fits six waves per SIMD)
+// the collision sort's key pass has a kernel of its own, so that it is given the registers of
+// its own path (it fits six waves per SIMD)
 template <class F>
 __global__ void __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(6))) k_fz_key_collision(FB<F> B, FP P, int R)
 {
-    key_pass<F, 1>(B, P, R);
+    __shared__ __align__(16) int hbuf[3 * KHASH];
+    __shared__ int lds[FT / 64];
+    __shared__ double red[16];
+    key_pass<F, 1>(B, P, unit_range(B.plan, R, U_KEY, B.xcd_order), hbuf, lds, red);
 }
+
 template <class F>
 __global__ void __launch_bounds__(FT) k_fz_key(FB<F> B, FP P, int R)
 {
-    key_pass<F, 0>(B, P, R);
+    __shared__ __align__(16) int hbuf[3 * KHASH];
+    __shared__ int lds[FT / 64];
+    __shared__ double red[16];
+    key_pass<F, 0>(B, P, unit_range(B.plan, R, U_KEY, B.xcd_order), hbuf, lds, red);
 }
 
 // S2: exclusive scan of the new cell counts inside tiles of SCAN_TILE cells (tile-local
 // offsets into slocal, tile totals into scan_sums); a unit is a tile
 template <class F>
-__global__ void __launch_bounds__(SCAN_T) k_fz_scan_tiles(FB<F> B, int R)
+__device__ inline void scan_pass(const FB<F> &B, const UnitRange &w, int *lds)
 {
-    __shared__ int lds[SCAN_T / 64];
-    const UnitRange w = unit_range(B.plan, R, U_SCAN, B.xcd_order);
     int a = -1;
     for (int64_t u = w.u0; u < w.u1; u += w.step) {
         if (a < 0 || u >= w.pre[a + 1]) a = find_unit(w.pre, w.nact, u);
@@ -1066,6 +1101,13 @@ __global__ void __launch_bounds__(SCAN_T) k_fz_scan_tiles(FB<F> B, int R)
     }
 }
 
+template <class F>
+__global__ void __launch_bounds__(SCAN_T) k_fz_scan_tiles(FB<F> B, int R)
+{
+    __shared__ int lds[SCAN_T / 64];
+    scan_pass<F>(B, unit_range(B.plan, R, U_SCAN, B.xcd_order), lds);
+}
+
 // S3: a unit is PT particles (pair[start + slot] = (reference position, storage index))
 // or PT cells (the final
 // cell_start = tile-local offset + tile prefix); the tile prefix of a replica is scanned
@@ -1075,13 +1117,10 @@ __global__ void __launch_bounds__(SCAN_T) k_fz_scan_tiles(FB<F> B, int R)
 // use (only those can hold a force; the gather copies forces only where they are
 // non-zero).
 template <class F>
-__global__ void __launch_bounds__(FT) k_fz_place(FB<F> B, int forced, int R)
+__device__ inline void place_pass(const FB<F> &B, int forced, const UnitRange &w, int *pre, int *lds, int &r_pre)
 {
     using Rl = typename F::real;
-    __shared__ int pre[MAX_TILES];
-    __shared__ int lds[FT / 64];
-    const UnitRange w = unit_range(B.plan, R, U_PLACE, B.xcd_order);
-    int a = -1, r_pre = -1;
+    int a = -1;
     for (int64_t u = w.u0; u < w.u1; u += w.step) {
         if (a < 0 || u >= w.pre[a + 1]) a = find_unit(w.pre, w.nact, u);
         const int r = (int)w.act[a];
@@ -1150,28 +1189,38 @@ __global__ void __launch_bounds__(FT) k_fz_place(FB<F> B, int forced, int R)
     }
 }
 
+template <class F>
+__global__ void __launch_bounds__(FT) k_fz_place(FB<F> B, int forced, int R)
+{
+    __shared__ int pre[MAX_TILES];
+    __shared__ int lds[FT / 64];
+    int r_pre = -1;
+    place_pass<F>(B, forced, unit_range(B.plan, R, U_PLACE, B.xcd_order), pre, lds, r_pre);
+}
+
 // The reference positions of the GHALO slots on either side of a unit's tile, so that
 // the rank of a particle in a cell that straddles the tile edge reads LDS only (a cell
 // holds far fewer than GHALO particles at the densities of the programs; a larger one
 // reads the rest from memory).
 __device__ inline void load_halo(int32_t *lv, int32_t *lk, const int2 *pair, const int32_t *dkey, int64_t t0,
-                                 int64_t n)
+                                 int gt, int64_t n)
 {
     for (int q = threadIdx.x; q < 2 * GHALO; q += FT) {
-        const int64_t j = q < GHALO ? t0 - GHALO + q : t0 + GT + (q - GHALO);
+        const int64_t j = q < GHALO ? t0 - GHALO + q : t0 + gt + (q - GHALO);
         const bool in = j >= 0 && j < n;
         const int2 pr = in ? pair[j] : make_int2(INT32_MAX, 0);
-        lv[q < GHALO ? q : GT + q] = pr.x;
-        if (dkey) lk[q < GHALO ? q : GT + q] = in ? dkey[pr.y] : INT32_MAX;
+        lv[q < GHALO ? q : gt + q] = pr.x;
+        if (dkey) lk[q < GHALO ? q : gt + q] = in ? dkey[pr.y] : INT32_MAX;
     }
 }
 
 // rank_in_cell when the previous extra sort was deferred: the reference order is (the
 // deferred sort's cell, then the order before it), lexicographic
 __device__ inline int rank_in_cell_deferred(const int32_t *lv, const int32_t *lk, const int2 *pair,
-                                            const int32_t *dkey, int64_t t0, int s, int m, int32_t ref, int32_t dk)
+                                            const int32_t *dkey, int64_t t0, int gt, int s, int m, int32_t ref,
+                                            int32_t dk)
 {
-    const int64_t w0 = t0 - GHALO, w1 = t0 + GT + GHALO;
+    const int64_t w0 = t0 - GHALO, w1 = t0 + gt + GHALO;
     const int lo = (int)(s > w0 ? s : w0), hi = (int)(s + m < w1 ? s + m : w1);
     int rank = 0;
     for (int e = lo; e < hi; ++e) {
@@ -1189,11 +1238,12 @@ __device__ inline int rank_in_cell_deferred(const int32_t *lv, const int32_t *lk
 }
 
 // The number of a cell's arrivals [s, s + m) whose reference position is below ref: the
-// window [t0 - GHALO, t0 + GT + GHALO) staged in LDS, anything outside it read from
+// window [t0 - GHALO, t0 + gt + GHALO) staged in LDS, anything outside it read from
 // memory (two separate loops, so that the common one is LDS only).
-__device__ inline int rank_in_cell(const int32_t *lv, const int2 *pair, int64_t t0, int s, int m, int32_t ref)
+__device__ inline int rank_in_cell(const int32_t *lv, const int2 *pair, int64_t t0, int gt, int s, int m,
+                                   int32_t ref)
 {
-    const int64_t w0 = t0 - GHALO, w1 = t0 + GT + GHALO;
+    const int64_t w0 = t0 - GHALO, w1 = t0 + gt + GHALO;
     const int lo = (int)(s > w0 ? s : w0), hi = (int)(s + m < w1 ? s + m : w1);
     int rank = 0;
     const int32_t *l = lv - w0;
@@ -1270,14 +1320,14 @@ __device__ inline void gather_pass(const FB<F> &B, const FP &P, int R)
             dk[h] = dkey ? dkey[vs[h]] : 0;
             if (dkey) lkey[GHALO + h * FT + threadIdx.x] = v[h] == INT32_MAX ? INT32_MAX : dk[h];
         }
-        load_halo(ltmp, lkey, pair, dkey, t0, n);
+        load_halo(ltmp, lkey, pair, dkey, t0, GT, n);
         __syncthreads();
         double vm = 0;
         for (int h = 0; h < GPT; ++h) {
             if (v[h] == INT32_MAX) continue;
             const int64_t d =
-                s0[h] + (dkey ? rank_in_cell_deferred(ltmp, lkey, pair, dkey, t0, s0[h], m0[h], v[h], dk[h])
-                              : rank_in_cell(ltmp, pair, t0, s0[h], m0[h], v[h]));
+                s0[h] + (dkey ? rank_in_cell_deferred(ltmp, lkey, pair, dkey, t0, GT, s0[h], m0[h], v[h], dk[h])
+                              : rank_in_cell(ltmp, pair, t0, GT, s0[h], m0[h], v[h]));
             const int fl = q[h].flags();
             const bool has_f = (fl & (MD_MASK | PAST_MD_MASK)) != 0;
             double v2 = 0;
@@ -1324,14 +1374,17 @@ __global__ void __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(8))) k_
 // read from LDS within the unit) gives its new reference position d: perm[d] = storage
 // index, inv[storage index] = d.  Clears the previous cell counts and the is_md/is_reac
 // marks like the gather.
-template <class F>
-__global__ void __launch_bounds__(FT) k_fz_rank(FB<F> B, int R)
+// up to kUnits units of one replica are taken together, their loads in flight together
+template <class F, int kUnits>
+__device__ inline void rank_pass(const FB<F> &B, const UnitRange &w, int32_t *lref, int32_t *lkey)
 {
-    __shared__ int32_t lref[GT + 2 * GHALO], lkey[GT + 2 * GHALO];
-    const UnitRange w = unit_range(B.plan, R, U_GATHER, B.xcd_order);
+    static_assert(GPT == 1, "a slot per thread and unit");
     int a = -1;
     for (int64_t u = w.u0; u < w.u1; u += w.step) {
         if (a < 0 || u >= w.pre[a + 1]) a = find_unit(w.pre, w.nact, u);
+        int64_t e = w.u1 < w.pre[a + 1] ? w.u1 : w.pre[a + 1];
+        if (e > u + kUnits || w.step > 1) e = u + (w.step > 1 ? 1 : kUnits);
+        const int Q = (int)(e - u), gt = Q * FT;
         const int r = (int)w.act[a];
         const int64_t t0 = (u - w.pre[a]) * GT;
         const CtlDev &C = B.ctl[r];
@@ -1342,43 +1395,159 @@ __global__ void __launch_bounds__(FT) k_fz_rank(FB<F> B, int R)
         int32_t *perm = B.perm + rp.p_off, *inv = B.inv + rp.p_off;
         const int32_t *start = B.start + rp.c_off, *cnt = B.count[C.cnt ^ 1] + rp.c_off;
         int32_t *old_cnt = B.count[C.cnt] + rp.c_off;
-        int32_t ref[GPT], sto[GPT], s0[GPT], m0[GPT];
+        int32_t ref[kUnits], sto[kUnits], s0[kUnits], m0[kUnits], dk[kUnits];
         __syncthreads();
-        for (int h = 0; h < GPT; ++h) {
+        for (int h = 0; h < kUnits; ++h) {
             const int64_t j = t0 + h * FT + threadIdx.x;
-            const int2 pr = pair[j < n ? j : n - 1];
-            ref[h] = j < n ? pr.x : INT32_MAX;
+            const bool in = h < Q && j < n;
+            const int2 pr = pair[in ? j : n - 1];
+            ref[h] = in ? pr.x : INT32_MAX;
             sto[h] = pr.y;
-            lref[GHALO + h * FT + threadIdx.x] = ref[h];
         }
         const int32_t *dkey = C.def ? B.dkey + rp.p_off : nullptr;
-        int32_t dk[GPT];
-        for (int h = 0; h < GPT; ++h) {
+        int c[kUnits];
+        for (int h = 0; h < kUnits; ++h) {
             dk[h] = dkey ? dkey[sto[h]] : 0;
-            if (dkey) lkey[GHALO + h * FT + threadIdx.x] = ref[h] == INT32_MAX ? INT32_MAX : dk[h];
+            c[h] = key[sto[h]];
         }
-        load_halo(lref, lkey, pair, dkey, t0, n);
-        for (int h = 0; h < GPT; ++h) {
-            const int c = key[sto[h]];
-            s0[h] = start[c];
-            m0[h] = cnt[c];
+        for (int h = 0; h < kUnits; ++h) {
+            s0[h] = start[c[h]];
+            m0[h] = cnt[c[h]];
         }
+        for (int h = 0; h < kUnits; ++h)
+            if (h < Q) {
+                lref[GHALO + h * FT + threadIdx.x] = ref[h];
+                if (dkey) lkey[GHALO + h * FT + threadIdx.x] = ref[h] == INT32_MAX ? INT32_MAX : dk[h];
+            }
+        load_halo(lref, lkey, pair, dkey, t0, gt, n);
         __syncthreads();
-        for (int h = 0; h < GPT; ++h) {
+        for (int h = 0; h < kUnits; ++h) {
             if (ref[h] == INT32_MAX) continue;
             const int32_t d =
-                s0[h] + (dkey ? rank_in_cell_deferred(lref, lkey, pair, dkey, t0, s0[h], m0[h], ref[h], dk[h])
-                              : rank_in_cell(lref, pair, t0, s0[h], m0[h], ref[h]));
+                s0[h] + (dkey ? rank_in_cell_deferred(lref, lkey, pair, dkey, t0, gt, s0[h], m0[h], ref[h], dk[h])
+                              : rank_in_cell(lref, pair, t0, gt, s0[h], m0[h], ref[h]));
             perm[d] = sto[h];
             inv[sto[h]] = d;
         }
-        for (int h = 0; h < GPT; ++h) {
+        for (int h = 0; h < Q; ++h) {
             const int64_t jc = t0 + h * FT + threadIdx.x;
             if (jc < nc) {
                 old_cnt[jc] = 0;
                 B.is_md[rp.c_off + jc] = 0;
                 B.is_reac[rp.c_off + jc] = 1;
             }
+        }
+        if (w.step == 1) u = e - 1;
+    }
+}
+
+template <class F>
+__global__ void __launch_bounds__(FT) k_fz_rank(FB<F> B, int R)
+{
+    __shared__ int32_t lref[GT + 2 * GHALO], lkey[GT + 2 * GHALO];
+    rank_pass<F, 1>(B, unit_range(B.plan, R, U_GATHER, B.xcd_order), lref, lkey);
+}
+
+// The particle passes of the sort that may follow an MD step: key, tile scan, place and rank
+// in one launch (see CHAIN_BYTES for when).  Mostly no sort is due, and four launches that only read the plan and return
+// took 10 us of the 26 us step of one L=24 box.  Each pass is dealt out by tickets (runs of
+// units), from a queue for each XCD's eighth of the units, then from the other queues; a
+// workgroup begins a pass when every unit of the pass before is done.  When a workgroup finds
+// all queues empty, each of their tickets is held by a workgroup that runs and waits for
+// nothing in this pass, so every wait ends whatever number of workgroups the device holds at
+// once.  Between two passes the L2 of each XCD that worked on the first is written back, once,
+// by the first of its workgroups to see that all units are done (a write-back by each workgroup
+// took 40 us a pass with 64 of them on an XCD).  A full sort takes longer than in four launches
+// (L=24 75 us against 39, L=64 300 against 196), but most steps have none: L=24 FP32 1.31 ->
+// 1.08 ms per cycle, L=48 FP64 1.96 -> 1.76, 4 x L=45 FP32 lazy 2.16 -> 1.96.
+template <class F>
+__global__ void __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4))) k_fz_extra_sort(FB<F> B, FP P, int R)
+{
+    __shared__ __align__(16) int buf[3 * KHASH];
+    static_assert(MAX_TILES <= 3 * KHASH && 2 * RANK_LDS <= 3 * KHASH, "the passes share their LDS");
+    static_assert(U_KEY == 0 && U_SCAN == 1 && U_PLACE == 2 && U_GATHER == 3 && SCAN_T == FT, "order of the passes");
+    __shared__ int lds[FT / 64], unit;
+    __shared__ double red[16];
+    if (B.plan[0] == 0) return;
+    const int xcc = (int)(__builtin_amdgcn_s_getreg(HWREG_XCC_ID) & (XCCS - 1));
+    int r_pre = -1;
+    for (int p = 0; p < U_KINDS; ++p) {
+        const int T = (int)B.plan[1 + p];
+        if (T == 0) return;  // deferred sorts alone: no pass after the keys
+        if (p > 0) {
+            if (threadIdx.x == 0) {
+                chain_wait(chain_line(B.chain, p - 1, CH_DONE), (int)B.plan[p]);
+                const int m = chain_load(chain_line(B.chain, p - 1, CH_XCCS));
+                int *wrote = chain_line(B.chain, p - 1, CH_WROTE);
+                if ((m >> xcc & 1) && atomicAdd(chain_line(B.chain, p - 1, CH_ELECT + xcc), 1) == 0) {
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+                    atomicAdd(wrote, 1);
+                }
+                chain_wait(wrote, __popc((unsigned)m));
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            }
+            __syncthreads();
+        }
+        const int eighth = (T + XCDS - 1) / XCDS, run = (T + CHAIN_RUNS * (int)gridDim.x - 1) / (CHAIN_RUNS * (int)gridDim.x);
+        int *next = chain_line(B.chain, p, CH_NEXT);
+        int x = (int)blockIdx.x % XCDS, mine = 0, t = 0;
+        if (threadIdx.x == 0) t = atomicAdd(&next[x * CHAIN_STRIDE], 1);
+        for (;;) {
+            if (threadIdx.x < 64) {
+                const int lane = threadIdx.x;
+                int u = -1;
+                for (;;) {
+                    const int in = __builtin_amdgcn_readfirstlane(t) * run;
+                    if (in < eighth && x * eighth + in < T) {
+                        u = x * eighth + in;
+                        break;
+                    }
+                    // this queue is empty: the first one after it that is not
+                    bool more = false;
+                    if (lane < XCDS) {
+                        const int c = chain_load(&next[lane * CHAIN_STRIDE]) * run;
+                        more = c < eighth && lane * eighth + c < T;
+                    }
+                    const unsigned m = (unsigned)__ballot(more);
+                    if (m == 0) break;
+                    const unsigned rot = (m | (m << XCDS)) >> x;
+                    x = (x + __builtin_ctz(rot)) % XCDS;
+                    if (lane == 0) t = atomicAdd(&next[x * CHAIN_STRIDE], 1);
+                }
+                if (lane == 0) {
+                    unit = u;
+                    // the ticket after this one arrives during its work
+                    if (u >= 0) t = atomicAdd(&next[x * CHAIN_STRIDE], 1);
+                }
+            }
+            __syncthreads();
+            const int u0 = unit;
+            x = u0 >= 0 ? u0 / eighth : x;
+            __syncthreads();
+            if (u0 < 0) break;
+            UnitRange w;
+            w.u0 = u0;
+            w.u1 = min(min(u0 + run, (x + 1) * eighth), T);
+            w.step = 1;
+            w.nact = (int)B.plan[0];
+            w.pre = plan_pre(B.plan, R, p);
+            w.act = plan_act(B.plan);
+            if (mine == 0 && threadIdx.x == 0) atomicOr(chain_line(B.chain, p, CH_XCCS), 1 << xcc);
+            mine += (int)(w.u1 - w.u0);
+            if (p == U_KEY)
+                key_pass<F, 0>(B, P, w, buf, lds, red);
+            else if (p == U_SCAN)
+                scan_pass<F>(B, w, lds);
+            else if (p == U_PLACE)
+                place_pass<F>(B, 0, w, buf, lds, r_pre);
+            else
+                rank_pass<F, RANK_UNITS>(B, w, buf, buf + RANK_LDS);
+        }
+        if (mine && p + 1 < U_KINDS) {
+            // every wave's stores have reached the L2
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (threadIdx.x == 0) atomicAdd(chain_line(B.chain, p, CH_DONE), mine);
         }
     }
 }
@@ -2091,6 +2260,7 @@ static FB<F> make_fb(DimerSim &s, int r0 = 0, int g = 0, int64_t gpart_off = 0)
     b.scan_sums = s.scan_sums;
     b.mslots = s.f_mslots;
     b.plan = s.f_plan + g * plan_len(s.R);
+    b.chain = s.f_chain + g * CHAIN_LEN;
     b.gpart = s.f_gpart + gpart_off;
     b.r0 = r0;
     b.mcount = s.f_mcount;
@@ -2150,16 +2320,11 @@ static int stream_blocks(const DimerSim &s)
     return (int)std::min<int64_t>((s.nmax_rep + per - 1) / per, cap);
 }
 
-// the grid of a sort pass after an MD step: no more workgroups than R of the largest replica
-// have units (a multiple of 8 for the XCD grouping)
-static unsigned extra_grid(const DimerSim &s, int R, int kind, int cap)
+// the grid of the sort that may follow an MD step: no more workgroups than R of the largest
+// replica have key units (more make the passes of an L=24 box 92 us instead of 75)
+static unsigned extra_grid(const DimerSim &s, int R)
 {
-    const int64_t n = s.nmax_rep, nc = s.ncmax_rep;
-    const int64_t u = kind == U_KEY     ? (n + KCHUNK - 1) / KCHUNK
-                      : kind == U_SCAN  ? (nc + SCAN_TILE - 1) / SCAN_TILE
-                      : kind == U_PLACE ? (n + PT - 1) / PT + (nc + PT - 1) / PT
-                                        : (std::max(n, nc) + GT - 1) / GT;
-    return (unsigned)std::min<int64_t>((u * R + XCDS - 1) / XCDS * XCDS, cap);
+    return (unsigned)std::min<int64_t>((s.nmax_rep + KCHUNK - 1) / KCHUNK * R, s.extra_blocks);
 }
 
 // (each enqueue_* works on the R replicas of b's group)
@@ -2167,15 +2332,22 @@ template <class F>
 static void enqueue_sort(DimerSim &s, const FB<F> &b, const FP &p, hipStream_t st, int R, int forced)
 {
     const unsigned Rr = (unsigned)R;
-    const int nb = s.sort_blocks, nx = s.extra_blocks;
+    const int nb = s.sort_blocks;
     if (!forced) {
-        // the sorts that may follow each MD step: when none is due their blocks only read
-        // the plan and return
+        // the sort that may follow an MD step: when none is due its blocks only read the plan
+        // and return
         if (R > 1) k_fz_plan<F><<<1, FT, 0, st>>>(b, 0, R);
-        k_fz_key<F><<<extra_grid(s, R, U_KEY, nx), FT, 0, st>>>(b, p, R);
-        k_fz_scan_tiles<F><<<extra_grid(s, R, U_SCAN, SCAN_BLOCKS), SCAN_T, 0, st>>>(b, R);
-        k_fz_place<F><<<extra_grid(s, R, U_PLACE, nx), FT, 0, st>>>(b, 0, R);
-        k_fz_rank<F><<<extra_grid(s, R, U_GATHER, nx), FT, 0, st>>>(b, R);
+        const int nx = s.extra_blocks;
+        int64_t n = 0;
+        for (int r = b.r0; r < b.r0 + R; ++r) n += s.rep[r].n;
+        if (R == 1 || s.cfg.lazy || 9 * (int64_t)sizeof(typename F::real) * n < CHAIN_BYTES) {
+            k_fz_extra_sort<F><<<extra_grid(s, R), FT, 0, st>>>(b, p, R);
+        } else {
+            k_fz_key<F><<<nx, FT, 0, st>>>(b, p, R);
+            k_fz_scan_tiles<F><<<nx, SCAN_T, 0, st>>>(b, R);
+            k_fz_place<F><<<nx, FT, 0, st>>>(b, 0, R);
+            k_fz_rank<F><<<nx, FT, 0, st>>>(b, R);
+        }
         k_fz_commit_list<F><<<dim3(2, Rr), 1024, 0, st>>>(b, p, 0, R);
         return;
     }
@@ -2460,6 +2632,7 @@ int fused_prepare(DimerSim &s)
     if ((rc = s.alloc((void **)&s.f_slocal, s.nctot * 4))) return rc;
     if ((rc = s.alloc((void **)&s.f_mslots, (size_t)s.R * 4 * s.nmax * 4))) return rc;
     if ((rc = s.alloc((void **)&s.f_plan, MAX_GROUPS * plan_len(s.R) * 8))) return rc;
+    if ((rc = s.alloc((void **)&s.f_chain, MAX_GROUPS * CHAIN_LEN * 4))) return rc;
     int64_t gunits = 0;
     for (const Replica &rp : s.rep) gunits += gather_units(rp);
     if ((rc = s.alloc((void **)&s.f_gpart, (size_t)gunits * 8))) return rc;

@@ -79,6 +79,7 @@ struct DimerSim {
     int32_t *f_key = nullptr, *f_slot = nullptr, *scan_sums = nullptr, *f_slocal = nullptr;
     int32_t *f_mslots = nullptr, *f_mcount = nullptr;
     int64_t *f_plan = nullptr;
+    int32_t *f_chain = nullptr;
     double *f_gpart = nullptr;
     double *part = nullptr;
     void *scratch = nullptr;

@@ -318,3 +318,24 @@ def test_many_extra_sorts_per_cycle(gpu, form):
     lazy.close()
     odd.close()
     flat.close()
+
+
+@pytest.mark.parametrize("form", [capi.FP64, capi.FP32])
+def test_extra_sort_workgroups(gpu, form):
+    """the sort after an MD step is one launch whose passes wait for each other: with one
+    workgroup, with fewer than there are XCDs, with a number that is no multiple of them and
+    with as many as there are units, for boxes of one and of several scan tiles, it must
+    give the same state bit for bit"""
+    Ls = [(24, 24, 20), (12, 16, 12)]
+    kw = dict(mode=capi.SIM_FUSED, n_md=40, tau=0.5, form=form, seed=77, replica_L=Ls, skin=0.6)
+    sims = [SingleDimer(**kw)] + [SingleDimer(extra_sort_blocks=b, groups=g, **kw)
+                                  for b, g in ((1, 1), (5, 2), (77, 1))]
+    for s in sims:
+        s.run(2)
+    for r in range(len(Ls)):
+        a = sims[0].download(r)
+        assert a["n_extra_sorting"] >= 4, "replica %d" % r
+        for k, s in enumerate(sims[1:]):
+            compare(a, s.download(r), "replica %d, launch shape %d" % (r, k), rtol=0.0)
+    for s in sims:
+        s.close()
