@@ -66,7 +66,7 @@ struct Schedule {
     // by link: a, b, distance; per particle: the links
     // touching it in link order (bit 31 set where it is the second particle)
     int32_t *d_la = nullptr, *d_lb = nullptr;
-        double *d_dist = nullptr;
+    double *d_dist = nullptr;
     int32_t *d_cstart = nullptr, *d_csr = nullptr;
     void *block = nullptr;
     BlockSched blocks[KMAX + 1];  // by K, built on first use
