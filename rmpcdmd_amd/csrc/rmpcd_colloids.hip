@@ -356,9 +356,7 @@ __global__ void __launch_bounds__(CG_T) k_cg_key(SolB<F> S, const ColCtl *C, int
                 }
                 CgRec<R> r;
                 for (int q = 0; q < 3; ++q) {
-                    const R ed = (R)b.edges[q];
-                    const int jump = (int)floor((double)(x[q] / ed));
-                    x[q] = x[q] - (R)jump * ed;
+                    const int jump = fold_pbc<R>(x[q], (R)b.edges[q]);
                     r.p[q] = x[q];
                     r.v[q] = vv[q];
                     r.im[q] = img[q * n + i] + jump;
@@ -442,16 +440,6 @@ __global__ void __launch_bounds__(CG_T) k_cg_key(SolB<F> S, const ColCtl *C, int
         __syncthreads();
     }
 }
-
-// the position in the particle's precision, wrapped as apply_pbc does
-template <class R>
-__device__ inline R cg_wrap(R x, double e, int &jump)
-{
-    const R ed = (R)e;
-    jump = (int)floor((double)(x / ed));
-    return x - (R)jump * ed;
-}
-
 
 // exclusive scan of nc int32 in tiles of CG_TILE: tile-local scan and tile totals, one block
 // for the totals, then each tile's offset (the total goes to *total when given); with a

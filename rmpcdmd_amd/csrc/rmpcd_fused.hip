@@ -863,10 +863,7 @@ __device__ inline void key_pass(const FB<F> &B, const FP &P, const UnitRange &w,
                         }
                     }
                     for (int k = 0; k < 3; ++k) {
-                        Rl e = (Rl)b.edges[k];
-                        int jump = (int)floor((double)(x[k] / e));
-                        x[k] = x[k] - (Rl)jump * e;
-                        jmp[k] = jump;
+                        jmp[k] = fold_pbc<Rl>(x[k], (Rl)b.edges[k]);
                     }
                     // the staging record: wrapped position (apply_pbc, md.f90:202-217), image,
                     // and the rest of the particle's state
@@ -904,9 +901,7 @@ __device__ inline void key_pass(const FB<F> &B, const FP &P, const UnitRange &w,
                         write = true;
                     }
                     for (int k = 0; k < 3; ++k) {
-                        Rl e = (Rl)b.edges[k];
-                        int jump = (int)floor((double)(x[k] / e));
-                        x[k] = x[k] - (Rl)jump * e;
+                        const int jump = fold_pbc<Rl>(x[k], (Rl)b.edges[k]);
                         if (jump != 0) {
                             img[k * n + i] += jump;
                             write = true;
