@@ -1,6 +1,6 @@
 // rmpcd_fused.hip -- the single-dimer MD step and collision cycle as fused device-side
 // kernels over a group of replicas at once (blockIdx.y = replica within the group),
-// captured as one hipGraph per collision cycle with one independent branch per group (a
+// captured as one hipGraph per group and collision cycle, each group on its own stream (a
 // group's latency-bound kernels run beside another group's streaming).
 //
 // Per MD step (programs/single_dimer_pbc.f90:306-383), one kernel k_fz_step: the
