@@ -22,7 +22,7 @@ enum Slot {
     WS_SLOT,        // per-particle place in its tile's list
     WS_TMP,         // the tiles' particle lists
     WS_TILE,        // sort tile starts
-    WS_TCOUNT,      // sort tile counts: zeroed when allocated, left zero by every sort
+    WS_TCOUNT,      // sort tile counts, zero between sorts
     WS_SCAN,        // scan tile sums
     WS_RED,         // reductions (doubles)
     WS_FLAG,        // status flags (ints)
@@ -30,10 +30,16 @@ enum Slot {
     WS_NLCNT,       // neighbour-list per-stencil-cell counts
     WS_PART,        // per-block partial sums
     WS_AUX,         // misc
-    WS_HEAD,        // chains of list entries by particle: zeroed when allocated, left zero by compute_force
+    WS_HEAD,        // chains of list entries by particle, zero between calls of compute_force
     WS_COUNT
 };
 void *workspace(Slot s, size_t bytes);
+// A slot whose words are zero between calls.  A call opens it before its first kernel that
+// writes there and closes it when the one that leaves the words zero is queued; the words of
+// a slot that is new, or that a call left open when it stopped at an error, are cleared when
+// it is opened next (by a kernel: a call may be captured).
+int zeroed_open(Slot s);
+void zeroed_close(Slot s);
 // host-pinned staging for synchronous scalar results
 void *pinned(size_t bytes);
 

@@ -28,6 +28,7 @@ hipStream_t stream() { return g_stream; }
 struct WsEntry {
     void *ptr = nullptr;
     size_t bytes = 0;
+    bool dirty = true, keep_dirty = false;  // of the slots that are zero between calls
 };
 static WsEntry g_ws[WS_COUNT];
 static void *g_pinned = nullptr;
@@ -52,13 +53,39 @@ void *workspace(Slot s, size_t bytes)
         e.ptr = nullptr;
         return nullptr;
     }
-    if ((s == WS_TCOUNT || s == WS_HEAD) && hipMemsetAsync(e.ptr, 0, want, g_stream) != hipSuccess) {
-        (void)hipFree(e.ptr);
-        e.ptr = nullptr;
-        return nullptr;
-    }
     e.bytes = want;
+    e.dirty = true;
     return e.ptr;
+}
+
+__global__ void k_clear_words(uint32_t *p, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] = 0;
+}
+
+int zeroed_open(Slot s)
+{
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    WsEntry &e = g_ws[s];
+    if (e.dirty) {
+        // cleared by a captured launch, the words are zero once the graph runs, not now
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (g_stream) RMPCD_HIP(hipStreamIsCapturing(g_stream, &cap));
+        e.keep_dirty = cap != hipStreamCaptureStatusNone;
+        const int64_t n = (int64_t)(e.bytes / 4);
+        k_clear_words<<<blocks_for(n, 256), 256, 0, g_stream>>>((uint32_t *)e.ptr, n);
+        RMPCD_LAUNCHED();
+    }
+    e.dirty = true;
+    return RMPCD_OK;
+}
+
+void zeroed_close(Slot s)
+{
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    g_ws[s].dirty = g_ws[s].keep_dirty;
+    g_ws[s].keep_dirty = false;
 }
 
 void *pinned(size_t bytes)

@@ -637,7 +637,7 @@ static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
         return set_error(RMPCD_ERR_HIP, "rmpcd_sort: workspace allocation failed");
     t.lut = hilbert_lut(t.b);
     if (!t.lut) return set_error(RMPCD_ERR_HIP, "rmpcd_sort: Hilbert table allocation failed");
-    return RMPCD_OK;
+    return zeroed_open(WS_TCOUNT);  // the keys' kernel comes next
 }
 
 // the sort after its keys
@@ -656,6 +656,7 @@ static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmp
         k_fill_i32<<<blocks_for(t.nt, 256), 256, 0, s>>>(t.count, t.nt, 0);
         RMPCD_LAUNCHED();
     }
+    zeroed_close(WS_TCOUNT);
     k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, t.key, t.shift, t.slot, t.start, t.list);
     RMPCD_LAUNCHED();
     const unsigned runs = (unsigned)((t.nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN));

@@ -1,5 +1,7 @@
 """shared fixtures for the parity tests: seeded synthetic states in the oracle layout
 and their device copies"""
+import ctypes as C
+
 import numpy as np
 
 from oracle import oracle as O
@@ -61,3 +63,13 @@ def same_bits(a, b):
     a = np.ascontiguousarray(a)
     b = np.ascontiguousarray(b)
     return a.shape == b.shape and a.tobytes() == b.tobytes()
+
+
+def leave_hip_error():
+    """a HIP error that no call has read yet, as a program's own failed allocation leaves it: the
+    library's next check after a launch reports it, with that call half queued"""
+    paths = {line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line}
+    assert len(paths) == 1, paths
+    hip = C.CDLL(paths.pop())
+    p = C.c_void_p()
+    assert hip.hipMalloc(C.byref(p), C.c_size_t(1 << 60)) != 0

@@ -12,7 +12,7 @@ from oracle import oracle as O
 from rmpcdmd_amd import capi
 from rmpcdmd_amd.system import CellSet, NeighborList, ParticleSet, lj_params
 
-from _helpers import cells_to_device, same_bits, solvent_state, sorted_state, to_device
+from _helpers import cells_to_device, leave_hip_error, same_bits, solvent_state, sorted_state, to_device
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-12
@@ -160,6 +160,35 @@ def test_sort_tiles(gpu, L, n, spread, form):
     for name in ("pos", "vel", "force", "force_old", "image", "id", "species", "flags"):
         assert (dst.host(name) == getattr(srt, name)).all(), name
     assert same_bits(i2i_d.cpu().numpy(), i2i)
+
+
+@pytest.mark.parametrize("L,n", [((24, 20, 12), 30000), ((256, 256, 128), 100000)])
+def test_sort_after_a_failed_sort(gpu, L, n):
+    """a sort that stops at an error with its key pass queued leaves tile counts behind; the
+    sorts after it must not add to them"""
+    rng = np.random.default_rng(n)
+    ps = O.PState(n)
+    ps.pos[:] = rng.uniform(0, 1, size=(n, 3)) * L
+    ps.id[:] = np.arange(n)
+    ps.species[:] = 1
+    c = O.cells_init(L)
+    srt, i2i, cnt, st = O.sort(c, ps)
+    src, dst, cs = to_device(ps), ParticleSet(n), cells_to_device(c)
+    i2i_d = torch.zeros(n, dtype=torch.int32, device="cuda")
+    for fails in (False, True, True, False, False):
+        dst.load(pos=np.zeros((n, 3)))
+        if fails:
+            leave_hip_error()
+            with pytest.raises(capi.RmpcdError) as e:
+                capi.call("rmpcd_sort", cs.boxp(), src.struct(), dst.struct(), ptr(i2i_d), cs.cellsp(), 0)
+            assert e.value.code == capi.RMPCD_ERR_HIP
+            torch.cuda.synchronize()
+            assert not dst.host("pos").any()  # it stopped before the move
+            continue
+        capi.call("rmpcd_sort", cs.boxp(), src.struct(), dst.struct(), ptr(i2i_d), cs.cellsp(), 0)
+        torch.cuda.synchronize()
+        assert same_bits(cs.cell_count.cpu().numpy(), cnt) and same_bits(cs.cell_start.cpu().numpy(), st)
+        assert same_bits(dst.host("pos"), srt.pos) and same_bits(dst.host("id"), srt.id)
 
 
 def test_maximum_displacement(gpu):
