@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(256)
 // the chains of k_force_nl: the thread of a chain's last arrival adds its entries in
 // colloid order (the next larger entry each time: two or three colloids meet at most) and
 // clears the head.  The other entries of the chain read a head that is not their own before
-// as after that.
+// as after that.  A chain holds no more than the launch's entries, so the walk ends.
 template <class F>
 __global__ void __launch_bounds__(256)
     k_force_nl_apply(PView<F64> c, PView<F> sol, const int32_t *__restrict__ list, const int32_t *__restrict__ nl,
@@ -200,6 +200,7 @@ __global__ void __launch_bounds__(256)
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= min(nl[i], nmax)) return;
     const uint32_t ent = (uint32_t)blockIdx.y * (uint32_t)nmax + (uint32_t)k + 1;
+    const uint32_t most = gridDim.y * (uint32_t)nmax;
     if (next[ent - 1] == OUTSIDE) return;
     const int idx = list[(int64_t)i * nmax + k];
     if (head[idx] != ent) return;
@@ -207,8 +208,8 @@ __global__ void __launch_bounds__(256)
     int fl = (int)sol.flags[idx];
     uint32_t done = 0;
     for (;;) {
-        uint32_t least = OUTSIDE;
-        for (uint32_t q = ent; q; q = next[q - 1])
+        uint32_t least = OUTSIDE, len = 0;
+        for (uint32_t q = ent; q && len < most; q = next[q - 1], ++len)
             if (q > done && q < least) least = q;
         if (least == OUTSIDE) break;
         done = least;
@@ -411,18 +412,20 @@ int force_list(const rmpcd_particles_t *ps1, const rmpcd_particles_t *ps2, const
         next = (uint32_t *)workspace(WS_AUX, sizeof(uint32_t) * (size_t)group * nmax);
     }
     if (np > 1 && (!head || !next)) return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
+    int rc;
+    if (np > 1 && (rc = zeroed_open(WS_HEAD))) return rc;
     hipStream_t s = stream();
     const LJ l = make_lj(lj);
     for (int c0 = 0; c0 < np; c0 += group) {
         const dim3 grid(nb, group < np - c0 ? group : np - c0);
         k_force_nl<F><<<grid, 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, part, c0, head,
                                            next);
-        RMPCD_LAUNCHED();
-        if (np == 1) break;
-        k_force_nl_apply<F><<<grid, 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, c0, head,
-                                                 next);
+        if (np > 1)
+            k_force_nl_apply<F><<<grid, 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, c0, head,
+                                                     next);
         RMPCD_LAUNCHED();
     }
+    if (np > 1) zeroed_close(WS_HEAD);
     return RMPCD_OK;
 }
 

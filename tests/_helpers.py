@@ -1,6 +1,7 @@
 """shared fixtures for the parity tests: seeded synthetic states in the oracle layout
 and their device copies"""
 import ctypes as C
+import os
 
 import numpy as np
 
@@ -73,3 +74,15 @@ def leave_hip_error():
     hip = C.CDLL(paths.pop())
     p = C.c_void_p()
     assert hip.hipMalloc(C.byref(p), C.c_size_t(1 << 60)) != 0
+
+
+def workspace_slot(name, n_bytes):
+    """the library's workspace slot as (index, device address), through its own C++ functions"""
+    import re
+    from rmpcdmd_amd import capi
+    path = os.path.join(os.path.dirname(capi.__file__), "csrc", "rmpcd_internal.hpp")
+    enum = re.search(r"enum Slot \{(.*?)\};", open(path).read(), re.S).group(1)
+    slot = re.findall(r"^\s*(WS_[A-Z]+)", enum, re.M).index(name)
+    f = capi.lib()._ZN5rmpcd9workspaceENS_4SlotEm
+    f.restype, f.argtypes = C.c_void_p, [C.c_int, C.c_size_t]
+    return slot, f(slot, n_bytes)

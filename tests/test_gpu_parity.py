@@ -12,7 +12,7 @@ from oracle import oracle as O
 from rmpcdmd_amd import capi
 from rmpcdmd_amd.system import CellSet, NeighborList, ParticleSet, lj_params
 
-from _helpers import cells_to_device, leave_hip_error, same_bits, solvent_state, sorted_state, to_device
+from _helpers import cells_to_device, leave_hip_error, same_bits, solvent_state, sorted_state, to_device, workspace_slot
 
 pytestmark = pytest.mark.gpu
 RTOL = 1e-12
@@ -521,6 +521,38 @@ def test_compute_force_colloid_order(gpu, n_col, nmax):
     # the colloid sums run over blocks of 256 entries: 1e-12 of the sum of the magnitudes
     assert abs(e.value - e_o) <= 1e-12 * abs(e_o)
     assert close(cd.host("force"), want_c.force, scale=np.abs(want_c.force - cp.force).sum() + 1.0)
+
+
+def test_compute_force_after_a_failed_call(gpu):
+    """a call that stopped between its two launches leaves chain heads behind: the next one must
+    clear them (an entry that finds its own number there would follow itself for ever)"""
+    L, n_col, nmax = (14, 12, 13), 3, 2501
+    c, srt, cnt, st = sorted_state(L, 10, 43)
+    cp = O.PState(n_col)
+    cp.pos[:] = [[5.0, 6.0, 6.0], [6.5, 6.0, 6.0], [6.0, 7.0, 6.0]]
+    cp.species[:] = 1
+    sig, eps = np.array([[1.5]]), np.array([[1.0]])
+    cut = sig * 2 ** (1 / 6)
+    radius = cut.max() + 1.0
+    lj_o = O.lj_params(eps, sig, cut)
+    lst, nl, is_md, is_reac = O.update_list(c, cnt, st, cp.pos, cp.species, srt.pos, srt.species, radius,
+                                            O.make_stencil(1.0, radius), lj_o, nmax)
+    lj, e = lj_params(eps, sig, cut), C.c_double()
+    ld, nd = torch.as_tensor(lst).cuda(), torch.as_tensor(nl).cuda()
+    slot, at = workspace_slot("WS_HEAD", 4 * srt.n)
+    for stopped in (False, True, False):
+        if stopped:  # opened, its heads set (each entry number of the first colloid), not closed
+            assert capi.lib()._ZN5rmpcd11zeroed_openENS_4SlotE(C.c_int(slot)) == 0
+            heads = np.zeros(srt.n, np.uint32)
+            heads[lst[0, :nl[0]]] = np.arange(1, nl[0] + 1)
+            capi.call("rmpcd_memcpy", C.c_void_p(at), heads.ctypes.data_as(C.c_void_p), heads.nbytes, 0)
+        d, cd = to_device(srt), to_device(cp)
+        want_s, want_c = srt.copy(), cp.copy()
+        O.compute_force(want_c.pos, want_c.species, want_c.force, want_s.pos, want_s.species, want_s.force,
+                        want_s.flags, lst, nl, L, lj_o)
+        capi.call("rmpcd_compute_force", cd.struct(), d.struct(), ptr(ld), ptr(nd), nmax, capi.d3(L), C.byref(lj),
+                  C.byref(e))
+        assert same_bits(d.host("force"), want_s.force) and same_bits(d.host("flags"), want_s.flags)
 
 
 def test_compute_force_and_helpers(gpu):
