@@ -145,6 +145,9 @@ __global__ void k_roll_md(int64_t n, typename F::small *flags)
 // latency of the entries' reads: a launch per colloid, which kept the order before, took
 // 390 us an MD step with 52 colloids (30.0 ms a cycle of 50 steps, 10.8 with the chains).
 constexpr uint32_t OUTSIDE = 0xffffffffu;
+// List entries of one launch's chains, 4 B each, which the workspace holds until the process
+// ends: 64 MiB.  More colloids are taken in several pairs of launches, in their order.
+constexpr int32_t CHAIN_ENTRIES = 1 << 24;
 
 template <class F>
 __global__ void __launch_bounds__(256)
@@ -404,28 +407,29 @@ int force_list(const rmpcd_particles_t *ps1, const rmpcd_particles_t *ps2, const
     const int np = (int)ps1->n;
     const unsigned nb = blocks_for(nmax, 256);
     const PView<F> sol = view<F>(ps2);
-    // colloids of one launch: their entries are counted in 32 bits
-    const int group = np == 1 ? 1 : (int)(nmax >= (1 << 30) ? 1 : np < (1 << 30) / nmax ? np : (1 << 30) / nmax);
+    // colloids of one launch
+    const int group = nmax >= CHAIN_ENTRIES ? 1 : np < CHAIN_ENTRIES / nmax ? np : CHAIN_ENTRIES / nmax;
+    const bool chains = group > 1;
     uint32_t *head = nullptr, *next = nullptr;
-    if (np > 1) {
+    int rc;
+    if (chains) {
         head = (uint32_t *)workspace(WS_HEAD, sizeof(uint32_t) * (size_t)sol.n);
         next = (uint32_t *)workspace(WS_AUX, sizeof(uint32_t) * (size_t)group * nmax);
+        if (!head || !next) return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
+        if ((rc = zeroed_open(WS_HEAD))) return rc;
     }
-    if (np > 1 && (!head || !next)) return set_error(RMPCD_ERR_HIP, "compute_force: workspace allocation failed");
-    int rc;
-    if (np > 1 && (rc = zeroed_open(WS_HEAD))) return rc;
     hipStream_t s = stream();
     const LJ l = make_lj(lj);
     for (int c0 = 0; c0 < np; c0 += group) {
         const dim3 grid(nb, group < np - c0 ? group : np - c0);
         k_force_nl<F><<<grid, 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, part, c0, head,
                                            next);
-        if (np > 1)
+        if (chains)
             k_force_nl_apply<F><<<grid, 256, 0, s>>>(view<F64>(ps1), sol, list, nl, nmax, L[0], L[1], L[2], l, c0, head,
                                                      next);
         RMPCD_LAUNCHED();
     }
-    if (np > 1) zeroed_close(WS_HEAD);
+    if (chains) zeroed_close(WS_HEAD);
     return RMPCD_OK;
 }
 

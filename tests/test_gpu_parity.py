@@ -490,10 +490,11 @@ def test_update_list_overflow(gpu):
     assert nlst.n.max().item() <= 50
 
 
-@pytest.mark.parametrize("n_col,nmax", [(1, 3000), (3, 2501), (70, 2600)])
+@pytest.mark.parametrize("n_col,nmax", [(1, 3000), (3, 2501), (70, 2600), (3, 6_000_000), (2, 9_000_000)])
 def test_compute_force_colloid_order(gpu, n_col, nmax):
     """overlapping colloids, so that particles lie inside the cutoff of several: their forces
-    are added in the reference's colloid order, bit for bit, onto what they hold"""
+    are added in the reference's colloid order, bit for bit, onto what they hold (by launches of
+    two and one colloid for the longer lists, of one each for the longest)"""
     L = (14, 12, 13)
     c, srt, cnt, st = sorted_state(L, 10, 41, frac2=0.3)
     rng = np.random.default_rng(n_col)
