@@ -35,10 +35,19 @@ namespace rmpcd {
 // fifty COLLOIDS steps 7.9 ms (L = 48, FP64, 52 colloids), 0.63 and 4.8 ms like this.
 constexpr unsigned STEP_BLOCKS = 1024;  // workgroups of a pass over all particles that leaves a partial each
 
-// SPHERE, before the decision: md_pos, maximum_displacement, and the solvent's force reset
-// of this step: the new force array (force_old until the switch) zeroed, the MD bits
-// rolled.  The reference makes the reset after a sort of the same step; the sort carries
-// zeros and bits along, so the state after it is the same.
+// The solvent's force reset of a SPHERE step (the new force array zeroed, the MD bits rolled;
+// neighbor_list.f90:180-188) falls on two kernels: the list's particles have it in
+// k_sphere_list, which marks them, the others in k_sphere_finish, which removes the mark.  A
+// step that stops at a failed list build has then touched neither, as in the reference.
+constexpr int LISTED_MASK = 1 << 7;  // a bit of the flags that no state shows between steps
+
+__device__ inline int roll_md(int f)
+{
+    f = (f & MD_MASK) ? (f | PAST_MD_MASK) : (f & ~PAST_MD_MASK);
+    return f & ~MD_MASK;
+}
+
+// SPHERE, before the decision: md_pos and maximum_displacement
 template <class F>
 __global__ void __launch_bounds__(256)
     k_sphere_move(PView<F> p, const typename F::real *__restrict__ pos_old, double dt, double *__restrict__ part)
@@ -52,11 +61,7 @@ __global__ void __launch_bounds__(256)
         for (int k = 0; k < 3; ++k) {
             const int64_t q = k * p.n + i;
             p.pos[q] = (p.pos[q] + rdt * p.vel[q]) + dt_sq * p.force[q];
-            p.force_old[q] = 0;
         }
-        int f = (int)p.flags[i];
-        f = (f & MD_MASK) ? (f | PAST_MD_MASK) : (f & ~PAST_MD_MASK);
-        p.flags[i] = (typename F::small)(f & ~MD_MASK);
         r_sq = fmax(r_sq, disp_sq<F>(p, pos_old, i));
     }
     const double m = block_max(r_sq, red);
@@ -80,11 +85,17 @@ __global__ void __launch_bounds__(256)
     if (k < n) {
         const int idx = list[k];
         int fl = (int)sol.flags[idx];
-        const int old = fl;
+        // (a stencil wider than the box lists a particle twice)
+        R g[3] = {0, 0, 0};
+        if (fl & LISTED_MASK)
+            for (int q = 0; q < 3; ++q) g[q] = sol.force[q * sol.n + idx];
+        else
+            fl = roll_md(fl) | LISTED_MASK;
         if (pair_force<F>(c, sol, 0, idx, L0, L1, L2, lj, f, &e)) {
-            for (int q = 0; q < 3; ++q) sol.force[q * sol.n + idx] = sol.force[q * sol.n + idx] - (R)f[q];
+            for (int q = 0; q < 3; ++q) g[q] = g[q] - (R)f[q];
             fl |= MD_MASK | (c.species[0] == 1 ? CATALYZED_MASK : 0);
         }
+        for (int q = 0; q < 3; ++q) sol.force[q * sol.n + idx] = g[q];
         if ((int)sol.species[idx] == 1) {
             const double d0 = min_image(c.pos[0] - (double)sol.pos[idx], L0);
             const double d1 = min_image(c.pos[c.n] - (double)sol.pos[sol.n + idx], L1);
@@ -95,7 +106,7 @@ __global__ void __launch_bounds__(256)
                 if (u01(a) <= prob) fl |= REAC_MASK;
             }
         }
-        if (fl != old) sol.flags[idx] = (typename F::small)fl;
+        sol.flags[idx] = (typename F::small)fl;
     }
     double *pp = part + 4 * (int64_t)blockIdx.x;
     if ((int)(blockIdx.x * blockDim.x) >= n) {
@@ -122,13 +133,21 @@ __global__ void __launch_bounds__(256)
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.n) return;
     const int old = (int)p.flags[i];
-    int f = old;
+    const bool listed = (old & LISTED_MASK) != 0;
+    int f = listed ? old & ~LISTED_MASK : roll_md(old);
+    R fn[3] = {0, 0, 0};
+    for (int k = 0; k < 3; ++k) {
+        if (listed)
+            fn[k] = p.force[k * p.n + i];
+        else
+            p.force[k * p.n + i] = 0;
+    }
     if (!(f & WALL_MASK)) {
         const R rdt = (R)dt;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const int64_t q = k * p.n + i;
-            p.vel[q] = p.vel[q] + (rdt * (p.force[q] + p.force_old[q])) / (R)2;
+            p.vel[q] = p.vel[q] + (rdt * (fn[k] + p.force_old[q])) / (R)2;
         }
     } else {
         f &= ~WALL_MASK;
@@ -194,9 +213,7 @@ __global__ void __launch_bounds__(256) k_force_reset(PView<F> p)
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= p.n) return;
     for (int k = 0; k < 3; ++k) p.force[k * p.n + i] = 0;
-    int f = (int)p.flags[i];
-    f = (f & MD_MASK) ? (f | PAST_MD_MASK) : (f & ~PAST_MD_MASK);
-    p.flags[i] = (typename F::small)(f & ~MD_MASK);
+    p.flags[i] = (typename F::small)roll_md((int)p.flags[i]);
 }
 
 // COLLOIDS, one workgroup per colloid: its list partials, compute_force_n2 and its Verlet
@@ -518,12 +535,11 @@ static int sphere_step_t(ProgramSim &m)
     const double *L = m.box.edges;
     k_sphere_list<F><<<lb, 256, 0, st>>>(view<F64>(&p), view<F>(&s), m.list, m.nlist, m.nmax, L[0], L[1], L[2],
                                          make_lj(&m.lj_sc), m.cfg.prob, m.seed, (uint64_t)m.md_steps, part);
-    RMPCD_LAUNCHED();
-    if ((rc = force_sum_unchecked(&p, part, (int)lb, m.dev_e1))) return rc;
-    m.have_e = true;
     k_sphere_finish<F><<<blocks_for(m.n, 256), 256, 0, st>>>(view<F>(&s), view<F64>(&p), m.dt, L[0], L[1], L[2],
                                                              m.lj_sc.cut_sq[0]);
     RMPCD_LAUNCHED();
+    if ((rc = force_sum_unchecked(&p, part, (int)lb, m.dev_e1))) return rc;
+    m.have_e = true;
     ++m.md_steps;
     return RMPCD_OK;
 }

@@ -123,6 +123,62 @@ def test_sphere_matches_oracle(gpu):
     prog.close()
 
 
+def test_sphere_failed_list_build(gpu):
+    """a step that stops at a list longer than its capacity leaves the state where the
+    reference stops: moved and sorted, the forces and the MD bits of the step before"""
+    from oracle.programs import SphereOracle
+
+    class Stop(Exception):
+        pass
+
+    class Capped(SphereOracle):
+        cap, builds, in_step = None, (), False
+
+        def update_list(self):
+            super().update_list()
+            self.builds = self.builds + ((self.in_step, int(self.nl[0])),)
+            if self.cap is not None and self.nl[0] > self.cap:
+                raise Stop
+
+        def md_step(self):
+            self.in_step = True
+            super().md_step()
+            self.in_step = False
+
+    L = (16, 16, 16)
+    kw = dict(L=L, n_md=10, tau=0.5, sigma=2.0, T=1.0, bulk_rate=0.05, prob=0.7, seed=19)
+    prog = Program(PROG_SPHERE, form=capi.FP64, **kw)
+    st = prog.download()
+    prog.close()
+    args = dict(sigma=2.0, prob=0.7, bulk_rate=0.05)
+    orc = Capped(st, L, 0.5, 10, 19, **args)
+    for _ in range(6):
+        orc.cycle()
+    # the capacity that a step's list exceeds first, after a few steps
+    n = [b[1] for b in orc.builds]
+    first = next(k for k, b in enumerate(orc.builds) if k > 2 and b[0] and b[1] > max(n[:k]))
+    cap = max(n[:first])
+    print("list lengths", n, "capacity", cap, flush=True)
+    prog = Program(PROG_SPHERE, form=capi.FP64, nmax_list=cap, **kw)
+    orc = Capped(st, L, 0.5, 10, 19, **args)
+    orc.cap = cap
+    with pytest.raises(capi.RmpcdError) as e:
+        prog.run(6)
+    assert e.value.code == capi.RMPCD_ERR_OVERFLOW
+    with pytest.raises(Stop):
+        for _ in range(6):
+            orc.cycle()
+    assert orc.in_step and (orc.s.flags & 4).any() and orc.s.force_old.any()
+    g = prog.download()
+    assert g["md_steps"] == orc.md_steps
+    for k in ("id", "species", "flags", "image"):
+        assert (g[k] == getattr(orc.s, k)).all(), k
+    for k in ("pos", "vel", "force", "force_old"):
+        assert close(g[k], getattr(orc.s, k)), k
+    assert close(g["e1"], orc.e1)
+    prog.close()
+
+
 def test_colloids_matches_oracle(gpu):
     from oracle.programs import ColloidsOracle
     L = (20, 20, 20)
