@@ -429,6 +429,10 @@ int rmpcd_dimer_destroy(rmpcd_dimer_t *sim);
  * duration of those launches in the last cycle run */
 int rmpcd_dimer_profile(rmpcd_dimer_t *sim, int32_t stride);
 int rmpcd_dimer_stream_time(rmpcd_dimer_t *sim, double *avg_ms, int32_t *samples);
+/* fused mode: the particle passes of the sorts that may follow an MD step in one launch (1) or
+ * in a launch each (4), instead of by the library's own rule on sizes (0); the same results
+ * either way */
+int rmpcd_dimer_extra_sort(rmpcd_dimer_t *sim, int32_t launches);
 
 /* ---- the other driver loops on device-resident state --------------------------------
  * RMPCD_PROG_FLUID     test/setup_simple_fluid.f90:89-127: SRD, streaming, grid shift,

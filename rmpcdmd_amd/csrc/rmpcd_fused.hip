@@ -2335,7 +2335,8 @@ static void enqueue_sort(DimerSim &s, const FB<F> &b, const FP &p, hipStream_t s
         const int nx = s.extra_blocks;
         int64_t n = 0;
         for (int r = b.r0; r < b.r0 + R; ++r) n += s.rep[r].n;
-        if (R == 1 || s.cfg.lazy || 9 * (int64_t)sizeof(typename F::real) * n < CHAIN_BYTES) {
+        const bool chained = R == 1 || s.cfg.lazy || 9 * (int64_t)sizeof(typename F::real) * n < CHAIN_BYTES;
+        if (s.extra_launches ? s.extra_launches == 1 : chained) {
             k_fz_extra_sort<F><<<extra_grid(s, R), FT, 0, st>>>(b, p, R);
         } else {
             k_fz_key<F><<<nx, FT, 0, st>>>(b, p, R);
@@ -2548,7 +2549,7 @@ static int build_cycle(DimerSim &s)
 int fused_set_profile(DimerSim &s, int stride)
 {
     if (!s.fused_ready) return set_error(RMPCD_ERR_ARG, "dimer: profiling needs the fused mode");
-    RMPCD_HIP(hipStreamSynchronize(s.gstreams[0]));
+    for (hipStream_t st : s.gstreams) RMPCD_HIP(hipStreamSynchronize(st));
     for (hipEvent_t e : s.prof_ev) (void)hipEventDestroy(e);
     s.prof_ev.clear();
     s.prof_stride = stride > 0 ? stride : 0;
@@ -2557,6 +2558,14 @@ int fused_set_profile(DimerSim &s, int stride)
         s.prof_ev.resize(2 * (size_t)pairs);
         for (hipEvent_t &e : s.prof_ev) RMPCD_HIP(hipEventCreate(&e));
     }
+    return build_cycle(s);
+}
+
+int fused_set_extra_sort(DimerSim &s, int launches)
+{
+    if (!s.fused_ready) return set_error(RMPCD_ERR_ARG, "dimer: the sort after an MD step belongs to the fused mode");
+    for (hipStream_t st : s.gstreams) RMPCD_HIP(hipStreamSynchronize(st));
+    s.extra_launches = launches;
     return build_cycle(s);
 }
 

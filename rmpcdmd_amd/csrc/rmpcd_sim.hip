@@ -479,6 +479,12 @@ int rmpcd_dimer_stream_time(rmpcd_dimer_t *sim, double *avg_ms, int32_t *samples
     return fused_stream_time(*(DimerSim *)sim, avg_ms, samples);
 }
 
+int rmpcd_dimer_extra_sort(rmpcd_dimer_t *sim, int32_t launches)
+{
+    RMPCD_CHECK(sim && (launches == 0 || launches == 1 || launches == 4), "rmpcd_dimer_extra_sort: bad argument");
+    return fused_set_extra_sort(*(DimerSim *)sim, launches);
+}
+
 int rmpcd_dimer_destroy(rmpcd_dimer_t *sim)
 {
     delete (DimerSim *)sim;

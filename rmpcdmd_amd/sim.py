@@ -64,6 +64,10 @@ class SingleDimer:
                   C.byref(cells), C.byref(st))
         return sol, col, box, cells, st
 
+    def extra_sort(self, launches):
+        """the sorts after MD steps in one launch (1), a launch per pass (4) or by rule (0)"""
+        capi.call("rmpcd_dimer_extra_sort", self._h, int(launches))
+
     @property
     def n_solvent(self):
         return self.state()[4].n_solvent

@@ -321,6 +321,41 @@ def test_many_extra_sorts_per_cycle(gpu, form):
 
 
 @pytest.mark.parametrize("form", [capi.FP64, capi.FP32])
+@pytest.mark.parametrize("kw", [
+    dict(n_md=50, tau=0.5, replica_L=[(16, 16, 16), (20, 16, 12)], skin=0.6),  # several sorts a cycle
+    dict(n_md=50, tau=0.5, replica_L=[(16, 16, 16), (20, 16, 12)], skin=0.6, lazy=1),
+    dict(n_md=10, tau=0.1, replica_L=[(12, 12, 12)], rho=40),  # cells beyond the halo, one replica
+    dict(n_md=30, tau=0.3, replica_L=[(24, 24, 24), (12, 12, 12), (13, 13, 13), (16, 24, 12)], skin=0.6),
+], ids=["two", "two-lazy", "dense", "four"])
+def test_extra_sort_launches(gpu, form, kw):
+    """the sort after an MD step in one launch and in a launch per pass: each against the
+    reference sequence, and against each other bit for bit, with units grouped by XCD and in
+    contiguous ranges, by grids of fewer workgroups than units and with one group and two"""
+    kw = dict(kw, form=form, seed=61)
+    ref = SingleDimer(mode=capi.SIM_REFERENCE, **{k: v for k, v in kw.items() if k != "lazy"})
+    ref.run(2)
+    first = {}
+    n = len(kw["replica_L"])
+    for launches in (1, 4):
+        for shape in (dict(), dict(sort_order=1), dict(sort_order=2, extra_sort_blocks=5, groups=1),
+                      dict(sort_order=1, extra_sort_blocks=3, groups=min(2, n))):
+            sim = SingleDimer(mode=capi.SIM_FUSED, **kw, **shape)
+            sim.extra_sort(launches)
+            sim.run(2)
+            for r in range(n):
+                g = sim.download(r)
+                msg = "%d launches, %s, replica %d" % (launches, shape, r)
+                if r not in first:
+                    compare(ref.download(r), g, msg, 1e-12 if form == capi.FP64 else 1e-5)
+                    first[r] = g
+                compare(first[r], g, msg, rtol=0.0)
+                assert g["pos_old"].tobytes() == first[r]["pos_old"].tobytes(), msg
+            sim.close()
+    assert min(g["n_extra_sorting"] for g in first.values()) >= (1 if "rho" in kw else 4)
+    ref.close()
+
+
+@pytest.mark.parametrize("form", [capi.FP64, capi.FP32])
 def test_extra_sort_workgroups(gpu, form):
     """the sort after an MD step is one launch whose passes wait for each other: with one
     workgroup, with fewer than there are XCDs, with a number that is no multiple of them and
