@@ -380,10 +380,11 @@ typedef struct rmpcd_dimer_config {
                                   moved only when read (at a sort or an exact skin test), by
                                   replaying their per-step additions; the same trajectory
                                   bit for bit, without the per-step pass over all solvent */
-    int32_t extra_sort_blocks; /* fused mode launch shape, 0: 512 or sort_blocks if fewer: at
-                                  most so many workgroups for the key, place and rank passes
-                                  of the sorts that may follow each MD step (they return at
-                                  once when none is due) */
+    int32_t extra_sort_blocks; /* fused mode launch shape: at most so many workgroups for the
+                                  key, place and rank passes of the sorts that may follow
+                                  each MD step (they return at once when none is due).  0:
+                                  512, or 1024 to 2048 for large boxes and where the skin is
+                                  so thin that sorts are due often, or sort_blocks if fewer */
     int32_t sort_order;        /* fused mode launch shape: how the sort passes' workgroups
                                   take their units.  0: default (2), 1: a contiguous range
                                   per workgroup, 2: XCD-grouped (the workgroups of one XCD,

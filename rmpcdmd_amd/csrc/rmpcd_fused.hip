@@ -54,14 +54,35 @@ constexpr int EXTRA_BLOCKS = 512;
 // lazy, 16 x L=64 (1.5 GB) 7.08, 7.11 and 6.91, 6.95; 4 x L=64 2.81, 2.84 and 2.74, 2.88.  Four
 // groups are slower at each of these sizes (4 x L=64: 5.81).
 constexpr int64_t GROUP_BYTES = 100000000;
-// Bytes that a step's eager streaming moves in a group of several replicas from which the sort
-// after the step has a launch for each particle pass: its launches run beside the other
+// Bytes that a step's eager streaming moves in a group from which the sort after the step has
+// a launch for each particle pass.  With several replicas its launches run beside the other
 // group's streaming there, and its passes are faster on their own.  One launch and four,
 // FP32, a cycle and the first one, in which all replicas sort several times: 16 x L=64 (0.75
 // GB a group) 16.18, 19.5 and 16.30, 18.9 ms; 8 x L=64 8.35, 10.3 and 8.52, 9.7; 4 x L=64
 // 4.48, 5.6 and 4.76, 5.4; FP64 8 x L=64 (0.75 GB) 15.7, 18.1 and 15.7, 17.2; lazy,
-// 16 x L=64 6.5 and 6.8 a cycle.
-constexpr int64_t CHAIN_BYTES = 500000000;
+// 16 x L=64 6.5 and 6.8 a cycle.  One replica, on 1024 workgroups, later cycles and the first:
+// L=112 FP64 (1.0 GB) 11.28, 12.6 and 11.45, 12.3 ms; L=128 FP64 (1.5 GB) 16.8, 18.6 and 16.4, 18.1.
+constexpr int64_t CHAIN_BYTES = 500000000, CHAIN_BYTES_ONE = 1200000000;
+// The share of MD steps with a sort due up to which one launch is the faster form: it saves 5
+// us at a step without a sort and loses at one with, more for more particles and most where
+// replicas sort together.  A group of one replica that streams m MB a step: up to
+// CHAIN_SHARE_ONE / cbrt(m), if that is more.  Measured with the skin from 2 (one sort in 50
+// steps) to 0.2; one launch and four (1024 workgroups), a cycle of 50 steps: L=24 FP32 (5 MB)
+// with 1 sort 1.00 and 1.26 ms, with 9 1.44 and 1.43; L=64 FP32 (94 MB) with 1 1.78 and 2.03,
+// with 3 2.14 and 2.19, with 5 2.51 and 2.38, with 10 3.62 and 2.91; L=96 FP64 (640 MB) with 1
+// 7.67 and 7.75, with 3 8.97 and 8.47; 4 x L=48 FP64 with 1 4.08 and 4.37, with 2.6 4.86 and
+// 4.61, with 10 8.21 and 5.72; 16 x L=24 FP32 with 1 2.38 and 2.57, with 2 2.75 and 2.54; lazy,
+// 4 x L=45 FP32 with 1 1.87 and 2.08, with 2.5 2.49 and 2.34; L=64 with 3 1.78 and 1.82.
+constexpr double CHAIN_SHARE = 0.03, CHAIN_SHARE_ONE = 0.3;
+// Workgroups of these sorts in groups that stream WIDE_BYTES or more a step: in one launch
+// where the group is one replica or lazy (first and later cycles on 512 and 1024 workgroups:
+// L=96 FP64 8.75, 7.71 and 8.62, 7.63 ms; L=128 FP32 10.9, 8.9 and 10.3, 8.9; lazy 5.9, 3.6 and
+// 5.2, 3.4; lazy, 8 x L=64 FP32 6.34, 3.98 and 5.76, 3.69; one L=64 FP32 box idles 3 % longer),
+// and in four launches where sorts are due often: EXTRA_BLOCKS, 1024, 2048 and 4096 with the
+// skin at 0.3, L=64 FP32 3.18, 2.91, 2.94, 2.99 ms a cycle; 4 x L=48 FP64 6.03, 5.72, 5.69, 5.81;
+// L=96 FP64 12.19, 11.32, 11.13, 10.88; 16 x L=64 FP32 29.3, 29.6, 28.0, 27.8.
+constexpr int64_t WIDE_BYTES = 150000000;
+constexpr int WIDE_BLOCKS = 1024, BUSY_BLOCKS = 1024, BUSY_BLOCKS_WIDE = 2048;
 constexpr int GATHER_GRID_MUL = 4;  // the collision sort's fused gather runs on this many times the sort grid
 constexpr int SCAN_BLOCKS = 1024;     // blocks of the cell-count tile scan (all replicas)
 constexpr int CT_DEFAULT = 128;  // cells per block in the collision kernel (64, 128 or 256; 12 particles per cell
@@ -2317,9 +2338,22 @@ static int stream_blocks(const DimerSim &s)
 
 // the grid of the sort that may follow an MD step: no more workgroups than R of the largest
 // replica have key units (more make the passes of an L=24 box 92 us instead of 75)
-static unsigned extra_grid(const DimerSim &s, int R)
+static unsigned extra_grid(const DimerSim &s, int R, int most)
 {
-    return (unsigned)std::min<int64_t>((s.nmax_rep + KCHUNK - 1) / KCHUNK * R, s.extra_blocks);
+    return (unsigned)std::min<int64_t>((s.nmax_rep + KCHUNK - 1) / KCHUNK * R, most);
+}
+
+// The share of MD steps after which a sort is to be expected: a sort is due when the fastest
+// solvent particle has moved 0.89 skin or a colloid 0.1 skin, and the collision's sort starts
+// anew.  The fastest of n thermal speeds is taken where n times the tail of the Maxwell
+// distribution is one, a colloid's as the root mean square.
+static double due_share(const DimerSim &s)
+{
+    const double n = (double)s.nmax_rep, T = s.cfg.T, x0 = sqrt(2 * log(n + 2));
+    const double v = sqrt(T * (x0 * x0 + 2 * log(0.8 * x0)));
+    const double vc = sqrt(3 * T / std::min(s.mass[0], s.mass[1]));
+    const double steps = s.skin / s.dt / std::max(v / 0.89, vc / 0.1);
+    return steps > 1 ? floor(s.cfg.n_md / steps) / s.cfg.n_md : 1;
 }
 
 // (each enqueue_* works on the R replicas of b's group)
@@ -2332,12 +2366,19 @@ static void enqueue_sort(DimerSim &s, const FB<F> &b, const FP &p, hipStream_t s
         // the sort that may follow an MD step: when none is due its blocks only read the plan
         // and return
         if (R > 1) k_fz_plan<F><<<1, FT, 0, st>>>(b, 0, R);
-        const int nx = s.extra_blocks;
         int64_t n = 0;
         for (int r = b.r0; r < b.r0 + R; ++r) n += s.rep[r].n;
-        const bool chained = R == 1 || s.cfg.lazy || 9 * (int64_t)sizeof(typename F::real) * n < CHAIN_BYTES;
-        if (s.extra_launches ? s.extra_launches == 1 : chained) {
-            k_fz_extra_sort<F><<<extra_grid(s, R), FT, 0, st>>>(b, p, R);
+        const int64_t bytes = 9 * (int64_t)sizeof(typename F::real) * n;
+        const double one = R == 1 ? CHAIN_SHARE_ONE / cbrt(1e-6 * (double)bytes) : 0;
+        const bool seldom = due_share(s) <= std::max(CHAIN_SHARE, one);
+        const bool chained = seldom && (s.cfg.lazy || bytes < (R == 1 ? CHAIN_BYTES_ONE : CHAIN_BYTES));
+        const bool in_one = s.extra_launches ? s.extra_launches == 1 : chained, wide = bytes >= WIDE_BYTES;
+        const int by_rule = in_one   ? (wide && (R == 1 || s.cfg.lazy) ? WIDE_BLOCKS : EXTRA_BLOCKS)
+                            : seldom ? (R == 1 ? WIDE_BLOCKS : EXTRA_BLOCKS)
+                                     : (wide ? BUSY_BLOCKS_WIDE : BUSY_BLOCKS);
+        const int nx = s.cfg.extra_sort_blocks > 0 ? s.cfg.extra_sort_blocks : std::min(s.sort_blocks, by_rule);
+        if (in_one) {
+            k_fz_extra_sort<F><<<extra_grid(s, R, nx), FT, 0, st>>>(b, p, R);
         } else {
             k_fz_key<F><<<nx, FT, 0, st>>>(b, p, R);
             k_fz_scan_tiles<F><<<nx, SCAN_T, 0, st>>>(b, R);
@@ -2593,11 +2634,10 @@ int fused_prepare(DimerSim &s)
     // every per-block partial of a replica must fit its PS slots
     s.stream_blocks = s.cfg.stream_blocks > 0 ? s.cfg.stream_blocks : STREAM_BLOCKS;
     s.sort_blocks = s.cfg.sort_blocks > 0 ? s.cfg.sort_blocks : SORT_BLOCKS;
-    s.extra_blocks = s.cfg.extra_sort_blocks > 0 ? s.cfg.extra_sort_blocks : std::min(s.sort_blocks, EXTRA_BLOCKS);
     RMPCD_CHECK(s.cfg.sort_order >= 0 && s.cfg.sort_order <= 2, "dimer: sort_order must be 0, 1 or 2");
     RMPCD_CHECK(s.cfg.groups >= 0 && s.cfg.groups <= MAX_GROUPS, "dimer: groups must be 0 to 8");
     s.sort_order = s.cfg.sort_order > 0 ? s.cfg.sort_order : 2;
-    RMPCD_CHECK(s.stream_blocks <= STREAM_BLOCKS && s.sort_blocks <= 65536 && s.extra_blocks <= 65536,
+    RMPCD_CHECK(s.stream_blocks <= STREAM_BLOCKS && s.sort_blocks <= 65536 && s.cfg.extra_sort_blocks <= 65536,
                 "dimer: stream_blocks must be at most 16384 and sort_blocks, extra_sort_blocks at most 65536");
     RMPCD_CHECK(s.cfg.collide_cells == 0 || s.cfg.collide_cells == 64 || s.cfg.collide_cells == 128 ||
                     s.cfg.collide_cells == 256,

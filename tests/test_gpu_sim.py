@@ -359,13 +359,14 @@ def test_extra_sort_launches(gpu, form, kw):
 def test_extra_sort_workgroups(gpu, form):
     """the sort after an MD step is one launch whose passes wait for each other: with one
     workgroup, with fewer than there are XCDs, with a number that is no multiple of them and
-    with as many as there are units, for boxes of one and of several scan tiles, it must
+    with as many as there are units, for boxes of two and of sixteen scan tiles, it must
     give the same state bit for bit"""
     Ls = [(24, 24, 20), (12, 16, 12)]
     kw = dict(mode=capi.SIM_FUSED, n_md=40, tau=0.5, form=form, seed=77, replica_L=Ls, skin=0.6)
     sims = [SingleDimer(**kw)] + [SingleDimer(extra_sort_blocks=b, groups=g, **kw)
                                   for b, g in ((1, 1), (5, 2), (77, 1))]
     for s in sims:
+        s.extra_sort(1)
         s.run(2)
     for r in range(len(Ls)):
         a = sims[0].download(r)
