@@ -432,8 +432,9 @@ int rmpcd_dimer_profile(rmpcd_dimer_t *sim, int32_t stride);
 int rmpcd_dimer_stream_time(rmpcd_dimer_t *sim, double *avg_ms, int32_t *samples);
 /* fused mode: the particle passes of the sorts that may follow an MD step in one launch (1) or
  * in a launch each (4), instead of by the library's own rule on sizes (0); the same results
- * either way */
-int rmpcd_dimer_extra_sort(rmpcd_dimer_t *sim, int32_t launches);
+ * either way.  The passes of one launch wait for each other, each wait at most max_polls polls
+ * (0: default, about ten seconds); one that gives up stops the replica with RMPCD_ERR_HIP */
+int rmpcd_dimer_extra_sort(rmpcd_dimer_t *sim, int32_t launches, int32_t max_polls);
 
 /* ---- the other driver loops on device-resident state --------------------------------
  * RMPCD_PROG_FLUID     test/setup_simple_fluid.f90:89-127: SRD, streaming, grid shift,

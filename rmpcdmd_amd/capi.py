@@ -187,7 +187,7 @@ SIGNATURES = {
     "rmpcd_dimer_destroy": [_P],
     "rmpcd_dimer_profile": [_P, _I],
     "rmpcd_dimer_stream_time": [_P, _D3, C.POINTER(_I)],
-    "rmpcd_dimer_extra_sort": [_P, _I],
+    "rmpcd_dimer_extra_sort": [_P, _I, _I],
     "rmpcd_threefry_uniform": [_U64, _U64, _U64, _I64, _P],
     "rmpcd_threefry2x64_20": [C.POINTER(_U64), C.POINTER(_U64), C.POINTER(_U64)],
 }

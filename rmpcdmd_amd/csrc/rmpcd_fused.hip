@@ -97,9 +97,10 @@ constexpr int KPT = 4, KCHUNK = FT * KPT;  // particles per thread and per chunk
 constexpr int KHASH_BITS = 11, KHASH = 1 << KHASH_BITS;  // LDS hash entries, 2 x KCHUNK
 constexpr int RANK_LDS = RANK_UNITS * GT + 2 * GHALO;
 // a replica's error flag: a list longer than its capacity (the reference's error stop),
-// or more particles near the colloids than a deferred extra sort can collect; every
-// kernel returns at once for a replica with the flag set, so it stops at that step
-constexpr int ERR_CANDIDATES = -100;
+// more particles near the colloids than a deferred extra sort can collect, or a wait of
+// k_fz_extra_sort that did not end; every kernel returns at once for a replica with the flag
+// set, so it stops at that step
+constexpr int ERR_CANDIDATES = -100, ERR_WAIT = -101;
 
 
 // The staging record of a sort: a particle's wrapped state, written by the key pass in
@@ -160,6 +161,7 @@ struct FB {
     int32_t *mslots, *mcount;  // per replica and sort buffer: the member slots of its last lists
     int64_t *plan;             // the replicas a sort chain works on (k_fz_plan)
     int32_t *chain;            // the counters of k_fz_extra_sort
+    int32_t max_polls;         // its waits give up after so many
     double *gpart;             // |v|^2 maximum per gather unit
     int32_t nmax;
     int32_t xcd_order;  // sort passes: units grouped by XCD (1) or a contiguous range per workgroup (0)
@@ -482,10 +484,11 @@ __device__ inline int64_t units_of(const RepDev &rp, int kind, bool fused_gather
 
 // k_fz_extra_sort's counters, a cache line each: per pass the units done, the XCDs that worked
 // on it (a bit each), those that have written their L2 back, each XCD's election of the
-// workgroup that does, and the next ticket of each queue
+// workgroup that does, and the next ticket of each queue; then whether a wait has given up
 constexpr int CHAIN_STRIDE = 32, XCCS = 16;
 enum { CH_DONE = 0, CH_XCCS, CH_WROTE, CH_ELECT, CH_NEXT = CH_ELECT + XCCS, CH_LINES = CH_NEXT + XCDS };
-constexpr int CHAIN_LEN = U_KINDS * CH_LINES * CHAIN_STRIDE;
+constexpr int CHAIN_STOP = U_KINDS * CH_LINES * CHAIN_STRIDE, CHAIN_LEN = CHAIN_STOP + CHAIN_STRIDE;
+constexpr int CHAIN_POLLS = 1 << 23;              // polls of a wait, 1 us or more each, before it gives up
 constexpr int CHAIN_RUNS = 8;                     // runs of units of a pass per workgroup
 constexpr int HWREG_XCC_ID = (31 << 11) | 20;     // s_getreg: all of HW_REG_XCC_ID
 __device__ inline int *chain_line(int *chain, int pass, int what)
@@ -496,9 +499,17 @@ __device__ inline int chain_load(const int *c)
 {
     return __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ inline void chain_wait(const int *c, int n)
+// waits for *c to reach n; false when it gave up, or another wait has
+__device__ inline bool chain_wait(const int *c, int n, int *chain, int max_polls)
 {
-    while (chain_load(c) < n) __builtin_amdgcn_s_sleep(16);
+    for (int k = 0; chain_load(c) < n; ++k) {
+        if (k >= max_polls || ((k & 255) == 255 && chain_load(&chain[CHAIN_STOP]))) {
+            atomicOr(&chain[CHAIN_STOP], 1);
+            return false;
+        }
+        __builtin_amdgcn_s_sleep(16);
+    }
+    return true;
 }
 // plan layout (int64), for a group of R replicas from r0 on: [0] active count, [1 + kind]
 // total units, then act[R] (replica of active index a), amap[R] (active index of replica
@@ -1473,7 +1484,11 @@ __global__ void __launch_bounds__(FT) k_fz_rank(FB<F> B, int R)
 // nothing in this pass, so every wait ends whatever number of workgroups the device holds at
 // once.  Between two passes the L2 of each XCD that worked on the first is written back, once,
 // by the first of its workgroups to see that all units are done (a write-back by each workgroup
-// took 40 us a pass with 64 of them on an XCD).  A full sort takes longer than in four launches
+// took 40 us a pass with 64 of them on an XCD).  That another workgroup than the writers makes it
+// rests on the hardware, not on the memory model: an XCD's workgroups share its L2, a store is
+// in it when vmcnt counts it done, and a release at agent scope writes all of it back.  Every
+// wait is bounded all the same: one that gives up stops the replicas of the sort with an error,
+// and the other workgroups with it.  A full sort takes longer than in four launches
 // (L=24 75 us against 39, L=64 300 against 196), but most steps have none: L=24 FP32 1.31 ->
 // 1.08 ms per cycle, L=48 FP64 1.96 -> 1.76, 4 x L=45 FP32 lazy 2.16 -> 1.96.
 template <class F>
@@ -1482,7 +1497,7 @@ __global__ void __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4))) k_
     __shared__ __align__(16) int buf[3 * KHASH];
     static_assert(MAX_TILES <= 3 * KHASH && 2 * RANK_LDS <= 3 * KHASH, "the passes share their LDS");
     static_assert(U_KEY == 0 && U_SCAN == 1 && U_PLACE == 2 && U_GATHER == 3 && SCAN_T == FT, "order of the passes");
-    __shared__ int lds[FT / 64], unit;
+    __shared__ int lds[FT / 64], unit, go;
     __shared__ double red[16];
     if (B.plan[0] == 0) return;
     const int xcc = (int)(__builtin_amdgcn_s_getreg(HWREG_XCC_ID) & (XCCS - 1));
@@ -1492,17 +1507,20 @@ __global__ void __launch_bounds__(FT) __attribute__((amdgpu_waves_per_eu(4))) k_
         if (T == 0) return;  // deferred sorts alone: no pass after the keys
         if (p > 0) {
             if (threadIdx.x == 0) {
-                chain_wait(chain_line(B.chain, p - 1, CH_DONE), (int)B.plan[p]);
+                go = chain_wait(chain_line(B.chain, p - 1, CH_DONE), (int)B.plan[p], B.chain, B.max_polls);
                 const int m = chain_load(chain_line(B.chain, p - 1, CH_XCCS));
                 int *wrote = chain_line(B.chain, p - 1, CH_WROTE);
-                if ((m >> xcc & 1) && atomicAdd(chain_line(B.chain, p - 1, CH_ELECT + xcc), 1) == 0) {
+                if (go && (m >> xcc & 1) && atomicAdd(chain_line(B.chain, p - 1, CH_ELECT + xcc), 1) == 0) {
                     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
                     atomicAdd(wrote, 1);
                 }
-                chain_wait(wrote, __popc((unsigned)m));
+                go = go && chain_wait(wrote, __popc((unsigned)m), B.chain, B.max_polls);
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                if (!go)
+                    for (int a = 0; a < (int)B.plan[0]; ++a) B.ctl[plan_act(B.plan)[a]].error = ERR_WAIT;
             }
             __syncthreads();
+            if (!go) return;
         }
         const int eighth = (T + XCDS - 1) / XCDS, run = (T + CHAIN_RUNS * (int)gridDim.x - 1) / (CHAIN_RUNS * (int)gridDim.x);
         int *next = chain_line(B.chain, p, CH_NEXT);
@@ -1722,6 +1740,7 @@ __global__ void __launch_bounds__(1024) k_fz_commit_list(FB<F> B, FP P, int forc
     // build; with no replica sorting the plan holds only its zero count); both blocks
     // read the same plan, so they agree even while one of them sets the error flag
     if (B.plan[0] == 0 || plan_amap(B.plan, R)[r - B.r0] < 0) return;
+    if (C.error == ERR_WAIT) return;  // a sort left half done (k_fz_extra_sort, the kernel before)
     __shared__ int skey[MAX_STENCIL], sstart[MAX_STENCIL], soff[MAX_STENCIL + 1], sflag[MAX_STENCIL];
     if (!forced && C.kind == 1) {
         __shared__ short dlut[DEFER_BOX];
@@ -2277,6 +2296,7 @@ static FB<F> make_fb(DimerSim &s, int r0 = 0, int g = 0, int64_t gpart_off = 0)
     b.mslots = s.f_mslots;
     b.plan = s.f_plan + g * plan_len(s.R);
     b.chain = s.f_chain + g * CHAIN_LEN;
+    b.max_polls = s.max_polls > 0 ? s.max_polls : CHAIN_POLLS;
     b.gpart = s.f_gpart + gpart_off;
     b.r0 = r0;
     b.mcount = s.f_mcount;
@@ -2602,11 +2622,12 @@ int fused_set_profile(DimerSim &s, int stride)
     return build_cycle(s);
 }
 
-int fused_set_extra_sort(DimerSim &s, int launches)
+int fused_set_extra_sort(DimerSim &s, int launches, int max_polls)
 {
     if (!s.fused_ready) return set_error(RMPCD_ERR_ARG, "dimer: the sort after an MD step belongs to the fused mode");
     for (hipStream_t st : s.gstreams) RMPCD_HIP(hipStreamSynchronize(st));
     s.extra_launches = launches;
+    s.max_polls = max_polls;
     return build_cycle(s);
 }
 
@@ -2782,13 +2803,15 @@ int DimerSim::sync_state()
         rp.e1 = c.e1;
         rp.e2 = c.e2;
         for (int k = 0; k < 3; ++k) rp.box.origin[k] = c.origin[k];
-        rp.error = c.error == ERR_CANDIDATES ? RMPCD_ERR_OVERFLOW : c.error;
+        rp.error = c.error == ERR_CANDIDATES ? RMPCD_ERR_OVERFLOW : c.error == ERR_WAIT ? RMPCD_ERR_HIP : c.error;
         if (c.error) err = c.error;
     }
     if (err == RMPCD_ERR_OVERFLOW) return set_error(RMPCD_ERR_OVERFLOW, "maximum of neighbor list reached");
     if (err == ERR_CANDIDATES)
         return set_error(RMPCD_ERR_OVERFLOW, "dimer: more particles near the colloids than the deferred extra "
                                              "sort's candidate buffer holds (%lld)", (long long)cand_cap);
+    if (err == ERR_WAIT)
+        return set_error(RMPCD_ERR_HIP, "dimer: a pass of the sort after an MD step waited in vain for the one before");
     if (err) return set_error(err, "dimer: device error %d", err);
     return RMPCD_OK;
 }

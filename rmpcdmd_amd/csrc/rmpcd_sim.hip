@@ -479,10 +479,11 @@ int rmpcd_dimer_stream_time(rmpcd_dimer_t *sim, double *avg_ms, int32_t *samples
     return fused_stream_time(*(DimerSim *)sim, avg_ms, samples);
 }
 
-int rmpcd_dimer_extra_sort(rmpcd_dimer_t *sim, int32_t launches)
+int rmpcd_dimer_extra_sort(rmpcd_dimer_t *sim, int32_t launches, int32_t max_polls)
 {
-    RMPCD_CHECK(sim && (launches == 0 || launches == 1 || launches == 4), "rmpcd_dimer_extra_sort: bad argument");
-    return fused_set_extra_sort(*(DimerSim *)sim, launches);
+    RMPCD_CHECK(sim && (launches == 0 || launches == 1 || launches == 4) && max_polls >= 0,
+                "rmpcd_dimer_extra_sort: bad argument");
+    return fused_set_extra_sort(*(DimerSim *)sim, launches, max_polls);
 }
 
 int rmpcd_dimer_destroy(rmpcd_dimer_t *sim)

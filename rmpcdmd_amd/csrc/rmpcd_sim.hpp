@@ -91,6 +91,7 @@ struct DimerSim {
     // its own for it
     int groups = 1;
     int extra_launches = 0;  // of the particle passes of the sort after an MD step, 0: by rule
+    int max_polls = 0;       // of a wait between them, 0: default
     std::vector<hipStream_t> gstreams;
     std::vector<hipGraph_t> graphs;
     std::vector<hipGraphExec_t> graph_execs;
@@ -122,6 +123,6 @@ int fused_prepare(DimerSim &s);
 int run_fused_cycles(DimerSim &s, int n_cycles);
 int fused_set_profile(DimerSim &s, int stride);
 int fused_stream_time(DimerSim &s, double *avg_ms, int32_t *samples);
-int fused_set_extra_sort(DimerSim &s, int launches);
+int fused_set_extra_sort(DimerSim &s, int launches, int max_polls);
 
 }  // namespace rmpcd

@@ -64,9 +64,9 @@ class SingleDimer:
                   C.byref(cells), C.byref(st))
         return sol, col, box, cells, st
 
-    def extra_sort(self, launches):
+    def extra_sort(self, launches, max_polls=0):
         """the sorts after MD steps in one launch (1), a launch per pass (4) or by rule (0)"""
-        capi.call("rmpcd_dimer_extra_sort", self._h, int(launches))
+        capi.call("rmpcd_dimer_extra_sort", self._h, int(launches), int(max_polls))
 
     @property
     def n_solvent(self):

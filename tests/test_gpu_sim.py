@@ -355,6 +355,32 @@ def test_extra_sort_launches(gpu, form, kw):
     ref.close()
 
 
+def test_extra_sort_wait_gives_up(gpu):
+    """a wait between the passes of the one-launch sort that reaches its bound (here one poll)
+    stops the replicas with an error, and the launch ends"""
+    kw = dict(mode=capi.SIM_FUSED, n_md=40, tau=0.5, form=capi.FP64, seed=78, L=(24, 24, 24), n_replicas=2, skin=0.6)
+    sim = SingleDimer(**kw)
+    sim.extra_sort(1, max_polls=1)
+    with pytest.raises(capi.RmpcdError) as e:
+        sim.run(1)
+    assert e.value.code == capi.RMPCD_ERR_HIP and "waited in vain" in e.value.msg
+    for again in (lambda: sim.run(1), lambda: sim.state(0)):  # a box left half sorted is not shown
+        with pytest.raises(capi.RmpcdError) as e:
+            again()
+        assert "waited in vain" in e.value.msg
+    sim.close()
+    # the counters are the group's own: a run with the default bound is not touched
+    ok, ref = SingleDimer(**kw), SingleDimer(**kw)
+    ok.extra_sort(1)
+    ref.extra_sort(4)
+    ok.run(2)
+    ref.run(2)
+    for r in range(2):
+        compare(ref.download(r), ok.download(r), "replica %d" % r, rtol=0.0)
+    ok.close()
+    ref.close()
+
+
 @pytest.mark.parametrize("form", [capi.FP64, capi.FP32])
 def test_extra_sort_workgroups(gpu, form):
     """the sort after an MD step is one launch whose passes wait for each other: with one
