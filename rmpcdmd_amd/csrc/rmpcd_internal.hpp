@@ -74,9 +74,10 @@ const int32_t *hilbert_lut(const Box &b);
 int check_particles(const rmpcd_particles_t *p, const char *who, bool need_force);
 int check_box(const rmpcd_box_t *b, const char *who);
 
-// rmpcd_sort on sets that the caller has checked; id_to_idx may be null (not written)
+// rmpcd_sort on sets that the caller has checked; id_to_idx may be null (not written); even:
+// the particles are known to lie about evenly in the box
 int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
-                   rmpcd_cells_t *cells, int wrap);
+                   rmpcd_cells_t *cells, int wrap, bool even);
 
 // a plain fluid's cycle on checked sets whose forces are zero: SRD on the cells of the last
 // sort, n_md streaming steps, then the sort under the next grid shift

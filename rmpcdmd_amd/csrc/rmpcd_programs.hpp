@@ -115,7 +115,7 @@ struct ProgramSim {
         rmpcd_particles_t s = sv(), d = alt();
         rmpcd_cells_t c = cells();
         // no id_to_idx: nothing in these programs reads it and the state does not show it
-        int rc = sort_unchecked(&box, &s, &d, nullptr, &c, pbc ? 1 : 0);
+        int rc = sort_unchecked(&box, &s, &d, nullptr, &c, pbc ? 1 : 0, true);
         if (rc) return rc;
         cur = 1 - cur;  // the switch() calls of particle_system.f90:346-353
         return RMPCD_OK;

@@ -3,7 +3,7 @@
 // src/particle_system.f90:304-355, src/md.f90:202-217 fused).
 //
 // Sort pipeline (all launches on the library stream).  The unit is a tile: 2^k cells with
-// consecutive Hilbert keys, about a thousand particles.
+// consecutive Hilbert keys, at most 1382 particles on average in FP32 and 460 in FP64.
 //   k_tile_key    per particle: optional periodic wrap, cell key from the box's Hilbert
 //                 table, and its place in its tile's list (an LDS hash counts the tiles of
 //                 1024 consecutive particles, one global atomic per tile met there)
@@ -12,6 +12,7 @@
 //   k_tile_gather one workgroup per tile: counts its cells (cell_count, cell_start), ranks
 //                 each particle among its cell's by original index, and moves the planes
 //                 through LDS, read in list order and written in slot order
+//   k_tile_spill  ranks and moves the particles of the tiles that the LDS does not hold
 // The order within a tile's list is not deterministic, the rank does not depend on it: the
 // result equals the reference's single-thread order, where each cell keeps increasing
 // original index.
@@ -390,12 +391,38 @@ __global__ void __launch_bounds__(1024)
     if (tid == 0) start[nt] = tot;
 }
 
+// Pieces of the tiles that hold more particles than the LDS: how many, and each one's tile
+// and number in it.
+struct SpillWork {
+    int32_t *count;
+    int2 *item;
+};
+constexpr int SPILL_PIECE = 512, SPILL_AHEAD = 8;
+// A tile's own workgroup moves up to `own` particles alone: SPILL_OWN (FP64: the LDS holds
+// fewer; L=32 with all particles in one half, 640 a tile: first sort 153 us, by k_tile_spill
+// 170), or any number in the device-resident programs, whose particles spread evenly from the
+// start, so that the launch of k_tile_spill would be for nothing (1.5 us of the 63 us cycle of an
+// L=32 FP64 fluid).
+constexpr int SPILL_OWN = 1024, SPILL_NEVER = INT32_MAX;
+constexpr unsigned SPILL_BLOCKS = 1024;  // the 512th below at 512 and 2048: 7.9, 4.6 ms; 2048 idle 1 us longer
+
+// a thread's next particles of such a tile and their cells, -1 beyond its m particles
+__device__ inline void spill_load(int32_t w[SPILL_AHEAD], int k[SPILL_AHEAD], const int32_t *__restrict__ list,
+                                  const int32_t *__restrict__ key, int cmask, int64_t q0, int m)
+{
+#pragma unroll
+    for (int u = 0; u < SPILL_AHEAD; ++u) w[u] = q0 + u * SORT_T < m ? list[q0 + u * SORT_T] : -1;
+#pragma unroll
+    for (int u = 0; u < SPILL_AHEAD; ++u) k[u] = w[u] >= 0 ? key[w[u]] & cmask : 0;
+}
+
 __global__ void k_tile_place(int64_t n, const int32_t *__restrict__ key, int shift,
                              const int32_t *__restrict__ slot, const int32_t *__restrict__ start,
-                             int32_t *__restrict__ list)
+                             int32_t *__restrict__ list, SpillWork work)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
+    if (i == 0) *work.count = 0;
     list[start[key[i] >> shift] + slot[i]] = (int32_t)i;
 }
 
@@ -425,6 +452,32 @@ __device__ inline void tile_store(T *__restrict__ plane, const T *lds, int m)
     }
 }
 
+// particle w of src to slot o of dst
+template <class F, bool FORCES>
+__device__ inline void spill_move(const Box &b, const PView<F> &src, const PView<F> &dst, int wrap, int32_t w, int64_t o,
+                                  int32_t *__restrict__ id_to_idx)
+{
+    using R = typename F::real;
+    const int64_t n = src.n;
+    for (int j = 0; j < 3; ++j) {
+        R x = src.pos[j * n + w];
+        int32_t im = src.image[j * n + w];
+        if (wrap) im += fold_pbc<R>(x, (R)b.edges[j]);
+        dst.pos[j * n + o] = x;
+        dst.image[j * n + o] = im;
+        dst.vel[j * n + o] = src.vel[j * n + w];
+        if (FORCES) {
+            dst.force[j * n + o] = src.force[j * n + w];
+            dst.force_old[j * n + o] = src.force_old[j * n + w];
+        }
+    }
+    const int32_t id = src.id[w];
+    dst.id[o] = id;
+    dst.species[o] = src.species[w];
+    dst.flags[o] = src.flags[w];
+    if (id_to_idx && (uint32_t)id < (uint32_t)n) id_to_idx[id] = (int32_t)o;
+}
+
 // The cell sort's move.  Bound by memory: FP32 it reads 74 B and writes 66 B per particle,
 // and fetches 1.33 times what it uses (tiles read the edges of their neighbours' stretches),
 // 164 B in 0.67 ms for 21 million particles, 5.1 TB/s.  Moved one particle per thread
@@ -437,7 +490,8 @@ template <class F, bool FORCES>
 __global__ void __launch_bounds__(SORT_T)
     k_tile_gather(Box b, PView<F> src, PView<F> dst, int wrap, int shift, int nt, const int32_t *__restrict__ key,
                   const int32_t *__restrict__ start, const int32_t *__restrict__ list, int32_t *__restrict__ spill,
-                  int32_t *__restrict__ cell_count, int32_t *__restrict__ cell_start, int32_t *__restrict__ id_to_idx)
+                  int32_t *__restrict__ cell_count, int32_t *__restrict__ cell_start, int own, SpillWork work,
+                  int32_t *__restrict__ id_to_idx)
 {
     using R = typename F::real;
     using S = typename F::small;
@@ -476,7 +530,14 @@ __global__ void __launch_bounds__(SORT_T)
 #pragma unroll
         for (int u = 0; u < N; ++u) d[u] = v[u] >= 0 ? atomicAdd(&lcnt[c[u]], 1) : 0;
     } else {
-        for (int q = tid; q < m; q += SORT_T) atomicAdd(&lcnt[key[list[s + q]] & cmask], 1);
+        for (int64_t q0 = tid; q0 < m; q0 += SPILL_AHEAD * SORT_T) {
+            int32_t w[SPILL_AHEAD];
+            int k[SPILL_AHEAD];
+            spill_load(w, k, list + s, key, cmask, q0, m);
+#pragma unroll
+            for (int u = 0; u < SPILL_AHEAD; ++u)
+                if (w[u] >= 0) atomicAdd(&lcnt[k[u]], 1);
+        }
     }
     __syncthreads();
     if (tid < 64) {  // one wave scans the tile's cells
@@ -547,40 +608,93 @@ __global__ void __launch_bounds__(SORT_T)
     }
     // more particles than the LDS holds: the list grouped by cell goes to memory (each
     // workgroup writes and reads its own stretch), and each particle is ranked and moved
-    // from there
+    // from there, or the pieces of a tile that is larger still go to k_tile_spill
     for (int k = tid; k < ncell; k += SORT_T) lcnt[k] = 0;
     __syncthreads();
-    for (int q = tid; q < m; q += SORT_T) {
-        const int32_t w = list[s + q];
-        const int k = key[w] & cmask;
-        spill[s + lstart[k] + atomicAdd(&lcnt[k], 1)] = w;
+    for (int64_t q0 = tid; q0 < m; q0 += SPILL_AHEAD * SORT_T) {
+        int32_t w[SPILL_AHEAD];
+        int k[SPILL_AHEAD];
+        spill_load(w, k, list + s, key, cmask, q0, m);
+#pragma unroll
+        for (int u = 0; u < SPILL_AHEAD; ++u)
+            if (w[u] >= 0) spill[s + lstart[k[u]] + atomicAdd(&lcnt[k[u]], 1)] = w[u];
     }
-    __threadfence_block();
+    if (m <= own) {
+        __threadfence_block();
+        __syncthreads();
+        for (int q = tid; q < m; q += SORT_T) {
+            const int32_t w = spill[s + q];
+            const int k = key[w] & cmask;
+            const int a = lstart[k], e = a + lcnt[k];
+            int rank = 0;
+            for (int y = a; y < e; ++y) rank += spill[s + y] < w ? 1 : 0;
+            spill_move<F, FORCES>(b, src, dst, wrap, w, s + a + rank, id_to_idx);
+        }
+        return;
+    }
+    const int pieces = (m - 1) / SPILL_PIECE + 1;
+    if (tid == 0) lv[0] = atomicAdd(work.count, pieces);
     __syncthreads();
-    for (int q = tid; q < m; q += SORT_T) {
-        const int32_t w = spill[s + q];
-        const int k = key[w] & cmask;
-        const int a = lstart[k], e = a + lcnt[k];
-        int rank = 0;
-        for (int y = a; y < e; ++y) rank += spill[s + y] < w ? 1 : 0;
-        const int64_t o = s + a + rank;
-        for (int j = 0; j < 3; ++j) {
-            R x = src.pos[j * n + w];
-            int32_t im = src.image[j * n + w];
-            if (wrap) im += fold_pbc<R>(x, (R)b.edges[j]);
-            dst.pos[j * n + o] = x;
-            dst.image[j * n + o] = im;
-            dst.vel[j * n + o] = src.vel[j * n + w];
-            if (FORCES) {
-                dst.force[j * n + o] = src.force[j * n + w];
-                dst.force_old[j * n + o] = src.force_old[j * n + w];
+    for (int k = tid; k < pieces; k += SORT_T) work.item[lv[0] + k] = make_int2(t, k);
+}
+
+// The tiles too large for their own workgroup, a piece of one per workgroup at a time: a
+// thread ranks two particles in their cells, the cells' lists staged in LDS, and moves them
+// straight between the planes.  Clustered particles fill few tiles, which would leave the rest
+// of the device idle: a sort with all particles in a half, an eighth, a 64th and a 512th of an
+// L=64 box (2.6 million FP32, in order) takes 0.30, 0.32, 0.87 and 5.3 ms; each tile by its own
+// workgroup 0.36, 1.02, 20.6 and 973; without tiles 0.42, 0.68, 1.7 and 9.7.  In no order 1.13,
+// 1.11, 1.51 and 5.2 ms; 1.14, 1.42, 22.5 and 987; 1.11, 1.10, 1.29 and 4.2.
+template <class F>
+__global__ void __launch_bounds__(SORT_T)
+    k_tile_spill(Box b, PView<F> src, PView<F> dst, int wrap, const int32_t *__restrict__ key,
+                 const int32_t *__restrict__ start, const int32_t *__restrict__ spill,
+                 const int32_t *__restrict__ cell_count, const int32_t *__restrict__ cell_start, SpillWork work,
+                 int32_t *__restrict__ id_to_idx)
+{
+    constexpr int P = SPILL_PIECE / SORT_T, STAGE = 2048;
+    __shared__ int32_t stage[STAGE];
+    __shared__ int64_t range[2];
+    const int tid = threadIdx.x;
+    const int items = *work.count;
+    for (int it = blockIdx.x; it < items; it += gridDim.x) {
+        const int2 e = work.item[it];
+        const int64_t q0 = start[e.x] + (int64_t)e.y * SPILL_PIECE, end = start[e.x + 1];
+        const int64_t q1 = q0 + SPILL_PIECE < end ? q0 + SPILL_PIECE : end;
+        int32_t w[P];
+        int64_t a[P], z[P];  // the particles' cells in the list
+        int rank[P];
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const int64_t q = q0 + tid + u * SORT_T;
+            w[u] = q < q1 ? spill[q] : -1;
+            const int c = w[u] >= 0 ? key[w[u]] : 0;
+            a[u] = w[u] >= 0 ? cell_start[c] : 0;
+            z[u] = w[u] >= 0 ? a[u] + cell_count[c] : 0;
+            rank[u] = 0;
+            // the list is grouped by cell: the piece's first and last particle bound the range
+            if (q == q0) range[0] = a[u];
+            if (q == q1 - 1) range[1] = z[u];
+        }
+        __syncthreads();
+        const int64_t r0 = range[0], r1 = range[1];
+        for (int64_t base = r0; base < r1; base += STAGE) {
+            __syncthreads();
+            for (int k = tid; k < STAGE && base + k < r1; k += SORT_T) stage[k] = spill[base + k];
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < P; ++u) {
+                const int lo = (int)(a[u] > base ? a[u] - base : 0);
+                const int hi = (int)(z[u] < base + STAGE ? z[u] - base : STAGE);
+                int r = 0;
+                for (int k = lo; k < hi; ++k) r += stage[k] < w[u] ? 1 : 0;
+                rank[u] += r;
             }
         }
-        const int32_t id = src.id[w];
-        dst.id[o] = id;
-        dst.species[o] = src.species[w];
-        dst.flags[o] = src.flags[w];
-        if (id_to_idx && (uint32_t)id < (uint32_t)n) id_to_idx[id] = (int32_t)o;
+#pragma unroll
+        for (int u = 0; u < P; ++u)
+            if (w[u] >= 0) spill_move<F, true>(b, src, dst, wrap, w[u], a[u] + rank[u], id_to_idx);
+        __syncthreads();
     }
 }
 
@@ -600,9 +714,11 @@ int count_impl(const rmpcd_box_t *box, const rmpcd_particles_t *pp, rmpcd_cells_
 }
 
 // cells per tile (a power of two): the most whose particles, at the mean density of the
-// cells inside the box, fill at most 0.9 of the LDS (a tile above that by chance still fits:
-// three standard deviations of 1400 particles are 112), and small enough that a box has two
-// workgroups for every compute unit (a floor of 1024 or 2048 tiles made no difference)
+// cells inside the box, fill at most 0.9 of the LDS (in FP32 a tile above that by chance still
+// fits: three standard deviations of 1382 particles are 112, and 154 are spare; in FP64 52 are
+// spare, 2.4 standard deviations of 460, and a tile above that is moved from memory), and small
+// enough that a box has two workgroups for every compute unit (a floor of 1024 or 2048 tiles made
+// no difference)
 static int tile_shift(const Box &b, int64_t n, int tile_max)
 {
     const double per_cell = (double)n / ((double)b.L[0] * b.L[1] * b.L[2]);
@@ -619,6 +735,7 @@ struct TileSort {
     const int32_t *lut;
     int shift, nt, stride;
     int32_t *key, *slot, *list, *start, *count;
+    SpillWork work;
 };
 
 template <class F>
@@ -631,7 +748,12 @@ static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
     t.key = (int32_t *)workspace(WS_KEY, sizeof(int32_t) * n);
     t.slot = (int32_t *)workspace(WS_SLOT, sizeof(int32_t) * n);
     t.list = (int32_t *)workspace(WS_TMP, sizeof(int32_t) * n);
-    t.start = (int32_t *)workspace(WS_TILE, sizeof(int32_t) * ((size_t)t.nt + 1));
+    // the tiles' starts, the spill pieces' number, the pieces: one per SPILL_PIECE particles, and
+    // a last, shorter one per tile that overflows
+    const size_t words = ((size_t)t.nt + 2 + 1) & ~(size_t)1;
+    const size_t most = (size_t)(n / SPILL_PIECE + n / SPILL_OWN + 1);
+    t.start = (int32_t *)workspace(WS_TILE, sizeof(int32_t) * words + sizeof(int2) * most);
+    if (t.start) t.work = {t.start + t.nt + 1, (int2 *)(t.start + words)};
     t.count = (int32_t *)workspace(WS_TCOUNT, sizeof(int32_t) * ((size_t)t.nt + 1) * t.stride);  // zero between sorts
     if (!t.key || !t.slot || !t.list || !t.start || !t.count)
         return set_error(RMPCD_ERR_HIP, "rmpcd_sort: workspace allocation failed");
@@ -643,7 +765,7 @@ static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
 // the sort after its keys
 template <class F, bool FORCES>
 static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
-                            int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap)
+                            int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, int own)
 {
     const int64_t n = src->n;
     hipStream_t s = stream();
@@ -657,19 +779,27 @@ static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmp
         RMPCD_LAUNCHED();
     }
     zeroed_close(WS_TCOUNT);
-    k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, t.key, t.shift, t.slot, t.start, t.list);
+    k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, t.key, t.shift, t.slot, t.start, t.list, t.work);
     RMPCD_LAUNCHED();
     const unsigned runs = (unsigned)((t.nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
     k_tile_gather<F, FORCES><<<8 * TILE_RUN * runs, SORT_T, 0, s>>>(t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt,
                                                                     t.key, t.start, t.list, t.slot, cells->cell_count,
-                                                                    cells->cell_start, id_to_idx);
+                                                                    cells->cell_start, own, t.work, id_to_idx);
     RMPCD_LAUNCHED();
+    if constexpr (FORCES) {  // the others are the programs'
+        if (n <= own || n <= TILE_MAX<F>) return RMPCD_OK;  // no tile holds more
+        const unsigned pieces = blocks_for(n, SPILL_PIECE);
+        k_tile_spill<F><<<pieces < SPILL_BLOCKS ? pieces : SPILL_BLOCKS, SORT_T, 0, s>>>(
+            t.b, view<F>(src), view<F>(dst), wrap, t.key, t.start, t.slot, cells->cell_count, cells->cell_start, t.work,
+            id_to_idx);
+        RMPCD_LAUNCHED();
+    }
     return RMPCD_OK;
 }
 
 template <class F>
 int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
-              int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap)
+              int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, int own)
 {
     TileSort t;
     int rc = tile_sort_begin<F>(box, src->n, t);
@@ -677,7 +807,7 @@ int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_partic
     k_tile_key<F><<<blocks_for(src->n, KEY_CHUNK), SORT_T, 0, stream()>>>(t.b, t.lut, view<F>(src), wrap, t.shift,
                                                                           t.stride, t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    return tile_sort_finish<F, true>(t, src, dst, id_to_idx, cells, wrap);
+    return tile_sort_finish<F, true>(t, src, dst, id_to_idx, cells, wrap, own);
 }
 
 template <class F>
@@ -694,7 +824,7 @@ int fluid_cycle_impl(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpc
         t.b, t.lut, view<F>(src), cells->cell_start, cells->cell_count, cshift, seed, step, n_md, dt, t.shift, t.stride,
         t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    return tile_sort_finish<F, false>(t, src, dst, nullptr, cells, 0);
+    return tile_sort_finish<F, false>(t, src, dst, nullptr, cells, 0, SPILL_NEVER);
 }
 
 int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
@@ -704,9 +834,9 @@ int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src,
 }
 
 int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
-                   rmpcd_cells_t *cells, int wrap)
+                   rmpcd_cells_t *cells, int wrap, bool even)
 {
-    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, wrap);
+    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, wrap, even ? SPILL_NEVER : SPILL_OWN);
 }
 
 template <class F>
@@ -775,7 +905,7 @@ int rmpcd_sort(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_parti
                     src->force_old != dst->force_old && src->image != dst->image &&
                     src->id != dst->id && src->species != dst->species && src->flags != dst->flags,
                 "rmpcd_sort: source and destination share an array (the sort is out of place)");
-    return sort_unchecked(box, src, dst, id_to_idx, cells, apply_pbc ? 1 : 0);
+    return sort_unchecked(box, src, dst, id_to_idx, cells, apply_pbc ? 1 : 0, false);
 }
 
 }  // extern "C"

@@ -162,6 +162,47 @@ def test_sort_tiles(gpu, L, n, spread, form):
     assert same_bits(i2i_d.cpu().numpy(), i2i)
 
 
+@pytest.mark.parametrize("form", [0, 1])
+@pytest.mark.parametrize("L,n,parts", [
+    ((32, 32, 32), 30000, [(0.9, (3, 3, 3)), (0.1, (32, 32, 32))]),        # a cluster in a thin gas
+    ((16, 16, 16), 20000, [(0.5, (1, 1, 1)), (0.25, (2, 1, 1)), (0.25, (16, 16, 16))]),  # cells beyond a piece
+    ((20, 10, 6), 2500, [(1.0, (5, 5, 5))]),
+])
+def test_sort_clusters(gpu, L, n, parts, form):
+    """the sort of clustered particles, whose tiles the LDS does not hold, with the periodic
+    wrap; positions are multiples of 2^-10, so both forms place them in the oracle's cells"""
+    rng = np.random.default_rng(n)
+    ps = O.PState(n)
+    a = 0
+    for share, hi in parts:
+        m = n - a if share == parts[-1][0] and hi == parts[-1][1] else int(share * n)
+        ps.pos[a:a + m] = rng.integers(0, np.array(hi) * 1024, size=(m, 3)) / 1024.0
+        a += m
+    ps.pos[:] += rng.integers(-1, 2, size=(n, 3)) * np.array(L)
+    ps.vel[:] = rng.integers(-999, 999, size=(n, 3)) / 256.0
+    ps.force[:] = rng.integers(-999, 999, size=(n, 3)) / 256.0
+    ps.force_old[:] = rng.integers(-999, 999, size=(n, 3)) / 256.0
+    ps.image[:] = rng.integers(-3, 4, size=(n, 3))
+    ps.species[:] = rng.integers(0, 4, size=n)
+    ps.flags[:] = rng.integers(0, 128, size=n)
+    ps.id[:] = rng.permutation(n).astype(np.int32)
+    order = rng.permutation(n)
+    for k in ("pos", "vel", "force", "force_old", "image", "species", "flags"):
+        getattr(ps, k)[:] = getattr(ps, k)[order]
+    c = O.cells_init(L)
+    src, dst, cs = to_device(ps, form=form), ParticleSet(n, form=form), cells_to_device(c)
+    O.apply_pbc(ps.pos, ps.image, tuple(float(v) for v in L))
+    srt, i2i, cnt, st = O.sort(c, ps)
+    i2i_d = torch.zeros(n, dtype=torch.int32, device="cuda")
+    for _ in range(2):
+        capi.call("rmpcd_sort", cs.boxp(), src.struct(), dst.struct(), ptr(i2i_d), cs.cellsp(), 1)
+    torch.cuda.synchronize()
+    assert same_bits(cs.cell_count.cpu().numpy(), cnt) and same_bits(cs.cell_start.cpu().numpy(), st)
+    for name in ("pos", "vel", "force", "force_old", "image", "id", "species", "flags"):
+        assert (dst.host(name) == getattr(srt, name)).all(), name
+    assert same_bits(i2i_d.cpu().numpy(), i2i)
+
+
 @pytest.mark.parametrize("L,n", [((24, 20, 12), 30000), ((256, 256, 128), 100000)])
 def test_sort_after_a_failed_sort(gpu, L, n):
     """a sort that stops at an error with its key pass queued leaves tile counts behind; the

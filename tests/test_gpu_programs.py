@@ -62,6 +62,7 @@ def test_fluid_matches_oracle(gpu, n_md):
 @pytest.mark.parametrize("L,rho,n_md", [
     ((13, 10, 7), 10, 2),   # workgroups of several cells, a padded box
     ((4, 4, 4), 900, 1),    # one cell holds more particles than a workgroup's LDS
+    ((4, 4, 4), 1700, 1),   # and than the LDS of the sort's move in either form
     ((9, 8, 8), 1, 1),      # cells with one particle or none
 ])
 def test_fluid_equals_entry_points(gpu, form, L, rho, n_md):
