@@ -321,6 +321,8 @@ __device__ inline double sqrt_mid(double x)
 // 1e200 on, and for 0, infinities and NaN
 constexpr uint32_t MID_LOW = (1023u - 665u) << 21, MID_SPAN = (665u + 664u) << 21;
 __device__ inline uint32_t mid_off(double x) { return ((uint32_t)__double2hiint(x) << 1) - MID_LOW; }
+// the same in single units for an x that has to be positive: more than MID_SPAN / 2 for the rest
+__device__ inline uint32_t mid_off_pos(double x) { return (uint32_t)__double2hiint(x) - MID_LOW / 2; }
 
 // The steps of a block for one wave.  A lane's update needs its entry, then the constants of
 // the entry's link (and with kG the update's multiplier from g): they are read from memory
@@ -381,7 +383,12 @@ __device__ inline void for_steps(const WaveView &w, const double *lc, const doub
 //
 // The square root and the division of an update are made without the general forms' scaling
 // and special cases; what they leave out is watched for (the largest mid_off of their
-// operands), and a block that met it is run again from its start with the general forms.
+// operands), and a block that met it is run again from its start with the general forms.  A
+// position's multiplier needs no watch of its own: with the root between 1e-100 and 1e100 its
+// numerator is +0, for which div_by is exact, or at least an ulp of the root, 1e-117, and it
+// is at most 1e155, beyond which the discriminant is not finite.  (Watched too, the zeros of
+// a body at rest or of links at their exact length sent blocks to the general forms: a
+// 60-bead shell with half its beads at rest 459 us a call, 372 like this.)
 //
 // Bound by one wave's issue and the latency of a step's chain of LDS reads and FP64
 // operations (one update after the other along the longest chain of links): 0.21 us a step.
@@ -473,7 +480,7 @@ __global__ void __launch_bounds__(WT)
                 const double disc = rs * rs - c[7] * (ssq - c[8]);
                 if (kFast) {
                     g = rs - sqrt_mid(disc);
-                    off = max(off, max(mid_off(disc), mid_off(g)));
+                    off = max(off, mid_off_pos(disc));
                 } else {
                     g = rs - sqrt(disc);
                 }
@@ -498,7 +505,7 @@ __global__ void __launch_bounds__(WT)
                 at[tid & 63] = g;
             }
         });
-        return !__any(off > MID_SPAN);
+        return !__any(off > (kPos ? MID_SPAN / 2 : MID_SPAN));
     };
     const std::true_type yes{};
     const std::false_type no{};

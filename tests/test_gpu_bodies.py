@@ -92,10 +92,10 @@ def test_rattle_body_pos_vel(gpu, n, radius, centre, edges):
     assert same_bits(g.host("vel"), want.vel)
 
 
-@pytest.mark.parametrize("case", ["at rest", "unsatisfiable", "far too large"])
+@pytest.mark.parametrize("case", ["at rest", "half at rest", "unsatisfiable", "far too large"])
 def test_rattle_body_edges(gpu, case):
-    """where the one-wave rattle leaves its usual way: multipliers of zero (a body at rest),
-    the last, shorter block of 1000 sweeps, a body beyond its 16-bit offsets and LDS"""
+    """where the one-wave rattle leaves its usual way: multipliers of zero (a body or a part of
+    it at rest), the last, shorter block of 1000 sweeps, a body beyond the LDS"""
     n, radius, edges = {"far too large": (2400, 14.0, np.array([60.0] * 3))}.get(case, (24, 2.0, EDGES))
     ps, links, d, rng = sphere_body(n, radius, edges / 2, 77)
     mass = np.array([1.0, 2.5])
@@ -103,6 +103,9 @@ def test_rattle_body_edges(gpu, case):
     precision = 1e-4 if case == "far too large" else 1e-11
     if case == "at rest":
         ps.vel[:] = 0
+    elif case == "half at rest":
+        ps.vel[:12] = 0
+        ps.pos[12:] += 0.001 * rng.normal(size=(12, 3))
     else:
         ps.pos[:] += 0.001 * rng.normal(size=ps.pos.shape)
     if case == "unsatisfiable":
