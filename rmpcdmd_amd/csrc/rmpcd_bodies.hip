@@ -34,7 +34,12 @@ constexpr int RATTLE_MAX = 1000;  // md.f90:341, :432
 constexpr int KMAX = 16;          // sweeps per block at most (4 bits of the entry)
 constexpr int AHEAD = 4;          // steps that a link's constants are read ahead of their use
 constexpr int LC = 10;            // doubles per link of its constants
-constexpr int WAVE_N = 2700;      // particles of the one-wave rattle at most (16-bit offsets)
+// particles of the one-wave rattle at most, for its 16-bit offsets (with 160 KiB of LDS the
+// snapshot of one sweep ends it at 1687 for positions and 2250 for velocities)
+constexpr int WAVE_N = 2700;
+// Entries of its schedule at most, 64 MiB: every step takes 64, however few updates may run
+// side by side, so a list that is one long chain would take 64 times its updates.
+constexpr int64_t WAVE_ENTRIES = 1 << 22;
 
 struct BodyMass {
     double m[16];    // particle_system%mass by species (species s at s - 1)
@@ -48,6 +53,7 @@ __device__ inline double dot3b(const double a[3], const double b[3]) { return (a
 // unchanged (compared by content on every call).
 struct BlockSched {
     int K = 0, n_steps = 0;   // n_steps a multiple of 2 AHEAD
+    bool too_long = false;    // more than WAVE_ENTRIES: not built
     // 64 per step, all as byte offsets that a lane can use as they are: {a | b << 16 in the
     // particles, the link's constants | sweep, where a's and b's state go in the snapshots}
     uint4 *d_ent = nullptr;
@@ -180,8 +186,9 @@ static int get_schedule(const int32_t *links, const double *dist, int n_links, i
     return RMPCD_OK;
 }
 
-// the unrolled schedule of K sweeps, built once per list and K: each step takes, of the
-// updates whose predecessors have run, the up to 64 with the longest chain behind them
+// the unrolled schedule of K sweeps, built once per list and K (null if it is too long): each
+// step takes, of the updates whose predecessors have run, the up to 64 with the longest chain
+// behind them
 static int get_block(Schedule &s, int K, const BlockSched **out)
 {
     BlockSched &b = s.blocks[K];
@@ -189,6 +196,8 @@ static int get_block(Schedule &s, int K, const BlockSched **out)
         *out = &b;
         return RMPCD_OK;
     }
+    *out = nullptr;
+    if (b.too_long || (int64_t)K * s.n_links > WAVE_ENTRIES) return RMPCD_OK;
     const int nl = s.n_links, nt = K * nl;
     const int32_t *links = s.links.data();
     // the next update of a's and of b's particle, the number of updates waited for, the
@@ -207,6 +216,10 @@ static int get_block(Schedule &s, int K, const BlockSched **out)
             }
         height[t] = h + 1;
         last[x[0]] = last[x[1]] = t;
+        if ((int64_t)height[t] * 64 > WAVE_ENTRIES) {
+            b.too_long = true;
+            return RMPCD_OK;
+        }
     }
     // the longest chain first, the earlier update among equals
     auto later = [&](int32_t p, int32_t q) { return height[p] != height[q] ? height[p] < height[q] : p > q; };
@@ -246,6 +259,10 @@ static int get_block(Schedule &s, int K, const BlockSched **out)
         while (ent.size() % 64) pad();
         if (ready.empty())  // idle steps up to a whole turn, and one more turn to read ahead
             while (ent.size() % (64 * 2 * AHEAD)) pad();
+        if ((int64_t)ent.size() > WAVE_ENTRIES) {
+            b.too_long = true;
+            return RMPCD_OK;
+        }
     }
     const size_t n_ent = ent.size();
     for (int k = 0; k < 64 * 2 * AHEAD; ++k) {
@@ -1035,7 +1052,7 @@ static int fetch_i32(const int32_t *dev, int32_t *host_out)
 }
 
 // which rattle runs: the one-wave one with the most sweeps per block whose snapshots fit in
-// LDS, else the global one
+// LDS and whose schedule is not too long, else the global one
 static int pick_k(Schedule &s, bool with_pr, const BlockSched **blk, size_t *lds)
 {
     *blk = nullptr;
@@ -1044,8 +1061,10 @@ static int pick_k(Schedule &s, bool with_pr, const BlockSched **blk, size_t *lds
     for (int K = KMAX; K >= 1; --K) {
         const size_t need = wave_lds_bytes(s.n, K, with_pr);
         if (need > (size_t)lds_limit()) continue;
+        int rc = get_block(s, K, blk);
+        if (rc) return rc;
         *lds = need;
-        return get_block(s, K, blk);
+        if (*blk) return RMPCD_OK;
     }
     return RMPCD_OK;
 }

@@ -56,8 +56,8 @@ def fold(x, edges=EDGES):
     return x - np.floor(x / edges) * edges
 
 
-# up to 900 beads the body and its schedule fit in LDS (12 sweeps overlapped for 300
-# beads, 1 or 2 for 900); 1400 beads (5800 links) run from global memory
+# 16 sweeps overlap for up to 300 beads, 4 for 900 (6 for the velocities), 1 for 1400 (2);
+# test_rattle_body_edges has a body that runs from global memory
 @pytest.mark.parametrize("n,radius,centre,edges", [
     (12, 2.0, (8.0, 6.0, 10.0), EDGES),
     (60, 2.0, (15.5, 0.3, 19.6), EDGES),
@@ -126,6 +126,31 @@ def test_rattle_body_edges(gpu, case):
     capi.call("rmpcd_rattle_body_vel", g.struct(), lk, dd, len(d), m, 2, 0.01, capi.d3(edges), precision, C.byref(it))
     assert it.value == it_v
     assert same_bits(g.host("pos"), want.pos) and same_bits(g.host("vel"), want.vel)
+
+
+def test_rattle_body_long_chain(gpu):
+    """a link list that is one chain of 72,000 updates: its one-wave schedule, of which a step
+    would hold one update, is not built, and the call takes no more than some MiB"""
+    n = 12
+    ps, _, _, rng = sphere_body(n, 2.0, EDGES / 2, 5)
+    ring = np.stack([np.arange(n), (np.arange(n) + 1) % n], 1).astype(np.int32)
+    links = np.ascontiguousarray(np.tile(ring, (6000, 1)))
+    d = np.ascontiguousarray(np.tile(np.linalg.norm(ps.pos[ring[:, 0]] - ps.pos[ring[:, 1]], axis=1), 6000))
+    mass, rattle = np.array([1.0, 2.5]), ps.pos.copy()
+    ps.pos[:] += 0.001 * rng.normal(size=ps.pos.shape)
+    g = to_device(ps)
+    rt, lk, dd, m, it = dev(rattle.T), host(links), host(d), (C.c_double * 2)(*mass), C.c_int32(0)
+    want, want_r = ps.copy(), rattle.copy()
+    it_p = O.rattle_body_pos(want.pos, want.vel, want_r, want.species, mass, links, d, 0.01, EDGES, 1e-9)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    capi.call("rmpcd_rattle_body_pos", g.struct(), ptr(rt), lk, dd, len(d), m, 2, 0.01, capi.d3(EDGES), 1e-9, C.byref(it))
+    assert it.value == it_p
+    assert same_bits(g.host("pos"), want.pos) and same_bits(g.host("vel"), want.vel)
+    it_v = O.rattle_body_vel(want.pos, want.vel, want.species, mass, links, d, 0.01, EDGES, 1e-9)
+    capi.call("rmpcd_rattle_body_vel", g.struct(), lk, dd, len(d), m, 2, 0.01, capi.d3(EDGES), 1e-9, C.byref(it))
+    assert it.value == it_v and same_bits(g.host("vel"), want.vel)
+    assert free - torch.cuda.mem_get_info()[0] < 64 << 20
 
 
 def test_rattle_body_without_links(gpu):
