@@ -61,14 +61,14 @@ __global__ void k_apply_pbc(int64_t n, typename F::real *__restrict__ pos, int32
     }
 }
 
-template <class F>
+template <class F, int LANES>
 __global__ void __launch_bounds__(256)
     k_cell_md_pos(Box b, const int32_t *__restrict__ start, const int32_t *__restrict__ count,
                   const uint8_t *__restrict__ is_md, PView<F> p, double dt, int md_flag, int wall_axis)
 {
     using R = typename F::real;
     const R rdt = (R)dt, dt_sq = (R)((dt * dt) / 2);
-    for_md_cells(b.ncells, start, count, is_md, md_flag, [&](int64_t j) {
+    for_md_cells<LANES>(b.ncells, start, count, is_md, md_flag, [&](int64_t j) {
         R x[3], v[3];
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -106,7 +106,7 @@ __global__ void __launch_bounds__(256)
     });
 }
 
-template <class F>
+template <class F, int LANES>
 __global__ void __launch_bounds__(256)
     k_cell_md_vel(int ncells, const int32_t *__restrict__ start,
                   const int32_t *__restrict__ count, const uint8_t *__restrict__ is_md,
@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(256)
 {
     using R = typename F::real;
     const R rdt = (R)dt;
-    for_md_cells(ncells, start, count, is_md, md_flag, [&](int64_t j) {
+    for_md_cells<LANES>(ncells, start, count, is_md, md_flag, [&](int64_t j) {
         int f = (int)p.flags[j];
         if (!(f & WALL_MASK)) {
 #pragma unroll
@@ -147,7 +147,7 @@ __global__ void __launch_bounds__(256)
 }
 
 // cell_maximum_displacement (particle_system.f90:380-410)
-template <class F>
+template <class F, int LANES>
 __global__ void __launch_bounds__(256)
     k_cell_max_disp(int ncells, const int32_t *__restrict__ start,
                     const int32_t *__restrict__ count, const uint8_t *__restrict__ is_md,
@@ -156,7 +156,7 @@ __global__ void __launch_bounds__(256)
 {
     __shared__ double red[16];
     double local = 0;
-    for_md_cells(ncells, start, count, is_md, 1, [&](int64_t j) { local = fmax(local, disp_sq<F>(p, pos_old, j)); });
+    for_md_cells<LANES>(ncells, start, count, is_md, 1, [&](int64_t j) { local = fmax(local, disp_sq<F>(p, pos_old, j)); });
     const double m = block_max(local, red);
     if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
@@ -266,8 +266,10 @@ int cell_md_pos_impl(const rmpcd_box_t *box, const rmpcd_cells_t *cells, rmpcd_p
                      double dt, int md_flag, int axis)
 {
     Box b = make_box(box);
-    k_cell_md_pos<F><<<cell_blocks(b.ncells), 256, 0, stream()>>>(
-        b, cells->cell_start, cells->cell_count, cells->is_md, view<F>(pp), dt, md_flag, axis);
+    by_density(box, pp->n, [&](auto lanes) {
+        k_cell_md_pos<F, decltype(lanes)::value><<<cell_blocks(b.ncells), 256, 0, stream()>>>(
+            b, cells->cell_start, cells->cell_count, cells->is_md, view<F>(pp), dt, md_flag, axis);
+    });
     RMPCD_LAUNCHED();
     return RMPCD_OK;
 }
@@ -275,8 +277,10 @@ template <class F>
 int cell_md_vel_impl(const rmpcd_box_t *box, const rmpcd_cells_t *cells, rmpcd_particles_t *pp,
                      double dt, int md_flag)
 {
-    k_cell_md_vel<F><<<cell_blocks(box->ncells), 256, 0, stream()>>>(
-        box->ncells, cells->cell_start, cells->cell_count, cells->is_md, view<F>(pp), dt, md_flag);
+    by_density(box, pp->n, [&](auto lanes) {
+        k_cell_md_vel<F, decltype(lanes)::value><<<cell_blocks(box->ncells), 256, 0, stream()>>>(
+            box->ncells, cells->cell_start, cells->cell_count, cells->is_md, view<F>(pp), dt, md_flag);
+    });
     RMPCD_LAUNCHED();
     return RMPCD_OK;
 }
@@ -313,9 +317,11 @@ int cell_max_disp_impl(const rmpcd_box_t *box, const rmpcd_cells_t *cells,
     const unsigned nb = cell_blocks(box->ncells);
     double *part = (double *)workspace(WS_PART, sizeof(double) * nb);
     if (!part) return set_error(RMPCD_ERR_HIP, "cell_maximum_displacement: workspace allocation failed");
-    k_cell_max_disp<F><<<nb, 256, 0, stream()>>>(
-        box->ncells, cells->cell_start, cells->cell_count, cells->is_md, p,
-        (const typename F::real *)pos_old, part);
+    by_density(box, pp->n, [&](auto lanes) {
+        k_cell_max_disp<F, decltype(lanes)::value><<<nb, 256, 0, stream()>>>(
+            box->ncells, cells->cell_start, cells->cell_count, cells->is_md, p,
+            (const typename F::real *)pos_old, part);
+    });
     RMPCD_LAUNCHED();
     int rc = fetch_max(part, nb, r);
     if (rc) return rc;

@@ -27,12 +27,11 @@ __device__ inline int stencil_key(const Box &b, const double *x, const int32_t *
 }
 
 // pass 1 (fill == 0) counts accepted particles per (point, stencil cell) and marks
-// is_md / is_reac; pass 2 (fill == 1) writes them at offset[point*ns + j].  NL_LANES lanes
+// is_md / is_reac; pass 2 (fill == 1) writes them at offset[point*ns + j].  LANES lanes
 // take a stencil cell, a particle each (a thread per cell walked its ten particles one
-// after the other: 15 us a pass for one point with 1500 stencil cells, FP64).
-constexpr int NL_LANES = 16;
-
-template <class F>
+// after the other: 15 us a pass for one point with 1500 stencil cells, FP64), fewer for
+// less dense cells (by_density).
+template <class F, int LANES>
 __global__ void __launch_bounds__(NL_THREADS)
     k_nl_pass(Box b, PView<F64> pts, PView<F> sol, const int32_t *__restrict__ start,
               const int32_t *__restrict__ count, const int32_t *__restrict__ st, int ns,
@@ -40,10 +39,10 @@ __global__ void __launch_bounds__(NL_THREADS)
               int32_t *__restrict__ cnt, uint8_t *__restrict__ is_md, uint8_t *__restrict__ is_reac,
               int fill, int32_t nmax, int32_t *__restrict__ list)
 {
-    const int j = (blockIdx.x * blockDim.x + threadIdx.x) / NL_LANES;
+    const int j = (blockIdx.x * blockDim.x + threadIdx.x) / LANES;
     const int i = blockIdx.y;
     if (j >= ns) return;  // all lanes of a cell alike
-    const int lane = threadIdx.x & 63, sub = lane & (NL_LANES - 1), first = lane - sub;
+    const int lane = threadIdx.x & 63, sub = lane & (LANES - 1), first = lane - sub;
     double x[3] = {pts.pos[i], pts.pos[pts.n + i], pts.pos[2 * pts.n + i]};
     int si = pts.species[i];
     int key = stencil_key(b, x, st, j);
@@ -52,7 +51,7 @@ __global__ void __launch_bounds__(NL_THREADS)
     int off = fill ? cnt[slot] : 0;
     int k = 0;
     bool noreac = false;
-    for (int q0 = s; q0 < s + n; q0 += NL_LANES) {
+    for (int q0 = s; q0 < s + n; q0 += LANES) {
         const int q = q0 + sub;
         const int sp = q < s + n ? (int)sol.species[q] : 0;
         bool in = false;
@@ -64,7 +63,7 @@ __global__ void __launch_bounds__(NL_THREADS)
             if (in && do_lj && rsq <= lj.cut_sq[(sp - 1) + lj.n1 * (si - 1)]) noreac = true;
         }
         // the accepted lanes of this cell, in the cell's order
-        const unsigned m = (unsigned)(__ballot(in) >> first) & ((1u << NL_LANES) - 1);
+        const unsigned m = (unsigned)(__ballot(in) >> first) & ((1u << LANES) - 1);
         if (fill && in) {
             const int pos = off + k + __popc(m & ((1u << sub) - 1));
             if (pos < nmax) list[(int64_t)i * nmax + pos] = q;
@@ -72,7 +71,7 @@ __global__ void __launch_bounds__(NL_THREADS)
         k += __popc(m);
     }
     if (!fill) {
-        const unsigned nr = (unsigned)(__ballot(noreac) >> first) & ((1u << NL_LANES) - 1);
+        const unsigned nr = (unsigned)(__ballot(noreac) >> first) & ((1u << LANES) - 1);
         if (sub == 0) {
             cnt[slot] = k;
             if (k > 0) {
@@ -382,16 +381,21 @@ int update_list_impl(const rmpcd_box_t *box, rmpcd_cells_t *cells, const rmpcd_p
     k_init_cells<<<blocks_for(b.ncells, 256), 256, 0, s>>>(b.ncells, cells->is_md, cells->is_reac);
     volatile int32_t *host = (int32_t *)(pin + 32);
     *host = 0;
-    dim3 grid(blocks_for((int64_t)ns * NL_LANES, NL_THREADS), np);
-    k_nl_pass<F><<<grid, NL_THREADS, 0, s>>>(b, view<F64>(points), view<F>(solvent), cells->cell_start,
-                                             cells->cell_count, stencil, ns, radius * radius, L0, L1, L2,
-                                             lj ? 1 : 0, l, cnt, cells->is_md, cells->is_reac, 0, nmax, list);
+    auto pass = [&](int fill) {
+        by_density(box, solvent->n, [&](auto lanes) {
+            constexpr int LANES = decltype(lanes)::value;
+            const dim3 grid(blocks_for((int64_t)ns * LANES, NL_THREADS), np);
+            k_nl_pass<F, LANES><<<grid, NL_THREADS, 0, s>>>(b, view<F64>(points), view<F>(solvent), cells->cell_start,
+                                                            cells->cell_count, stencil, ns, radius * radius, L0, L1, L2,
+                                                            lj ? 1 : 0, l, cnt, cells->is_md, cells->is_reac, fill, nmax,
+                                                            list);
+        });
+    };
+    pass(0);
     RMPCD_LAUNCHED();
     k_nl_scan<<<np, 1024, 0, s>>>(cnt, ns, nmax, n, (int32_t *)(pin + 32));
     RMPCD_LAUNCHED();
-    k_nl_pass<F><<<grid, NL_THREADS, 0, s>>>(b, view<F64>(points), view<F>(solvent), cells->cell_start,
-                                             cells->cell_count, stencil, ns, radius * radius, L0, L1, L2,
-                                             lj ? 1 : 0, l, cnt, cells->is_md, cells->is_reac, 1, nmax, list);
+    pass(1);
     RMPCD_LAUNCHED();
     RMPCD_HIP(hipStreamSynchronize(s));
     if (*host) return set_error(RMPCD_ERR_OVERFLOW, "maximum of neighbor list reached");

@@ -165,7 +165,7 @@ __global__ void __launch_bounds__(256)
 }
 
 // COLLOIDS: cell_md_pos with md_flag true and cell_maximum_displacement over the same cells
-template <class F>
+template <class F, int LANES>
 __global__ void __launch_bounds__(256)
     k_cells_move(int ncells, const int32_t *__restrict__ start, const int32_t *__restrict__ count,
                  const uint8_t *__restrict__ is_md, PView<F> p, const typename F::real *__restrict__ pos_old, double dt,
@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(256)
     __shared__ double red[16];
     const R rdt = (R)dt, dt_sq = (R)((dt * dt) / 2);
     double r_sq = 0;
-    for_md_cells(ncells, start, count, is_md, 1, [&](int64_t j) {
+    for_md_cells<LANES>(ncells, start, count, is_md, 1, [&](int64_t j) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             const int64_t q = k * p.n + j;
@@ -581,8 +581,11 @@ static int colloids_step_t(ProgramSim &m)
     const size_t moves = (size_t)nb + cb, lists = 4 * (size_t)lb * m.nc;
     double *part = (double *)workspace(WS_PART, sizeof(double) * (moves > lists ? moves : lists));
     if (!part) return set_error(RMPCD_ERR_HIP, "program: workspace allocation failed");
-    k_cells_move<F><<<nb, 256, 0, st>>>(m.box.ncells, c.cell_start, c.cell_count, c.is_md, view<F>(&s),
-                                        (const typename F::real *)m.alt().pos, m.dt, part);
+    by_density(&m.box, m.n, [&](auto lanes) {
+        k_cells_move<F, decltype(lanes)::value><<<nb, 256, 0, st>>>(m.box.ncells, c.cell_start, c.cell_count, c.is_md,
+                                                                    view<F>(&s), (const typename F::real *)m.alt().pos,
+                                                                    m.dt, part);
+    });
     RMPCD_LAUNCHED();
     k_colloids_move<<<cb, 256, 0, st>>>(view<F64>(&p), m.col_mass, m.col_pos_old, m.dt, part + nb);
     RMPCD_LAUNCHED();

@@ -2,6 +2,8 @@
 // rmpcd_nlist.hip) and the programs that fuse them (rmpcd_programs.hip): the walk over the
 // cells with is_md set or clear, displacements and their maximum, the pair force.
 #pragma once
+#include <type_traits>
+
 #include "rmpcd_internal.hpp"
 
 namespace rmpcd {
@@ -9,18 +11,19 @@ namespace rmpcd {
 // cell_md_pos / cell_md_vel / cell_md_pos_{y,z}wall (md.f90:79-263) and
 // cell_maximum_displacement (particle_system.f90:380-410) touch the particles of the cells
 // with is_md equal to md_flag.  A wave takes CELL_WAVE consecutive cells: it reads their
-// marks, starts and counts together, then goes through those that qualify, four at a time
-// with CELL_LANES lanes each, so that neighbouring lanes move neighbouring particles (a
-// thread per cell walked its ten particles one after the other, each wave's lanes ten
-// particles apart: for the velocities, positions and displacements of the md cells of an
-// L = 48 box with 52 colloids, FP64, 33, 24 and 22 us then, 16, 10 and 12 us now).
-constexpr int CELL_WAVE = 32, CELL_LANES = 16;
+// marks, starts and counts together, then goes through those that qualify with LANES lanes
+// each, so that neighbouring lanes move neighbouring particles (a thread per cell walked its
+// ten particles one after the other, each wave's lanes ten particles apart: for the
+// velocities, positions and displacements of the md cells of an L = 48 box with 52 colloids,
+// FP64, 33, 24 and 22 us then, 16, 10 and 12 us now).  LANES by the density: see by_density.
+constexpr int CELL_WAVE = 32;
 
-template <class Fn>
+template <int LANES, class Fn>
 __device__ inline void for_md_cells(int ncells, const int32_t *__restrict__ start, const int32_t *__restrict__ count,
                                     const uint8_t *__restrict__ is_md, int md_flag, Fn each)
 {
-    const int lane = threadIdx.x & 63, sub = lane & (CELL_LANES - 1), grp = lane / CELL_LANES;
+    constexpr int GROUPS = 64 / LANES;
+    const int lane = threadIdx.x & 63, sub = lane & (LANES - 1), grp = lane / LANES;
     const int64_t wave = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int64_t c = wave * CELL_WAVE + (lane & (CELL_WAVE - 1));
     int s = 0, m = 0;
@@ -32,18 +35,44 @@ __device__ inline void for_md_cells(int ncells, const int32_t *__restrict__ star
     }
     // one bit per cell (the two halves of the wave hold the same cells)
     uint32_t todo = (uint32_t)__ballot(on);
+    if constexpr (LANES < 16) {  // every cell in its turn: one or two rounds
+        if (todo == 0) return;
+        for (int r = 0; r < CELL_WAVE / GROUPS; ++r) {
+            const int from = r * GROUPS + grp;
+            const int cs = __shfl(s, from), cm = __shfl(m, from);
+            const int n = todo >> from & 1 ? cm : 0;
+            for (int j = sub; j < n; j += LANES) each((int64_t)cs + j);
+        }
+        return;
+    }
     while (todo) {
         uint32_t t = todo;
         for (int k = 0; k < grp; ++k) t &= t - 1;
         const int from = t ? __ffs(t) - 1 : 0;
         const int cs = __shfl(s, from), cm = __shfl(m, from);
         const int n = t ? cm : 0;
-        for (int j = sub; j < n; j += CELL_LANES) each((int64_t)cs + j);
-        for (int k = 0; k < 64 / CELL_LANES; ++k) todo &= todo - 1;
+        for (int j = sub; j < n; j += LANES) each((int64_t)cs + j);
+        for (int k = 0; k < GROUPS; ++k) todo &= todo - 1;
     }
 }
 
 inline unsigned cell_blocks(int ncells) { return blocks_for(ncells, 256 / 64 * CELL_WAVE); }
+
+// The lanes that take a cell, by the mean number of particles in one.  Lists of 1000 points,
+// L = 64, FP64, at 1, 3 and 10 particles a cell: 54, 73 and 162 us; 16 lanes throughout 158, 159
+// and 162; a thread per cell 62, 91 and 380.  Velocities of all cells, L = 100, FP64: 46 us at 1
+// (16 lanes 86, a thread per cell 49) and 248 at 10 (a thread per cell 1536).
+template <class Fn>
+inline void by_density(const rmpcd_box_t *box, int64_t n, Fn fn)
+{
+    const double per_cell = (double)n / ((double)box->L[0] * box->L[1] * box->L[2]);
+    if (per_cell >= 6)
+        fn(std::integral_constant<int, 16>{});
+    else if (per_cell >= 1.5)
+        fn(std::integral_constant<int, 4>{});
+    else
+        fn(std::integral_constant<int, 2>{});
+}
 
 // the squared displacement of particle j from pos_old (particle_system.f90:357-378)
 template <class F>

@@ -440,6 +440,34 @@ def test_cell_md(gpu, axis, bc):
         assert same_bits(d.host(name), getattr(want, name)), name
 
 
+@pytest.mark.parametrize("L,rho,clump", [((9, 14, 11), 1, 0), ((16, 16, 16), 1, 40), ((13, 8, 10), 3, 0),
+                                         ((16, 8, 16), 3, 70)])
+def test_cell_passes_of_thin_gases(gpu, L, rho, clump):
+    """few particles a cell take fewer lanes: cell-wise Verlet and displacements, with a cell of
+    far more particles than the mean (clump)"""
+    ps = solvent_state(L, rho, 51)
+    if clump:
+        ps.pos[:clump] = np.array([3.0, 2.0, 5.0]) + 0.4 * np.random.default_rng(52).random((clump, 3))
+    ps.id[:] = np.arange(ps.n)
+    c = O.cells_init(L)
+    srt, i2i, cnt, st = O.sort(c, ps)
+    assert not clump or cnt.max() >= clump
+    is_md = (np.random.default_rng(53).random(c.N) < 0.6).astype(np.uint8)
+    old = srt.pos.copy()
+    d, cs = to_device(srt), cells_to_device(c, cnt, st)
+    cs.is_md.copy_(torch.as_tensor(is_md))
+    want, old_d, r = srt.copy(), torch.as_tensor(np.ascontiguousarray(old.T)).cuda(), C.c_double()
+    for flag in (True, False):
+        O.cell_md_pos(c, cnt, st, is_md, want.pos, want.vel, want.force, 0.3, flag)
+        capi.call("rmpcd_cell_md_pos", cs.boxp(), cs.cellsp(), d.struct(), 0.3, int(flag))
+        O.cell_md_vel(c, cnt, st, is_md, want.vel, want.force, want.force_old, want.flags, 0.3, flag)
+        capi.call("rmpcd_cell_md_vel", cs.boxp(), cs.cellsp(), d.struct(), 0.3, int(flag))
+        capi.call("rmpcd_cell_maximum_displacement", cs.boxp(), cs.cellsp(), d.struct(), ptr(old_d), 0.0, C.byref(r))
+        assert r.value == O.cell_maximum_displacement(c, cnt, st, is_md, want.pos, old, want.species, 0.0)
+    for name in ("pos", "vel", "flags"):
+        assert same_bits(d.host(name), getattr(want, name)), name
+
+
 def colloid_pair(L, seed):
     rng = np.random.default_rng(seed)
     cp = O.PState(2)
@@ -490,7 +518,8 @@ def dimer_setup(L, rho, seed, sigma=(2.0, 2.0), frac2=0.2):
 
 
 @pytest.mark.parametrize("L,rho,with_lj", [((16, 16, 16), 10, True), ((24, 20, 28), 10, False),
-                                           ((32, 32, 32), 10, True)])
+                                           ((32, 32, 32), 10, True), ((16, 16, 16), 1, True),
+                                           ((20, 16, 18), 3, True)])
 def test_update_list(gpu, L, rho, with_lj):
     c, srt, cnt, st, cp, eps, sig, cut = dimer_setup(L, rho, 27)
     radius = cut.max() + 2.0
