@@ -21,7 +21,6 @@
 #include <math.h>
 #include <string.h>
 
-#include <queue>
 #include <type_traits>
 #include <vector>
 
@@ -221,21 +220,37 @@ static int get_block(Schedule &s, int K, const BlockSched **out)
             return RMPCD_OK;
         }
     }
-    // the longest chain first, the earlier update among equals
-    auto later = [&](int32_t p, int32_t q) { return height[p] != height[q] ? height[p] < height[q] : p > q; };
-    std::priority_queue<int32_t, std::vector<int32_t>, decltype(later)> ready(later);
+    // the longest chain first, the one that became ready first among equals: a list per height
+    int top = 0;
     for (int t = 0; t < nt; ++t)
-        if (wait[t] == 0) ready.push(t);
+        if (height[t] > top) top = height[t];
+    std::vector<int32_t> front((size_t)top + 1, -1), back((size_t)top + 1), behind((size_t)nt);
+    auto push = [&](int32_t t) {
+        const int h = height[t];
+        behind[t] = -1;
+        if (front[h] < 0)
+            front[h] = t;
+        else
+            behind[back[h]] = t;
+        back[h] = t;
+        if (h > top) top = h;
+    };
+    auto any_ready = [&] {
+        while (top > 0 && front[top] < 0) --top;
+        return top > 0;
+    };
+    for (int t = 0; t < nt; ++t)
+        if (wait[t] == 0) push(t);
     std::vector<uint4> ent;
     const uint32_t spare = (uint32_t)(K * s.n * 24);  // in the snapshots: a place per lane
     const uint4 idle{(uint32_t)(s.n * 24) | ((uint32_t)((s.n + 1) * 24) << 16), (uint32_t)nl * LC * 8, 0, 0};
     std::vector<int32_t> step;
     ent.reserve(2 * (size_t)nt);
-    while (!ready.empty()) {
+    while (any_ready()) {
         step.clear();
-        while (!ready.empty() && step.size() < 64) {
-            step.push_back(ready.top());
-            ready.pop();
+        while (step.size() < 64 && any_ready()) {
+            step.push_back(front[top]);
+            front[top] = behind[front[top]];
         }
         for (const int32_t t : step) {
             const int l = t % nl, q = t / nl, a = links[2 * l], c = links[2 * l + 1];
@@ -248,7 +263,7 @@ static int get_block(Schedule &s, int K, const BlockSched **out)
             ent.push_back(e);
             for (int k = 0; k < 2; ++k) {
                 const int32_t w = next[2 * (size_t)t + k];
-                if (w >= 0 && --wait[w] == 0) ready.push(w);
+                if (w >= 0 && --wait[w] == 0) push(w);
             }
         }
         auto pad = [&] {
@@ -257,7 +272,7 @@ static int get_block(Schedule &s, int K, const BlockSched **out)
             ent.push_back(e);
         };
         while (ent.size() % 64) pad();
-        if (ready.empty())  // idle steps up to a whole turn, and one more turn to read ahead
+        if (!any_ready())  // idle steps up to a whole turn, and one more turn to read ahead
             while (ent.size() % (64 * 2 * AHEAD)) pad();
         if ((int64_t)ent.size() > WAVE_ENTRIES) {
             b.too_long = true;
