@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(256)
 // as after that.  The first CHAIN_REG entries are read once and kept; a longer chain's rest is
 // walked for each addition, and holds no more than the launch's entries, so the walk ends.
 // (200 overlapping colloids in an L = 16 box, FP64, a call: 56 us walking the chain for each
-// addition, 49 like this.)
+// addition, 52.5 like this.)
 constexpr int CHAIN_REG = 8;
 
 template <class F>

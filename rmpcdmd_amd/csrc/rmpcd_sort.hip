@@ -16,6 +16,8 @@
 // The order within a tile's list is not deterministic, the rank does not depend on it: the
 // result equals the reference's single-thread order, where each cell keeps increasing
 // original index.
+#include <type_traits>
+
 #include "rmpcd_internal.hpp"
 #include "rmpcd_srdtile.hpp"
 
@@ -153,7 +155,14 @@ constexpr int TILE_MAX = SORT_T * TILE_ITEMS<F>;
 // runs of 16, 485 with 4, 64 or 256; 21 million particles in order: 1.38 ms, 1.35 ms with
 // runs of 4 to 64).
 constexpr int TILE_RUN = 16;
-constexpr int TILE_CELLS = 128;                               // cells of a tile at most
+// Cells of a tile at most: TILE_CELLS, or TILE_THIN where the particles of twice as many still
+// fit.  (1 particle a cell: a tile of 128 cells, half of them outside an L=100 box, gives a
+// workgroup 60 particles, a sort of a million FP32 152 us; 84 like this; 102 without tiles.  The
+// larger counts cost the move two of six workgroups per CU where a tile is full.)
+constexpr int TILE_CELLS = 128, TILE_THIN = 1024;
+// Particles per tile on average up to which a thread takes two at most (a small box's tiles:
+// 5120 FP32 particles 39.1 us a sort with room for six a thread, 35.8 like this).
+constexpr int TILE_FEW = 200;
 constexpr int SCAN1_TILES = 1 << 14;                          // tile counts that one workgroup scans
 // The counts of up to SCAN1_TILES tiles are spread over 128 KiB, a cache line each up to 2048:
 // particles in no order (the first sort of a run) meet a few thousand counts from
@@ -486,7 +495,7 @@ __device__ inline void spill_move(const Box &b, const PView<F> &src, const PView
 // that the stores are contiguous too.  id_to_idx costs 0.42 ms of the 1.09 ms with it: its
 // 4-byte stores go anywhere once the particles have mixed.  FORCES false leaves the force
 // planes out, for a program whose forces are zero in both buffers.
-template <class F, bool FORCES>
+template <class F, bool FORCES, int CELLS, int N>
 __global__ void __launch_bounds__(SORT_T)
     k_tile_gather(Box b, PView<F> src, PView<F> dst, int wrap, int shift, int nt, const int32_t *__restrict__ key,
                   const int32_t *__restrict__ start, const int32_t *__restrict__ list, int32_t *__restrict__ spill,
@@ -495,10 +504,10 @@ __global__ void __launch_bounds__(SORT_T)
 {
     using R = typename F::real;
     using S = typename F::small;
-    constexpr int N = TILE_ITEMS<F>, M = TILE_MAX<F>, PLANES = FORCES ? 4 : 2;
+    constexpr int M = SORT_T * N, PLANES = FORCES ? 4 : 2;
     __shared__ R buf[3][M];
     __shared__ int lv[M];
-    __shared__ int lcnt[TILE_CELLS], lstart[TILE_CELLS];
+    __shared__ int lcnt[CELLS], lstart[CELLS];
     // consecutive workgroups go to the XCDs in turn: each XCD takes runs of TILE_RUN tiles,
     // so that the tiles in flight there read neighbouring stretches.  The runs are short
     // enough that the empty cells of a padded box fall to all XCDs alike.
@@ -719,11 +728,11 @@ int count_impl(const rmpcd_box_t *box, const rmpcd_particles_t *pp, rmpcd_cells_
 // spare, 2.4 standard deviations of 460, and a tile above that is moved from memory), and small
 // enough that a box has two workgroups for every compute unit (a floor of 1024 or 2048 tiles made
 // no difference)
-static int tile_shift(const Box &b, int64_t n, int tile_max)
+static int tile_shift(const Box &b, int64_t n, int tile_max, int tile_cells)
 {
     const double per_cell = (double)n / ((double)b.L[0] * b.L[1] * b.L[2]);
     int shift = 0;
-    while ((2 << shift) <= TILE_CELLS && (2 << shift) <= b.ncells && per_cell * (2 << shift) <= tile_max * 0.9 &&
+    while ((2 << shift) <= tile_cells && (2 << shift) <= b.ncells && per_cell * (2 << shift) <= tile_max * 0.9 &&
            (b.ncells >> (shift + 1)) >= 512)
         ++shift;
     return shift;
@@ -742,7 +751,7 @@ template <class F>
 static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
 {
     t.b = make_box(box);
-    t.shift = tile_shift(t.b, n, TILE_MAX<F>);
+    t.shift = tile_shift(t.b, n, TILE_MAX<F>, TILE_THIN);
     t.nt = t.b.ncells >> t.shift;
     t.stride = count_stride(t.nt);
     t.key = (int32_t *)workspace(WS_KEY, sizeof(int32_t) * n);
@@ -782,9 +791,19 @@ static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmp
     k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, t.key, t.shift, t.slot, t.start, t.list, t.work);
     RMPCD_LAUNCHED();
     const unsigned runs = (unsigned)((t.nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
-    k_tile_gather<F, FORCES><<<8 * TILE_RUN * runs, SORT_T, 0, s>>>(t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt,
-                                                                    t.key, t.start, t.list, t.slot, cells->cell_count,
-                                                                    cells->cell_start, own, t.work, id_to_idx);
+    auto move = [&](auto cells_max, auto items) {
+        k_tile_gather<F, FORCES, decltype(cells_max)::value, decltype(items)::value><<<8 * TILE_RUN * runs, SORT_T, 0, s>>>(
+            t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt, t.key, t.start, t.list, t.slot, cells->cell_count,
+            cells->cell_start, own, t.work, id_to_idx);
+    };
+    using Items = std::integral_constant<int, TILE_ITEMS<F>>;
+    using Few = std::integral_constant<int, 2>;
+    if ((1 << t.shift) > TILE_CELLS)
+        move(std::integral_constant<int, TILE_THIN>{}, Items{});
+    else if (n <= (int64_t)t.nt * TILE_FEW)
+        move(std::integral_constant<int, TILE_CELLS>{}, Few{});
+    else
+        move(std::integral_constant<int, TILE_CELLS>{}, Items{});
     RMPCD_LAUNCHED();
     if constexpr (FORCES) {  // the others are the programs'
         if (n <= own || n <= TILE_MAX<F>) return RMPCD_OK;  // no tile holds more
@@ -818,8 +837,7 @@ int fluid_cycle_impl(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpc
     int rc = tile_sort_begin<F>(next, src->n, t);
     if (rc) return rc;
     // the collision's cells per workgroup, by the same rule as a tile's
-    int cshift = tile_shift(t.b, src->n, FLUID_MAX<F>);
-    while ((1 << cshift) > SRD_CELLS) --cshift;
+    int cshift = tile_shift(t.b, src->n, FLUID_MAX<F>, SRD_CELLS);
     k_fluid_key<F><<<(unsigned)(t.b.ncells >> cshift), SORT_T, 0, stream()>>>(
         t.b, t.lut, view<F>(src), cells->cell_start, cells->cell_count, cshift, seed, step, n_md, dt, t.shift, t.stride,
         t.count, t.key, t.slot);

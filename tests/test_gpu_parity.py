@@ -132,7 +132,8 @@ def test_sort_outside_box_and_empty_cells(gpu):
     ((16, 16, 16), 3000, "one cell"),       # every particle in one cell
     ((32, 32, 32), 60000, "octant"),        # tiles of many cells fuller than their LDS
     ((37, 5, 21), 41, "even"),              # fewer particles than tiles
-    ((256, 256, 128), 200000, "even"),      # more tiles than one workgroup scans
+    ((256, 256, 128), 200000, "even"),      # tiles of many nearly empty cells
+    ((33, 65, 65), 1_390_000, "even"),      # in FP64 more tiles than one workgroup scans
 ])
 def test_sort_tiles(gpu, L, n, spread, form):
     """the tile sort where tiles overflow, are empty or are many; positions and grid shift are
@@ -203,7 +204,7 @@ def test_sort_clusters(gpu, L, n, parts, form):
     assert same_bits(i2i_d.cpu().numpy(), i2i)
 
 
-@pytest.mark.parametrize("L,n", [((24, 20, 12), 30000), ((256, 256, 128), 100000)])
+@pytest.mark.parametrize("L,n", [((24, 20, 12), 30000), ((33, 65, 65), 1_390_000)])
 def test_sort_after_a_failed_sort(gpu, L, n):
     """a sort that stops at an error with its key pass queued leaves tile counts behind; the
     sorts after it must not add to them"""

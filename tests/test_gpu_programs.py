@@ -64,6 +64,7 @@ def test_fluid_matches_oracle(gpu, n_md):
     ((4, 4, 4), 900, 1),    # one cell holds more particles than a workgroup's LDS
     ((4, 4, 4), 1700, 1),   # and than the LDS of the sort's move in either form
     ((9, 8, 8), 1, 1),      # cells with one particle or none
+    ((64, 64, 64), 1, 1),   # and tiles of many of them
 ])
 def test_fluid_equals_entry_points(gpu, form, L, rho, n_md):
     """the fused cycle against simple_mpcd_step, mpcd_stream_periodic and sort, bit for bit"""
