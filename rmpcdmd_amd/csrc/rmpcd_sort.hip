@@ -160,8 +160,9 @@ constexpr int TILE_RUN = 16;
 // workgroup 60 particles, a sort of a million FP32 152 us; 84 like this; 102 without tiles.  The
 // larger counts cost the move two of six workgroups per CU where a tile is full.)
 constexpr int TILE_CELLS = 128, TILE_THIN = 1024;
-// Particles per tile on average up to which a thread takes two at most (a small box's tiles:
-// 5120 FP32 particles 39.1 us a sort with room for six a thread, 35.8 like this).
+// Particles on average in a tile inside the box up to which a thread takes two at most (a
+// small box's tiles: 5120 FP32 particles 39.1 us a sort with room for six a thread, 35.8 like
+// this).
 constexpr int TILE_FEW = 200;
 constexpr int SCAN1_TILES = 1 << 14;                          // tile counts that one workgroup scans
 // The counts of up to SCAN1_TILES tiles are spread over 128 KiB, a cache line each up to 2048:
@@ -407,13 +408,16 @@ struct SpillWork {
     int2 *item;
 };
 constexpr int SPILL_PIECE = 512, SPILL_AHEAD = 8;
-// A tile's own workgroup moves up to `own` particles alone: SPILL_OWN (FP64: the LDS holds
-// fewer; L=32 with all particles in one half, 640 a tile: first sort 153 us, by k_tile_spill
-// 170), or any number in the device-resident programs, whose particles spread evenly from the
-// start, so that the launch of k_tile_spill would be for nothing (1.5 us of the 63 us cycle of an
-// L=32 FP64 fluid).
-constexpr int SPILL_OWN = 1024, SPILL_NEVER = INT32_MAX;
-constexpr unsigned SPILL_BLOCKS = 1024;  // the 512th below at 512 and 2048: 7.9, 4.6 ms; 2048 idle 1 us longer
+// A tile's own workgroup moves any number of particles alone, or, where k_tile_spill follows,
+// up to SPILL_OWN.  It follows in sorts of SPREAD_FROM particles or more that may be clustered:
+// its launch is 2 us, mostly for nothing, of a step's 50 for 80,000 FP64 particles, 200 for 1.25
+// million.  Below that, clusters cost more: 327,680 FP64 particles in a half, an eighth, a 64th
+// and a 512th of the box (in order) take 0.06, 0.12, 1.7 and 85 ms a sort; with it 0.07, 0.09, 0.24
+// and 1.4; without tiles 0.08, 0.14, 0.56 and 3.2.  The device-resident programs, whose particles
+// spread evenly from the start, go without it.
+constexpr int SPILL_OWN = 1024;
+constexpr int64_t SPREAD_FROM = 1 << 21;
+constexpr unsigned SPILL_BLOCKS = 1024;  // 2048 idle 1 us longer
 
 // a thread's next particles of such a tile and their cells, -1 beyond its m particles
 __device__ inline void spill_load(int32_t w[SPILL_AHEAD], int k[SPILL_AHEAD], const int32_t *__restrict__ list,
@@ -487,6 +491,53 @@ __device__ inline void spill_move(const Box &b, const PView<F> &src, const PView
     if (id_to_idx && (uint32_t)id < (uint32_t)n) id_to_idx[id] = (int32_t)o;
 }
 
+// Particles [q0, q1) of a list that is grouped by cell, at most P a thread: a thread ranks its
+// own in their cells by original index, the cells' lists staged in LDS, and moves them straight
+// between the planes.  All threads call.
+constexpr int SPILL_STAGE = 1536;
+template <class F, bool FORCES, int P>
+__device__ inline void spill_piece(const Box &b, const PView<F> &src, const PView<F> &dst, int wrap,
+                                   const int32_t *key, const int32_t *list, const int32_t *cell_count,
+                                   const int32_t *cell_start, int64_t q0, int64_t q1, int32_t *stage, int *range,
+                                   int32_t *__restrict__ id_to_idx)
+{
+    const int tid = threadIdx.x;
+    int32_t w[P];
+    int a[P], z[P], rank[P];  // the particles' cells in the list
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+        const int64_t q = q0 + tid + u * SORT_T;
+        w[u] = q < q1 ? list[q] : -1;
+        const int c = w[u] >= 0 ? key[w[u]] : 0;
+        a[u] = w[u] >= 0 ? cell_start[c] : 0;
+        z[u] = w[u] >= 0 ? a[u] + cell_count[c] : 0;
+        rank[u] = 0;
+        // the piece's first and last particle bound the cells that are needed
+        if (q == q0) range[0] = a[u];
+        if (q == q1 - 1) range[1] = z[u];
+    }
+    __syncthreads();
+    const int r0 = range[0], r1 = range[1];
+    for (int base = r0; base < r1; base += SPILL_STAGE) {
+        const int m = r1 - base < SPILL_STAGE ? r1 - base : SPILL_STAGE;
+        __syncthreads();
+        for (int k = tid; k < m; k += SORT_T) stage[k] = list[base + k];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < P; ++u) {
+            const int lo = a[u] > base ? a[u] - base : 0, hi = z[u] - base < m ? z[u] - base : m;
+            int r = 0;
+#pragma unroll 4
+            for (int k = lo; k < hi; ++k) r += stage[k] < w[u] ? 1 : 0;
+            rank[u] += r;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < P; ++u)
+        if (w[u] >= 0) spill_move<F, FORCES>(b, src, dst, wrap, w[u], (int64_t)a[u] + rank[u], id_to_idx);
+    __syncthreads();
+}
+
 // The cell sort's move.  Bound by memory: FP32 it reads 74 B and writes 66 B per particle,
 // and fetches 1.33 times what it uses (tiles read the edges of their neighbours' stretches),
 // 164 B in 0.67 ms for 21 million particles, 5.1 TB/s.  Moved one particle per thread
@@ -494,12 +545,14 @@ __device__ inline void spill_move(const Box &b, const PView<F> &src, const PView
 // ms; in list order a tile's loads run along the source, and LDS puts them in slot order so
 // that the stores are contiguous too.  id_to_idx costs 0.42 ms of the 1.09 ms with it: its
 // 4-byte stores go anywhere once the particles have mixed.  FORCES false leaves the force
-// planes out, for a program whose forces are zero in both buffers.
-template <class F, bool FORCES, int CELLS, int N>
-__global__ void __launch_bounds__(SORT_T)
+// planes out, for a program whose forces are zero in both buffers.  With two particles a thread
+// it is held to eight waves per SIMD, which its scalar registers would make seven (a step of
+// 390,000 FP64 particles 95 us, 90 with eight).
+template <class F, bool FORCES, int CELLS, int N, bool SPREAD>
+__global__ void __launch_bounds__(SORT_T, CELLS > TILE_CELLS ? 1 : N == 2 ? 8 : 6)
     k_tile_gather(Box b, PView<F> src, PView<F> dst, int wrap, int shift, int nt, const int32_t *__restrict__ key,
                   const int32_t *__restrict__ start, const int32_t *__restrict__ list, int32_t *__restrict__ spill,
-                  int32_t *__restrict__ cell_count, int32_t *__restrict__ cell_start, int own, SpillWork work,
+                  int32_t *__restrict__ cell_count, int32_t *__restrict__ cell_start, SpillWork work,
                   int32_t *__restrict__ id_to_idx)
 {
     using R = typename F::real;
@@ -628,17 +681,13 @@ __global__ void __launch_bounds__(SORT_T)
         for (int u = 0; u < SPILL_AHEAD; ++u)
             if (w[u] >= 0) spill[s + lstart[k[u]] + atomicAdd(&lcnt[k[u]], 1)] = w[u];
     }
-    if (m <= own) {
+    if (!SPREAD || m <= SPILL_OWN) {
         __threadfence_block();
         __syncthreads();
-        for (int q = tid; q < m; q += SORT_T) {
-            const int32_t w = spill[s + q];
-            const int k = key[w] & cmask;
-            const int a = lstart[k], e = a + lcnt[k];
-            int rank = 0;
-            for (int y = a; y < e; ++y) rank += spill[s + y] < w ? 1 : 0;
-            spill_move<F, FORCES>(b, src, dst, wrap, w, s + a + rank, id_to_idx);
-        }
+        static_assert(sizeof(buf) >= SPILL_STAGE * sizeof(int32_t), "the lists' stage");
+        for (int64_t q = s; q < s + m; q += SORT_T)
+            spill_piece<F, FORCES, 1>(b, src, dst, wrap, key, spill, cell_count, cell_start, q,
+                                      q + SORT_T < s + m ? q + SORT_T : s + m, (int32_t *)buf, lv, id_to_idx);
         return;
     }
     const int pieces = (m - 1) / SPILL_PIECE + 1;
@@ -647,13 +696,11 @@ __global__ void __launch_bounds__(SORT_T)
     for (int k = tid; k < pieces; k += SORT_T) work.item[lv[0] + k] = make_int2(t, k);
 }
 
-// The tiles too large for their own workgroup, a piece of one per workgroup at a time: a
-// thread ranks two particles in their cells, the cells' lists staged in LDS, and moves them
-// straight between the planes.  Clustered particles fill few tiles, which would leave the rest
-// of the device idle: a sort with all particles in a half, an eighth, a 64th and a 512th of an
-// L=64 box (2.6 million FP32, in order) takes 0.30, 0.32, 0.87 and 5.3 ms; each tile by its own
-// workgroup 0.36, 1.02, 20.6 and 973; without tiles 0.42, 0.68, 1.7 and 9.7.  In no order 1.13,
-// 1.11, 1.51 and 5.2 ms; 1.14, 1.42, 22.5 and 987; 1.11, 1.10, 1.29 and 4.2.
+// The tiles too large for their own workgroup, a piece of one per workgroup at a time.
+// Clustered particles fill few tiles, which would leave the rest of the device idle: a sort
+// with all particles in a half, an eighth, a 64th and a 512th of an L=64 box (2.6 million FP32, in
+// order) takes 0.29, 0.30, 0.66 and 3.6 ms; without tiles 0.42, 0.68, 1.7 and 9.7.  In no order 1.13,
+// 1.12, 1.43 and 3.6 ms; without tiles 1.11, 1.10, 1.29 and 4.2.
 template <class F>
 __global__ void __launch_bounds__(SORT_T)
     k_tile_spill(Box b, PView<F> src, PView<F> dst, int wrap, const int32_t *__restrict__ key,
@@ -661,49 +708,14 @@ __global__ void __launch_bounds__(SORT_T)
                  const int32_t *__restrict__ cell_count, const int32_t *__restrict__ cell_start, SpillWork work,
                  int32_t *__restrict__ id_to_idx)
 {
-    constexpr int P = SPILL_PIECE / SORT_T, STAGE = 2048;
-    __shared__ int32_t stage[STAGE];
-    __shared__ int64_t range[2];
-    const int tid = threadIdx.x;
+    __shared__ int32_t stage[SPILL_STAGE];
+    __shared__ int range[2];
     const int items = *work.count;
     for (int it = blockIdx.x; it < items; it += gridDim.x) {
         const int2 e = work.item[it];
         const int64_t q0 = start[e.x] + (int64_t)e.y * SPILL_PIECE, end = start[e.x + 1];
-        const int64_t q1 = q0 + SPILL_PIECE < end ? q0 + SPILL_PIECE : end;
-        int32_t w[P];
-        int64_t a[P], z[P];  // the particles' cells in the list
-        int rank[P];
-#pragma unroll
-        for (int u = 0; u < P; ++u) {
-            const int64_t q = q0 + tid + u * SORT_T;
-            w[u] = q < q1 ? spill[q] : -1;
-            const int c = w[u] >= 0 ? key[w[u]] : 0;
-            a[u] = w[u] >= 0 ? cell_start[c] : 0;
-            z[u] = w[u] >= 0 ? a[u] + cell_count[c] : 0;
-            rank[u] = 0;
-            // the list is grouped by cell: the piece's first and last particle bound the range
-            if (q == q0) range[0] = a[u];
-            if (q == q1 - 1) range[1] = z[u];
-        }
-        __syncthreads();
-        const int64_t r0 = range[0], r1 = range[1];
-        for (int64_t base = r0; base < r1; base += STAGE) {
-            __syncthreads();
-            for (int k = tid; k < STAGE && base + k < r1; k += SORT_T) stage[k] = spill[base + k];
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < P; ++u) {
-                const int lo = (int)(a[u] > base ? a[u] - base : 0);
-                const int hi = (int)(z[u] < base + STAGE ? z[u] - base : STAGE);
-                int r = 0;
-                for (int k = lo; k < hi; ++k) r += stage[k] < w[u] ? 1 : 0;
-                rank[u] += r;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < P; ++u)
-            if (w[u] >= 0) spill_move<F, true>(b, src, dst, wrap, w[u], a[u] + rank[u], id_to_idx);
-        __syncthreads();
+        spill_piece<F, true, SPILL_PIECE / SORT_T>(b, src, dst, wrap, key, spill, cell_count, cell_start, q0,
+                             q0 + SPILL_PIECE < end ? q0 + SPILL_PIECE : end, stage, range, id_to_idx);
     }
 }
 
@@ -743,6 +755,7 @@ struct TileSort {
     Box b;
     const int32_t *lut;
     int shift, nt, stride;
+    double per_tile;  // particles, in tiles inside the box
     int32_t *key, *slot, *list, *start, *count;
     SpillWork work;
 };
@@ -753,6 +766,7 @@ static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
     t.b = make_box(box);
     t.shift = tile_shift(t.b, n, TILE_MAX<F>, TILE_THIN);
     t.nt = t.b.ncells >> t.shift;
+    t.per_tile = (double)n / ((double)t.b.L[0] * t.b.L[1] * t.b.L[2]) * (1 << t.shift);
     t.stride = count_stride(t.nt);
     t.key = (int32_t *)workspace(WS_KEY, sizeof(int32_t) * n);
     t.slot = (int32_t *)workspace(WS_SLOT, sizeof(int32_t) * n);
@@ -774,7 +788,7 @@ static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
 // the sort after its keys
 template <class F, bool FORCES>
 static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
-                            int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, int own)
+                            int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, bool spread)
 {
     const int64_t n = src->n;
     hipStream_t s = stream();
@@ -791,22 +805,35 @@ static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmp
     k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, t.key, t.shift, t.slot, t.start, t.list, t.work);
     RMPCD_LAUNCHED();
     const unsigned runs = (unsigned)((t.nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
-    auto move = [&](auto cells_max, auto items) {
-        k_tile_gather<F, FORCES, decltype(cells_max)::value, decltype(items)::value><<<8 * TILE_RUN * runs, SORT_T, 0, s>>>(
-            t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt, t.key, t.start, t.list, t.slot, cells->cell_count,
-            cells->cell_start, own, t.work, id_to_idx);
+    auto move = [&](auto cells_max, auto items, auto spread_c) {
+        k_tile_gather<F, FORCES, decltype(cells_max)::value, decltype(items)::value, decltype(spread_c)::value>
+            <<<8 * TILE_RUN * runs, SORT_T, 0, s>>>(t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt, t.key, t.start,
+                                                    t.list, t.slot, cells->cell_count, cells->cell_start, t.work,
+                                                    id_to_idx);
     };
-    using Items = std::integral_constant<int, TILE_ITEMS<F>>;
-    using Few = std::integral_constant<int, 2>;
-    if ((1 << t.shift) > TILE_CELLS)
-        move(std::integral_constant<int, TILE_THIN>{}, Items{});
-    else if (n <= (int64_t)t.nt * TILE_FEW)
-        move(std::integral_constant<int, TILE_CELLS>{}, Few{});
-    else
-        move(std::integral_constant<int, TILE_CELLS>{}, Items{});
+    const std::integral_constant<int, TILE_CELLS> some{};
+    const std::integral_constant<int, TILE_THIN> thin{};
+    const std::integral_constant<int, TILE_ITEMS<F>> items{};
+    const std::integral_constant<int, 2> few{};
+    const bool is_thin = (1 << t.shift) > TILE_CELLS;
+    if constexpr (FORCES)  // the others are the programs'
+        if (spread) {
+            if (is_thin)
+                move(thin, items, std::true_type{});
+            else
+                move(some, items, std::true_type{});
+        }
+    if (!spread) {
+        if (is_thin)
+            move(thin, items, std::false_type{});
+        else if (t.per_tile <= TILE_FEW)
+            move(some, few, std::false_type{});
+        else
+            move(some, items, std::false_type{});
+    }
     RMPCD_LAUNCHED();
-    if constexpr (FORCES) {  // the others are the programs'
-        if (n <= own || n <= TILE_MAX<F>) return RMPCD_OK;  // no tile holds more
+    if constexpr (FORCES) {
+        if (!spread) return RMPCD_OK;
         const unsigned pieces = blocks_for(n, SPILL_PIECE);
         k_tile_spill<F><<<pieces < SPILL_BLOCKS ? pieces : SPILL_BLOCKS, SORT_T, 0, s>>>(
             t.b, view<F>(src), view<F>(dst), wrap, t.key, t.start, t.slot, cells->cell_count, cells->cell_start, t.work,
@@ -818,7 +845,7 @@ static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmp
 
 template <class F>
 int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
-              int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, int own)
+              int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, bool spread)
 {
     TileSort t;
     int rc = tile_sort_begin<F>(box, src->n, t);
@@ -826,7 +853,7 @@ int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_partic
     k_tile_key<F><<<blocks_for(src->n, KEY_CHUNK), SORT_T, 0, stream()>>>(t.b, t.lut, view<F>(src), wrap, t.shift,
                                                                           t.stride, t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    return tile_sort_finish<F, true>(t, src, dst, id_to_idx, cells, wrap, own);
+    return tile_sort_finish<F, true>(t, src, dst, id_to_idx, cells, wrap, spread);
 }
 
 template <class F>
@@ -842,7 +869,7 @@ int fluid_cycle_impl(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpc
         t.b, t.lut, view<F>(src), cells->cell_start, cells->cell_count, cshift, seed, step, n_md, dt, t.shift, t.stride,
         t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    return tile_sort_finish<F, false>(t, src, dst, nullptr, cells, 0, SPILL_NEVER);
+    return tile_sort_finish<F, false>(t, src, dst, nullptr, cells, 0, false);
 }
 
 int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
@@ -854,7 +881,7 @@ int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src,
 int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
                    rmpcd_cells_t *cells, int wrap, bool even)
 {
-    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, wrap, even ? SPILL_NEVER : SPILL_OWN);
+    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, wrap, !even && src->n >= SPREAD_FROM);
 }
 
 template <class F>

@@ -168,6 +168,7 @@ def test_sort_tiles(gpu, L, n, spread, form):
     ((32, 32, 32), 30000, [(0.9, (3, 3, 3)), (0.1, (32, 32, 32))]),        # a cluster in a thin gas
     ((16, 16, 16), 20000, [(0.5, (1, 1, 1)), (0.25, (2, 1, 1)), (0.25, (16, 16, 16))]),  # cells beyond a piece
     ((20, 10, 6), 2500, [(1.0, (5, 5, 5))]),
+    ((64, 64, 64), (1 << 21) + 37, [(0.9, (32, 32, 32)), (0.05, (8, 4, 4)), (0.05, (64, 64, 64))]),  # by all workgroups
 ])
 def test_sort_clusters(gpu, L, n, parts, form):
     """the sort of clustered particles, whose tiles the LDS does not hold, with the periodic
