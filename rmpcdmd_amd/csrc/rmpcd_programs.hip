@@ -135,13 +135,10 @@ __global__ void __launch_bounds__(256)
     const int old = (int)p.flags[i];
     const bool listed = (old & LISTED_MASK) != 0;
     int f = listed ? old & ~LISTED_MASK : roll_md(old);
-    R fn[3] = {0, 0, 0};
-    for (int k = 0; k < 3; ++k) {
-        if (listed)
-            fn[k] = p.force[k * p.n + i];
-        else
-            p.force[k * p.n + i] = 0;
-    }
+    R fn[3];  // read beside the flags, not after them
+    for (int k = 0; k < 3; ++k) fn[k] = p.force[k * p.n + i];
+    if (!listed)
+        for (int k = 0; k < 3; ++k) p.force[k * p.n + i] = fn[k] = 0;
     if (!(f & WALL_MASK)) {
         const R rdt = (R)dt;
 #pragma unroll
