@@ -234,6 +234,52 @@ def test_sort_after_a_failed_sort(gpu, L, n):
         assert same_bits(dst.host("pos"), srt.pos) and same_bits(dst.host("id"), srt.id)
 
 
+def test_sort_captured_after_a_failed_sort(gpu):
+    """a captured sort clears the counts that a stopped one left when the graph runs, not before:
+    eager sorts before and between the replays are right too"""
+    L, n = (24, 20, 12), 30000
+    rng = np.random.default_rng(9)
+    ps = O.PState(n)
+    ps.pos[:] = rng.uniform(0, 1, size=(n, 3)) * L
+    ps.id[:] = np.arange(n)
+    ps.species[:] = 1
+    c = O.cells_init(L)
+    srt, i2i, cnt, st = O.sort(c, ps)
+    src, dst, cs = to_device(ps), ParticleSet(n), cells_to_device(c)
+    i2i_d = torch.zeros(n, dtype=torch.int32, device="cuda")
+
+    def sort():
+        capi.call("rmpcd_sort", cs.boxp(), src.struct(), dst.struct(), ptr(i2i_d), cs.cellsp(), 0)
+
+    def check():
+        torch.cuda.synchronize()
+        assert same_bits(dst.host("pos"), srt.pos) and same_bits(cs.cell_count.cpu().numpy(), cnt)
+        dst.pos.zero_()
+        torch.cuda.synchronize()
+
+    stream = torch.cuda.Stream()
+    capi.call("rmpcd_set_stream", C.c_void_p(stream.cuda_stream))
+    try:
+        sort()
+        check()
+        slot, at = workspace_slot("WS_TCOUNT", 4)
+        assert capi.lib()._ZN5rmpcd11zeroed_openENS_4SlotE(C.c_int(slot)) == 0  # opened and left so
+        ones = np.ones(64, np.int32)
+        capi.call("rmpcd_memcpy", C.c_void_p(at), ones.ctypes.data_as(C.c_void_p), ones.nbytes, 0)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            sort()
+        sort()
+        check()
+        for _ in range(3):
+            graph.replay()
+            check()
+            sort()
+            check()
+    finally:
+        capi.call("rmpcd_set_stream", None)
+
+
 def test_maximum_displacement(gpu):
     ps = solvent_state((10, 10, 10), 10, 12)
     old = ps.pos.copy()
