@@ -538,14 +538,16 @@ __device__ inline void spill_piece(const Box &b, const PView<F> &src, const PVie
     __syncthreads();
 }
 
-// The cell sort's move.  Bound by memory: FP32 it reads 74 B and writes 66 B per particle,
-// and fetches 1.33 times what it uses (tiles read the edges of their neighbours' stretches),
-// 164 B in 0.67 ms for 21 million particles, 5.1 TB/s.  Moved one particle per thread
+// The cell sort's move.  Bound by memory: FP32 it reads 74 B and writes 66 B per particle.
+// For 21 million particles on a newly shifted grid it fetches 110 B (tiles read the edges of
+// their neighbours' stretches) and writes 67 in 0.70 ms, 5.3 TB/s; on the grid of the last sort
+// 78 and 67 B in 0.645 ms.  Moved one particle per thread
 // straight from the planes, each load touched a cache line per lane and the pass took 2.08
 // ms; in list order a tile's loads run along the source, and LDS puts them in slot order so
-// that the stores are contiguous too.  id_to_idx costs 0.42 ms of the 1.09 ms with it: its
-// 4-byte stores go anywhere once the particles have mixed.  FORCES false leaves the force
-// planes out, for a program whose forces are zero in both buffers.  With two particles a thread
+// that the stores are contiguous too.  id_to_idx costs 0.43 ms of the 1.13 ms with it: its
+// 4-byte stores go anywhere once the particles have mixed, each fetching and writing a piece of
+// a line (170 and 100 B a particle in all).  FORCES false leaves the force planes out, for a
+// program whose forces are zero in both buffers (72 and 43 B, 0.43 ms).  With two particles a thread
 // it is held to eight waves per SIMD, which its scalar registers would make seven (a step of
 // 390,000 FP64 particles 95 us, 90 with eight).
 template <class F, bool FORCES, int CELLS, int N, bool SPREAD>
