@@ -12,7 +12,8 @@
 //   k_tile_gather one workgroup per tile: counts its cells (cell_count, cell_start), ranks
 //                 each particle among its cell's by original index, and moves the planes
 //                 through LDS, read in list order and written in slot order
-//   k_tile_spill  ranks and moves the particles of the tiles that the LDS does not hold
+//   k_tile_spill  ranks and moves the particles of the tiles that the LDS does not hold (in
+//                 smaller sorts the first workgroups of k_tile_gather do)
 // The order within a tile's list is not deterministic, the rank does not depend on it: the
 // result equals the reference's single-thread order, where each cell keeps increasing
 // original index.
@@ -407,17 +408,25 @@ struct SpillWork {
     int32_t *count;
     int2 *item;
 };
-constexpr int SPILL_PIECE = 512, SPILL_AHEAD = 8;
-// A tile's own workgroup moves any number of particles alone, or, where k_tile_spill follows,
-// up to SPILL_OWN.  It follows in sorts of SPREAD_FROM particles or more that may be clustered:
-// its launch is 2 us, mostly for nothing, of a step's 50 for 80,000 FP64 particles, 200 for 1.25
-// million.  Below that, clusters cost more: 327,680 FP64 particles in a half, an eighth, a 64th
-// and a 512th of the box (in order) take 0.06, 0.12, 1.7 and 85 ms a sort; with it 0.07, 0.09, 0.24
-// and 1.4; without tiles 0.08, 0.14, 0.56 and 3.2.  The device-resident programs, whose particles
-// spread evenly from the start, go without it.
-constexpr int SPILL_OWN = 1024;
-constexpr int64_t SPREAD_FROM = 1 << 21;
+// Who moves such a tile's particles.  Its own workgroup any number of them (ALONE), or up to
+// HELP_OWN and above that the first HELPERS workgroups of the launch (HELPED), or up to SPILL_OWN
+// and above that the launch of k_tile_spill that follows (SPREAD): clustered particles fill
+// few tiles, and would leave the rest of the device idle.  The helpers wait for nobody, so each
+// counts and groups the cells that it moves from the tile's whole list; k_tile_spill finds
+// them grouped, but its launch takes 2 us, mostly for nothing.  It follows sorts of SPREAD_FROM
+// particles or more (200 us a step and above).  The device-resident programs, whose particles
+// spread evenly from the start, go alone.
+enum Spill { ALONE, HELPED, SPREAD };
+constexpr int64_t SPREAD_FROM = 1 << 20;
+constexpr int SPILL_PIECE = 512, SPILL_AHEAD = 8, SPILL_OWN = 1024;
 constexpr unsigned SPILL_BLOCKS = 1024;  // 2048 idle 1 us longer
+// The helpers' units are of about SPILL_PIECE particles; a cell of more than HELP_CELL is shared by
+// all units of its tile.  327,680 particles in an eighth, a 64th and a 512th of the box (in
+// order): FP64 0.10, 0.17 and 3.3 ms a sort, FP32 0.07, 0.24 and 3.7; by the tiles' own workgroups
+// 0.10, 1.7, 85 and 0.17, 2.9, 138; without tiles FP64 0.14, 0.56 and 3.2.  (256 and 512 helpers: 0.34
+// and 0.25 for the FP64 64th.)  Where no tile overflows they cost nothing that shows: 5120 to
+// 327,680 particles, 21 to 88 us a sort with and without.
+constexpr int HELPERS = 1024, HELP_OWN = 4096, HELP_CELL = 8192;
 
 // a thread's next particles of such a tile and their cells, -1 beyond its m particles
 __device__ inline void spill_load(int32_t w[SPILL_AHEAD], int k[SPILL_AHEAD], const int32_t *__restrict__ list,
@@ -491,14 +500,55 @@ __device__ inline void spill_move(const Box &b, const PView<F> &src, const PView
     if (id_to_idx && (uint32_t)id < (uint32_t)n) id_to_idx[id] = (int32_t)o;
 }
 
-// Particles [q0, q1) of a list that is grouped by cell, at most P a thread: a thread ranks its
-// own in their cells by original index, the cells' lists staged in LDS, and moves them straight
-// between the planes.  All threads call.
+// Of a tile of m particles: the counts of its cells, added to lcnt, and their starts in the tile.
+// All threads call, with a barrier before and after.
+__device__ inline void spill_count(int *lcnt, const int32_t *list, const int32_t *key, int cmask, int m)
+{
+    for (int64_t q0 = threadIdx.x; q0 < m; q0 += SPILL_AHEAD * SORT_T) {
+        int32_t w[SPILL_AHEAD];
+        int k[SPILL_AHEAD];
+        spill_load(w, k, list, key, cmask, q0, m);
+#pragma unroll
+        for (int u = 0; u < SPILL_AHEAD; ++u)
+            if (w[u] >= 0) atomicAdd(&lcnt[k[u]], 1);
+    }
+}
+__device__ inline void cell_starts(int *lstart, const int *lcnt, int ncell)
+{
+    if (threadIdx.x >= 64) return;  // one wave scans the tile's cells
+    int carry = 0;
+    for (int c0 = 0; c0 < ncell; c0 += 64) {
+        const int k = c0 + (int)threadIdx.x, w = k < ncell ? lcnt[k] : 0;
+        const int inc = wave_inclusive_scan(w);
+        if (k < ncell) lstart[k] = carry + inc - w;
+        carry += __shfl(inc, 63);
+    }
+}
+
+// the list's particles of the cells [c0, c1] grouped by cell, to a stretch that starts with the
+// tile; those cells' lcnt is zero before and their counts after
+__device__ inline void spill_group(int32_t *grouped, int *lcnt, const int *lstart, const int32_t *list, const int32_t *key,
+                                   int cmask, int m, int c0, int c1)
+{
+    for (int64_t q0 = threadIdx.x; q0 < m; q0 += SPILL_AHEAD * SORT_T) {
+        int32_t w[SPILL_AHEAD];
+        int k[SPILL_AHEAD];
+        spill_load(w, k, list, key, cmask, q0, m);
+#pragma unroll
+        for (int u = 0; u < SPILL_AHEAD; ++u)
+            if (w[u] >= 0 && k[u] >= c0 && k[u] <= c1) grouped[lstart[k[u]] + atomicAdd(&lcnt[k[u]], 1)] = w[u];
+    }
+}
+
+// Particles [q0, q1) of a tile's list that is grouped by cell, at most P a thread: a thread ranks
+// its own in their cells by original index, the cells' lists staged in LDS, and moves them
+// straight between the planes, to slots from s on.  lcnt and lstart are the tile's cells in that
+// list.  All threads call.
 constexpr int SPILL_STAGE = 1536;
 template <class F, bool FORCES, int P>
-__device__ inline void spill_piece(const Box &b, const PView<F> &src, const PView<F> &dst, int wrap,
-                                   const int32_t *key, const int32_t *list, const int32_t *cell_count,
-                                   const int32_t *cell_start, int64_t q0, int64_t q1, int32_t *stage, int *range,
+__device__ inline void spill_piece(const Box &b, const PView<F> &src, const PView<F> &dst, int wrap, int64_t s,
+                                   const int32_t *key, int cmask, const int32_t *grouped, const int *lcnt,
+                                   const int *lstart, int q0, int q1, int32_t *stage, int *range,
                                    int32_t *__restrict__ id_to_idx)
 {
     const int tid = threadIdx.x;
@@ -506,11 +556,11 @@ __device__ inline void spill_piece(const Box &b, const PView<F> &src, const PVie
     int a[P], z[P], rank[P];  // the particles' cells in the list
 #pragma unroll
     for (int u = 0; u < P; ++u) {
-        const int64_t q = q0 + tid + u * SORT_T;
-        w[u] = q < q1 ? list[q] : -1;
-        const int c = w[u] >= 0 ? key[w[u]] : 0;
-        a[u] = w[u] >= 0 ? cell_start[c] : 0;
-        z[u] = w[u] >= 0 ? a[u] + cell_count[c] : 0;
+        const int q = q0 + tid + u * SORT_T;
+        w[u] = q < q1 ? grouped[q] : -1;
+        const int c = w[u] >= 0 ? key[w[u]] & cmask : 0;
+        a[u] = w[u] >= 0 ? lstart[c] : 0;
+        z[u] = w[u] >= 0 ? a[u] + lcnt[c] : 0;
         rank[u] = 0;
         // the piece's first and last particle bound the cells that are needed
         if (q == q0) range[0] = a[u];
@@ -521,7 +571,7 @@ __device__ inline void spill_piece(const Box &b, const PView<F> &src, const PVie
     for (int base = r0; base < r1; base += SPILL_STAGE) {
         const int m = r1 - base < SPILL_STAGE ? r1 - base : SPILL_STAGE;
         __syncthreads();
-        for (int k = tid; k < m; k += SORT_T) stage[k] = list[base + k];
+        for (int k = tid; k < m; k += SORT_T) stage[k] = grouped[base + k];
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < P; ++u) {
@@ -534,8 +584,132 @@ __device__ inline void spill_piece(const Box &b, const PView<F> &src, const PVie
     }
 #pragma unroll
     for (int u = 0; u < P; ++u)
-        if (w[u] >= 0) spill_move<F, FORCES>(b, src, dst, wrap, w[u], (int64_t)a[u] + rank[u], id_to_idx);
+        if (w[u] >= 0) spill_move<F, FORCES>(b, src, dst, wrap, w[u], s + a[u] + rank[u], id_to_idx);
     __syncthreads();
+}
+
+// Particles [q0, q0 + SPILL_PIECE) of a tile's list, those in cells of more than HELP_CELL: ranked by
+// cell and original index among all of the tile's.  All threads call.
+template <class F>
+__device__ inline void help_cells(const Box &b, const PView<F> &src, const PView<F> &dst, int wrap, int64_t s,
+                                  const int32_t *key, int cmask, const int32_t *list, int m, const int *lcnt, int q0,
+                                  uint64_t *stage, int32_t *__restrict__ id_to_idx)
+{
+    constexpr int P = SPILL_PIECE / SORT_T, STAGE = SPILL_STAGE / 2;
+    const int tid = threadIdx.x;
+    int32_t w[P];
+    uint64_t o[P];
+    int rank[P];
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+        const int q = q0 + tid + u * SORT_T;
+        w[u] = q < m ? list[q] : -1;
+        const int c = w[u] >= 0 ? key[w[u]] & cmask : 0;
+        if (lcnt[c] <= HELP_CELL) w[u] = -1;
+        o[u] = (uint64_t)c << 32 | (uint32_t)w[u];
+        rank[u] = 0;
+    }
+    for (int base = 0; base < m; base += STAGE) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < STAGE / SORT_T; ++u) {
+            const int q = base + tid + u * SORT_T;
+            const int32_t x = q < m ? list[q] : -1;
+            stage[tid + u * SORT_T] = x >= 0 ? (uint64_t)(key[x] & cmask) << 32 | (uint32_t)x : ~(uint64_t)0;
+        }
+        __syncthreads();
+#pragma unroll 4
+        for (int k = 0; k < STAGE; ++k) {
+            const uint64_t y = stage[k];
+#pragma unroll
+            for (int u = 0; u < P; ++u) rank[u] += y < o[u] ? 1 : 0;
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < P; ++u)
+        if (w[u] >= 0) spill_move<F, true>(b, src, dst, wrap, w[u], s + rank[u], id_to_idx);
+    __syncthreads();
+}
+
+// The tiles of more than HELP_OWN particles, their units to the HELPERS workgroups in turn.  A
+// unit is the cells that begin in SPILL_PIECE consecutive places of the tile (that are not shared by
+// all units), their list made in the unit's own stretch of `spill`.  `some` holds
+// HELP_WORDS words: the particles of SORT_T tiles, which of them are large, flags and ranges.
+constexpr int HELP_MASK = SORT_T, HELP_FLAG = HELP_MASK + SORT_T / 32, HELP_RANGE = HELP_FLAG + 2,
+              HELP_WORDS = HELP_RANGE + 4;
+template <class F>
+__device__ inline void help(const Box &b, const PView<F> &src, const PView<F> &dst, int wrap, int shift, int nt,
+                            const int32_t *key, const int32_t *start, const int32_t *list, int32_t *spill, int *lcnt,
+                            int *lstart, void *stage, int *some, int32_t *__restrict__ id_to_idx)
+{
+    const int tid = threadIdx.x, ncell = 1 << shift, cmask = ncell - 1;
+    int any = 0;
+#pragma unroll 4
+    for (int t = tid; t < nt; t += SORT_T) any |= start[t + 1] - start[t] > HELP_OWN;
+    if (tid == 0) some[HELP_FLAG] = 0;
+    __syncthreads();
+    if (any) some[HELP_FLAG] = 1;
+    __syncthreads();
+    if (!some[HELP_FLAG]) return;
+    int unit = blockIdx.x;  // the next one of this workgroup, counted from the tile at hand
+    for (int t0 = 0; t0 < nt; t0 += SORT_T) {
+        const int mine = t0 + tid < nt ? start[t0 + tid + 1] - start[t0 + tid] : 0;
+        const uint64_t large = __ballot(mine > HELP_OWN);
+        some[tid] = mine;
+        if ((tid & 31) == 0) some[HELP_MASK + tid / 32] = (int)(large >> (tid & 32));
+        __syncthreads();
+        for (int word = 0; word < SORT_T / 32; ++word) {
+            for (uint32_t left = (uint32_t)some[HELP_MASK + word]; left; left &= left - 1) {
+                const int t = 32 * word + __ffs(left) - 1, m = some[t], units = (m - 1) / SPILL_PIECE + 1;
+                if (unit >= units) {
+                    unit -= units;
+                    continue;
+                }
+                const int64_t s = start[t0 + t];
+                for (int c = tid; c < ncell; c += SORT_T) lcnt[c] = 0;
+                if (tid == 0) some[HELP_FLAG + 1] = 0;
+                __syncthreads();
+                spill_count(lcnt, list + s, key, cmask, m);
+                __syncthreads();
+                cell_starts(lstart, lcnt, ncell);
+                for (int c = tid; c < ncell; c += SORT_T)
+                    if (lcnt[c] > HELP_CELL) some[HELP_FLAG + 1] = 1;
+                __syncthreads();
+                for (; unit < units; unit += HELPERS) {
+                    int *range = some + HELP_RANGE;  // the unit's cells, first and last
+                    __syncthreads();
+                    if (tid == 0) range[0] = ncell, range[1] = -1;
+                    __syncthreads();
+                    for (int c = tid; c < ncell; c += SORT_T)
+                        if (lstart[c] / SPILL_PIECE == unit && lcnt[c] > 0 && lcnt[c] <= HELP_CELL) {
+                            atomicMin(&range[0], c);
+                            atomicMax(&range[1], c);
+                        }
+                    __syncthreads();
+                    const int c0 = range[0], c1 = range[1];
+                    if (c0 <= c1) {
+                        const int q0 = lstart[c0], q1 = lstart[c1] + lcnt[c1];
+                        __syncthreads();
+                        for (int c = c0 + tid; c <= c1; c += SORT_T) lcnt[c] = 0;
+                        __syncthreads();
+                        spill_group(spill + s, lcnt, lstart, list + s, key, cmask, m, c0, c1);
+                        __threadfence_block();
+                        __syncthreads();
+                        for (int q = q0; q < q1; q += SPILL_PIECE)
+                            spill_piece<F, true, SPILL_PIECE / SORT_T>(
+                                b, src, dst, wrap, s, key, cmask, spill + s, lcnt, lstart, q,
+                                q + SPILL_PIECE < q1 ? q + SPILL_PIECE : q1, (int32_t *)stage, range + 2, id_to_idx);
+                    }
+                    if (some[HELP_FLAG + 1])
+                        help_cells<F>(b, src, dst, wrap, s, key, cmask, list + s, m, lcnt, unit * SPILL_PIECE,
+                                      (uint64_t *)stage, id_to_idx);
+                }
+                unit -= units;
+                __syncthreads();
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // The cell sort's move.  Bound by memory: FP32 it reads 74 B and writes 66 B per particle.
@@ -550,7 +724,7 @@ __device__ inline void spill_piece(const Box &b, const PView<F> &src, const PVie
 // program whose forces are zero in both buffers (72 and 43 B, 0.43 ms).  With two particles a thread
 // it is held to eight waves per SIMD, which its scalar registers would make seven (a step of
 // 390,000 FP64 particles 95 us, 90 with eight).
-template <class F, bool FORCES, int CELLS, int N, bool SPREAD>
+template <class F, bool FORCES, int CELLS, int N, Spill MODE>
 __global__ void __launch_bounds__(SORT_T, CELLS > TILE_CELLS ? 1 : N == 2 ? 8 : FORCES ? 6 : 1)
     k_tile_gather(Box b, PView<F> src, PView<F> dst, int wrap, int shift, int nt, const int32_t *__restrict__ key,
                   const int32_t *__restrict__ start, const int32_t *__restrict__ list, int32_t *__restrict__ spill,
@@ -560,14 +734,21 @@ __global__ void __launch_bounds__(SORT_T, CELLS > TILE_CELLS ? 1 : N == 2 ? 8 : 
     using R = typename F::real;
     using S = typename F::small;
     constexpr int M = SORT_T * N, PLANES = FORCES ? 4 : 2;
-    __shared__ R buf[3][M];
+    __shared__ alignas(8) R buf[3][M];
     __shared__ int lv[M];
     __shared__ int lcnt[CELLS], lstart[CELLS];
+    constexpr int OWN = MODE == ALONE ? INT32_MAX : MODE == HELPED ? HELP_OWN : SPILL_OWN > M ? SPILL_OWN : M;
+    static_assert(sizeof(buf) >= SPILL_STAGE * sizeof(int32_t) && M >= HELP_WORDS && M <= OWN, "the stages");
+    if constexpr (MODE == HELPED)
+        if (blockIdx.x < HELPERS) {
+            help<F>(b, src, dst, wrap, shift, nt, key, start, list, spill, lcnt, lstart, buf, lv, id_to_idx);
+            return;
+        }
     // consecutive workgroups go to the XCDs in turn: each XCD takes runs of TILE_RUN tiles,
     // so that the tiles in flight there read neighbouring stretches.  The runs are short
     // enough that the empty cells of a padded box fall to all XCDs alike.
-    const int j = (int)blockIdx.x >> 3;
-    const int t = ((j / TILE_RUN) * 8 + ((int)blockIdx.x & 7)) * TILE_RUN + j % TILE_RUN;
+    const int block = (int)blockIdx.x - (MODE == HELPED ? HELPERS : 0), j = block >> 3;
+    const int t = ((j / TILE_RUN) * 8 + (block & 7)) * TILE_RUN + j % TILE_RUN;
     if (t >= nt) return;
     const int tid = threadIdx.x;
     const int64_t n = src.n;
@@ -594,25 +775,10 @@ __global__ void __launch_bounds__(SORT_T, CELLS > TILE_CELLS ? 1 : N == 2 ? 8 : 
 #pragma unroll
         for (int u = 0; u < N; ++u) d[u] = v[u] >= 0 ? atomicAdd(&lcnt[c[u]], 1) : 0;
     } else {
-        for (int64_t q0 = tid; q0 < m; q0 += SPILL_AHEAD * SORT_T) {
-            int32_t w[SPILL_AHEAD];
-            int k[SPILL_AHEAD];
-            spill_load(w, k, list + s, key, cmask, q0, m);
-#pragma unroll
-            for (int u = 0; u < SPILL_AHEAD; ++u)
-                if (w[u] >= 0) atomicAdd(&lcnt[k[u]], 1);
-        }
+        spill_count(lcnt, list + s, key, cmask, m);
     }
     __syncthreads();
-    if (tid < 64) {  // one wave scans the tile's cells
-        int carry = 0;
-        for (int c0 = 0; c0 < ncell; c0 += 64) {
-            const int k = c0 + tid, w = k < ncell ? lcnt[k] : 0;
-            const int inc = wave_inclusive_scan(w);
-            if (k < ncell) lstart[k] = carry + inc - w;
-            carry += __shfl(inc, 63);
-        }
-    }
+    cell_starts(lstart, lcnt, ncell);
     __syncthreads();
     for (int k = tid; k < ncell; k += SORT_T) {
         cell_count[((int64_t)t << shift) + k] = lcnt[k];
@@ -671,54 +837,46 @@ __global__ void __launch_bounds__(SORT_T, CELLS > TILE_CELLS ? 1 : N == 2 ? 8 : 
         return;
     }
     // more particles than the LDS holds: the list grouped by cell goes to memory (each
-    // workgroup writes and reads its own stretch), and each particle is ranked and moved
-    // from there, or the pieces of a tile that is larger still go to k_tile_spill
+    // workgroup writes and reads its own stretch), and each particle is ranked and moved from
+    // there, by the helpers, or by k_tile_spill
+    if (MODE == HELPED && m > OWN) return;
     for (int k = tid; k < ncell; k += SORT_T) lcnt[k] = 0;
     __syncthreads();
-    for (int64_t q0 = tid; q0 < m; q0 += SPILL_AHEAD * SORT_T) {
-        int32_t w[SPILL_AHEAD];
-        int k[SPILL_AHEAD];
-        spill_load(w, k, list + s, key, cmask, q0, m);
-#pragma unroll
-        for (int u = 0; u < SPILL_AHEAD; ++u)
-            if (w[u] >= 0) spill[s + lstart[k[u]] + atomicAdd(&lcnt[k[u]], 1)] = w[u];
-    }
-    if (!SPREAD || m <= SPILL_OWN) {
-        __threadfence_block();
+    spill_group(spill + s, lcnt, lstart, list + s, key, cmask, m, 0, ncell - 1);
+    if (MODE == SPREAD && m > OWN) {
+        const int pieces = (m - 1) / SPILL_PIECE + 1;
+        if (tid == 0) lv[0] = atomicAdd(work.count, pieces);
         __syncthreads();
-        static_assert(sizeof(buf) >= SPILL_STAGE * sizeof(int32_t), "the lists' stage");
-        if constexpr (FORCES) {
-            for (int64_t q = s; q < s + m; q += SORT_T)
-                spill_piece<F, true, 1>(b, src, dst, wrap, key, spill, cell_count, cell_start, q,
-                                        q + SORT_T < s + m ? q + SORT_T : s + m, (int32_t *)buf, lv, id_to_idx);
-        } else {
-            // an even fluid's tile overflows where one cell does; what is above costs its usual
-            // way registers (21 million FP32 particles 953 us a cycle, 941 like this)
-            for (int q = tid; q < m; q += SORT_T) {
-                const int32_t w = spill[s + q];
-                const int k = key[w] & cmask;
-                const int a = lstart[k], e = a + lcnt[k];
-                int rank = 0;
-                for (int y = a; y < e; ++y) rank += spill[s + y] < w ? 1 : 0;
-                spill_move<F, false>(b, src, dst, wrap, w, s + a + rank, id_to_idx);
-            }
-        }
+        for (int k = tid; k < pieces; k += SORT_T) work.item[lv[0] + k] = make_int2(t, k);
         return;
     }
-    const int pieces = (m - 1) / SPILL_PIECE + 1;
-    if (tid == 0) lv[0] = atomicAdd(work.count, pieces);
+    __threadfence_block();
     __syncthreads();
-    for (int k = tid; k < pieces; k += SORT_T) work.item[lv[0] + k] = make_int2(t, k);
+    if constexpr (FORCES) {
+        for (int q = 0; q < m; q += SORT_T)
+            spill_piece<F, true, 1>(b, src, dst, wrap, s, key, cmask, spill + s, lcnt, lstart, q,
+                                    q + SORT_T < m ? q + SORT_T : m, (int32_t *)buf, lv, id_to_idx);
+    } else {
+        // an even fluid's tile overflows where one cell does; what is above costs its usual
+        // way registers (21 million FP32 particles 953 us a cycle, 941 like this)
+        for (int q = tid; q < m; q += SORT_T) {
+            const int32_t w = spill[s + q];
+            const int k = key[w] & cmask;
+            const int a = lstart[k], e = a + lcnt[k];
+            int rank = 0;
+            for (int y = a; y < e; ++y) rank += spill[s + y] < w ? 1 : 0;
+            spill_move<F, false>(b, src, dst, wrap, w, s + a + rank, id_to_idx);
+        }
+    }
 }
 
-// The tiles too large for their own workgroup, a piece of one per workgroup at a time.
-// Clustered particles fill few tiles, which would leave the rest of the device idle: a sort
+// The tiles too large for their own workgroup, a piece of one per workgroup at a time: a sort
 // with all particles in a half, an eighth, a 64th and a 512th of an L=64 box (2.6 million FP32, in
-// order) takes 0.29, 0.30, 0.66 and 3.6 ms; without tiles 0.42, 0.68, 1.7 and 9.7.  In no order 1.13,
-// 1.12, 1.43 and 3.6 ms; without tiles 1.11, 1.10, 1.29 and 4.2.
+// order) takes 0.29, 0.30, 0.66 and 3.6 ms; without tiles 0.42, 0.68, 1.7 and 9.7; by helpers 0.27, 0.72,
+// 3.2 and 15.  In no order 1.13, 1.12, 1.43 and 3.6 ms; without tiles 1.11, 1.10, 1.29 and 4.2.
 template <class F>
 __global__ void __launch_bounds__(SORT_T)
-    k_tile_spill(Box b, PView<F> src, PView<F> dst, int wrap, const int32_t *__restrict__ key,
+    k_tile_spill(Box b, PView<F> src, PView<F> dst, int wrap, int shift, const int32_t *__restrict__ key,
                  const int32_t *__restrict__ start, const int32_t *__restrict__ spill,
                  const int32_t *__restrict__ cell_count, const int32_t *__restrict__ cell_start, SpillWork work,
                  int32_t *__restrict__ id_to_idx)
@@ -728,9 +886,11 @@ __global__ void __launch_bounds__(SORT_T)
     const int items = *work.count;
     for (int it = blockIdx.x; it < items; it += gridDim.x) {
         const int2 e = work.item[it];
-        const int64_t q0 = start[e.x] + (int64_t)e.y * SPILL_PIECE, end = start[e.x + 1];
-        spill_piece<F, true, SPILL_PIECE / SORT_T>(b, src, dst, wrap, key, spill, cell_count, cell_start, q0,
-                             q0 + SPILL_PIECE < end ? q0 + SPILL_PIECE : end, stage, range, id_to_idx);
+        const int q0 = start[e.x] + e.y * SPILL_PIECE, end = start[e.x + 1];
+        const int64_t c = (int64_t)e.x << shift;  // (the lists' starts are the box's)
+        spill_piece<F, true, SPILL_PIECE / SORT_T>(b, src, dst, wrap, 0, key, (1 << shift) - 1, spill, cell_count + c,
+                                                   cell_start + c, q0, end - q0 > SPILL_PIECE ? q0 + SPILL_PIECE : end,
+                                                   stage, range, id_to_idx);
     }
 }
 
@@ -803,10 +963,11 @@ static int tile_sort_begin(const rmpcd_box_t *box, int64_t n, TileSort &t)
 // the sort after its keys
 template <class F, bool FORCES>
 static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
-                            int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, bool spread)
+                            int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, bool even)
 {
     const int64_t n = src->n;
     hipStream_t s = stream();
+    const Spill mode = even ? ALONE : n >= SPREAD_FROM || t.nt > SCAN1_TILES ? SPREAD : HELPED;
     if (t.nt <= SCAN1_TILES) {
         k_tile_scan<<<1, 1024, 0, s>>>(t.count, t.stride, t.nt, t.start);
         RMPCD_LAUNCHED();
@@ -820,39 +981,35 @@ static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmp
     k_tile_place<<<blocks_for(n, 256), 256, 0, s>>>(n, t.key, t.shift, t.slot, t.start, t.list, t.work);
     RMPCD_LAUNCHED();
     const unsigned runs = (unsigned)((t.nt + 8 * TILE_RUN - 1) / (8 * TILE_RUN));
-    auto move = [&](auto cells_max, auto items, auto spread_c) {
-        k_tile_gather<F, FORCES, decltype(cells_max)::value, decltype(items)::value, decltype(spread_c)::value>
-            <<<8 * TILE_RUN * runs, SORT_T, 0, s>>>(t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt, t.key, t.start,
-                                                    t.list, t.slot, cells->cell_count, cells->cell_start, t.work,
-                                                    id_to_idx);
+    auto move = [&](auto cells_max, auto items, auto spill) {
+        constexpr Spill MODE = decltype(spill)::value;
+        k_tile_gather<F, FORCES, decltype(cells_max)::value, decltype(items)::value, MODE>
+            <<<(MODE == HELPED ? HELPERS : 0) + 8 * TILE_RUN * runs, SORT_T, 0, s>>>(
+                t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.nt, t.key, t.start, t.list, t.slot, cells->cell_count,
+                cells->cell_start, t.work, id_to_idx);
     };
-    const std::integral_constant<int, TILE_CELLS> some{};
-    const std::integral_constant<int, TILE_THIN> thin{};
-    const std::integral_constant<int, TILE_ITEMS<F>> items{};
-    const std::integral_constant<int, 2> few{};
-    const bool is_thin = (1 << t.shift) > TILE_CELLS;
-    if constexpr (FORCES)  // the others are the programs'
-        if (spread) {
-            if (is_thin)
-                move(thin, items, std::true_type{});
-            else
-                move(some, items, std::true_type{});
-        }
-    if (!spread) {
-        if (is_thin)
-            move(thin, items, std::false_type{});
+    auto tiles = [&](auto spill) {
+        const std::integral_constant<int, TILE_ITEMS<F>> items{};
+        const std::integral_constant<int, TILE_CELLS> some{};
+        if ((1 << t.shift) > TILE_CELLS)
+            move(std::integral_constant<int, TILE_THIN>{}, items, spill);
         else if (t.per_tile <= TILE_FEW)
-            move(some, few, std::false_type{});
+            move(some, std::integral_constant<int, 2>{}, spill);
         else
-            move(some, items, std::false_type{});
+            move(some, items, spill);
+    };
+    if (mode == ALONE) tiles(std::integral_constant<Spill, ALONE>{});
+    if constexpr (FORCES) {  // the others are the programs'
+        if (mode == HELPED) tiles(std::integral_constant<Spill, HELPED>{});
+        if (mode == SPREAD) tiles(std::integral_constant<Spill, SPREAD>{});
     }
     RMPCD_LAUNCHED();
     if constexpr (FORCES) {
-        if (!spread) return RMPCD_OK;
+        if (mode != SPREAD) return RMPCD_OK;
         const unsigned pieces = blocks_for(n, SPILL_PIECE);
         k_tile_spill<F><<<pieces < SPILL_BLOCKS ? pieces : SPILL_BLOCKS, SORT_T, 0, s>>>(
-            t.b, view<F>(src), view<F>(dst), wrap, t.key, t.start, t.slot, cells->cell_count, cells->cell_start, t.work,
-            id_to_idx);
+            t.b, view<F>(src), view<F>(dst), wrap, t.shift, t.key, t.start, t.slot, cells->cell_count, cells->cell_start,
+            t.work, id_to_idx);
         RMPCD_LAUNCHED();
     }
     return RMPCD_OK;
@@ -860,7 +1017,7 @@ static int tile_sort_finish(const TileSort &t, const rmpcd_particles_t *src, rmp
 
 template <class F>
 int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
-              int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, bool spread)
+              int32_t *id_to_idx, rmpcd_cells_t *cells, int wrap, bool even)
 {
     TileSort t;
     int rc = tile_sort_begin<F>(box, src->n, t);
@@ -868,7 +1025,7 @@ int sort_impl(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_partic
     k_tile_key<F><<<blocks_for(src->n, KEY_CHUNK), SORT_T, 0, stream()>>>(t.b, t.lut, view<F>(src), wrap, t.shift,
                                                                           t.stride, t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    return tile_sort_finish<F, true>(t, src, dst, id_to_idx, cells, wrap, spread);
+    return tile_sort_finish<F, true>(t, src, dst, id_to_idx, cells, wrap, even);
 }
 
 template <class F>
@@ -884,7 +1041,7 @@ int fluid_cycle_impl(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpc
         t.b, t.lut, view<F>(src), cells->cell_start, cells->cell_count, cshift, seed, step, n_md, dt, t.shift, t.stride,
         t.count, t.key, t.slot);
     RMPCD_LAUNCHED();
-    return tile_sort_finish<F, false>(t, src, dst, nullptr, cells, 0, false);
+    return tile_sort_finish<F, false>(t, src, dst, nullptr, cells, 0, true);
 }
 
 int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src, rmpcd_particles_t *dst,
@@ -896,7 +1053,7 @@ int fluid_cycle_unchecked(const rmpcd_box_t *next, const rmpcd_particles_t *src,
 int sort_unchecked(const rmpcd_box_t *box, const rmpcd_particles_t *src, rmpcd_particles_t *dst, int32_t *id_to_idx,
                    rmpcd_cells_t *cells, int wrap, bool even)
 {
-    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, wrap, !even && src->n >= SPREAD_FROM);
+    return RMPCD_DISPATCH_FORM(src, sort_impl, box, src, dst, id_to_idx, cells, wrap, even);
 }
 
 template <class F>

@@ -168,7 +168,16 @@ def test_sort_tiles(gpu, L, n, spread, form):
     ((32, 32, 32), 30000, [(0.9, (3, 3, 3)), (0.1, (32, 32, 32))]),        # a cluster in a thin gas
     ((16, 16, 16), 20000, [(0.5, (1, 1, 1)), (0.25, (2, 1, 1)), (0.25, (16, 16, 16))]),  # cells beyond a piece
     ((20, 10, 6), 2500, [(1.0, (5, 5, 5))]),
-    ((64, 64, 64), (1 << 21) + 37, [(0.9, (32, 32, 32)), (0.05, (8, 4, 4)), (0.05, (64, 64, 64))]),  # by all workgroups
+    ((64, 64, 64), (1 << 21) + 37, [(0.9, (32, 32, 32)), (0.05, (8, 4, 4)), (0.05, (64, 64, 64))]),  # a launch of their own
+    ((48, 48, 48), (1 << 20) - 1, [(0.9, (24, 24, 24)), (0.05, (8, 4, 4)), (0.05, (48, 48, 48))]),   # the first workgroups
+    ((8, 8, 8), 1537, [(1.0, (1, 1, 1))]),
+    # tiles that their own workgroup moves and the next larger, cells that all units share and not
+    ((16, 16, 16), 4096 + 8192, [(1 / 3, (1, 1, 1)), (2 / 3, (16, 16, 16))]),
+    ((8, 8, 8), 4097, [(1.0, (1, 1, 1))]), ((8, 8, 8), 8192, [(1.0, (1, 1, 1))]), ((8, 8, 8), 8193, [(1.0, (1, 1, 1))]),
+    ((32, 32, 32), 60000, [(0.5, (1, 1, 1)), (0.3, (2, 2, 2)), (0.2, (8, 8, 8))]),
+    ((100, 100, 100), 50000, [(0.9, (9, 9, 9)), (0.1, (100, 100, 100))]),           # tiles of 1024 cells
+    ((100, 100, 100), 100000, [(0.5, (1, 1, 1)), (0.5, (10, 10, 10))]),
+    ((512, 129, 129), 6000, [(0.5, (2, 2, 2)), (0.5, (512, 129, 129))]),            # more tiles than one workgroup scans
 ])
 def test_sort_clusters(gpu, L, n, parts, form):
     """the sort of clustered particles, whose tiles the LDS does not hold, with the periodic
