@@ -420,13 +420,19 @@ enum Spill { ALONE, HELPED, SPREAD };
 constexpr int64_t SPREAD_FROM = 1 << 20;
 constexpr int SPILL_PIECE = 512, SPILL_AHEAD = 8, SPILL_OWN = 1024;
 constexpr unsigned SPILL_BLOCKS = 1024;  // 2048 idle 1 us longer
-// The helpers' units are of about SPILL_PIECE particles; a cell of more than HELP_CELL is shared by
-// all units of its tile.  327,680 particles in an eighth, a 64th and a 512th of the box (in
-// order): FP64 0.10, 0.17 and 3.3 ms a sort, FP32 0.07, 0.24 and 3.7; by the tiles' own workgroups
+// The helpers' units are of about SPILL_PIECE particles.  327,680 particles in an eighth, a 64th and a 512th of the box (in
+// order): FP64 0.08, 0.17 and 3.3 ms a sort, FP32 0.07, 0.24 and 3.7; by the tiles' own workgroups
 // 0.10, 1.7, 85 and 0.17, 2.9, 138; without tiles FP64 0.14, 0.56 and 3.2.  (256 and 512 helpers: 0.34
 // and 0.25 for the FP64 64th.)  Where no tile overflows they cost nothing that shows: 5120 to
 // 327,680 particles, 21 to 88 us a sort with and without.
-constexpr int HELPERS = 1024, HELP_OWN = 4096, HELP_CELL = 8192;
+constexpr int HELPERS = 1024, HELP_OWN = 2048, HELP_CELL = 2048;
+// A cell of a tile of m particles that all units share: each unit of 512 then looks through all of
+// the tile instead of the cell, but one workgroup is not left with the whole cell (64 cells
+// of 5000 FP64 particles 2.7 ms a sort, shared 0.24).
+__device__ inline bool help_shared(int count, int m)
+{
+    return count > HELP_CELL && (int64_t)count * count > (int64_t)1024 * m;
+}
 
 // a thread's next particles of such a tile and their cells, -1 beyond its m particles
 __device__ inline void spill_load(int32_t w[SPILL_AHEAD], int k[SPILL_AHEAD], const int32_t *__restrict__ list,
@@ -588,7 +594,7 @@ __device__ inline void spill_piece(const Box &b, const PView<F> &src, const PVie
     __syncthreads();
 }
 
-// Particles [q0, q0 + SPILL_PIECE) of a tile's list, those in cells of more than HELP_CELL: ranked by
+// Particles [q0, q0 + SPILL_PIECE) of a tile's list, those in cells that all units share: ranked by
 // cell and original index among all of the tile's.  All threads call.
 template <class F>
 __device__ inline void help_cells(const Box &b, const PView<F> &src, const PView<F> &dst, int wrap, int64_t s,
@@ -605,7 +611,7 @@ __device__ inline void help_cells(const Box &b, const PView<F> &src, const PView
         const int q = q0 + tid + u * SORT_T;
         w[u] = q < m ? list[q] : -1;
         const int c = w[u] >= 0 ? key[w[u]] & cmask : 0;
-        if (lcnt[c] <= HELP_CELL) w[u] = -1;
+        if (!help_shared(lcnt[c], m)) w[u] = -1;
         o[u] = (uint64_t)c << 32 | (uint32_t)w[u];
         rank[u] = 0;
     }
@@ -673,7 +679,7 @@ __device__ inline void help(const Box &b, const PView<F> &src, const PView<F> &d
                 __syncthreads();
                 cell_starts(lstart, lcnt, ncell);
                 for (int c = tid; c < ncell; c += SORT_T)
-                    if (lcnt[c] > HELP_CELL) some[HELP_FLAG + 1] = 1;
+                    if (help_shared(lcnt[c], m)) some[HELP_FLAG + 1] = 1;
                 __syncthreads();
                 for (; unit < units; unit += HELPERS) {
                     int *range = some + HELP_RANGE;  // the unit's cells, first and last
@@ -681,7 +687,7 @@ __device__ inline void help(const Box &b, const PView<F> &src, const PView<F> &d
                     if (tid == 0) range[0] = ncell, range[1] = -1;
                     __syncthreads();
                     for (int c = tid; c < ncell; c += SORT_T)
-                        if (lstart[c] / SPILL_PIECE == unit && lcnt[c] > 0 && lcnt[c] <= HELP_CELL) {
+                        if (lstart[c] / SPILL_PIECE == unit && lcnt[c] > 0 && !help_shared(lcnt[c], m)) {
                             atomicMin(&range[0], c);
                             atomicMax(&range[1], c);
                         }

@@ -173,7 +173,8 @@ def test_sort_tiles(gpu, L, n, spread, form):
     ((8, 8, 8), 1537, [(1.0, (1, 1, 1))]),
     # tiles that their own workgroup moves and the next larger, cells that all units share and not
     ((16, 16, 16), 4096 + 8192, [(1 / 3, (1, 1, 1)), (2 / 3, (16, 16, 16))]),
-    ((8, 8, 8), 4097, [(1.0, (1, 1, 1))]), ((8, 8, 8), 8192, [(1.0, (1, 1, 1))]), ((8, 8, 8), 8193, [(1.0, (1, 1, 1))]),
+    ((8, 8, 8), 2048, [(1.0, (1, 1, 1))]), ((8, 8, 8), 2049, [(1.0, (1, 1, 1))]), ((8, 8, 8), 8193, [(1.0, (1, 1, 1))]),
+    ((16, 16, 16), 6400, [(0.3, (1, 1, 1)), (0.7, (2, 2, 2))]), ((16, 16, 16), 6400, [(0.4, (1, 1, 1)), (0.6, (2, 2, 2))]),
     ((32, 32, 32), 60000, [(0.5, (1, 1, 1)), (0.3, (2, 2, 2)), (0.2, (8, 8, 8))]),
     ((100, 100, 100), 50000, [(0.9, (9, 9, 9)), (0.1, (100, 100, 100))]),           # tiles of 1024 cells
     ((100, 100, 100), 100000, [(0.5, (1, 1, 1)), (0.5, (10, 10, 10))]),
