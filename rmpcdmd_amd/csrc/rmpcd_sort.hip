@@ -420,11 +420,13 @@ enum Spill { ALONE, HELPED, SPREAD };
 constexpr int64_t SPREAD_FROM = 1 << 20;
 constexpr int SPILL_PIECE = 512, SPILL_AHEAD = 8, SPILL_OWN = 1024;
 constexpr unsigned SPILL_BLOCKS = 1024;  // 2048 idle 1 us longer
-// The helpers' units are of about SPILL_PIECE particles.  327,680 particles in an eighth, a 64th and a 512th of the box (in
-// order): FP64 0.08, 0.17 and 3.3 ms a sort, FP32 0.07, 0.24 and 3.7; by the tiles' own workgroups
-// 0.10, 1.7, 85 and 0.17, 2.9, 138; without tiles FP64 0.14, 0.56 and 3.2.  (256 and 512 helpers: 0.34
-// and 0.25 for the FP64 64th.)  Where no tile overflows they cost nothing that shows: 5120 to
-// 327,680 particles, 21 to 88 us a sort with and without.
+// The helpers' units are of about SPILL_PIECE particles.  327,680 particles in an eighth, a 64th
+// and a 512th of the box (in order): FP64 0.08, 0.17 and 3.3 ms a sort, FP32 0.07, 0.24 and 3.7;
+// by the tiles' own workgroups 0.10, 1.7, 85 and 0.17, 2.9, 138; without tiles FP64 0.14, 0.56 and
+// 3.2.  (256 and 512 helpers: 0.34 and 0.25 for the FP64 64th.)  Where no tile overflows they cost
+// nothing that shows with 5120 to 327,680 particles (21 to 88 us a sort), and 1 us of the 154 of
+// a step of 837,000 FP64 particles.  A flag from the scan or the place pass instead of
+// their own look at the starts, and helpers that have moved a tile first, were not faster.
 constexpr int HELPERS = 1024, HELP_OWN = 2048, HELP_CELL = 2048;
 // A cell of a tile of m particles that all units share: each unit of 512 then looks through all of
 // the tile instead of the cell, but one workgroup is not left with the whole cell (64 cells
